@@ -153,7 +153,10 @@ struct Handle {
   // local expansions per sublevel.
   DBuf<cplx> per_M, per_part;
 
-  // Ewald summation: waves (kx, ky, kz as doubles, re, im) and results.
+  // Ewald summation: the wave rows, the forward transform's partial sums and
+  // the scaled wave table, and slots of partial results.
+  DBuf<int> ew_rows;
+  int ew_ksize = 0, ew_nrows = 0, ew_nsrows = 0;  // what ew_rows holds
   DBuf<double> ew_waves;
   DBuf<double4> ew_trg;
 
