@@ -15,10 +15,11 @@
 // descending.
 //
 // The upward pass follows the reference's operation order without FMA
-// contraction (multipoles bit-identical to the reference).  M2L pairs are
-// batched per target cell: each lane builds one pair's derivative tensor
-// (Taylor recurrence) in LDS, then the lanes run a host-built, load-balanced
-// schedule of (a, b) terms over the whole batch.
+// contraction (multipoles bit-identical to the reference).  M2L takes one
+// wave per target cell and, at P = 4 and 6, one lane per pair with everything
+// in registers; at P = 8 each lane builds one pair's derivative tensor in LDS
+// and the lanes run a host-built, load-balanced schedule of (a, b) terms over
+// the whole batch.
 #include <algorithm>
 #include <vector>
 
@@ -49,14 +50,21 @@ __host__ __device__ inline void cmi(int t, int &a, int &b, int &c) {
   a = n - m;
 }
 
+// v / i correctly rounded for a small whole number i: the quotient by the
+// rounded reciprocal, corrected once by its exact remainder.
+__device__ inline double div_small(double v, int i) {
+  const double y = kInv.v[i], q = v * y;
+  return fma(fma(-q, (double)i, v), y, q);
+}
+
 // One coefficient of Kernels::power (:183-186,213-216,243-246): the chain
 // C_(a,0,0) = C_(a-1,0,0) dx / a, C_(a,b,0) = C_(a,b-1,0) dy / b,
 // C_(a,b,c) = C_(a,b,c-1) dz / c, started from v.
 __device__ inline double cpow(double v, int a, int b, int c, double dx, double dy, double dz) {
 #pragma clang fp contract(off)
-  for (int i = 1; i <= a; i++) v = v * dx / i;
-  for (int i = 1; i <= b; i++) v = v * dy / i;
-  for (int i = 1; i <= c; i++) v = v * dz / i;
+  for (int i = 1; i <= a; i++) v = div_small(v * dx, i);
+  for (int i = 1; i <= b; i++) v = div_small(v * dy, i);
+  for (int i = 1; i <= c; i++) v = div_small(v * dz, i);
   return v;
 }
 
@@ -101,105 +109,168 @@ __host__ __device__ inline bool m2l_term(int P, int da, int db) {
   return da + db <= P - 1 && !(P <= 7 && da == 0 && db == P - 1);
 }
 
+// Index tables of the packed coefficients.
+template <int P>
+struct CartTab {
+  static constexpr int NT = Cart<P>::NT;
+  int x[NT], y[NT], z[NT];
+  int prev[NT], dir[NT];  // the factor of power's chain: index less one in direction dir
+  constexpr CartTab() : x(), y(), z(), prev(), dir() {
+    int t = 0;
+    for (int n = 0; n < P; n++)
+      for (int a = n; a >= 0; a--)
+        for (int b = n - a; b >= 0; b--, t++) {
+          const int c = n - a - b;
+          x[t] = a;
+          y[t] = b;
+          z[t] = c;
+          dir[t] = c > 0 ? 2 : b > 0 ? 1 : 0;
+          prev[t] = n == 0 ? 0 : idx(a - (dir[t] == 0), b - (dir[t] == 1), c - (dir[t] == 2));
+        }
+  }
+  static constexpr int idx(int a, int b, int c) {
+    const int n = a + b + c, m = b + c;
+    return n * (n + 1) * (n + 2) / 6 + m * (m + 1) / 2 + c;
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Upward pass: P2M (:590-598) at leaves, M2M (:600-612) at parents, then
 // setRmax and R /= theta as in the spherical pass.
+
+__device__ inline void cart_radius(double4 *cX, int c, double rb, double rmax, double theta, int useRmax) {
+  double R = rb;
+  if (useRmax) R = R < rmax ? R : rmax;
+  R /= theta;
+  cX[c].w = R;
+}
+
+__device__ inline double wave_max(double v) {  // exact in any order
+  for (int d = 32; d >= 1; d >>= 1) {
+    const double o = __shfl_xor(v, d);
+    v = o > v ? o : v;
+  }
+  return v;
+}
+
+// Every leaf among `cells`, one wave each: lanes own bodies and run power's
+// chain once for all coefficients, then own coefficients and add the bodies
+// in order.  (A lane per coefficient, each with its own chain of up to P - 1
+// divisions per body, took 84 us for 4096 leaves of 27 bodies at P = 6;
+// this takes 16 us.)
 template <int P>
 __global__ void __launch_bounds__(64)
-    k_upward_cart(const int *__restrict__ cells, const double4 *__restrict__ body, double4 *__restrict__ cX,
-                  const double *__restrict__ cRb, const int *__restrict__ cChild, const int *__restrict__ cNChild,
-                  const int *__restrict__ cBody, const int *__restrict__ cNBody, cplx *__restrict__ M, double theta,
-                  int useRmax) {
+    k_p2m_cart(const int *__restrict__ cells, const double4 *__restrict__ body, double4 *__restrict__ cX,
+               const double *__restrict__ cRb, const int *__restrict__ cNChild, const int *__restrict__ cBody,
+               const int *__restrict__ cNBody, cplx *__restrict__ M, double theta, int useRmax) {
 #pragma clang fp contract(off)
   constexpr int NT = Cart<P>::NT;
   constexpr int NO = (NT + 63) / 64;
-  __shared__ double4 sb[64];
-  __shared__ double sC[NT];
-  __shared__ double sM[NT];
-  __shared__ double sred[64];
+  constexpr int CH = P <= 6 ? 64 : 32;  // bodies at a time (29 to 32 KB of LDS)
+  constexpr CartTab<P> tab{};
+  __shared__ double sR[NT][CH + 1];
   const int c = cells[blockIdx.x];
+  if (cNChild[c] != 0) return;
   const int lane = threadIdx.x;
   const double4 Xc = cX[c];
-  const int nchild = cNChild[c];
-  int ka[NO], kb[NO], kc[NO];
-  double acc[NO];
+  double acc[NO], rmax = 0;
 #pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const int t = lane + 64 * o;
-    cmi(t < NT ? t : 0, ka[o], kb[o], kc[o]);
-    acc[o] = 0;
-  }
-  double rmax = 0;
-  if (nchild == 0) {
-    const int b0 = cBody[c], nb = cNBody[c];
-    for (int base = 0; base < nb; base += 64) {
-      const int cnt = min(64, nb - base);
-      if (lane < cnt) {
-        const double4 v = body[b0 + base + lane];
-        sb[lane] = make_double4(Xc.x - v.x, Xc.y - v.y, Xc.z - v.z, v.w);
-        const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
-        rmax = r > rmax ? r : rmax;
-      }
-      __syncthreads();
-      for (int k = 0; k < cnt; k++) {
-        const double4 d = sb[k];
+  for (int o = 0; o < NO; o++) acc[o] = 0;
+  const int b0 = cBody[c], nb = cNBody[c];
+  for (int base = 0; base < nb; base += CH) {
+    const int cnt = min(CH, nb - base);
+    __syncthreads();
+    if (lane < cnt) {
+      const double4 v = body[b0 + base + lane];
+      const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
+      rmax = r > rmax ? r : rmax;
+      const double d[3] = {Xc.x - v.x, Xc.y - v.y, Xc.z - v.z};
+      double C[NT];
+      C[0] = v.w;
+      sR[0][lane] = v.w;
 #pragma unroll
-        for (int o = 0; o < NO; o++)
-          if (lane + 64 * o < NT) acc[o] += cpow(d.w, ka[o], kb[o], kc[o], d.x, d.y, d.z);
+      for (int t = 1; t < NT; t++) {
+        const int k = tab.dir[t], i = k == 0 ? tab.x[t] : k == 1 ? tab.y[t] : tab.z[t];
+        const double w = C[tab.prev[t]] * d[k];
+        C[t] = i == 1 ? w : div_small(w, i);
+        sR[t][lane] = C[t];
       }
-      __syncthreads();
     }
-  } else {
-    const int ch0 = cChild[c];
-    for (int ci = 0; ci < nchild; ci++) {
-      const int cc = ch0 + ci;
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < NO; o++) {
+      const int t = lane + 64 * o;
+      if (t < NT)
+        for (int k = 0; k < cnt; k++) acc[o] += sR[t][k];
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < NO; o++)
+    if (lane + 64 * o < NT) M[(size_t)c * NT + lane + 64 * o] = {acc[o], 0.0};
+  rmax = wave_max(rmax);
+  if (lane == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
+}
+
+// The parents among `cells` (one level), one wave per child; the children's
+// two sums per coefficient are then added in child order, as one lane walking
+// the children would.  Latency-bound: 21 us per level of up to 512 parents,
+// 97 us with one wave for all 8 children.
+template <int P>
+__global__ void __launch_bounds__(512)
+    k_m2m_cart(const int *__restrict__ cells, double4 *__restrict__ cX, const double *__restrict__ cRb,
+               const int *__restrict__ cChild, const int *__restrict__ cNChild, cplx *__restrict__ M, double theta,
+               int useRmax) {
+#pragma clang fp contract(off)
+  constexpr int NT = Cart<P>::NT;
+  __shared__ double sC[8][NT], sM[8][NT], s0[8][NT], s1[8][NT];
+  __shared__ double sred[8];
+  const int c = cells[blockIdx.x];
+  const int nchild = cNChild[c];
+  if (nchild == 0) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double4 Xc = cX[c];
+  double acc = 0, rmax = 0;
+  for (int base = 0; base < nchild; base += 8) {  // (an octree cell has 8 at most)
+    const int cnt = min(8, nchild - base);
+    __syncthreads();
+    if (wave < cnt) {
+      const int cc = cChild[c] + base + wave;
       const double4 Xj = cX[cc];
       const double dx = Xc.x - Xj.x, dy = Xc.y - Xj.y, dz = Xc.z - Xj.z;
       for (int t = lane; t < NT; t += 64) {
         int a, b, cz;
         cmi(t, a, b, cz);
-        sC[t] = cpow(1.0, a, b, cz, dx, dy, dz);
-        sM[t] = M[(size_t)cc * NT + t].re;
+        sC[wave][t] = cpow(1.0, a, b, cz, dx, dy, dz);
+        sM[wave][t] = M[(size_t)cc * NT + t].re;
       }
-      if (lane == 0) {
-        const double r = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
-        rmax = r > rmax ? r : rmax;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int o = 0; o < NO; o++) {
-        const int t = lane + 64 * o;
-        if (t >= NT) continue;
-        acc[o] += sC[t] * sM[0];
-        if (t == 0) continue;
+      if (lane == 0) sred[wave] = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
+    }
+    __syncthreads();
+    if (wave < cnt)
+      for (int t = lane; t < NT; t += 64) {
+        s0[wave][t] = sC[wave][t] * sM[wave][0];
+        int ka, kb, kc;
+        cmi(t, ka, kb, kc);
         // MultipoleSum: 0 <= k <= n, k != 0, lexicographic (kx, ky, kz).
         double sum = 0;
-        for (int a = 0; a <= ka[o]; a++)
-          for (int b = 0; b <= kb[o]; b++)
-            for (int cz = 0; cz <= kc[o]; cz++) {
+        for (int a = 0; a <= ka; a++)
+          for (int b = 0; b <= kb; b++)
+            for (int cz = 0; cz <= kc; cz++) {
               if (a == 0 && b == 0 && cz == 0) continue;
-              sum += sC[cidx(ka[o] - a, kb[o] - b, kc[o] - cz)] * sM[cidx(a, b, cz)];
+              sum += sC[wave][cidx(ka - a, kb - b, kc - cz)] * sM[wave][cidx(a, b, cz)];
             }
-        acc[o] += sum;
+        s1[wave][t] = sum;
       }
-      __syncthreads();
-    }
+    __syncthreads();
+    if ((int)threadIdx.x < NT)
+      for (int w = 0; w < cnt; w++) {
+        acc += s0[w][threadIdx.x];
+        if (threadIdx.x > 0) acc += s1[w][threadIdx.x];
+        rmax = sred[w] > rmax ? sred[w] : rmax;
+      }
   }
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const int t = lane + 64 * o;
-    if (t < NT) M[(size_t)c * NT + t] = {acc[o], 0.0};
-  }
-  sred[lane] = rmax;
-  __syncthreads();
-  if (lane == 0) {
-    double rm = 0;
-    for (int i = 0; i < 64; i++) rm = sred[i] > rm ? sred[i] : rm;
-    double R = cRb[c];
-    if (useRmax) R = R < rm ? R : rm;
-    R /= theta;
-    cX[c].w = R;
-  }
+  if ((int)threadIdx.x < NT) M[(size_t)c * NT + threadIdx.x] = {acc, 0.0};
+  if (threadIdx.x == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
 }
 
 // ---------------------------------------------------------------------------
@@ -460,39 +531,122 @@ __global__ void __launch_bounds__(64)
   }
 }
 
-template <int P, int IPL>
-static void m2l_cart_launch(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L,
-                            const uint32_t *desc, const int *slot0, const int *outslot, int maxc) {
-  hipLaunchKernelGGL((k_m2l_cart<P, IPL>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img,
-                     cX, M, L, desc, slot0, outslot, maxc, h.cfg.cycle, h.cfg.mass);
+// Real parts of the multipoles, packed (what k_m2l_cart_reg reads).
+__global__ void k_cart_pack(const cplx *__restrict__ M, int64_t n, double *__restrict__ Mp) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) Mp[i] = M[i].re;
 }
 
-// Items per lane, rounded up to the compiled register budgets.
+// P = 4 and 6: one wave per target cell and one lane per pair, the pair's
+// derivative tensor and the target's sums in registers (2 x 56 doubles at P =
+// 6, two waves per SIMD), every index fixed at compile time; the lanes' sums
+// are added in lane order through LDS at the end.  A pair is 462 multiply-adds
+// and about 400 operations of the recurrence at P = 6, and 448 bytes of its
+// source's multipole.  1.41 M pairs over 4680 targets: 315 us; 2180 us with a
+// batch of tensors in LDS and a term list per lane (62 KB for one wave left
+// two waves per CU), which stays for P = 8, whose 2 x 120 doubles do not fit.
 template <int P>
-struct CartIPL;
-template <>
-struct CartIPL<4> {
-  static constexpr int V = 8;
-};
-template <>
-struct CartIPL<6> {
-  static constexpr int V = 16;
-};
-template <>
-struct CartIPL<8> {
-  static constexpr int V = 40;
-};
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+    k_m2l_cart_reg(const int *__restrict__ tgt_list, const int *__restrict__ off, const int *__restrict__ src,
+                   const unsigned char *__restrict__ img, const double4 *__restrict__ cX,
+                   const double *__restrict__ Mp, cplx *__restrict__ L, double cycle, int mass) {
+  constexpr int NT = Cart<P>::NT;
+  constexpr CartTab<P> tab{};
+  constexpr int kRow = 28;  // outputs reduced at a time
+  __shared__ double sh[kRow][65];
+  const int c = tgt_list[blockIdx.x], lane = threadIdx.x;
+  const double4 Xi = cX[c];
+  const double mi0 = mass ? Mp[(size_t)c * NT] : 1.0;
+  double l[NT];
+#pragma unroll
+  for (int a = 0; a < NT; a++) l[a] = 0;
+  const int e0 = off[c], e1 = off[c + 1];
+  for (int e = e0 + lane; e < e1; e += 64) {
+    const int s = src[e], im = img[e];
+    const double4 Xj = cX[s];
+    const double2 *mp = reinterpret_cast<const double2 *>(Mp + (size_t)s * NT);
+    const double px = (im / 9 - 1) * cycle, py = ((im / 3) % 3 - 1) * cycle, pz = (im % 3 - 1) * cycle;
+    const double d[3] = {Xi.x - Xj.x - px, Xi.y - Xj.y - py, Xi.z - Xj.z - pz};
+    const double invR2 = 1 / (d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+    // Taylor coefficients (Kernels::derivative, :187-191), then times k!.
+    double C[NT];
+    C[0] = (mass ? mi0 * Mp[(size_t)s * NT] : 1.0) * sqrt(invR2);
+#pragma unroll
+    for (int t = 1; t < NT; t++) {
+      const int k[3] = {tab.x[t], tab.y[t], tab.z[t]}, n = k[0] + k[1] + k[2];
+      double s1 = 0, s2 = 0;
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        const int ux = q == 0, uy = q == 1, uz = q == 2;
+        if (k[q] >= 1) s1 += d[q] * C[CartTab<P>::idx(k[0] - ux, k[1] - uy, k[2] - uz)];
+        if (k[q] >= 2) s2 += C[CartTab<P>::idx(k[0] - 2 * ux, k[1] - 2 * uy, k[2] - 2 * uz)];
+      }
+      C[t] = ((1.0 - 2 * n) / n * s1 + (1.0 - n) / n * s2) * invR2;
+    }
+#pragma unroll
+    for (int t = 1; t < NT; t++) {
+      int f = 1;
+#pragma unroll
+      for (int q = 2; q < P; q++) f *= (tab.x[t] >= q ? q : 1) * (tab.y[t] >= q ? q : 1) * (tab.z[t] >= q ? q : 1);
+      C[t] *= f;
+    }
+#pragma unroll
+    for (int b2 = 0; b2 < NT / 2; b2++) {
+      const double2 m2 = mp[b2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int b = 2 * b2 + u;
+        const double m = u == 0 ? (mass && b == 0 ? 1.0 : m2.x) : m2.y;
+#pragma unroll
+        for (int a = 0; a < NT; a++)
+          if (m2l_term(P, tab.x[a] + tab.y[a] + tab.z[a], tab.x[b] + tab.y[b] + tab.z[b]))
+            l[a] += m * C[CartTab<P>::idx(tab.x[a] + tab.x[b], tab.y[a] + tab.y[b], tab.z[a] + tab.z[b])];
+      }
+    }
+  }
+#pragma unroll
+  for (int a0 = 0; a0 < NT; a0 += kRow) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRow; r++)
+      if (a0 + r < NT) sh[r][lane] = l[a0 + r];
+    __syncthreads();
+    const int r = lane >> 1, half = 32 * (lane & 1);  // two lanes per output
+    double v = 0;
+    if (r < kRow)
+      for (int i = 0; i < 32; i++) v += sh[r][half + i];
+    v += __shfl_xor(v, 1);
+    if (r < kRow && a0 + r < NT && half == 0) {
+      cplx o = L[(size_t)c * NT + a0 + r];
+      o.re += v;
+      L[(size_t)c * NT + a0 + r] = o;
+    }
+  }
+}
 
 template <int P>
-static void m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L) {
-  using S = CartM2LShape<P>;
-  const int key = 1000 + P;
+static void m2l_cart_reg(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int64_t nc, cplx *L) {
+  constexpr int NT = Cart<P>::NT;
+  if (lst.ntgt == 0) return;
+  h.cart_M.resize(nc * NT);
+  hipLaunchKernelGGL(k_cart_pack, dim3(div_up(nc * NT, 256)), dim3(256), 0, h.stream, M, nc * NT, h.cart_M.p);
+  hipLaunchKernelGGL(k_m2l_cart_reg<P>, dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img, cX,
+                     h.cart_M.p, L, h.cfg.cycle, h.cfg.mass);
+  EXA_HIP(hipGetLastError());
+}
+
+// Items per lane at P = 8, rounded up to the compiled register budget.
+constexpr int kCartIPL8 = 40;
+
+static void m2l_cart_sched8(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L) {
+  using S = CartM2LShape<8>;
+  const int key = 1008;
   if (h.m2l_sched_P != key) {
-    const CartSchedule sc = build_cart_schedule(P);
-    if (sc.ipl > CartIPL<P>::V || sc.nslots > S::NCHUNK)
+    const CartSchedule sc = build_cart_schedule(8);
+    if (sc.ipl > kCartIPL8 || sc.nslots > S::NCHUNK)
       throw Error(EXAFMM_HIP_EUNSUP, "Cartesian M2L schedule exceeds its compiled budget");
     std::vector<uint32_t> blob(sc.desc);
-    blob.resize((size_t)CartIPL<P>::V * 64, (uint32_t)S::NT);  // pad to the compiled item count
+    blob.resize((size_t)kCartIPL8 * 64, (uint32_t)S::NT);  // pad to the compiled item count
     for (int v : sc.slot0) blob.push_back((uint32_t)v);
     for (int v : sc.outslot) blob.push_back((uint32_t)v);
     h.m2l_sched.resize(blob.size());
@@ -503,162 +657,161 @@ static void m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, co
     h.cart_maxc = sc.maxc;
   }
   const uint32_t *desc = h.m2l_sched.p;
-  const int *slot0 = reinterpret_cast<const int *>(desc + 64 * CartIPL<P>::V);
+  const int *slot0 = reinterpret_cast<const int *>(desc + 64 * kCartIPL8);
   const int *outslot = slot0 + 64;
-  if (lst.ntgt > 0) m2l_cart_launch<P, CartIPL<P>::V>(h, lst, cX, M, L, desc, slot0, outslot, h.cart_maxc);
+  if (lst.ntgt > 0)
+    hipLaunchKernelGGL((k_m2l_cart<8, kCartIPL8>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src,
+                       lst.img, cX, M, L, desc, slot0, outslot, h.cart_maxc, h.cfg.cycle, h.cfg.mass);
   EXA_HIP(hipGetLastError());
 }
 
-template <int P>
-static void m2l_cart_impl(Handle &h) {
-  m2l_cart_arrays<P>(h, M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p}, h.cX.p, h.M.p,
-                     h.L.p);
+// The pairs of `lst` on arrays of nc cells.
+static void m2l_cart(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int64_t nc, cplx *L) {
+  switch (h.cfg.P) {
+    case 4: m2l_cart_reg<4>(h, lst, cX, M, nc, L); break;
+    case 6: m2l_cart_reg<6>(h, lst, cX, M, nc, L); break;
+    case 8: m2l_cart_sched8(h, lst, cX, M, L); break;
+    default: throw Error(EXAFMM_HIP_EUNSUP, "Cartesian P must be one of 4, 6, 8");
+  }
 }
 
 // ---------------------------------------------------------------------------
-// traversePeriodic (traversal.h:127-185) in the Cartesian basis.
+// traversePeriodic (traversal.h:127-185) in the Cartesian basis, by lattice
+// sums as in the spherical one (periodic.hip): the derivative tensors of a
+// sublevel's 702 offsets are summed once, in units of the cycle, and so are
+// the 26 neighbours' powers (6 us at P = 6 and 3 levels; 1.9 ms as single
+// translations, whose recurrence ran on one lane).  Both sums vanish unless all three
+// indices are even (and, for the derivatives, at degree 2).
 template <int P>
-__global__ void __launch_bounds__(64)
-    k_periodic_cart_m2l(const double4 *__restrict__ cX, const cplx *__restrict__ M, const cplx *__restrict__ Mp,
-                        double cycle, int mass, cplx *__restrict__ part) {
+__global__ void __launch_bounds__(1024) k_periodic_cart_table(double *__restrict__ tab, double *__restrict__ rows) {
   constexpr int NT = Cart<P>::NT;
-  constexpr int NO = (NT + 63) / 64;
-  __shared__ double sC[NT];
-  __shared__ double sM[NT];
-  const int lane = threadIdx.x;
-  const int r = blockIdx.x < 13 ? blockIdx.x : blockIdx.x + 1;
-  const int ix = r / 9 - 1, iy = (r / 3) % 3 - 1, iz = r % 3 - 1;
-  for (int t = lane; t < NT; t += 64) sM[t] = (t == 0 && mass) ? 1.0 : Mp[t].re;
-  const double mi0 = M[0].re, mj0 = Mp[0].re;
-  double acc[NO];
-  for (int o = 0; o < NO; o++) acc[o] = 0;
-  const double4 X = cX[0];
-  for (int cx = -1; cx <= 1; cx++)
-    for (int cy = -1; cy <= 1; cy++)
-      for (int cz = -1; cz <= 1; cz++) {
-        const double dx = X.x - X.x - (ix * 3 + cx) * cycle, dy = X.y - X.y - (iy * 3 + cy) * cycle,
-                     dz = X.z - X.z - (iz * 3 + cz) * cycle;
-        __syncthreads();
-        if (lane == 0) {
-          double r2 = 0;
-          r2 += dx * dx;
-          r2 += dy * dy;
-          r2 += dz * dz;
-          const double invR2 = 1 / r2;
-          const double invR = mass ? mi0 * mj0 * sqrt(invR2) : sqrt(invR2);
-          cart_coef<P>(sC, dx, dy, dz, invR2, invR);
-        }
-        __syncthreads();
-        for (int o = 0; o < NO; o++) {
-          const int a = lane + 64 * o;
-          if (a >= NT) continue;
-          int xa, ya, za;
-          cmi(a, xa, ya, za);
-          const int da = xa + ya + za;
-          double sum = 0;
-          for (int b = 0; b < NT; b++) {
-            int xb, yb, zb;
-            cmi(b, xb, yb, zb);
-            if (m2l_term(P, da, xb + yb + zb)) sum += sM[b] * sC[cidx(xa + xb, ya + yb, za + zb)];
-          }
-          acc[o] += sum;
-        }
-      }
-  for (int o = 0; o < NO; o++) {
-    const int a = lane + 64 * o;
-    if (a < NT) part[(size_t)blockIdx.x * NT + a] = {acc[o], 0.0};
+  const int tid = threadIdx.x;
+  // One offset per lane: its tensor (or powers) in its own row, then lane
+  // t adds coefficient t of every row, in offset order.
+  const int x = tid / 81 - 4, y = (tid / 9) % 9 - 4, z = tid % 9 - 4;
+  const int far = max(max(abs(x), abs(y)), abs(z));
+  if (tid < 729 && far >= 2) {
+    const double invR2 = 1.0 / (x * x + y * y + z * z);
+    cart_coef<P>(rows + (size_t)tid * NT, x, y, z, invR2, sqrt(invR2));
+  } else if (tid < 729 && far == 1) {
+    for (int t = 0; t < NT; t++) {
+      int a, b, c;
+      cmi(t, a, b, c);
+      rows[(size_t)tid * NT + t] = cpow(1.0, a, b, c, x, y, z);
+    }
   }
+  __threadfence_block();
+  __syncthreads();
+  if (tid >= NT) return;
+  int a, b, c;
+  cmi(tid, a, b, c);
+  double s = 0, r = 0;
+  for (int v = 0; v < 729; v++) {
+    const int m = max(max(abs(v / 81 - 4), abs((v / 9) % 9 - 4)), abs(v % 9 - 4));
+    if (m >= 2) s += rows[(size_t)v * NT + tid];
+    if (m == 1) r += rows[(size_t)v * NT + tid];
+  }
+  const bool odd = (a | b | c) & 1;
+  tab[tid] = odd || a + b + c == 2 ? 0.0 : s;
+  tab[NT + tid] = odd ? 0.0 : r;
 }
 
+// The nsub sublevels, 8 lanes per output (they split the terms and add their
+// sums in lane order); multipoles in units of the current cycle.
 template <int P>
-__global__ void __launch_bounds__(64)
-    k_periodic_cart_update(const double4 *__restrict__ cX, cplx *__restrict__ L, const cplx *__restrict__ part,
-                           cplx *__restrict__ Mp, double cycle, int mass, int last) {
-#pragma clang fp contract(off)
+__global__ void __launch_bounds__(1024)
+    k_periodic_cart_far(const cplx *__restrict__ M, cplx *__restrict__ L, const double *__restrict__ tab,
+                        double cycle, int nsub, int mass) {
   constexpr int NT = Cart<P>::NT;
-  constexpr int NO = (NT + 63) / 64;
-  __shared__ double sM[NT];
-  __shared__ double sC[NT];
-  __shared__ double sN[NT];
-  const int lane = threadIdx.x;
-  for (int t = lane; t < NT; t += 64) {
-    cplx l = L[t];
-    for (int b = 0; b < 26; b++) l.re += part[(size_t)b * NT + t].re;
-    L[t] = l;
-  }
-  if (last) return;
-  const double m0 = Mp[0].re;
-  for (int t = lane; t < NT; t += 64) sM[t] = (mass && t > 0) ? Mp[t].re * m0 : Mp[t].re;
-  double acc[NO];
-  int ka[NO], kb[NO], kc[NO];
-  for (int o = 0; o < NO; o++) {
-    acc[o] = 0;
-    const int t = lane + 64 * o;
-    cmi(t < NT ? t : 0, ka[o], kb[o], kc[o]);
-  }
-  const double4 X = cX[0];
-  for (int ix = -1; ix <= 1; ix++)
-    for (int iy = -1; iy <= 1; iy++)
-      for (int iz = -1; iz <= 1; iz++) {
-        if (ix == 0 && iy == 0 && iz == 0) continue;
-        const double dx = X.x - (X.x + ix * cycle), dy = X.y - (X.y + iy * cycle), dz = X.z - (X.z + iz * cycle);
-        __syncthreads();
-        for (int t = lane; t < NT; t += 64) {
-          int a, b, cz;
-          cmi(t, a, b, cz);
-          sC[t] = cpow(1.0, a, b, cz, dx, dy, dz);
-        }
-        __syncthreads();
-        for (int o = 0; o < NO; o++) {
-          const int t = lane + 64 * o;
-          if (t >= NT) continue;
-          acc[o] += sC[t] * sM[0];
-          if (t == 0) continue;
-          double sum = 0;
-          for (int a = 0; a <= ka[o]; a++)
-            for (int b = 0; b <= kb[o]; b++)
-              for (int cz = 0; cz <= kc[o]; cz++) {
-                if (a == 0 && b == 0 && cz == 0) continue;
-                sum += sC[cidx(ka[o] - a, kb[o] - b, kc[o] - cz)] * sM[cidx(a, b, cz)];
-              }
-          acc[o] += sum;
-        }
-      }
-  for (int o = 0; o < NO; o++) {
-    const int t = lane + 64 * o;
-    if (t < NT) sN[t] = acc[o];
+  static_assert(8 * NT <= 1024, "8 lanes per output");
+  __shared__ double sM[NT], sN[NT], sC[NT], sR[NT];
+  __shared__ unsigned char sx[NT], sy[NT], sz[NT];
+  const int tid = threadIdx.x, o = tid >> 3, part = tid & 7;
+  const double icycle = 1 / cycle;
+  if (tid < NT) {
+    int a, b, c;
+    cmi(tid, a, b, c);
+    sx[tid] = a;
+    sy[tid] = b;
+    sz[tid] = c;
+    double f = 1;
+    for (int i = 0; i < a + b + c; i++) f *= icycle;
+    sM[tid] = M[tid].re * f;
+    sC[tid] = tab[tid];
+    sR[tid] = tab[NT + tid];
   }
   __syncthreads();
-  const double n0 = sN[0];
-  for (int t = lane; t < NT; t += 64) Mp[t] = {(mass && t > 0) ? sN[t] / n0 : sN[t], 0.0};
+  const bool on = o < NT;
+  const int xa = on ? sx[o] : 0, ya = on ? sy[o] : 0, za = on ? sz[o] : 0, da = xa + ya + za;
+  const double mi0 = M[0].re;
+  auto sum8 = [](double v) {  // of the 8 lanes of an output
+    v += __shfl_xor(v, 1);
+    v += __shfl_xor(v, 2);
+    return v + __shfl_xor(v, 4);
+  };
+  double iu = icycle, l = 0, third = 1;
+  for (int i = 0; i < da; i++) third *= 1.0 / 3;
+  for (int lev = 0; lev < nsub; lev++, iu /= 3) {
+    const double m0 = sM[0];
+    double s = 0;
+    if (on)
+      for (int b = part; b < NT; b += 8) {
+        const int xb = sx[b], yb = sy[b], zb = sz[b];
+        if (m2l_term(P, da, xb + yb + zb))
+          s += (mass && b == 0 ? 1.0 : sM[b]) * sC[cidx(xa + xb, ya + yb, za + zb)];
+      }
+    double f = mass ? mi0 * m0 * iu : iu;
+    for (int i = 0; i < da; i++) f *= iu;
+    l += f * sum8(s);
+    if (lev == nsub - 1) break;
+    // M2M of the 26 copies: sum over k <= a of R_(a - k) M_k.
+    s = 0;
+    if (on)
+      for (int b = part; b <= o; b += 8) {
+        const int xb = sx[b], yb = sy[b], zb = sz[b];
+        if (xb <= xa && yb <= ya && zb <= za)
+          s += (mass && b > 0 ? sM[b] * m0 : sM[b]) * sR[cidx(xa - xb, ya - yb, za - zb)];
+      }
+    s = sum8(s);
+    if (on && part == 0) sN[o] = s;
+    __syncthreads();
+    const double n0 = sN[0];
+    if (on && part == 0) sM[o] = third * (mass && o > 0 ? s / n0 : s);
+    __syncthreads();
+  }
+  if (on && part == 0) {
+    cplx v = L[o];
+    v.re += l;
+    L[o] = v;
+  }
 }
 
 template <int P>
 static void periodic_cart_impl(Handle &h) {
   constexpr int NT = Cart<P>::NT;
-  h.per_M.resize(NT);
-  h.per_part.resize(26 * NT);
-  EXA_HIP(hipMemcpyAsync(h.per_M.p, h.M.p, NT * sizeof(cplx), hipMemcpyDeviceToDevice, h.stream));
-  double cycle = h.cfg.cycle;
-  for (int lev = 0; lev < h.cfg.images - 1; lev++) {
-    hipLaunchKernelGGL((k_periodic_cart_m2l<P>), dim3(26), dim3(64), 0, h.stream, h.cX.p, h.M.p, h.per_M.p, cycle,
-                       h.cfg.mass, h.per_part.p);
-    hipLaunchKernelGGL((k_periodic_cart_update<P>), dim3(1), dim3(64), 0, h.stream, h.cX.p, h.L.p, h.per_part.p,
-                       h.per_M.p, cycle, h.cfg.mass, lev == h.cfg.images - 2 ? 1 : 0);
-    cycle *= 3;
+  if (h.cfg.images <= 1) return;
+  if (!h.per_ready) {
+    h.per_tab.resize((2 + 729) * NT);  // the sums, and the rows they are made from
+    hipLaunchKernelGGL(k_periodic_cart_table<P>, dim3(1), dim3(1024), 0, h.stream, h.per_tab.p,
+                       h.per_tab.p + 2 * NT);
+    h.per_ready = true;
   }
+  hipLaunchKernelGGL(k_periodic_cart_far<P>, dim3(1), dim3(1024), 0, h.stream, h.M.p, h.L.p, h.per_tab.p, h.cfg.cycle,
+                     h.cfg.images - 1, h.cfg.mass);
   EXA_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
+// All leaves first (they need nothing), then the parents level by level.
 template <int P>
 static void upward_cart_impl(Handle &h) {
-  for (int t = h.nlevels - 1; t >= 0; t--) {
+  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells), dim3(64), 0, h.stream, h.lvl_cells.p, h.body4.p, h.cX.p, h.cRb.p,
+                     h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
+  for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;
-    hipLaunchKernelGGL(k_upward_cart<P>, dim3(cnt), dim3(64), 0, h.stream, h.lvl_cells.p + h.lvl_off[t], h.body4.p,
-                       h.cX.p, h.cRb.p, h.cChild.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta,
-                       h.cfg.useRmax);
+    hipLaunchKernelGGL(k_m2m_cart<P>, dim3(cnt), dim3(512), 0, h.stream, h.lvl_cells.p + h.lvl_off[t], h.cX.p,
+                       h.cRb.p, h.cChild.p, h.cNChild.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
   }
   EXA_HIP(hipGetLastError());
 }
@@ -687,7 +840,8 @@ void run_upward_cart(Handle &h) { EXA_DISPATCH_CART(upward_cart_impl, h); }
 void run_downward_cart(Handle &h) { EXA_DISPATCH_CART(downward_cart_impl, h); }
 void run_m2l_cart(Handle &h) {
   if (h.nm2l_tgt == 0) return;
-  EXA_DISPATCH_CART(m2l_cart_impl, h);
+  m2l_cart(h, M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p}, h.cX.p, h.M.p, h.ncells,
+           h.L.p);
 }
 void run_periodic_cart(Handle &h) {
   if (h.cfg.images <= 0 || h.ncells == 0) return;
@@ -697,8 +851,10 @@ void run_periodic_cart(Handle &h) {
 // The Cartesian pass kernels on a caller-built cell set (per-cell operators).
 template <int P>
 static void upward_cart_cells_impl(Handle &h, const CellSetView &v) {
-  hipLaunchKernelGGL(k_upward_cart<P>, dim3(v.ncell), dim3(64), 0, h.stream, v.cells, v.body, v.cX, v.cRb, v.cChild,
-                     v.cNChild, v.cBody, v.cNBody, v.M, h.cfg.theta, h.cfg.useRmax);
+  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(v.ncell), dim3(64), 0, h.stream, v.cells, v.body, v.cX, v.cRb, v.cNChild,
+                     v.cBody, v.cNBody, v.M, h.cfg.theta, h.cfg.useRmax);
+  hipLaunchKernelGGL(k_m2m_cart<P>, dim3(v.ncell), dim3(512), 0, h.stream, v.cells, v.cX, v.cRb, v.cChild, v.cNChild,
+                     v.M, h.cfg.theta, h.cfg.useRmax);
 }
 
 template <int P>
@@ -723,13 +879,8 @@ void launch_downward_cart_cells(Handle &h, const CellSetView &v) {
   EXA_DISPATCH_CART2(downward_cart_cells_impl, h, v);
   EXA_HIP(hipGetLastError());
 }
-void launch_m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L) {
-  switch (h.cfg.P) {
-    case 4: m2l_cart_arrays<4>(h, lst, cX, M, L); break;
-    case 6: m2l_cart_arrays<6>(h, lst, cX, M, L); break;
-    case 8: m2l_cart_arrays<8>(h, lst, cX, M, L); break;
-    default: throw Error(EXAFMM_HIP_EUNSUP, "Cartesian P must be one of 4, 6, 8");
-  }
+void launch_m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L) {
+  m2l_cart(h, lst, cX, M, nc, L);
 }
 
 }  // namespace exafmm

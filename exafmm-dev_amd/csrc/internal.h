@@ -149,9 +149,9 @@ struct Handle {
   DBuf<int> at_start, at_count, at_parent, at_leaf, at_level, at_first, at_nchild, at_astart, at_acount, at_agid,
       at_idx2, at_nnode, at_cellid, at_cursor, at_nl;
 
-  // Periodic far field: the periodic parent's multipole and 26 partial
-  // local expansions per sublevel.
-  DBuf<cplx> per_M, per_part;
+  // Periodic far field: the lattice sums of the handle's order and basis.
+  DBuf<double> per_tab;
+  bool per_ready = false;
 
   // Ewald summation: the wave rows, the forward transform's partial sums and
   // the scaled wave table, and slots of partial results.
@@ -209,6 +209,7 @@ struct Handle {
   // M2L lane schedule (a pure function of P, the basis and the table type).
   DBuf<uint32_t> m2l_sched;
   int m2l_sched_P = -1;
+  DBuf<double> cart_M;  // real parts of the multipoles, packed (Cartesian M2L)
   int cart_maxc = 0;  // Cartesian schedule: chunks per output (outslot row length)
 
   // Scratch.
@@ -356,10 +357,10 @@ void launch_upward_cells(Handle &h, const CellSetView &v);
 void launch_downward_cells(Handle &h, const CellSetView &v);
 void launch_upward_cart_cells(Handle &h, const CellSetView &v);
 void launch_downward_cart_cells(Handle &h, const CellSetView &v);
-// M2L of the pairs of `lst` on explicit centre and expansion arrays in FP64
+// M2L of the pairs of `lst` on explicit centre and expansion arrays of nc cells in FP64
 // (spherical per-pair kernel, or the Cartesian kernel for basis 1).
-void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L);
-void launch_m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L);
+void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L);
+void launch_m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L);
 
 // Zero / copy device memory with a kernel (bytes a multiple of 8), so the
 // work can be recorded in a HIP graph (no memset or copy nodes).

@@ -328,8 +328,8 @@ static void m2l_impl(Handle &h, const M2LList &lst) {
   m2l_launch<P>(h, lst, h.cX.p, h.M.p, h.L.p, h.cfg.precision == 1, true);
 }
 
-void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L) {
-  if (h.cfg.basis == 1) return launch_m2l_cart_arrays(h, lst, cX, M, L);
+void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L) {
+  if (h.cfg.basis == 1) return launch_m2l_cart_arrays(h, lst, cX, M, nc, L);
   switch (h.cfg.P) {
     case 4: m2l_launch<4>(h, lst, cX, M, L, false, false); break;
     case 6: m2l_launch<6>(h, lst, cX, M, L, false, false); break;

@@ -9,9 +9,15 @@
 // parent in the reference, NCHILD = 26), and cycle triples.  MASS mode
 // denormalises around the M2M and finally divides the root's L by M0.
 //
-// Work: 702 M2L per sublevel, into one cell.  One workgroup per ring cell
-// (26) does its 27 translations; a one-workgroup kernel adds the 26 partial
-// local expansions in ring order and forms the next sublevel's multipole.
+// Work: every sublevel's 702 translations read one multipole and add into one
+// cell, so they are one translation by the lattice sum of the harmonics, and
+// the M2M of the 26 copies one translation by their sum.  The offsets are
+// integer vectors times the sublevel's cycle and the harmonics homogeneous:
+// the two sums over the integer vectors depend on the order alone and are
+// kept by the handle, and one workgroup walks the sublevels (10 us at P = 10,
+// 3 levels; 750 us as 702 translations per sublevel on 26 workgroups).  By
+// the cube's symmetry the sums are real and vanish unless n is even, not 2,
+// and m a multiple of 4.
 //
 // getDipole / dipoleCorrection (include/up_down_pass.h:151-168).
 #include <cmath>
@@ -21,153 +27,173 @@
 
 namespace exafmm {
 
-// Partial local expansion of ring cell blockIdx.x (ix, iy, iz != 0) at this
-// sublevel: sum over its 27 children of M2L(root <- parent image at Xp).
-template <int P>
-__global__ void __launch_bounds__(64)
-    k_periodic_m2l(const double4 *__restrict__ cX, const cplx *__restrict__ M, const cplx *__restrict__ Mp,
-                   double cycle, int mass, cplx *__restrict__ part) {
-  constexpr int NT = Expn<P>::NT;
-  constexpr int NO = (NT + 63) / 64;
-  __shared__ cplx sS[P * P];
-  __shared__ cplx sM[NT];
-  const int lane = threadIdx.x;
-  int r = blockIdx.x < 13 ? blockIdx.x : blockIdx.x + 1;  // skip the centre (13)
-  const int ix = r / 9 - 1, iy = (r / 3) % 3 - 1, iz = r % 3 - 1;
-  for (int t = lane; t < NT; t += 64) sM[t] = Mp[t];
-  const double mi0 = M[0].re, mj0 = Mp[0].re;
-  double ar[NO], ai[NO];
-  int tj[NO], tk[NO];
-#pragma unroll
-  for (int o = 0; o < NO; o++) {
-    ar[o] = ai[o] = 0;
-    coef_nm(lane + 64 * o < NT ? lane + 64 * o : 0, tj[o], tk[o]);
+// Sum of the values that the 64 k lanes of a workgroup hold, in a fixed
+// order (sh: blockDim.x doubles; every lane gets it).
+__device__ inline double block_sum(double v, double *sh) {
+  sh[threadIdx.x] = v;
+  __syncthreads();
+  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    __syncthreads();
   }
-  const double4 X = cX[0];
-  for (int cx = -1; cx <= 1; cx++)
-    for (int cy = -1; cy <= 1; cy++)
-      for (int cz = -1; cz <= 1; cz++) {
-        const double px = (ix * 3 + cx) * cycle, py = (iy * 3 + cy) * cycle, pz = (iz * 3 + cz) * cycle;
-        // dX = X_root - X_parent - Xp, with the parent a copy of the root.
-        const Geom g = make_geom(X.x - X.x - px, X.y - X.y - py, X.z - X.z - pz);
-        __syncthreads();
-        for (int t = lane; t < NT; t += 64) {
-          int a, b;
-          coef_nm(t, a, b);
-          double re, im;
-          singular_nm(a, b, g, re, im);
-          sS[a * a + a + b] = {re, im};
-          if (b > 0) sS[a * a + a - b] = {re, -im};
-        }
-        __syncthreads();
-#pragma unroll
-        for (int o = 0; o < NO; o++) {
-          if (lane + 64 * o >= NT) continue;
-          const int j = tj[o], k = tk[o];
-          // LaplaceSphericalCPU.cxx:149-191 (MASS: :157-172) for one (j, k).
-          const double Cnm = (mass ? mi0 * mj0 : 1.0) * ((j & 1) ? -1.0 : 1.0);
-          double lr = 0, li = 0;
-          int n0 = 0;
-          if (mass) {
-            const cplx y = sS[j * j + j - k];
-            lr += Cnm * y.re;
-            li += Cnm * y.im;
-            n0 = 1;
-          }
-          for (int n = n0; n < P - j; n++) {
-            const int a = j + n;
-            for (int m = -n; m < 0; m++) {  // conj(M_n^{-m}) S_{j+n}^{m-k}
-              const cplx mv = sM[tri(n) - m];
-              const cplx y = sS[a * a + a + m - k];
-              lr += Cnm * (mv.re * y.re + mv.im * y.im);
-              li += Cnm * (mv.re * y.im - mv.im * y.re);
-            }
-            for (int m = 0; m <= n; m++) {
-              const double c2 = Cnm * ((((k - m) * (k < m) + m) & 1) ? -1.0 : 1.0);
-              const cplx mv = sM[tri(n) + m];
-              const cplx y = sS[a * a + a + m - k];
-              lr += c2 * (mv.re * y.re - mv.im * y.im);
-              li += c2 * (mv.re * y.im + mv.im * y.re);
-            }
-          }
-          ar[o] += lr;
-          ai[o] += li;
-        }
-      }
-#pragma unroll
-  for (int o = 0; o < NO; o++)
-    if (lane + 64 * o < NT) part[(size_t)blockIdx.x * NT + lane + 64 * o] = {ar[o], ai[o]};
+  return sh[0];
 }
 
-// L_root += sum of the 26 partials (ring order); then, unless this was the
-// last sublevel, Mp <- M2M of the 26 neighbour copies of the periodic parent.
+// Lattice sums of coefficient t = blockIdx.x: tab[t] = sum of S_n^m over the
+// integer vectors 3 i + c (i, c in {-1, 0, 1}^3, i != 0), tab[NT + t] = sum of
+// R_n^m over the 26 neighbour vectors.
 template <int P>
-__global__ void __launch_bounds__(64)
-    k_periodic_update(const double4 *__restrict__ cX, cplx *__restrict__ L, const cplx *__restrict__ part,
-                      cplx *__restrict__ Mp, double cycle, int mass, int last) {
+__global__ void __launch_bounds__(256) k_periodic_table(double *__restrict__ tab) {
   constexpr int NT = Expn<P>::NT;
-  __shared__ cplx sM[NT];
-  __shared__ cplx sY[NT];
-  __shared__ double m0s;
-  const int lane = threadIdx.x;
-  for (int t = lane; t < NT; t += 64) {
-    cplx l = L[t];
-    for (int b = 0; b < 26; b++) {
-      l.re += part[(size_t)b * NT + t].re;
-      l.im += part[(size_t)b * NT + t].im;
+  __shared__ double sh[256];
+  int n, m;
+  coef_nm(blockIdx.x, n, m);
+  double s = 0, r = 0;
+  for (int v = threadIdx.x; v < 729; v += 256) {
+    const int x = v / 81 - 4, y = (v / 9) % 9 - 4, z = v % 9 - 4;
+    const int far = max(max(abs(x), abs(y)), abs(z));
+    if (far == 0) continue;
+    const Geom g = make_geom(x, y, z);
+    double re, im;
+    if (far >= 2) {
+      singular_nm(n, m, g, re, im);
+      s += re;
+    } else {
+      regular_nm(n, m, g, re, im);
+      r += re;
     }
-    L[t] = l;
   }
-  if (last) return;
-  if (lane == 0) m0s = Mp[0].re;
+  const bool zero = (n & 1) || (m & 3) || n == 2;
+  s = block_sum(s, sh);
   __syncthreads();
-  for (int t = lane; t < NT; t += 64) {
-    cplx v = Mp[t];
-    if (mass && t > 0) {  // traversal.h:155-156
-      v.re *= m0s;
-      v.im *= m0s;
-    }
-    sM[t] = v;
+  r = block_sum(r, sh);
+  if (threadIdx.x == 0) {
+    tab[blockIdx.x] = zero ? 0.0 : s;
+    tab[NT + blockIdx.x] = zero ? 0.0 : r;
   }
-  const double4 X = cX[0];
-  double acc_re[2] = {0, 0}, acc_im[2] = {0, 0};
-  for (int ix = -1; ix <= 1; ix++)
-    for (int iy = -1; iy <= 1; iy++)
-      for (int iz = -1; iz <= 1; iz++) {
-        if (ix == 0 && iy == 0 && iz == 0) continue;
-        const double xj = X.x + ix * cycle, yj = X.y + iy * cycle, zj = X.z + iz * cycle;
-        const Geom g = make_geom(X.x - xj, X.y - yj, X.z - zj);
-        __syncthreads();
-        for (int t = lane; t < NT; t += 64) {
-          int n, m;
-          coef_nm(t, n, m);
-          double re, im;
-          regular_nm(n, m, g, re, im);
-          sY[t] = {re, im};
-        }
-        __syncthreads();
-        for (int o = 0; o < 2; o++) {
-          const int t = lane + 64 * o;
-          if (t >= NT) continue;
-          int j, k;
-          coef_nm(t, j, k);
-          m2m_lane(j, k, sM, sY, acc_re[o], acc_im[o]);
+}
+
+// The nsub sublevels.  Multipoles are kept in units of the current cycle
+// (M_n cycle^-n), so both sums apply as they are.  Work items are (output
+// (j, k), n); an output's items are added in n order.
+template <int P>
+__global__ void __launch_bounds__(512)
+    k_periodic_far(const cplx *__restrict__ M, cplx *__restrict__ L, const double *__restrict__ tab, double cycle,
+                   int nsub, int mass) {
+  constexpr int NT = Expn<P>::NT;
+  __shared__ cplx sM[NT], sL[NT], sp[NT * P];
+  __shared__ double sS[NT], sR[NT];
+  const int tid = threadIdx.x;
+  const double icycle = 1 / cycle;
+  for (int t = tid; t < NT; t += 512) {
+    int n, m;
+    coef_nm(t, n, m);
+    double f = 1;
+    for (int i = 0; i < n; i++) f *= icycle;
+    sM[t] = {M[t].re * f, M[t].im * f};
+    sL[t] = {0, 0};
+    sS[t] = tab[t];
+    sR[t] = tab[NT + t];
+  }
+  const double mi0 = M[0].re;
+  double iu = icycle;  // 1 / cycle of the sublevel
+  __syncthreads();
+  for (int lev = 0; lev < nsub; lev++, iu /= 3) {
+    // M2L (LaplaceSphericalCPU.cxx:149-191; MASS: :157-172, where the source's
+    // M_0 counts as 1 and the translation is scaled by both M_0).
+    const double m0 = sM[0].re;
+    for (int i = tid; i < NT * P; i += 512) {
+      const int t = i / P, n = i % P;
+      int j, k;
+      coef_nm(t, j, k);
+      const int a = j + n;
+      double lr = 0, li = 0;
+      if (a < P && !(a & 1)) {
+        for (int m = -n + ((n + k) & 3); m <= n; m += 4) {  // m = k mod 4
+          const double y = sS[tri(a) + abs(m - k)];
+          cplx v = sM[tri(n) + abs(m)];
+          if (mass && n == 0) v = {1, 0};
+          if (m < 0) {  // conj(M_n^-m)
+            lr += v.re * y;
+            li -= v.im * y;
+          } else {
+            const double f = (((k - m) * (k < m) + m) & 1) ? -y : y;
+            lr += f * v.re;
+            li += f * v.im;
+          }
         }
       }
-  __syncthreads();
-  for (int o = 0; o < 2; o++) {
-    const int t = lane + 64 * o;
-    if (t < NT) sY[t] = {acc_re[o], acc_im[o]};
-  }
-  __syncthreads();
-  const double m0 = sY[0].re;
-  for (int t = lane; t < NT; t += 64) {
-    cplx v = sY[t];
-    if (mass && t > 0) {  // traversal.h:176-178
-      v.re /= m0;
-      v.im /= m0;
+      sp[i] = {lr, li};
     }
-    Mp[t] = v;
+    __syncthreads();
+    for (int t = tid; t < NT; t += 512) {
+      int j, k;
+      coef_nm(t, j, k);
+      double f = ((j & 1) ? -iu : iu) * (mass ? mi0 * m0 : 1.0);
+      for (int i = 0; i < j; i++) f *= iu;
+      double lr = 0, li = 0;
+      for (int n = 0; n < P - j; n++) {
+        lr += sp[t * P + n].re;
+        li += sp[t * P + n].im;
+      }
+      sL[t].re += f * lr;
+      sL[t].im += f * li;
+    }
+    __syncthreads();
+    if (lev == nsub - 1) break;
+    if (mass) {  // traversal.h:155-156
+      for (int t = tid; t < NT; t += 512)
+        if (t > 0) {
+          sM[t].re *= m0;
+          sM[t].im *= m0;
+        }
+      __syncthreads();
+    }
+    // M2M of the 26 copies (LaplaceSphericalCPU.cxx:120-147 with the real,
+    // even sums), then the next sublevel's units.
+    for (int i = tid; i < NT * P; i += 512) {
+      const int t = i / P, n = i % P;
+      int j, k;
+      coef_nm(t, j, k);
+      double lr = 0, li = 0;
+      if (n <= j && !(n & 1)) {
+        for (int m = -(n & ~3); m <= n; m += 4) {
+          const double y = sR[tri(n) + abs(m)];
+          if (m < k && m >= -j + k + n) {
+            const cplx v = sM[tri(j - n) + k - m];
+            lr += v.re * y;
+            li += v.im * y;
+          } else if (m >= k && m <= j + k - n) {
+            const cplx v = sM[tri(j - n) + m - k];
+            const double f = (k & 1) ? -y : y;
+            lr += f * v.re;
+            li -= f * v.im;
+          }
+        }
+      }
+      sp[i] = {lr, li};
+    }
+    __syncthreads();
+    const double n0 = sp[0].re;  // of t = 0 (n = 0 alone)
+    for (int t = tid; t < NT; t += 512) {
+      int j, k;
+      coef_nm(t, j, k);
+      double f = mass && t > 0 ? 1 / n0 : 1.0;  // traversal.h:176-178
+      for (int i = 0; i < j; i++) f *= 1.0 / 3;
+      double lr = 0, li = 0;
+      for (int n = 0; n <= j; n++) {
+        lr += sp[t * P + n].re;
+        li += sp[t * P + n].im;
+      }
+      sM[t] = {f * lr, f * li};
+    }
+    __syncthreads();
+  }
+  for (int t = tid; t < NT; t += 512) {
+    cplx l = L[t];
+    l.re += sL[t].re;
+    l.im += sL[t].im;
+    L[t] = l;
   }
 }
 
@@ -182,17 +208,14 @@ __global__ void k_periodic_mass_L(const cplx *__restrict__ M, cplx *__restrict__
 template <int P>
 static void periodic_impl(Handle &h) {
   constexpr int NT = Expn<P>::NT;
-  h.per_M.resize(NT);
-  h.per_part.resize(26 * NT);
-  copy_device(h.per_M.p, h.M.p, NT * sizeof(cplx), h.stream);
-  double cycle = h.cfg.cycle;
-  for (int lev = 0; lev < h.cfg.images - 1; lev++) {
-    hipLaunchKernelGGL((k_periodic_m2l<P>), dim3(26), dim3(64), 0, h.stream, h.cX.p, h.M.p, h.per_M.p, cycle,
-                       h.cfg.mass, h.per_part.p);
-    hipLaunchKernelGGL((k_periodic_update<P>), dim3(1), dim3(64), 0, h.stream, h.cX.p, h.L.p, h.per_part.p,
-                       h.per_M.p, cycle, h.cfg.mass, lev == h.cfg.images - 2 ? 1 : 0);
-    cycle *= 3;
+  if (!h.per_ready) {
+    h.per_tab.resize(2 * NT);
+    hipLaunchKernelGGL(k_periodic_table<P>, dim3(NT), dim3(256), 0, h.stream, h.per_tab.p);
+    h.per_ready = true;
   }
+  if (h.cfg.images > 1)
+    hipLaunchKernelGGL(k_periodic_far<P>, dim3(1), dim3(512), 0, h.stream, h.M.p, h.L.p, h.per_tab.p, h.cfg.cycle,
+                       h.cfg.images - 1, h.cfg.mass);
   if (h.cfg.mass) hipLaunchKernelGGL(k_periodic_mass_L, dim3(1), dim3(64), 0, h.stream, h.M.p, h.L.p, NT);
   EXA_HIP(hipGetLastError());
 }
