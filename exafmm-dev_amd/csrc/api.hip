@@ -76,12 +76,12 @@ static void do_build(Handle &h) {
   h.key_lvloff = h.nsys == 1 && h.cfg.builder == 1;
   h.have_tree = true;
   h.have_up = h.have_trav = false;
-  h.lat_ms_ready = false;  // scaled multipoles of an older tree
+  h.lat_ms_ready = h.lat_tiles_ready = false;  // of an older tree
 }
 
 static void do_upward(Handle &h) {
   ensure(h.have_tree, "upward_pass: tree not built");
-  h.lat_ms_ready = false;  // the lattice M2L rescales these multipoles itself
+  h.lat_ms_ready = h.lat_tiles_ready = false;  // the lattice M2L rescales these multipoles itself
   run_upward(h);
   run_ropt(h);
   h.have_up = true;
@@ -173,6 +173,7 @@ int exafmm_hip_create(const exafmm_hip_config *cfg, exafmm_hip_handle **out) {
     EXA_HIP(hipEventCreate(&H->h.ev_mult));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_cnt, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_lists, hipEventDisableTiming));
+    EXA_HIP(hipEventCreateWithFlags(&H->h.ev_tiles, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_p2pcnt, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_bounds, hipEventDisableTiming));
     EXA_HIP(hipHostMalloc((void **)&H->h.hpin, Handle::kPinWords * sizeof(int), hipHostMallocDefault));
@@ -265,7 +266,7 @@ int exafmm_hip_build_tree(exafmm_hip_handle *H, const double *xmin3, const doubl
         h.xmin[d] = xmin3[d];
         h.xmax[d] = xmax3[d];
       }
-      h.bounds_dev_stale = true;
+      h.bounds_dev_stale = h.bounds_given = true;
       h.have_bounds = true;
     }
     do_build(h);
@@ -620,7 +621,7 @@ int exafmm_hip_get_stats(exafmm_hip_handle *H, exafmm_hip_stats *s) {
     h.stats.num_cells = h.ncells;
     h.stats.num_levels = h.nlevels;
     h.stats.num_m2l_lattice = h.lat_stats_pairs;
-    h.stats.num_m2l_offsets = h.lat_stats_noff;
+    h.stats.num_m2l_offsets = h.have_trav ? lattice_offsets_used(h) : 0;
     h.stats.num_m2l_tiles = h.lat_stats_tiles;
     h.stats.num_m2l_steps = h.lat_stats_steps;
     *s = h.stats;

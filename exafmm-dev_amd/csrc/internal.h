@@ -89,6 +89,7 @@ struct Handle {
   bool mult_pending = false;     // the main stream has not joined ev_mult yet
   bool mult_enqueue = false;     // run_upward_mult not enqueued yet (the traversal does it)
   hipEvent_t ev_cnt = nullptr;   // a device count copied into hpin
+  hipEvent_t ev_tiles = nullptr; // lattice tiles done on stream3 (split upward pass)
   hipEvent_t ev_lists = nullptr; // raw lists done (the P2P grouping on stream2 waits for it)
   hipEvent_t ev_p2pcnt = nullptr; // P2P target count copied into hpin[9] (stream2)
   hipEvent_t ev_bounds = nullptr; // bounds copied into hpin[kPinBounds..] (main stream)
@@ -120,6 +121,7 @@ struct Handle {
   // values were set by the caller and the device copy is out of date.
   DBuf<double> box;
   bool bounds_pending = false, bounds_dev_stale = false;
+  bool bounds_given = false;  // by the caller: they may not enclose every body
   bool have_bounds = false, have_tree = false, have_up = false, have_trav = false;
 
   // Cells (reference Cell order).
@@ -131,6 +133,7 @@ struct Handle {
   DBuf<uint64_t> cKey;
   DBuf<cplx> M, L;                 // ncells * nterm
   std::vector<int> lvl_off;        // level-order offsets (host), size nlevels+1
+  std::vector<int> lvl_par;        // cells of each level that have children, or a bound on their number
   DBuf<int> lvl_cells;             // cells sorted by level (stable)
 
   // Interaction lists (CSR by target cell).
@@ -179,30 +182,35 @@ struct Handle {
   // (k_p2p_f64_rb / k_p2p_mixed_rb).
   int p2p_kmax = 1;
   DBuf<double> ud_ops;
-  DBuf<int> lat_tkey, lat_tval, lat_thist, lat_gb, lat_act, lat_aidx, lat_alist, lat_step0;
+  DBuf<int> lat_tkey, lat_tval, lat_aidx, lat_alist, lat_step0, lat_tcnt;
+  DBuf<unsigned char> lat_act;  // state of the set-up (LatState), then flags of the (tile, offset) steps in use
   DBuf<double> lat_part;
-  DBuf<int> lat_pkey, lat_hist, lat_flag, lat_kscan, lat_okey, lat_ookey, lat_tile_tgt, lat_tile_of, lat_col_of, lat_slot, lat_irr,
-      lat_scan, irr_off, irr_src, irr_tgt;
+  DBuf<int> lat_flag, lat_kscan, lat_tile_tgt, lat_tile_of, lat_col_of, lat_slot, lat_irr, lat_scan, irr_off, irr_src,
+      irr_tgt;
   DBuf<unsigned char> irr_img;
-  DBuf<int> lat_cnt;            // irregular-pair counter
-  DBuf<int> lat_has;            // cells with M2L pairs
   DBuf<int> irr_rt, irr_rs;     // irregular pairs in emission order (target, source)
   DBuf<unsigned char> irr_ri;   // ... and image
-  DBuf<int> lat_pslot;          // per-pair step, then slot (-1: not a lattice pair)
+  DBuf<int> lat_pslot;          // per-pair step (-1: irregular)
   // T(d) table kept across evaluations: offset key -> row of lat_T / lat_Tf
   // (-1: not computed yet), for expansion order lat_tc_P and FP32 or FP64.
   DBuf<int> lat_tc_map, lat_tc_flag, lat_tc_scan, lat_tc_keys;
+  // Offsets known so far, numbered in key order: key -> number (-1: not
+  // known), number -> T row; flags of offsets met that were not known.
+  DBuf<int> lat_ookey, lat_orow;
+  DBuf<unsigned char> lat_hist;
+  int lat_noff = 0;
   int lat_tc_rows = 0, lat_tc_P = 0, lat_tc_max = 16384;  // rows; a fuller table starts afresh
   bool lat_tc_f32 = false;
   bool lat_ms_ready = false;     // lat_Ms / lat_Msf already queued for this evaluation
   bool lat_begun = false;        // lattice set-up's first part queued (m2l_begin)
-  bool lat_tile_alt = false;     // sorted tile keys in the second half of lat_tkey / lat_tval
+  bool lat_tiles_ready = false;  // tiles of this tree queued on the third stream (ev_tiles)
+  int lat_ntiles = 0;            // tile slots of the tree
   DBuf<double> lat_T, lat_Ms;
   DBuf<float> lat_Tf, lat_Msf;
   int lat_run_ntiles = 0, lat_run_ngrid = 0;  // the last contraction's tiles and grid (0 tiles: none ran)
   M2LList m2l_last{};                          // the pairs the last run_m2l gave the per-pair kernel
   int64_t lat_stats_pairs = 0;
-  int lat_stats_noff = 0, lat_stats_tiles = 0;
+  int lat_stats_tiles = 0;
   int64_t lat_stats_steps = 0;
   bool lat_timed = false, pair_timed = false;  // ev[12..13]: MFMA kernel, ev[14..15]: per-pair kernel
 
@@ -218,6 +226,7 @@ struct Handle {
   // list grouping on the main stream.
   DBuf<int> g2a, g2b, g2c, g2d, g2e;
   DBuf<unsigned char> tmp2;
+  DBuf<unsigned char> tmp3;        // ... and of sorts on stream3
   DBuf<uint64_t> k64a, k64b;
   DBuf<int> ia, ib, ic, id, ie, ifl;
   DBuf<int2> fa, fb;               // traversal frontiers (ci, cj | img << 27)
@@ -337,6 +346,9 @@ void run_mass_normalise(Handle &h);
 void run_ropt(Handle &h);
 bool run_m2l_lattice(Handle &h, M2LList &irr);
 void run_lattice_mscale(Handle &h, hipStream_t st);
+// Target tiles of the lattice contraction for the current tree.
+void run_lattice_tiles(Handle &h, hipStream_t st);
+int lattice_offsets_used(Handle &h);
 bool updown_mfma_enabled(const Handle &h);
 bool lattice_applies(const Handle &h);
 void run_m2m_level_mfma(Handle &h, const int *cells, int cnt, hipStream_t st);

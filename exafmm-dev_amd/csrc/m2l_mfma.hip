@@ -105,33 +105,69 @@ struct MfmaAcc<float> {
 };
 
 // ---------------------------------------------------------------------------
-// Pair classification: key of the lattice offset, or -1 (ptgt: the target
-// cell of every CSR entry).
-__global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restrict__ src,
-                               const unsigned char *__restrict__ img, int64_t np, const double4 *__restrict__ cX,
-                               const double *__restrict__ cRb, int *__restrict__ pkey, int *__restrict__ hist) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= np) return;
-  const int t = ptgt[e], s = src[e];
-  int key = -1;
+// What the set-up kernels leave for the host and for the contraction.
+struct LatState {
+  int unknown;  // pairs with an offset that the table does not know yet: nothing of this set-up is used
+  int nirr;     // irregular pairs
+  int nsteps;   // (tile, offset) steps
+  int ntiles;   // tiles with steps
+};
+
+// Key of the lattice offset of target t and source s (image im), or -1.
+__device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ cX, const double *__restrict__ cRb) {
   // Same level or one level apart: then the offset's residue mod 4 fixes
   // the level relation (0: same, 2: source one up, odd: source one down).
   const double rt = cRb[t], rs = cRb[s];
-  if (img[e] == 13 && (rs == rt || rs == 2 * rt || 2 * rs == rt)) {
-    // Offsets in units of u = 2 R_t / kLatUnit; the lattice values are whole
-    // numbers to far better than the 1e-6 test below.
-    const double iu = kLatUnit / (2 * rt);
-    const double4 a = cX[t], b = cX[s];
-    const double dx = (a.x - b.x) * iu, dy = (a.y - b.y) * iu, dz = (a.z - b.z) * iu;
-    const double rx = rint(dx), ry = rint(dy), rz = rint(dz);
-    if (fabs(dx - rx) < 1e-6 && fabs(dy - ry) < 1e-6 && fabs(dz - rz) < 1e-6 && fabs(rx) <= kLatD &&
-        fabs(ry) <= kLatD && fabs(rz) <= kLatD)
-      key = (((int)rx + kLatD) * kLatSide + ((int)ry + kLatD)) * kLatSide + ((int)rz + kLatD);
+  if (im != 13 || !(rs == rt || rs == 2 * rt || 2 * rs == rt)) return -1;
+  // Offsets in units of u = 2 R_t / kLatUnit; the lattice values are whole
+  // numbers to far better than the 1e-6 test below.
+  const double iu = kLatUnit / (2 * rt);
+  const double4 a = cX[t], b = cX[s];
+  const double dx = (a.x - b.x) * iu, dy = (a.y - b.y) * iu, dz = (a.z - b.z) * iu;
+  const double rx = rint(dx), ry = rint(dy), rz = rint(dz);
+  if (fabs(dx - rx) < 1e-6 && fabs(dy - ry) < 1e-6 && fabs(dz - rz) < 1e-6 && fabs(rx) <= kLatD &&
+      fabs(ry) <= kLatD && fabs(rz) <= kLatD)
+    return (((int)rx + kLatD) * kLatSide + ((int)ry + kLatD)) * kLatSide + ((int)rz + kLatD);
+  return -1;
+}
+
+// Every M2L pair's step, tile * noff + o (o: number of its offset among the
+// noff known ones), into pstep, -1 for a pair that is not on the lattice (or
+// whose target is in no tile); act flags the steps in use.  A pair with an
+// unknown offset flags it in hist and makes the set-up unusable.  (A fixed grid
+// and one atomic per workgroup for the irregular count: one per wave took 500 us
+// in a periodic list of 11 M pairs, a fifth of them irregular.)
+__global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restrict__ src,
+                               const unsigned char *__restrict__ img, int64_t np, const double4 *__restrict__ cX,
+                               const double *__restrict__ cRb, const int *__restrict__ o_of_key,
+                               const int *__restrict__ tile_of, int noff, unsigned char *__restrict__ act,
+                               int *__restrict__ pstep, unsigned char *__restrict__ hist, LatState *__restrict__ st) {
+  __shared__ int sn;
+  if (threadIdx.x == 0) sn = 0;
+  __syncthreads();
+  int nirr = 0;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < np; e += (int64_t)gridDim.x * blockDim.x) {
+    const int t = ptgt[e];
+    const int key = lat_key(t, src[e], img[e], cX, cRb);
+    const int tile = tile_of[t];
+    int v = -1;
+    if (key >= 0 && tile >= 0) {
+      const int o = o_of_key[key];
+      if (o < 0) {
+        // A read first, so that the many pairs of one offset do not all store.
+        if (!hist[key]) hist[key] = 1;
+        if (!st->unknown) st->unknown = 1;
+      } else {
+        v = tile * noff + o;
+        act[v] = 1;
+      }
+    }
+    pstep[e] = v;
+    nirr += v < 0;
   }
-  pkey[e] = key;
-  // Presence flag (no counting): a read first, so the many pairs of a
-  // common offset do not all store to one address.
-  if (key >= 0 && hist[key] == 0) hist[key] = 1;
+  if (nirr) atomicAdd(&sn, nirr);
+  __syncthreads();
+  if (threadIdx.x == 0 && sn) atomicAdd(&st->nirr, sn);
 }
 
 // T(d) rows in memory and LDS: TE entries padded to whole 1 KiB chunks (one
@@ -212,9 +248,8 @@ __global__ void __launch_bounds__(64) k_lat_tmat(const int *__restrict__ okey, R
   for (int i = S::NBLK * 64 + lane; i < TPad<P, R>::TEP; i += 64) T[(size_t)o * TPad<P, R>::TEP + i] = 0;
 }
 
-// Target tiles: cells with M2L pairs grouped by (level, octant), and inside
-// a group ordered by face class, then cell order (a radix sort keeps cell
-// order among equal keys).  The face class is the six distances of the cell
+// Target tiles: cells grouped by (level, octant), and inside a group ordered
+// by face class, then cell order.  The face class is the six distances of the cell
 // to the faces of its level's grid, each clipped at kTileK: cells near the
 // domain boundary lack the offsets that point outside it, and cells of one
 // class lack the same ones, so tiles cut from class-ordered cells have
@@ -225,7 +260,7 @@ constexpr int kTileClassBits = 14;  // (kTileK + 1)^6 = 15625 classes
 static_assert((kTileK + 1) * (kTileK + 1) * (kTileK + 1) * (kTileK + 1) * (kTileK + 1) * (kTileK + 1) <=
                   (1 << kTileClassBits),
               "face classes fit their key bits");
-constexpr int kTileNoGroup = 255 << kTileClassBits;  // cells without pairs sort last
+constexpr int kTileNoGroup = 255 << kTileClassBits;  // cells in no group sort last
 
 // Face class of the cell whose Morton index on its level's grid is kk
 // (coordinate bits interleaved x, y, z from bit 0).
@@ -242,153 +277,270 @@ __device__ inline int face_class(uint64_t kk, int l) {
   return cls;
 }
 
-__global__ void k_tile_key(int nc, const int *__restrict__ has, const int *__restrict__ lvl,
-                           const uint64_t *__restrict__ ckey, bool key_lvloff, int *__restrict__ key,
-                           int *__restrict__ val) {
+// Tile slots are laid out by what the tree can hold, so that no count has to
+// reach the host: a level's octant group has at most one cell per parent (the
+// builders leave their number), and level l gets 8 ceil(parents / 64) slots
+// from base[l] on, chunk q of octant o at base[l] + 8 q + o (consecutive
+// tiles cover one region of space).  Slots without cells are skipped later.
+constexpr int kTileLevels = 32;  // deeper cells are in no tile (their pairs go per pair)
+struct TileLevels {
+  int nlevels;
+  int off[kTileLevels + 1];   // cells of level l: lvl_cells[off[l] .. off[l + 1])
+  int cap[kTileLevels + 1];   // most cells of one octant
+  int base[kTileLevels + 1];  // first tile slot of level l
+};
+
+// What cKey adds to the Morton index of a level's cells.
+__device__ inline uint64_t level_offset(int l, bool key_lvloff) {
+  return key_lvloff ? ((1ull << (3 * l)) - 1) / 7 : 0;
+}
+
+// One workgroup per (octant, level): its cells in cell order, sorted by class
+// in LDS.  For groups of up to kTileSort cells; the class and the cell's place
+// in its level share a word.  (One launch for all levels, beside the
+// traversal; the radix sort of all cells, about 10 launches and 60 us of the
+// main stream at 4700 cells, stays for larger levels.)
+constexpr int kTileSort = 4096;
+constexpr int kTilePosBits = 15;  // 8 kTileSort places
+static_assert(kTileClassBits + kTilePosBits < 32 && 8 * kTileSort <= (1 << kTilePosBits), "sort words");
+__global__ void __launch_bounds__(1024)
+    k_tiles(TileLevels tl, const int *__restrict__ lvl_cells, const uint64_t *__restrict__ ckey, bool key_lvloff,
+            int *__restrict__ tile_tgt, int *__restrict__ tile_of, int *__restrict__ col_of) {
+  extern __shared__ unsigned skey[];
+  __shared__ int swave[17];
+  const int oct = blockIdx.x, l = blockIdx.y + 1, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int *cells = lvl_cells + tl.off[l];
+  const uint64_t lvloff = level_offset(l, key_lvloff);
+  const int nl = tl.off[l + 1] - tl.off[l], cap = tl.cap[l];
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = tid; i < tl.off[1]; i += 1024) tile_of[lvl_cells[i]] = -1;  // roots
+  int m = 0;
+  for (int b = 0; b < nl; b += 1024) {
+    const int i = b + tid;
+    uint64_t kk = 0;
+    if (i < nl) kk = ckey[cells[i]] - lvloff;
+    const int o = i < nl ? (int)(kk & 7) : -1;
+    const unsigned long long in = __ballot(o == oct);
+    __syncthreads();
+    if (lane == 0) swave[wave] = (int)__popcll(in);
+    __syncthreads();
+    int before = m;
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) before += swave[w];
+      m += swave[w];
+    }
+    before += (int)__popcll(in & ((1ull << lane) - 1));
+    if (o == oct && before < cap)
+      skey[before] = ((unsigned)face_class(kk, l) << kTilePosBits) | (unsigned)i;
+    else if (o == oct)
+      tile_of[cells[i]] = -1;
+  }
+  m = min(m, cap);
+  int p2 = 1;
+  while (p2 < m) p2 *= 2;
+  for (int i = m + tid; i < p2; i += 1024) skey[i] = ~0u;
+  __syncthreads();
+  for (int k = 2; k <= p2; k *= 2)
+    for (int j = k / 2; j > 0; j /= 2) {
+      for (int i = tid; i < p2; i += 1024) {
+        const int x = i ^ j;
+        if (x > i) {
+          const unsigned u = skey[i], v = skey[x];
+          if ((u > v) == ((i & k) == 0)) {
+            skey[i] = v;
+            skey[x] = u;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  const int nslot = 8 * (tl.base[l + 1] - tl.base[l]);  // columns of this octant's slots
+  for (int r = tid; r < nslot; r += 1024) {
+    const int t = tl.base[l] + (r / 64) * 8 + oct, col = r % 64;
+    int c = -1;
+    if (r < m) {
+      c = cells[skey[r] & ((1u << kTilePosBits) - 1)];
+      tile_of[c] = t;
+      col_of[c] = col;
+    }
+    tile_tgt[t * 64 + col] = c;
+  }
+}
+
+// The same by a radix sort over all cells, keys (level, octant, class).
+__global__ void k_tile_key(int nc, const int *__restrict__ lvl, const uint64_t *__restrict__ ckey, bool key_lvloff,
+                           int *__restrict__ key, int *__restrict__ val) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nc) return;
   int k = kTileNoGroup;
   const int l = lvl[c];
-  if (has[c] && l > 0 && l < 31) {
-    const uint64_t lvloff = key_lvloff ? ((1ull << (3 * l)) - 1) / 7 : 0;
-    const uint64_t kk = ckey[c] - lvloff;
+  if (l > 0 && l < kTileLevels - 1) {
+    const uint64_t kk = ckey[c] - level_offset(l, key_lvloff);
     k = ((l * 8 + (int)(kk & 7)) << kTileClassBits) | face_class(kk, l);
   }
   key[c] = k;
   val[c] = c;
 }
 
-// has[t] = 1 for every target t of the M2L list (plain stores of 1).
-__global__ void k_mark_has(const int *__restrict__ tgt, int64_t np, int *__restrict__ has) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < np) has[tgt[e]] = 1;
-}
-
-// Group sizes from the sorted keys: hist[g] = end - start of group g.
-__global__ void k_tile_hist(int nc, const int *__restrict__ key, int *__restrict__ hist) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nc) return;
-  const int k = key[p] >> kTileClassBits;
-  if (k >= 255) return;
-  if (p == 0 || key[p - 1] >> kTileClassBits != k) atomicSub(&hist[k], p);  // one start per group
-  if (p == nc - 1 || key[p + 1] >> kTileClassBits != k) atomicAdd(&hist[k], p + 1);  // one end per group
-}
-
-// gb[0..255] = group start in sorted order, gb[256..511] = first chunk of
-// the group; tmap[chunk] = tile number (chunks of the 8 octant groups of a
-// level interleaved, so consecutive tiles cover one region of space).
-__global__ void k_tile_assign(int nc, const int *__restrict__ skey, const int *__restrict__ sval,
-                              const int *__restrict__ gb, const int *__restrict__ tmap, int *__restrict__ tile_tgt,
-                              int *__restrict__ tile_of, int *__restrict__ col_of) {
+__global__ void k_tile_assign(int nc, TileLevels tl, const int *__restrict__ skey, const int *__restrict__ sval,
+                              int *__restrict__ tile_tgt, int *__restrict__ tile_of, int *__restrict__ col_of) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nc) return;
   const int g = skey[p] >> kTileClassBits, c = sval[p];
-  if (g >= 255) {
+  if (g >= (kTileNoGroup >> kTileClassBits)) {
     tile_of[c] = -1;
     return;
   }
-  const int r = p - gb[g];
-  const int t = tmap[gb[256 + g] + r / 64], col = r % 64;
+  int lo = 0, hi = p;  // first entry of the group
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((skey[mid] >> kTileClassBits) < g)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  const int r = p - lo, t = tl.base[g >> 3] + (r / 64) * 8 + (g & 7), col = r % 64;
   tile_tgt[t * 64 + col] = c;
   tile_of[c] = t;
   col_of[c] = col;
 }
 
-// Mark the (tile, offset) steps that have at least one pair; pstep[e] = the
-// pair's step tile * noff + o, or -1 (not a lattice pair).
-__global__ void k_lat_mark(const int *__restrict__ ptgt, int64_t np, const int *__restrict__ pkey,
-                           const int *__restrict__ o_of_key, const int *__restrict__ tile_of, int noff,
-                           int *__restrict__ act, int *__restrict__ pstep) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= np) return;
-  int v = -1;
-  const int key = pkey[e];
-  const int o = key >= 0 ? o_of_key[key] : -1;
-  if (o >= 0) {
-    const int tile = tile_of[ptgt[e]];
-    if (tile >= 0) {
-      v = tile * noff + o;
-      act[v] = 1;
+// Steps per tile: the flags of its row of act.
+__global__ void __launch_bounds__(256)
+    k_lat_count(const unsigned char *__restrict__ act, int noff, int *__restrict__ cnt) {
+  __shared__ int sw[4];
+  const unsigned char *a = act + (size_t)blockIdx.x * noff;
+  int n = 0;
+  for (int o = threadIdx.x; o < noff; o += 256) n += a[o];
+  for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
+  if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) cnt[blockIdx.x] = sw[0] + sw[1] + sw[2] + sw[3];
+}
+
+// The tile's steps, in offset order, from step0[tile] = the counts of the
+// tiles before it: aidx[tile * noff + o] = step, alist[step] = the offset's T
+// row; their slots are emptied.
+__global__ void __launch_bounds__(256)
+    k_lat_steps(const unsigned char *__restrict__ act, const int *__restrict__ cnt, int noff,
+                const int *__restrict__ orow, int *__restrict__ aidx, int *__restrict__ step0,
+                int *__restrict__ alist, int4 *__restrict__ slot, LatState *__restrict__ st) {
+  __shared__ int sw[4], sn[4];
+  const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int base = 0, full = 0;
+  for (int t = tid; t < tile; t += 256) {
+    const int c = cnt[t];
+    base += c;
+    full += c > 0;
+  }
+  for (int d = 32; d >= 1; d >>= 1) {
+    base += __shfl_xor(base, d);
+    full += __shfl_xor(full, d);
+  }
+  if (lane == 0) {
+    sw[wave] = base;
+    sn[wave] = full;
+  }
+  __syncthreads();
+  base = sw[0] + sw[1] + sw[2] + sw[3];
+  const int mine = cnt[tile];
+  if (tid == 0) {
+    step0[tile] = base;
+    if (tile == (int)gridDim.x - 1) {
+      step0[tile + 1] = base + mine;
+      st->nsteps = base + mine;
+      st->ntiles = sn[0] + sn[1] + sn[2] + sn[3] + (mine > 0);
     }
   }
-  pstep[e] = v;
-}
-
-// Compact step list: alist[k] = offset of step k (steps of a tile in offset order).
-// Active step i = (tile, offset o): its T row, row_of_key[okey[o]].
-__global__ void k_lat_alist(const int *__restrict__ act, const int *__restrict__ aidx, int64_t n, int noff,
-                            const int *__restrict__ okey, const int *__restrict__ row_of_key, int *__restrict__ alist) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && act[i]) alist[aidx[i]] = row_of_key[okey[i % noff]];
-}
-
-// Lattice pairs and their (step, column) slots, in two passes of plain
-// stores: (1) each lattice pair's slot aidx[step] * 64 + column (kept in
-// pslot[e]) takes the pair's index; (2) a pair whose slot holds another
-// index (a repeated source: same target and offset) and every non-lattice
-// pair is irregular, counted per wave into *nirr, and the pair a slot holds
-// writes its source cell s there as -2 - s (never equal to a pair index, so
-// the comparisons of other pairs stay right in any order).  Slots left at -1
-// are empty columns.
-__global__ void k_lat_slots(const int *__restrict__ ptgt, int64_t np, const int *__restrict__ col_of,
-                            const int *__restrict__ aidx, int *__restrict__ pslot, int *__restrict__ slot) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= np) return;
-  const int v = pslot[e];  // the step, from k_lat_mark
-  if (v < 0) return;
-  const int k = aidx[v] * 64 + col_of[ptgt[e]];
-  pslot[e] = k;
-  slot[k] = (int)e;
-}
-
-__global__ void k_lat_check(int64_t np, const int *__restrict__ pslot, const int *__restrict__ src,
-                            int *__restrict__ slot, int *__restrict__ irr, int *__restrict__ nirr) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool ir = false;
-  if (e < np) {
-    const int k = pslot[e];
-    ir = k < 0 || slot[k] != (int)e;
-    if (!ir) slot[k] = -2 - src[e];
-    irr[e] = ir ? 1 : 0;
+  if (mine == 0) return;
+  for (int i = tid; i < mine * 16; i += 256) slot[(size_t)base * 16 + i] = make_int4(-1, -1, -1, -1);
+  for (int b = 0; b < noff; b += 256) {
+    const int o = b + tid;
+    const bool in = o < noff && act[(size_t)tile * noff + o];
+    const unsigned long long m = __ballot(in);
+    __syncthreads();
+    if (lane == 0) sw[wave] = (int)__popcll(m);
+    __syncthreads();
+    int k = base + (int)__popcll(m & ((1ull << lane) - 1));
+    for (int w = 0; w < 4; w++) {
+      if (w < wave) k += sw[w];
+      base += sw[w];
+    }
+    if (in) {
+      aidx[(size_t)tile * noff + o] = k;
+      alist[k] = orow[o];
+    }
   }
-  const unsigned long long m = __ballot(ir);
-  if (m && (threadIdx.x & 63) == __ffsll((long long)m) - 1) atomicAdd(nirr, (int)__popcll(m));
 }
 
-// v into p[0 .. 64 * (*nsteps)) (the step count is on the device).
-__global__ void k_fill_slots(int *__restrict__ p, const int *__restrict__ nsteps, int v) {
-  const int64_t n = (int64_t)*nsteps * 64;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = v;
+// Every lattice pair's source cell s into its (step, column) slot, as -2 - s.
+// No two pairs share a slot: the traversal visits a pair of cells once, the
+// key fixes the source's level and position, and cells of one level differ in
+// position.  That holds for bounds that enclose the bodies; with bounds from
+// the caller (CHECK) a taken slot makes the later pair irregular.  (The
+// exchange costs more than the store: 250 against 95 us for 6.7 M pairs.)
+template <bool CHECK>
+__global__ void k_lat_slots(const int *__restrict__ ptgt, const int *__restrict__ src, int64_t np,
+                            const int *__restrict__ col_of, const int *__restrict__ aidx, int *__restrict__ pstep,
+                            int *__restrict__ slot, LatState *__restrict__ st) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= np || st->unknown) return;
+  const int v = pstep[e];
+  if (v < 0) return;
+  int *p = &slot[aidx[v] * 64 + col_of[ptgt[e]]];
+  const int w = -2 - src[e];
+  if (!CHECK) {
+    *p = w;
+  } else if (atomicCAS(p, -1, w) != -1) {
+    pstep[e] = -1;
+    atomicAdd(&st->nirr, 1);
+  }
 }
 
-// Offsets present in the list (numbered in key order), and those of them
-// with no row in the T table yet.
-__global__ void k_lat_flag(const int *__restrict__ hist, const int *__restrict__ row_of_key, int n,
-                           int *__restrict__ flag, int *__restrict__ nflag) {
+__global__ void k_irr_flag(const int *__restrict__ pstep, int64_t np, int *__restrict__ irr) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e <= np) irr[e] = e < np && pstep[e] < 0 ? 1 : 0;
+}
+
+// Offsets known after this set-up (the known ones and those hist flags, to
+// be numbered in key order), and those of them with no row in the T table.
+__global__ void k_lat_flag(const unsigned char *__restrict__ hist, const int *__restrict__ o_of_key,
+                           const int *__restrict__ row_of_key, int n, int *__restrict__ flag,
+                           int *__restrict__ nflag) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k > n) return;
-  const bool used = k < n && hist[k] != 0;
+  const bool used = k < n && (hist[k] || o_of_key[k] >= 0);
   flag[k] = used ? 1 : 0;
   nflag[k] = used && row_of_key[k] < 0 ? 1 : 0;
 }
 
-// New rows base + scan[k] of the T table for the flagged keys.
-__global__ void k_tc_assign(const int *__restrict__ nflag, const int *__restrict__ scan, int n, int base,
-                            int *__restrict__ row_of_key, int *__restrict__ keys) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n && nflag[k]) {
-    row_of_key[k] = base + scan[k];
-    keys[scan[k]] = k;
-  }
-}
-
-__global__ void k_lat_number(const int *__restrict__ flag, const int *__restrict__ scan, int n,
-                             int *__restrict__ o_of_key, int *__restrict__ okey) {
+// Numbers the flagged offsets (o_of_key, orow: number -> T row), gives the
+// new ones the rows from `base` on and clears hist.
+__global__ void k_lat_number(const int *__restrict__ flag, const int *__restrict__ scan,
+                             const int *__restrict__ nflag, const int *__restrict__ nscan, int n, int base,
+                             int *__restrict__ row_of_key, int *__restrict__ keys, int *__restrict__ o_of_key,
+                             int *__restrict__ orow, unsigned char *__restrict__ hist) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  o_of_key[k] = flag[k] ? scan[k] : -1;
-  if (flag[k]) okey[scan[k]] = k;
+  hist[k] = 0;
+  if (!flag[k]) return;
+  int row = row_of_key[k];
+  if (nflag[k]) {
+    row = base + nscan[k];
+    row_of_key[k] = row;
+    keys[nscan[k]] = k;
+  }
+  o_of_key[k] = scan[k];
+  orow[scan[k]] = row;
+}
+
+// Offsets in use: flags of any tile.
+__global__ void k_lat_used(const unsigned char *__restrict__ act, int ntiles, int noff, int *__restrict__ count) {
+  const int o = blockIdx.x * blockDim.x + threadIdx.x;
+  bool u = false;
+  for (int t = 0; o < noff && t < ntiles && !u; t++) u = act[(size_t)t * noff + o];
+  const unsigned long long m = __ballot(u);
+  if (m && (threadIdx.x & 63) == 0) atomicAdd(count, (int)__popcll(m));
 }
 
 __global__ void k_fill_int(int *__restrict__ p, int64_t n, int v) {
@@ -396,7 +548,6 @@ __global__ void k_fill_int(int *__restrict__ p, int64_t n, int v) {
   if (i < n) p[i] = v;
 }
 
-// CSR of the irregular pairs: offsets from the exclusive scan of the flags.
 // The irregular pairs (irr[e] = 1) in emission order.
 __global__ void k_irr_compact(const int *__restrict__ irr, const int *__restrict__ scan, int64_t np,
                               const int *__restrict__ tgt, const int *__restrict__ src,
@@ -441,9 +592,8 @@ __global__ void __launch_bounds__(256)
 // 8 XCDs), so an XCD only ever needs the T(d) of one eighth of the offsets
 // and keeps them in its L2.
 constexpr int kLatSeg = 8;
-// Words of Handle::hpin the lattice set-up reads back.
-constexpr int kPinGhist = 64, kPinNoff = 64 + 256, kPinNnew = 64 + 257, kPinSteps = 64 + 258;
-static_assert(kPinSteps < Handle::kPinWords, "pinned words");
+// Words of Handle::hpin the lattice set-up reads back (LatState; registration counts).
+constexpr int kPinLat = 64, kPinNoff = 64 + 8, kPinNnew = 64 + 9;
 
 typedef __attribute__((address_space(3))) void lds_void;
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt left alone.
@@ -466,7 +616,7 @@ template <int P, typename R>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 10 ? 2 : 1, 2)))
     k_m2l_mfma(int nc, int nitems, const int *__restrict__ step0, const int *__restrict__ alist,
                const int *__restrict__ slot, const R *__restrict__ T, const R *__restrict__ Ms,
-               double *__restrict__ part) {
+               double *__restrict__ part, const LatState *__restrict__ st) {
   using S = MfmaShape<P>;
   using A = MfmaAcc<R>;
   using TP = TPad<P, R>;
@@ -478,6 +628,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 1
   __shared__ __attribute__((aligned(16))) R sT0[TEP];
   __shared__ __attribute__((aligned(16))) R sT1[TEP];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (st->unknown) return;  // the set-up is redone
   // Items (tile, segment) = (item / 8, item % 8); a grid that is a multiple
   // of 8 keeps every item of a segment on one XCD.
   for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
@@ -485,6 +636,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 1
     const int col = wave * 16 + (lane & 15);
     const int kq = lane >> 4;
     const int a0 = step0[tile], a1 = step0[tile + 1];
+    if (a0 == a1) continue;  // a tile without steps
     const int i0 = a0 + (a1 - a0) * seg / kLatSeg, i1 = a0 + (a1 - a0) * (seg + 1) / kLatSeg;
     typename A::type acc[RB];
     v4d acc64[F32 ? RB : 1];
@@ -576,12 +728,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 1
 // of a tile share a level, not necessarily a size: batched systems).
 template <int P>
 __global__ void __launch_bounds__(256)
-    k_lat_reduce(const int *__restrict__ tile_tgt, const double *__restrict__ cRb, const double *__restrict__ part,
-                 cplx *__restrict__ L) {
+    k_lat_reduce(const int *__restrict__ tile_tgt, const int *__restrict__ step0, const double *__restrict__ cRb,
+                 const double *__restrict__ part, cplx *__restrict__ L, const LatState *__restrict__ st) {
   using S = MfmaShape<P>;
   constexpr int NR = S::NR, NRP = S::RB * 16;
   constexpr DegreeTable<P> deg{};
   const int tile = blockIdx.x;
+  if (st->unknown || step0[tile] == step0[tile + 1]) return;
   double *Lr = reinterpret_cast<double *>(L);
   // Rows r0 .. r0 + 15 of the tile: the segment sums read column-fastest
   // (as the partials lie), then written row-fastest through LDS (the 16 rows
@@ -631,14 +784,16 @@ static void mscale_impl(Handle &h, hipStream_t st) {
 // Largest slot array sized by the all-steps-active bound (512 MB of int).
 constexpr int64_t kSlotBound = (int64_t)1 << 27;
 
-// An empty T table for expansion order P in FP32 or FP64.
+// An empty T table for expansion order P in FP32 or FP64, no offset known.
 static void tc_reset(Handle &h, int P, bool f32) {
   h.lat_tc_map.resize(kLatKeys + 1);
-  h.lat_tc_flag.resize(kLatKeys + 1);
-  h.lat_tc_scan.resize(kLatKeys + 1);
-  hipLaunchKernelGGL(k_fill_int, dim3(div_up(kLatKeys + 1, 256)), dim3(256), 0, h.stream, h.lat_tc_map.p,
-                     (int64_t)kLatKeys + 1, -1);
-  h.lat_tc_rows = 0;
+  h.lat_ookey.resize(kLatKeys + 1);
+  h.lat_hist.resize(kLatKeys + 8);
+  for (int *p : {h.lat_tc_map.p, h.lat_ookey.p})
+    hipLaunchKernelGGL(k_fill_int, dim3(div_up(kLatKeys + 1, 256)), dim3(256), 0, h.stream, p, (int64_t)kLatKeys + 1,
+                       -1);
+  zero_device(h.lat_hist.p, kLatKeys + 7, h.stream);
+  h.lat_tc_rows = h.lat_noff = 0;
   h.lat_tc_P = P;
   h.lat_tc_f32 = f32;
 }
@@ -659,6 +814,8 @@ static void grow_keep_rows(Handle &h, DBuf<R> &b, size_t want, size_t keep) {
   nb.cap = 0;
 }
 
+static LatState *lat_state(Handle &h) { return reinterpret_cast<LatState *>(h.lat_act.p); }
+
 // The contraction and the reduction of the last lattice set-up (its step
 // lists, slots and tiles), on the main stream.
 template <int P>
@@ -666,113 +823,140 @@ static void lattice_contract(Handle &h) {
   const int nitems = h.lat_run_ntiles * kLatSeg;
   if (h.cfg.precision == 1)
     hipLaunchKernelGGL((k_m2l_mfma<P, float>), dim3(h.lat_run_ngrid), dim3(256), 0, h.stream, h.ncells, nitems,
-                       h.lat_step0.p, h.lat_alist.p, h.lat_slot.p, h.lat_Tf.p, h.lat_Msf.p, h.lat_part.p);
+                       h.lat_step0.p, h.lat_alist.p, h.lat_slot.p, h.lat_Tf.p, h.lat_Msf.p, h.lat_part.p, lat_state(h));
   else
     hipLaunchKernelGGL((k_m2l_mfma<P, double>), dim3(h.lat_run_ngrid), dim3(256), 0, h.stream, h.ncells, nitems,
-                       h.lat_step0.p, h.lat_alist.p, h.lat_slot.p, h.lat_T.p, h.lat_Ms.p, h.lat_part.p);
+                       h.lat_step0.p, h.lat_alist.p, h.lat_slot.p, h.lat_T.p, h.lat_Ms.p, h.lat_part.p, lat_state(h));
   EXA_HIP(hipGetLastError());
 }
 
 template <int P>
 static void lattice_reduce(Handle &h) {
   hipLaunchKernelGGL(k_lat_reduce<P>, dim3(h.lat_run_ntiles, MfmaShape<P>::RB), dim3(256), 0, h.stream,
-                     h.lat_tile_tgt.p, h.cRb.p, h.lat_part.p, h.L.p);
+                     h.lat_tile_tgt.p, h.lat_step0.p, h.cRb.p, h.lat_part.p, h.L.p, lat_state(h));
   EXA_HIP(hipGetLastError());
 }
 
-template <int P>
-static void lattice_begin(Handle &h) {
-  const int nc = h.ncells;
-  const int64_t np = h.nm2l;
-  const int TPB = 256;
-  const int gp = div_up(np, TPB);
-  const bool f32 = h.cfg.precision == 1;
-  // 0. Source multipoles scaled per cell (independent of the pair lists;
-  // already queued behind the multipoles when the upward pass was split).
-  if (!h.lat_ms_ready) mscale_impl<P>(h, h.stream);
-  h.lat_ms_ready = false;
-  // 1. Classify pairs (offset key, target cell) and flag the offsets used.
-  // The raw (emission-order) M2L list: target, source, image per pair.
-  const int *ptgt = h.raw_mi.p, *psrc = h.raw_mj.p;
-  const unsigned char *pimg = h.raw_mimg.p;
-  h.lat_pkey.resize(np > 0 ? np : 1);
-  h.lat_hist.resize(kLatKeys);
-  hipLaunchKernelGGL(k_fill_int, dim3(div_up(kLatKeys, TPB)), dim3(TPB), 0, h.stream, h.lat_hist.p, (int64_t)kLatKeys,
-                     0);
-  hipLaunchKernelGGL(k_lat_classify, dim3(gp), dim3(TPB), 0, h.stream, ptgt, psrc, pimg, np,
-                     h.cX.p, h.cRb.p, h.lat_pkey.p, h.lat_hist.p);
-  // 2. Offsets present, numbered in key order; offsets without a T row.
-  if (h.lat_tc_P != P || h.lat_tc_f32 != f32) tc_reset(h, P, f32);
-  h.lat_flag.resize(kLatKeys + 1);
-  h.lat_kscan.resize(kLatKeys + 1);
-  h.lat_ookey.resize(kLatKeys);
-  h.lat_okey.resize(kLatKeys);
-  hipLaunchKernelGGL(k_lat_flag, dim3(div_up(kLatKeys + 1, TPB)), dim3(TPB), 0, h.stream, h.lat_hist.p,
-                     h.lat_tc_map.p, kLatKeys, h.lat_flag.p, h.lat_tc_flag.p);
-  exclusive_scan_int(h, h.lat_flag.p, h.lat_kscan.p, kLatKeys + 1);
-  exclusive_scan_int(h, h.lat_tc_flag.p, h.lat_tc_scan.p, kLatKeys + 1);
-  hipLaunchKernelGGL(k_lat_number, dim3(div_up(kLatKeys, TPB)), dim3(TPB), 0, h.stream, h.lat_flag.p, h.lat_kscan.p,
-                     kLatKeys, h.lat_ookey.p, h.lat_okey.p);
-  // 3. Target tiles of one level and one octant (face class, then cell order).
-  h.lat_tkey.resize(2 * (size_t)nc);
-  h.lat_tval.resize(2 * (size_t)nc);
-  h.lat_thist.resize(256);
-  int *tk = h.lat_tkey.p, *tv = h.lat_tval.p;
-  h.lat_has.resize(nc);
-  hipLaunchKernelGGL(k_fill_int, dim3(div_up(nc, TPB)), dim3(TPB), 0, h.stream, h.lat_has.p, (int64_t)nc, 0);
-  hipLaunchKernelGGL(k_mark_has, dim3(gp), dim3(TPB), 0, h.stream, ptgt, np, h.lat_has.p);
-  hipLaunchKernelGGL(k_tile_key, dim3(div_up(nc, TPB)), dim3(TPB), 0, h.stream, nc, h.lat_has.p, h.cLevel.p, h.cKey.p,
-                     h.key_lvloff, tk, tv);
-  bool alt = false;
-  sort_pairs_int_int(h, tk, tk + nc, tv, tv + nc, nc, 8 + kTileClassBits, alt);
-  h.lat_tile_alt = alt;
-  const int *skey = alt ? tk + nc : tk;
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, h.stream, h.lat_thist.p, (int64_t)256, 0);
-  hipLaunchKernelGGL(k_tile_hist, dim3(div_up(nc, TPB)), dim3(TPB), 0, h.stream, nc, skey, h.lat_thist.p);
-  // Tile histogram, offset count and new-row count for the host (read by
-  // lattice_run after the main stream has passed these copies).
-  EXA_HIP(hipMemcpyAsync(h.hpin + kPinGhist, h.lat_thist.p, 256 * sizeof(int), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipMemcpyAsync(h.hpin + kPinNoff, h.lat_kscan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipMemcpyAsync(h.hpin + kPinNnew, h.lat_tc_scan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost,
-                         h.stream));
-  h.lat_begun = true;
+// Target tiles of the current tree, on stream st (its own scratch: this runs
+// beside the traversal).
+void run_lattice_tiles(Handle &h, hipStream_t st) {
+  if (!lattice_applies(h)) return;
+  const int nc = h.ncells, TPB = 256;
+  TileLevels tl{};
+  int base = 0, most = 0;
+  tl.nlevels = std::min(h.nlevels, kTileLevels - 1);
+  for (int l = 0; l <= kTileLevels; l++) {
+    tl.off[l] = h.lvl_off[std::min(l, h.nlevels)];
+    tl.base[l] = base;
+    if (l == 0 || l >= tl.nlevels) continue;
+    const int group = std::min(h.lvl_par[l - 1], h.lvl_off[l + 1] - h.lvl_off[l]);
+    tl.cap[l] = group;
+    most = std::max(most, group);
+    base += 8 * div_up(group, 64);
+  }
+  h.lat_ntiles = base;
+  h.lat_tile_of.resize(nc);
+  h.lat_col_of.resize(nc);
+  h.lat_tile_tgt.resize((size_t)std::max(1, base) * 64);
+  if (base == 0) {
+    hipLaunchKernelGGL(k_fill_int, dim3(div_up(nc, TPB)), dim3(TPB), 0, st, h.lat_tile_of.p, (int64_t)nc, -1);
+  } else if (most <= kTileSort && h.nlevels < kTileLevels) {
+    int p2 = 1;
+    while (p2 < most) p2 *= 2;
+    hipLaunchKernelGGL(k_tiles, dim3(8, tl.nlevels - 1), dim3(1024), p2 * sizeof(unsigned), st, tl, h.lvl_cells.p,
+                       h.cKey.p, h.key_lvloff, h.lat_tile_tgt.p, h.lat_tile_of.p, h.lat_col_of.p);
+  } else {
+    h.lat_tkey.resize(2 * (size_t)nc);
+    h.lat_tval.resize(2 * (size_t)nc);
+    int *tk = h.lat_tkey.p, *tv = h.lat_tval.p;
+    hipLaunchKernelGGL(k_tile_key, dim3(div_up(nc, TPB)), dim3(TPB), 0, st, nc, h.cLevel.p, h.cKey.p, h.key_lvloff, tk,
+                       tv);
+    bool alt = false;
+    sort_pairs_int_int(tk, tk + nc, tv, tv + nc, nc, 8 + kTileClassBits, alt, st, h.tmp3);
+    hipLaunchKernelGGL(k_fill_int, dim3(div_up((int64_t)base * 64, TPB)), dim3(TPB), 0, st, h.lat_tile_tgt.p,
+                       (int64_t)base * 64, -1);
+    hipLaunchKernelGGL(k_tile_assign, dim3(div_up(nc, TPB)), dim3(TPB), 0, st, nc, tl, alt ? tk + nc : tk,
+                       alt ? tv + nc : tv, h.lat_tile_tgt.p, h.lat_tile_of.p, h.lat_col_of.p);
+  }
+  EXA_HIP(hipGetLastError());
 }
 
-// The rest of the lattice M2L, after lattice_begin (which the evaluation
-// queues before P2P, so the set-up's first kernels start while the P2P
-// list is grouped, before P2P fills the GPU).
-template <int P>
-static void lattice_run(Handle &h, M2LList &irr) {
-  using S = MfmaShape<P>;
-  const int nc = h.ncells;
-  const int64_t np = h.nm2l;
-  const int TPB = 256;
-  const int gp = div_up(np, TPB);
-  const bool f32 = h.cfg.precision == 1;
-  if (!h.lat_begun) lattice_begin<P>(h);
-  h.lat_begun = false;
+// Steps and slots of the current M2L list with the offsets known so far.
+// Nothing waits for the device; whether every offset was known, and how many
+// pairs are irregular, is read back behind it (ev_cnt).
+static void lattice_steps(Handle &h) {
+  const int64_t np = h.nm2l, nall = (int64_t)h.lat_ntiles * h.lat_noff;
+  const int TPB = 256, gp = div_up(np, TPB);
   const int *ptgt = h.raw_mi.p, *psrc = h.raw_mj.p;
-  const unsigned char *pimg = h.raw_mimg.p;
-  const int *tk = h.lat_tkey.p, *tv = h.lat_tval.p;
-  const int *skey = h.lat_tile_alt ? tk + nc : tk, *sval = h.lat_tile_alt ? tv + nc : tv;
-  EXA_HIP(hipStreamSynchronize(h.stream));
-  int ghist[256];
-  std::copy(h.hpin + kPinGhist, h.hpin + kPinGhist + 256, ghist);
-  const int noff = h.hpin[kPinNoff];
-  int nnew = h.hpin[kPinNnew];
-  if (h.lat_tc_rows + nnew > h.lat_tc_max) {  // start the table afresh
-    tc_reset(h, P, f32);
-    hipLaunchKernelGGL(k_lat_flag, dim3(div_up(kLatKeys + 1, TPB)), dim3(TPB), 0, h.stream, h.lat_hist.p,
-                       h.lat_tc_map.p, kLatKeys, h.lat_flag.p, h.lat_tc_flag.p);
-    exclusive_scan_int(h, h.lat_tc_flag.p, h.lat_tc_scan.p, kLatKeys + 1);
-    nnew = noff;
+  if (nall > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
+  h.lat_act.resize(sizeof(LatState) + nall + 8);
+  h.lat_aidx.resize(nall + 1);
+  h.lat_pslot.resize(np);
+  h.lat_tcnt.resize(h.lat_ntiles + 1);
+  h.lat_step0.resize(h.lat_ntiles + 1);
+  unsigned char *act = h.lat_act.p + sizeof(LatState);
+  zero_device(h.lat_act.p, sizeof(LatState) + (nall + 7) / 8 * 8, h.stream);
+  hipLaunchKernelGGL(k_lat_classify, dim3(std::min(gp, 4096)), dim3(TPB), 0, h.stream, ptgt, psrc, h.raw_mimg.p, np,
+                     h.cX.p, h.cRb.p, h.lat_ookey.p, h.lat_tile_of.p, h.lat_noff, act, h.lat_pslot.p, h.lat_hist.p,
+                     lat_state(h));
+  if (nall > 0) {
+    hipLaunchKernelGGL(k_lat_count, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_noff, h.lat_tcnt.p);
+    // Step lists sized for every (tile, offset) being in use, so that the
+    // host need not wait for the count, unless that bound is large.
+    int64_t nact = nall;
+    if (nall * 64 > kSlotBound) {
+      std::vector<int> cnt(h.lat_ntiles);
+      EXA_HIP(hipMemcpyAsync(cnt.data(), h.lat_tcnt.p, h.lat_ntiles * sizeof(int), hipMemcpyDeviceToHost, h.stream));
+      EXA_HIP(hipStreamSynchronize(h.stream));
+      nact = 0;
+      for (int c : cnt) nact += c;
+    }
+    if (nact * 64 > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
+    h.lat_alist.resize(nact > 0 ? nact : 1);
+    h.lat_slot.resize(nact > 0 ? nact * 64 : 4);
+    hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff,
+                       h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
+                       reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h));
+    hipLaunchKernelGGL(h.bounds_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
+                       psrc, np, h.lat_col_of.p, h.lat_aidx.p, h.lat_pslot.p, h.lat_slot.p, lat_state(h));
   }
-  // T(d) of the offsets not in the table yet: runs while the host lays out
-  // the tiles and steps.
+  EXA_HIP(hipMemcpyAsync(h.hpin + kPinLat, lat_state(h), sizeof(LatState), hipMemcpyDeviceToHost, h.stream));
+  EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
+  EXA_HIP(hipGetLastError());
+}
+
+// The offsets that the last lattice_steps flagged as unknown: numbers for
+// them (and new numbers for the others: in key order, so that a tile's steps
+// come in the same order whatever the table held before) and rows of T(d).
+template <int P>
+static void lattice_register(Handle &h) {
+  const int TPB = 256, gk = div_up(kLatKeys + 1, TPB);
+  const bool f32 = h.lat_tc_f32;
+  h.lat_flag.resize(kLatKeys + 1);
+  h.lat_kscan.resize(kLatKeys + 1);
+  h.lat_tc_flag.resize(kLatKeys + 1);
+  h.lat_tc_scan.resize(kLatKeys + 1);
+  for (int again = 0;; again++) {
+    hipLaunchKernelGGL(k_lat_flag, dim3(gk), dim3(TPB), 0, h.stream, h.lat_hist.p, h.lat_ookey.p, h.lat_tc_map.p,
+                       kLatKeys, h.lat_flag.p, h.lat_tc_flag.p);
+    exclusive_scan_int(h, h.lat_flag.p, h.lat_kscan.p, kLatKeys + 1);
+    exclusive_scan_int(h, h.lat_tc_flag.p, h.lat_tc_scan.p, kLatKeys + 1);
+    EXA_HIP(hipMemcpyAsync(h.hpin + kPinNoff, h.lat_kscan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost, h.stream));
+    EXA_HIP(hipMemcpyAsync(h.hpin + kPinNnew, h.lat_tc_scan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost,
+                           h.stream));
+    EXA_HIP(hipStreamSynchronize(h.stream));
+    if (again || h.lat_tc_rows == 0 || h.lat_tc_rows + h.hpin[kPinNnew] <= h.lat_tc_max) break;
+    tc_reset(h, P, f32);  // start the table afresh with this list's offsets alone
+    lattice_steps(h);
+  }
+  const int noff = h.hpin[kPinNoff], nnew = h.hpin[kPinNnew];
+  h.lat_tc_keys.resize(std::max(1, nnew));
+  h.lat_orow.resize(std::max(1, noff));
+  hipLaunchKernelGGL(k_lat_number, dim3(gk), dim3(TPB), 0, h.stream, h.lat_flag.p, h.lat_kscan.p, h.lat_tc_flag.p,
+                     h.lat_tc_scan.p, kLatKeys, h.lat_tc_rows, h.lat_tc_map.p, h.lat_tc_keys.p, h.lat_ookey.p,
+                     h.lat_orow.p, h.lat_hist.p);
+  h.lat_noff = noff;
   if (nnew > 0) {
-    h.lat_tc_keys.resize(nnew);
-    hipLaunchKernelGGL(k_tc_assign, dim3(div_up(kLatKeys, TPB)), dim3(TPB), 0, h.stream, h.lat_tc_flag.p,
-                       h.lat_tc_scan.p, kLatKeys, h.lat_tc_rows, h.lat_tc_map.p, h.lat_tc_keys.p);
     if (f32) {
       constexpr size_t TEP = TPad<P, float>::TEP;
       grow_keep_rows(h, h.lat_Tf, (size_t)(h.lat_tc_rows + nnew) * TEP, (size_t)h.lat_tc_rows * TEP);
@@ -786,129 +970,110 @@ static void lattice_run(Handle &h, M2LList &irr) {
     }
     h.lat_tc_rows += nnew;
   }
-  int gb[512], ntiles = 0, start = 0;
-  for (int g = 0; g < 256; g++) {
-    gb[g] = start;
-    gb[256 + g] = ntiles;
-    start += g < 255 ? ghist[g] : 0;
-    ntiles += g < 255 ? div_up(ghist[g], 64) : 0;
+  EXA_HIP(hipGetLastError());
+}
+
+// The set-up, queued before P2P so that it runs while the P2P list is
+// grouped, before P2P fills the GPU.
+template <int P>
+static void lattice_begin(Handle &h) {
+  const bool f32 = h.cfg.precision == 1;
+  // Source multipoles scaled per cell and the tiles (independent of the
+  // lists; already queued behind the radii when the upward pass was split).
+  if (!h.lat_ms_ready) mscale_impl<P>(h, h.stream);
+  h.lat_ms_ready = false;
+  if (h.lat_tiles_ready)
+    EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_tiles, 0));
+  else
+    run_lattice_tiles(h, h.stream);
+  h.lat_tiles_ready = false;
+  if (h.lat_tc_P != P || h.lat_tc_f32 != f32 || (int64_t)h.lat_ntiles * h.lat_noff > INT_MAX) tc_reset(h, P, f32);
+  lattice_steps(h);
+  if (h.lat_noff == 0) {  // no offset known yet: register them before P2P fills the GPU
+    EXA_HIP(hipEventSynchronize(h.ev_cnt));
+    if (reinterpret_cast<const LatState *>(h.hpin + kPinLat)->unknown) {
+      lattice_register<P>(h);
+      lattice_steps(h);
+    }
   }
-  // Tile numbers: per level, chunk q of octant 0..7, then chunk q + 1, ...
-  std::vector<int> tmap(ntiles > 0 ? ntiles : 1);
-  for (int l = 0, id = 0; l < 32; l++) {
-    int qmax = 0;
-    for (int o = 0; o < 8 && l * 8 + o < 255; o++) qmax = std::max(qmax, div_up(ghist[l * 8 + o], 64));
-    for (int q = 0; q < qmax; q++)
-      for (int o = 0; o < 8 && l * 8 + o < 255; o++) {
-        const int g = l * 8 + o;
-        if (q < div_up(ghist[g], 64)) tmap[gb[256 + g] + q] = id++;
-      }
-  }
-  h.lat_gb.resize(512 + tmap.size());
-  EXA_HIP(hipMemcpyAsync(h.lat_gb.p, gb, sizeof(gb), hipMemcpyHostToDevice, h.stream));
-  EXA_HIP(hipMemcpyAsync(h.lat_gb.p + 512, tmap.data(), tmap.size() * sizeof(int), hipMemcpyHostToDevice, h.stream));
-  h.lat_tile_tgt.resize((size_t)(ntiles > 0 ? ntiles : 1) * 64);
-  h.lat_tile_of.resize(nc);
-  h.lat_col_of.resize(nc);
-  if (ntiles)
-    hipLaunchKernelGGL(k_fill_int, dim3(div_up((int64_t)ntiles * 64, TPB)), dim3(TPB), 0, h.stream, h.lat_tile_tgt.p,
-                       (int64_t)ntiles * 64, -1);
-  hipLaunchKernelGGL(k_tile_assign, dim3(div_up(nc, TPB)), dim3(TPB), 0, h.stream, nc, skey, sval, h.lat_gb.p,
-                     h.lat_gb.p + 512, h.lat_tile_tgt.p, h.lat_tile_of.p, h.lat_col_of.p);
-  // 4. Steps: (tile, offset) with at least one pair, compacted per tile.
-  const int64_t nsteps_all = (int64_t)ntiles * noff;
-  h.lat_act.resize(nsteps_all + 1);
-  h.lat_aidx.resize(nsteps_all + 1);
-  hipLaunchKernelGGL(k_fill_int, dim3(div_up(nsteps_all + 1, TPB)), dim3(TPB), 0, h.stream, h.lat_act.p,
-                     nsteps_all + 1, 0);
-  h.lat_pslot.resize(np);
-  hipLaunchKernelGGL(k_lat_mark, dim3(gp), dim3(TPB), 0, h.stream, ptgt, np, h.lat_pkey.p, h.lat_ookey.p,
-                     h.lat_tile_of.p, noff, h.lat_act.p, h.lat_pslot.p);
-  exclusive_scan_int(h, h.lat_act.p, h.lat_aidx.p, (int)(nsteps_all + 1));
-  // Step lists sized for every (tile, offset) being active, so the host need
-  // not wait for the active count (the device has it in aidx[nsteps_all]),
-  // unless that bound is large; then the count is read back.
-  int64_t nact = nsteps_all;
-  if (nsteps_all * 64 > kSlotBound) {
-    int na = 0;
-    EXA_HIP(hipMemcpyAsync(&na, h.lat_aidx.p + nsteps_all, sizeof(int), hipMemcpyDeviceToHost, h.stream));
-    EXA_HIP(hipStreamSynchronize(h.stream));
-    nact = na;
-  }
-  if (nact * 64 > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
-  h.lat_alist.resize(nact > 0 ? nact : 1);
-  h.lat_step0.resize(ntiles + 1);
-  if (nsteps_all) {
-    hipLaunchKernelGGL(k_lat_alist, dim3(div_up(nsteps_all, TPB)), dim3(TPB), 0, h.stream, h.lat_act.p, h.lat_aidx.p,
-                       nsteps_all, noff, h.lat_okey.p, h.lat_tc_map.p, h.lat_alist.p);
-    // step0[t] = aidx[t * noff]: a strided copy.
-    EXA_HIP(hipMemcpy2DAsync(h.lat_step0.p, sizeof(int), h.lat_aidx.p, (size_t)noff * sizeof(int), sizeof(int),
-                             ntiles + 1, hipMemcpyDeviceToDevice, h.stream));
-  }
-  // 5. Slots of the lattice pairs; the rest (and repeats) are irregular.
-  const int64_t nslot = nact * 64;
-  h.lat_slot.resize(nslot > 0 ? nslot : 1);
-  if (nslot)
-    hipLaunchKernelGGL(k_fill_slots, dim3(std::min<int64_t>(div_up(nslot, TPB), 4096)), dim3(TPB), 0, h.stream,
-                       h.lat_slot.p, h.lat_aidx.p + nsteps_all, -1);
-  h.lat_irr.resize(np + 1);
-  h.lat_cnt.resize(1);
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, h.stream, h.lat_cnt.p, (int64_t)1, 0);
-  hipLaunchKernelGGL(k_lat_slots, dim3(gp), dim3(TPB), 0, h.stream, ptgt, np, h.lat_col_of.p, h.lat_aidx.p,
-                     h.lat_pslot.p, h.lat_slot.p);
-  hipLaunchKernelGGL(k_lat_check, dim3(gp), dim3(TPB), 0, h.stream, np, h.lat_pslot.p, psrc, h.lat_slot.p,
-                     h.lat_irr.p, h.lat_cnt.p);
-  // The irregular count (and the step count, for the statistics) is read
-  // back behind the contraction's launch (pinned host words; the copies
-  // complete before the contraction starts).
-  EXA_HIP(hipMemcpyAsync(h.hpin, h.lat_cnt.p, sizeof(int), hipMemcpyDeviceToHost, h.stream));
-  if (nsteps_all)
-    EXA_HIP(hipMemcpyAsync(h.hpin + kPinSteps, h.lat_aidx.p + nsteps_all, sizeof(int), hipMemcpyDeviceToHost,
-                           h.stream));
-  EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
-  h.lat_stats_noff = noff;
-  h.lat_stats_tiles = ntiles;
-  // 6. The contraction (timed by ev[12..13]) and the reduction.
-  const bool run_mfma = noff > 0 && ntiles > 0 && nsteps_all > 0;
+  h.lat_begun = true;
+}
+
+template <int P>
+static void lattice_run(Handle &h, M2LList &irr) {
+  using S = MfmaShape<P>;
+  const int64_t np = h.nm2l;
+  const int TPB = 256;
+  const int gp = div_up(np, TPB);
+  if (!h.lat_begun) lattice_begin<P>(h);
+  h.lat_begun = false;
+  const LatState *ls = reinterpret_cast<const LatState *>(h.hpin + kPinLat);
+  const int ntiles = h.lat_ntiles;
+  h.lat_stats_tiles = 0;
   join_multipoles(h);  // the set-up above did not need them
-  h.lat_run_ntiles = 0;
-  if (run_mfma) {
-    h.lat_part.resize((size_t)ntiles * kLatSeg * S::RB * 16 * 64);
-    // One workgroup per item, or lat_wg_cu workgroups per CU looping over
-    // the items (room left on every CU for the P2P waves of the other stream).
-    const int nitems = ntiles * kLatSeg;
-    int ngrid = nitems;
-    if (h.lat_wg_cu > 0) ngrid = std::min(ngrid, std::max(kLatSeg, (h.lat_wg_cu * h.ncu) / kLatSeg * kLatSeg));
-    h.lat_run_ntiles = ntiles;
-    h.lat_run_ngrid = ngrid;
-    if (h.serial_heavy) EXA_HIP(hipStreamWaitEvent(h.stream, h.ev[10], 0));  // P2P's end (second stream)
-    EXA_HIP(hipEventRecord(h.ev[12], h.stream));
-    h.lat_timed = true;
-    lattice_contract<P>(h);
-    EXA_HIP(hipEventRecord(h.ev[13], h.stream));
-    lattice_reduce<P>(h);
+  // The contraction (timed by ev[12..13]) and the reduction: queued on the
+  // set-up as it is; both do nothing if it met an unknown offset, and are
+  // queued again after that offset has its row.
+  for (int again = 0;; again++) {
+    h.lat_run_ntiles = 0;
+    if (h.lat_noff > 0 && ntiles > 0) {
+      h.lat_part.resize((size_t)ntiles * kLatSeg * S::RB * 16 * 64);
+      // One workgroup per item, or lat_wg_cu workgroups per CU looping over
+      // the items (room left on every CU for the P2P waves of the other stream).
+      const int nitems = ntiles * kLatSeg;
+      int ngrid = nitems;
+      if (h.lat_wg_cu > 0) ngrid = std::min(ngrid, std::max(kLatSeg, (h.lat_wg_cu * h.ncu) / kLatSeg * kLatSeg));
+      h.lat_run_ntiles = ntiles;
+      h.lat_run_ngrid = ngrid;
+      if (h.serial_heavy) EXA_HIP(hipStreamWaitEvent(h.stream, h.ev[10], 0));  // P2P's end (second stream)
+      EXA_HIP(hipEventRecord(h.ev[12], h.stream));
+      h.lat_timed = true;
+      lattice_contract<P>(h);
+      EXA_HIP(hipEventRecord(h.ev[13], h.stream));
+      lattice_reduce<P>(h);
+    }
+    EXA_HIP(hipEventSynchronize(h.ev_cnt));
+    if (!ls->unknown) break;
+    if (again) throw Error(EXAFMM_HIP_EDEVICE, "lattice M2L: offsets unknown after their registration");
+    lattice_register<P>(h);
+    lattice_steps(h);
   }
-  EXA_HIP(hipEventSynchronize(h.ev_cnt));
-  const int nirr = *h.hpin;
-  h.lat_stats_steps = nsteps_all ? h.hpin[kPinSteps] : 0;
-  // 7. The irregular pairs (none for a uniform free-space tree), in
-  // emission order, grouped by target (a stable sort: within a target the
-  // order of the full list grouped by target), queued behind the contraction.
+  const int nirr = ls->nirr;
+  h.lat_stats_steps = h.lat_run_ntiles ? ls->nsteps : 0;
+  h.lat_stats_tiles = h.lat_run_ntiles ? ls->ntiles : 0;
+  // The irregular pairs (none for a uniform free-space tree), in emission
+  // order, grouped by target (a stable sort: within a target the order of the
+  // full list grouped by target), queued behind the contraction.
   int nitl = 0;
   if (nirr) {
+    h.lat_irr.resize(np + 1);
     h.lat_scan.resize(np + 1);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, h.stream, h.lat_irr.p + np, (int64_t)1, 0);
+    hipLaunchKernelGGL(k_irr_flag, dim3(div_up(np + 1, TPB)), dim3(TPB), 0, h.stream, h.lat_pslot.p, np, h.lat_irr.p);
     exclusive_scan_int(h, h.lat_irr.p, h.lat_scan.p, (int)(np + 1));
     h.irr_rt.resize(nirr);
     h.irr_rs.resize(nirr);
     h.irr_ri.resize(nirr);
-    hipLaunchKernelGGL(k_irr_compact, dim3(gp), dim3(TPB), 0, h.stream, h.lat_irr.p, h.lat_scan.p, np, ptgt, psrc,
-                       pimg, h.irr_rt.p, h.irr_rs.p, h.irr_ri.p);
+    hipLaunchKernelGGL(k_irr_compact, dim3(gp), dim3(TPB), 0, h.stream, h.lat_irr.p, h.lat_scan.p, np, h.raw_mi.p,
+                       h.raw_mj.p, h.raw_mimg.p, h.irr_rt.p, h.irr_rs.p, h.irr_ri.p);
     group_pairs(h, nirr, h.irr_rt, h.irr_rs, h.irr_ri, h.irr_off, h.irr_src, h.irr_img, h.irr_tgt, nitl);
   }
   irr = M2LList{h.irr_tgt.p, nitl, h.irr_off.p, h.irr_src.p, h.irr_img.p};
   h.lat_stats_pairs = np - nirr;
   EXA_HIP(hipGetLastError());
+}
+
+// Distinct offsets of the last contraction (a reduction over its step flags).
+int lattice_offsets_used(Handle &h) {
+  if (h.lat_run_ntiles == 0) return 0;
+  h.cnt.reserve(4);
+  int n = 0;
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, h.stream, h.cnt.p, (int64_t)1, 0);
+  hipLaunchKernelGGL(k_lat_used, dim3(div_up(h.lat_noff, 256)), dim3(256), 0, h.stream, h.lat_act.p + sizeof(LatState),
+                     h.lat_run_ntiles, h.lat_noff, h.cnt.p);
+  EXA_HIP(hipGetLastError());
+  EXA_HIP(hipMemcpyAsync(&n, h.cnt.p, sizeof(int), hipMemcpyDeviceToHost, h.stream));
+  EXA_HIP(hipStreamSynchronize(h.stream));
+  return n;
 }
 
 bool lattice_applies(const Handle &h) {
@@ -933,7 +1098,7 @@ void run_lattice_mscale(Handle &h, hipStream_t st) {
 void m2l_begin(Handle &h) {
   h.lat_begun = false;
   if (!lattice_applies(h) || h.nm2l == 0) {
-    h.lat_ms_ready = false;  // queued scaled multipoles (if any) go unused
+    h.lat_ms_ready = h.lat_tiles_ready = false;  // queued scaled multipoles and tiles (if any) go unused
     return;
   }
   switch (h.cfg.P) {
@@ -963,10 +1128,10 @@ bool run_m2l_lattice(Handle &h, M2LList &irr) {
   h.lat_timed = false;
   h.lat_run_ntiles = 0;
   h.lat_stats_pairs = 0;
-  h.lat_stats_noff = h.lat_stats_tiles = 0;
+  h.lat_stats_tiles = 0;
   h.lat_stats_steps = 0;
   if (!lattice_applies(h) || h.nm2l == 0) {
-    h.lat_ms_ready = false;
+    h.lat_ms_ready = h.lat_tiles_ready = false;
     return false;
   }
   switch (h.cfg.P) {

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__
 // xmax) arrives behind ev_bounds and is read by sync_bounds when needed.
 void run_bounds(Handle &h) {
   h.box.reserve(16);
-  h.bounds_dev_stale = false;
+  h.bounds_dev_stale = h.bounds_given = false;
   if (h.n == 0) {
     sync_bounds(h);
     for (int d = 0; d < 3; d++) h.xmin[d] = h.xmax[d] = 0;
@@ -404,6 +404,7 @@ void run_build_uniform(Handle &h) {
                      h.cBody.p, h.cNBody.p, h.cKey.p, h.cLevel.p);
   // Level order: the layout is already level-contiguous.
   h.lvl_off.assign(off.begin(), off.begin() + L + 2);
+  h.lvl_par = counts;  // (all but the leaves)
   h.lvl_cells.resize(nc);
   hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
   EXA_HIP(hipGetLastError());
@@ -681,6 +682,7 @@ void run_build_forest(Handle &h) {
                        h.cLevel.p);
   }
   h.lvl_off.assign(loff.begin(), loff.begin() + L + 2);
+  h.lvl_par = counts;  // a bound: shallower systems end above
   h.lvl_cells.resize(nc);
   hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
   EXA_HIP(hipGetLastError());

@@ -372,6 +372,7 @@ void run_build_adaptive(Handle &h) {
                      nfirst.p, nnch.p, Xc[0], Xc[1], Xc[2], n, ncrit, aX.p, astart.p, acount.p, agid.p);
   std::vector<NodeLevel> levels;
   levels.push_back({1, 0});
+  h.lvl_par.assign(1, 0);
   int total = 1;
   int nact = n > ncrit ? 1 : 0;
   int na = nact ? n : 0;  // bodies of the active nodes
@@ -463,6 +464,8 @@ void run_build_adaptive(Handle &h) {
     EXA_HIP(hipMemcpyAsync(hcnt, h.cnt.p + 1, 3 * sizeof(int), hipMemcpyDeviceToHost, h.stream));
     EXA_HIP(hipStreamSynchronize(h.stream));
     const int nchildren = hcnt[0];
+    h.lvl_par.back() = nact;
+    h.lvl_par.push_back(0);
     levels.push_back({nchildren, total});
     total += nchildren;
     nact = hcnt[1];
