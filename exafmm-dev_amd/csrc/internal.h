@@ -68,6 +68,14 @@ struct cplx {
   double re, im;
 };
 
+// Scratch of one list grouping: entry indices (grouped, and a second array for
+// long ranges), counts per target (all zero between groupings if `zero`) and
+// the scan's chunk totals.
+struct GroupScratch {
+  DBuf<int> ord, aux, cnt, tot;
+  bool zero = false;
+};
+
 // A CSR interaction list by target cell (targets with work listed in tgt).
 struct M2LList {
   const int *tgt;
@@ -89,7 +97,7 @@ struct Handle {
   bool mult_pending = false;     // the main stream has not joined ev_mult yet
   bool mult_enqueue = false;     // run_upward_mult not enqueued yet (the traversal does it)
   hipEvent_t ev_cnt = nullptr;   // a device count copied into hpin
-  hipEvent_t ev_tiles = nullptr; // lattice tiles done on stream3 (split upward pass)
+  hipEvent_t ev_tiles = nullptr; // lattice tiles done on stream2 (split upward pass)
   hipEvent_t ev_lists = nullptr; // raw lists done (the P2P grouping on stream2 waits for it)
   hipEvent_t ev_p2pcnt = nullptr; // P2P target count copied into hpin[9] (stream2)
   hipEvent_t ev_bounds = nullptr; // bounds copied into hpin[kPinBounds..] (main stream)
@@ -203,7 +211,7 @@ struct Handle {
   bool lat_tc_f32 = false;
   bool lat_ms_ready = false;     // lat_Ms / lat_Msf already queued for this evaluation
   bool lat_begun = false;        // lattice set-up's first part queued (m2l_begin)
-  bool lat_tiles_ready = false;  // tiles of this tree queued on the third stream (ev_tiles)
+  bool lat_tiles_ready = false;  // tiles of this tree queued on the second stream (ev_tiles)
   int lat_ntiles = 0;            // tile slots of the tree
   DBuf<double> lat_T, lat_Ms;
   DBuf<float> lat_Tf, lat_Msf;
@@ -222,11 +230,10 @@ struct Handle {
 
   // Scratch.
   DBuf<unsigned char> tmp;         // hipCUB temporary storage
-  // Scratch of the P2P list grouping, which runs on stream2 beside the M2L
-  // list grouping on the main stream.
-  DBuf<int> g2a, g2b, g2c, g2d, g2e;
-  DBuf<unsigned char> tmp2;
-  DBuf<unsigned char> tmp3;        // ... and of sorts on stream3
+  // Scratch of the list groupings on the main stream and, beside it, of the
+  // P2P list's on stream2.
+  GroupScratch grp1, grp2;
+  DBuf<unsigned char> tmp3;        // ... and of sorts on stream2
   DBuf<uint64_t> k64a, k64b;
   DBuf<int> ia, ib, ic, id, ie, ifl;
   DBuf<int2> fa, fb;               // traversal frontiers (ci, cj | img << 27)

@@ -252,12 +252,7 @@ __global__ void __launch_bounds__(64)
           s.z += o.z;
           s.w += o.w;
         }
-        double4 tv = trg[tb0 + tfirst + lane];
-        tv.x += s.x;
-        tv.y -= s.y;
-        tv.z -= s.z;
-        tv.w -= s.w;
-        trg[tb0 + tfirst + lane] = tv;
+        trg[tb0 + tfirst + lane] = make_double4(s.x, -s.y, -s.z, -s.w);
       }
     };
     for (int tbase = 0; tbase < tn; tbase += 64) {
@@ -538,12 +533,7 @@ __device__ void rb_block(int lane, int c, int tb0, int tbase, int nt, int e0, in
         s.z += o.z;
         s.w += o.w;
       }
-      double4 tv = trg[tb0 + tbase + t];
-      tv.x += s.x;
-      tv.y -= s.y;
-      tv.z -= s.z;
-      tv.w -= s.w;
-      trg[tb0 + tbase + t] = tv;
+      trg[tb0 + tbase + t] = make_double4(s.x, -s.y, -s.z, -s.w);
     }
   }
 }
@@ -730,12 +720,7 @@ __global__ void __launch_bounds__(64)
           s.z += o.z;
           s.w += o.w;
         }
-        double4 tv = trg[tb0 + tfirst + lane];
-        tv.x += s.x;
-        tv.y -= s.y;
-        tv.z -= s.z;
-        tv.w -= s.w;
-        trg[tb0 + tfirst + lane] = tv;
+        trg[tb0 + tfirst + lane] = make_double4(s.x, -s.y, -s.z, -s.w);
       }
     };
     for (int tbase = 0; tbase < tn; tbase += 64) {
@@ -975,12 +960,7 @@ __device__ void rb_block32(int lane, int c, int tb0, int tbase, int nt, int e0, 
         s.z += o.z;
         s.w += o.w;
       }
-      double4 tv = trg[tb0 + tbase + ti];
-      tv.x += s.x;
-      tv.y -= s.y;
-      tv.z -= s.z;
-      tv.w -= s.w;
-      trg[tb0 + tbase + ti] = tv;
+      trg[tb0 + tbase + ti] = make_double4(s.x, -s.y, -s.z, -s.w);
     }
   }
 }
@@ -1039,7 +1019,8 @@ __global__ void k_count_body_pairs(const int *__restrict__ tgt_list, int ntl, co
 }
 
 void run_p2p(Handle &h, hipStream_t st) {
-  zero_device(h.trg4.p, (size_t)h.n * sizeof(double4), st);
+  // Every body belongs to a leaf that is in its own list, and every target is
+  // written once: the results need no clearing.
   if (h.np2p_tgt == 0) return;
   // A resident grid of p2p_wpc waves per CU that claims target leaves from a
   // counter (0: one wave per leaf).  A resident grid leaves the rest of each

@@ -444,8 +444,10 @@ void run_upward_radii(Handle &h) {
 void run_upward_mult(Handle &h) {
   EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev[16], 0));
   EXA_HIP(hipEventRecord(h.ev[17], h.stream3));
-  run_lattice_tiles(h, h.stream3);
-  EXA_HIP(hipEventRecord(h.ev_tiles, h.stream3));
+  // The tiles on the second stream, idle until the lists are there.
+  EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev[16], 0));
+  run_lattice_tiles(h, h.stream2);
+  EXA_HIP(hipEventRecord(h.ev_tiles, h.stream2));
   h.lat_tiles_ready = true;
   EXA_DISPATCH_P3(upward_impl, h, 1, h.stream3);
   run_lattice_mscale(h, h.stream3);  // the lattice M2L's input
