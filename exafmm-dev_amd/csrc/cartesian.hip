@@ -805,8 +805,9 @@ static void periodic_cart_impl(Handle &h) {
 // All leaves first (they need nothing), then the parents level by level.
 template <int P>
 static void upward_cart_impl(Handle &h) {
-  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells), dim3(64), 0, h.stream, h.lvl_cells.p, h.body4.p, h.cX.p, h.cRb.p,
-                     h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
+  const int l0 = h.lvl_off[std::min(h.leaf_level, h.nlevels - 1)];  // the cells that can be leaves
+  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells - l0), dim3(64), 0, h.stream, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
+                     h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
   for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;

@@ -141,6 +141,7 @@ struct Handle {
   DBuf<uint64_t> cKey;
   DBuf<cplx> M, L;                 // ncells * nterm
   std::vector<int> lvl_off;        // level-order offsets (host), size nlevels+1
+  int leaf_level = 0;              // no cell above this level is a leaf
   std::vector<int> lvl_par;        // cells of each level that have children, or a bound on their number
   DBuf<int> lvl_cells;             // cells sorted by level (stable)
 

@@ -1,10 +1,12 @@
-// Upward pass (P2M, M2M, setRmax, R /= theta) and downward pass (L2L, L2P),
-// level-synchronous: one 64-lane workgroup per cell, one launch per level.
+// Upward pass (P2M, M2M, setRmax, R /= theta) and downward pass (L2L, L2P):
+// P2M, leaf radii and L2P in one launch each where they can be, M2M and L2L
+// level by level.
 //
 // Reference: include/up_down_pass.h:45-148 and
 // kernels/LaplaceSphericalCPU.cxx:103-147,193-256.  Lanes own expansion
 // coefficients (P2M, M2M, L2L) or bodies (L2P).  Bodies are summed in body
 // order and children in child order, as the reference does.
+#include <algorithm>
 #include <cmath>
 
 #include "harmonics.h"
@@ -44,82 +46,73 @@ __device__ inline void p2m_rows(const Geom &g, double q, int b, double (*sR)[kP2
   }
 }
 
+// P2M (LaplaceSphericalCPU.cxx:103-118) of the leaves among `cells`, one wave
+// each: M_n^m = sum q conj(R_n^m(x_b - X_c)) over the cell's bodies, in order.
+// Chunks of kP2MChunk bodies: each body's lane writes its charge-weighted
+// table (all n, m by recurrence) into LDS, then lanes own coefficients and add
+// the chunk's rows in body order.  One launch for the leaves of every level.
 template <int P>
 __global__ void __launch_bounds__(64)
-    k_upward(const int *__restrict__ cells, const double4 *__restrict__ body, double4 *__restrict__ cX,
-             const double *__restrict__ cRb, const int *__restrict__ cChild, const int *__restrict__ cNChild,
-             const int *__restrict__ cBody, const int *__restrict__ cNBody, cplx *__restrict__ M, double theta,
-             int useRmax, int m2m, int what) {
-  // what: 1 = multipoles (P2M; M2M unless it runs as an MFMA product),
-  //       2 = radii (setRmax, R /= theta), 3 = both.
+    k_p2m(const int *__restrict__ cells, const double4 *__restrict__ body, const double4 *__restrict__ cX,
+          const int *__restrict__ cNChild, const int *__restrict__ cBody, const int *__restrict__ cNBody,
+          cplx *__restrict__ M) {
   constexpr int NT = Expn<P>::NT;
   constexpr int NO = (NT + 63) / 64;  // coefficients per lane
-  __shared__ double sR[2 * NT][kP2MChunk + 1];  // P2M rows (padded against bank conflicts)
-  __shared__ cplx sY[NT];
-  __shared__ cplx sM[NT];
-  __shared__ double sred[64];
+  __shared__ double sR[2 * NT][kP2MChunk + 1];  // rows (padded against bank conflicts)
   const int c = cells[blockIdx.x];
+  if (cNChild[c] != 0) return;
   const int lane = threadIdx.x;
   const double4 Xc = cX[c];
-  const int nchild = cNChild[c];
   double acc_re[NO], acc_im[NO];
-  int tn[NO], tm[NO];
-  for (int o = 0; o < NO; o++) {
-    acc_re[o] = acc_im[o] = 0;
-    const int t = lane + 64 * o;
-    coef_nm(t < NT ? t : 0, tn[o], tm[o]);
-  }
-  double rmax = 0;
-  if (nchild == 0) {
-    const int b0 = cBody[c], nb = cNBody[c];
-    if (!(what & 1)) {
-      for (int i = lane; i < nb; i += 64) {
-        const double4 v = body[b0 + i];
-        const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
-        rmax = r > rmax ? r : rmax;
-      }
-    } else {
-      // P2M: M_n^m += q conj(R_n^m(x_b - X_c)) over the cell's bodies, in
-      // order.  Chunks of kP2MChunk bodies: each body's lane writes its
-      // charge-weighted table (all n, m by recurrence) into LDS, then lanes
-      // own coefficients and add the chunk's rows in body order.
-      for (int base = 0; base < nb; base += kP2MChunk) {
-        const int cnt = min(kP2MChunk, nb - base);
-        __syncthreads();  // the previous chunk's rows are consumed
-        if (lane < cnt) {
-          const double4 v = body[b0 + base + lane];
-          if (what & 2) {
-            const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
-            rmax = r > rmax ? r : rmax;
-          }
-          p2m_rows<P>(make_geom(v.x - Xc.x, v.y - Xc.y, v.z - Xc.z), v.w, lane, sR);
-        }
-        __syncthreads();
 #pragma unroll
-        for (int o = 0; o < NO; o++) {
-          const int t = lane + 64 * o;
-          if (t < NT)
-            for (int k = 0; k < cnt; k++) {
-              acc_re[o] += sR[2 * t][k];
-              acc_im[o] += sR[2 * t + 1][k];
-            }
-        }
-      }
+  for (int o = 0; o < NO; o++) acc_re[o] = acc_im[o] = 0;
+  const int b0 = cBody[c], nb = cNBody[c];
+  for (int base = 0; base < nb; base += kP2MChunk) {
+    const int cnt = min(kP2MChunk, nb - base);
+    __syncthreads();  // the previous chunk's rows are consumed
+    if (lane < cnt) {
+      const double4 v = body[b0 + base + lane];
+      p2m_rows<P>(make_geom(v.x - Xc.x, v.y - Xc.y, v.z - Xc.z), v.w, lane, sR);
     }
-  } else if (!m2m || !(what & 1)) {
-    // M2M runs as a batched MFMA product (or is not asked for): Rmax only.
-    const int ch0 = cChild[c];
-    if (lane == 0)
-      for (int ci = 0; ci < nchild; ci++) {
-        const double4 Xj = cX[ch0 + ci];
-        const double r = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
-        rmax = r > rmax ? r : rmax;
-      }
-  } else {
-    // M2M (LaplaceSphericalCPU.cxx:120-147): child multipoles shifted to X_c.
-    const int ch0 = cChild[c];
-    for (int ci = 0; ci < nchild; ci++) {
-      const int cc = ch0 + ci;
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < NO; o++) {
+      const int t = lane + 64 * o;
+      if (t < NT)
+        for (int k = 0; k < cnt; k++) {
+          acc_re[o] += sR[2 * t][k];
+          acc_im[o] += sR[2 * t + 1][k];
+        }
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < NO; o++)
+    if (lane + 64 * o < NT) M[(size_t)c * NT + lane + 64 * o] = {acc_re[o], acc_im[o]};
+}
+
+// M2M (LaplaceSphericalCPU.cxx:120-147) of the parents among `cells` (one
+// level), where it does not run as a product on the matrix cores: one wave
+// per child, whose shifted multipoles are then added in child order.
+// Latency-bound (the longest coefficient adds 100 products one after another
+// at P = 10): 20 us per level of up to 512 parents and 107 us for 4096, against
+// 66 to 98 us and 279 us with one wave for all 8 children.
+template <int P>
+__global__ void __launch_bounds__(512)
+    k_m2m(const int *__restrict__ cells, const double4 *__restrict__ cX, const int *__restrict__ cChild,
+          const int *__restrict__ cNChild, cplx *__restrict__ M) {
+  constexpr int NT = Expn<P>::NT;
+  __shared__ cplx sY[8][NT], sM[8][NT];
+  const int c = cells[blockIdx.x];
+  const int nchild = cNChild[c];
+  if (nchild == 0) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double4 Xc = cX[c];
+  cplx acc{0, 0};
+  for (int base = 0; base < nchild; base += 8) {  // (an octree cell has 8 at most)
+    const int cnt = min(8, nchild - base);
+    __syncthreads();
+    if (wave < cnt) {
+      const int cc = cChild[c] + base + wave;
       const double4 Xj = cX[cc];
       const Geom g = make_geom(Xc.x - Xj.x, Xc.y - Xj.y, Xc.z - Xj.z);
       for (int t = lane; t < NT; t += 64) {
@@ -127,78 +120,110 @@ __global__ void __launch_bounds__(64)
         coef_nm(t, n, m);
         double re, im;
         regular_nm(n, m, g, re, im);
-        sY[t] = {re, im};
-        sM[t] = M[(size_t)cc * NT + t];
+        sY[wave][t] = {re, im};
+        sM[wave][t] = M[(size_t)cc * NT + t];
       }
-      if (lane == 0) {
-        const double r = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
-        rmax = r > rmax ? r : rmax;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int o = 0; o < NO; o++) {
-        if (lane + 64 * o >= NT) continue;
-        double lr = 0, li = 0;
-        m2m_lane(tn[o], tm[o], sM, sY, lr, li);
-        acc_re[o] += lr;
-        acc_im[o] += li;
-      }
-      __syncthreads();
     }
-  }
+    __syncthreads();
+    cplx r[(NT + 63) / 64];
+    if (wave < cnt)
 #pragma unroll
-  for (int o = 0; o < NO; o++) {
-    const int t = lane + 64 * o;
-    if (t < NT && (what & 1) && (nchild == 0 || m2m)) M[(size_t)c * NT + t] = {acc_re[o], acc_im[o]};
+      for (int o = 0; o < (NT + 63) / 64; o++) {
+        const int t = lane + 64 * o;
+        r[o] = {0, 0};
+        if (t >= NT) continue;
+        int j, k;
+        coef_nm(t, j, k);
+        m2m_lane(j, k, sM[wave], sY[wave], r[o].re, r[o].im);
+      }
+    __syncthreads();
+    if (wave < cnt)
+#pragma unroll
+      for (int o = 0; o < (NT + 63) / 64; o++)
+        if (lane + 64 * o < NT) sM[wave][lane + 64 * o] = r[o];
+    __syncthreads();
+    if ((int)threadIdx.x < NT)
+      for (int w = 0; w < cnt; w++) {
+        acc.re += sM[w][threadIdx.x].re;
+        acc.im += sM[w][threadIdx.x].im;
+      }
   }
-  if (!(what & 2)) return;
-  // setRmax (up_down_pass.h:51-67) and R /= theta (:82).
-  sred[lane] = rmax;
-  __syncthreads();
-  if (lane == 0) {
-    double rm = 0;
-    for (int i = 0; i < 64; i++) rm = sred[i] > rm ? sred[i] : rm;
-    double R = cRb[c];
-    if (useRmax) R = R < rm ? R : rm;
-    R /= theta;
-    cX[c].w = R;
-  }
+  if ((int)threadIdx.x < NT) M[(size_t)c * NT + threadIdx.x] = acc;
 }
 
-// Radii alone (what = 2 of k_upward: setRmax, up_down_pass.h:51-67, and
-// R /= theta, :82), one wave per cell and four cells per workgroup, without
-// k_upward's P2M tables in LDS (which held it to two waves per CU: the leaf
-// level took 85 us).  The maximum is exact in any order.
+// Radii: setRmax (up_down_pass.h:51-67) and R /= theta (:82).  The maximum is
+// exact in any order.
+__device__ inline void store_radius(double4 *cX, const double *cRb, int c, double rmax, double theta, int useRmax) {
+  double R = cRb[c];
+  if (useRmax) R = R < rmax ? R : rmax;
+  R /= theta;
+  cX[c].w = R;
+}
+
+__device__ inline void parent_radius(double4 *cX, const double *cRb, const int *cChild, int nchild, int c,
+                                     double theta, int useRmax) {
+  const double4 Xc = cX[c];
+  double rmax = 0;
+  for (int k = 0; k < nchild; k++) {
+    const double4 Xj = cX[cChild[c] + k];
+    const double r = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
+    rmax = r > rmax ? r : rmax;
+  }
+  store_radius(cX, cRb, c, rmax, theta, useRmax);
+}
+
+// The leaves among `cells`, one wave per leaf and four per workgroup.
 __global__ void __launch_bounds__(256)
-    k_radii(const int *__restrict__ cells, int ncell, const double4 *__restrict__ body, double4 *__restrict__ cX,
-            const double *__restrict__ cRb, const int *__restrict__ cChild, const int *__restrict__ cNChild,
-            const int *__restrict__ cBody, const int *__restrict__ cNBody, double theta, int useRmax) {
+    k_radii_leaves(const int *__restrict__ cells, int ncell, const double4 *__restrict__ body,
+                   double4 *__restrict__ cX, const double *__restrict__ cRb, const int *__restrict__ cNChild,
+                   const int *__restrict__ cBody, const int *__restrict__ cNBody, double theta, int useRmax) {
   const int w = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (w >= ncell) return;  // wave-uniform
   const int c = cells[w];
+  if (cNChild[c] != 0) return;
   const double4 Xc = cX[c];
-  const int nchild = cNChild[c];
+  const int b0 = cBody[c], nb = cNBody[c];
   double rmax = 0;
-  if (nchild == 0) {
-    const int b0 = cBody[c], nb = cNBody[c];
-    for (int i = lane; i < nb; i += 64) {
-      const double4 v = body[b0 + i];
-      const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
-      rmax = r > rmax ? r : rmax;
-    }
-  } else if (lane < nchild) {
-    const double4 Xj = cX[cChild[c] + lane];
-    rmax = exact_dist(Xc.x, Xc.y, Xc.z, Xj.x, Xj.y, Xj.z) + Xj.w;
+  for (int i = lane; i < nb; i += 64) {
+    const double4 v = body[b0 + i];
+    const double r = exact_dist(Xc.x, Xc.y, Xc.z, v.x, v.y, v.z);
+    rmax = r > rmax ? r : rmax;
   }
   for (int d = 32; d >= 1; d >>= 1) {
     const double o = __shfl_xor(rmax, d);
     rmax = o > rmax ? o : rmax;
   }
-  if (lane == 0) {
-    double R = cRb[c];
-    if (useRmax) R = R < rmax ? R : rmax;
-    R /= theta;
-    cX[c].w = R;
+  if (lane == 0) store_radius(cX, cRb, c, rmax, theta, useRmax);
+}
+
+// The parents of one large level, and those of all levels above it in one
+// workgroup (kRadiiTop cells per level at most): one thread per parent.
+constexpr int kRadiiTop = 1024;
+__global__ void __launch_bounds__(256)
+    k_radii_level(const int *__restrict__ cells, int ncell, double4 *cX, const double *__restrict__ cRb,
+                  const int *__restrict__ cChild, const int *__restrict__ cNChild, double theta, int useRmax) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= ncell) return;
+  const int c = cells[i], n = cNChild[c];
+  if (n > 0) parent_radius(cX, cRb, cChild, n, c, theta, useRmax);
+}
+
+struct TopLevels {
+  int n;
+  int off[33];
+};
+
+__global__ void __launch_bounds__(kRadiiTop)
+    k_radii_top(TopLevels tl, const int *__restrict__ lvl_cells, double4 *cX, const double *__restrict__ cRb,
+                const int *__restrict__ cChild, const int *__restrict__ cNChild, double theta, int useRmax) {
+  for (int l = tl.n - 1; l >= 0; l--) {
+    const int i = tl.off[l] + threadIdx.x;
+    if (i < tl.off[l + 1]) {
+      const int c = lvl_cells[i], n = cNChild[c];
+      if (n > 0) parent_radius(cX, cRb, cChild, n, c, theta, useRmax);
+    }
+    __threadfence_block();
+    __syncthreads();
   }
 }
 
@@ -347,22 +372,45 @@ __global__ void __launch_bounds__(64)
   }
 }
 
+// The cells that can be leaves: lvl_cells from the first such level on.
+static int first_leaf(const Handle &h) { return h.lvl_off[std::min(h.leaf_level, h.nlevels - 1)]; }
+
 template <int P>
-static void upward_impl(Handle &h, int what, hipStream_t st) {
+static void multipoles_impl(Handle &h, hipStream_t st) {
   const bool mf = updown_mfma_enabled(h);
-  for (int t = h.nlevels - 1; t >= 0; t--) {
+  const int l0 = first_leaf(h);
+  hipLaunchKernelGGL(k_p2m<P>, dim3(h.ncells - l0), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
+                     h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p);
+  for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;
     const int *cells = h.lvl_cells.p + h.lvl_off[t];
-    if (what == 2) {
-      hipLaunchKernelGGL(k_radii, dim3(div_up(cnt, 4)), dim3(256), 0, st, cells, cnt, h.body4.p, h.cX.p, h.cRb.p,
-                         h.cChild.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cfg.theta, h.cfg.useRmax);
-      continue;
-    }
-    hipLaunchKernelGGL(k_upward<P>, dim3(cnt), dim3(64), 0, st, cells, h.body4.p, h.cX.p, h.cRb.p, h.cChild.p,
-                       h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax, mf ? 0 : 1, what);
-    if ((what & 1) && mf && t + 1 < h.nlevels) run_m2m_level_mfma(h, cells, cnt, st);
+    if (mf)
+      run_m2m_level_mfma(h, cells, cnt, st);
+    else
+      hipLaunchKernelGGL(k_m2m<P>, dim3(cnt), dim3(512), 0, st, cells, h.cX.p, h.cChild.p, h.cNChild.p, h.M.p);
   }
+  EXA_HIP(hipGetLastError());
+}
+
+// Leaves of every level first, then the parents from the bottom up.
+static void run_radii(Handle &h) {
+  const int l0 = first_leaf(h), nleaf = h.ncells - l0;
+  hipLaunchKernelGGL(k_radii_leaves, dim3(div_up(nleaf, 4)), dim3(256), 0, h.stream, h.lvl_cells.p + l0, nleaf,
+                     h.body4.p, h.cX.p, h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cfg.theta, h.cfg.useRmax);
+  TopLevels tl{};
+  const int np = h.nlevels - 1;  // levels that can hold parents
+  while (tl.n < np && tl.n < 32 && h.lvl_off[tl.n + 1] - h.lvl_off[tl.n] <= kRadiiTop) tl.n++;
+  for (int l = 0; l <= tl.n; l++) tl.off[l] = h.lvl_off[l];
+  for (int t = np - 1; t >= tl.n; t--) {
+    const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
+    if (cnt > 0)
+      hipLaunchKernelGGL(k_radii_level, dim3(div_up(cnt, 256)), dim3(256), 0, h.stream, h.lvl_cells.p + h.lvl_off[t],
+                         cnt, h.cX.p, h.cRb.p, h.cChild.p, h.cNChild.p, h.cfg.theta, h.cfg.useRmax);
+  }
+  if (tl.n > 0)
+    hipLaunchKernelGGL(k_radii_top, dim3(1), dim3(kRadiiTop), 0, h.stream, tl, h.lvl_cells.p, h.cX.p, h.cRb.p,
+                       h.cChild.p, h.cNChild.p, h.cfg.theta, h.cfg.useRmax);
   EXA_HIP(hipGetLastError());
 }
 
@@ -370,7 +418,7 @@ template <int P>
 static void downward_impl(Handle &h) {
   // MASS mode divides each child's own L by its M_0 before the L2L
   // (LaplaceSphericalCPU.cxx MASS branch): kept in the per-cell kernel.
-  const bool mf = updown_mfma_enabled(h) && !h.cfg.mass;
+  const bool mf = h.updown_mfma && h.cfg.basis == 0 && !h.cfg.mass;
   if (mf) {
     // L2L level by level on the matrix cores, then L2P of every leaf with
     // bodies (the P2P target list holds exactly those: a leaf is always in
@@ -409,22 +457,14 @@ static void downward_impl(Handle &h) {
     default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");    \
   }
 
-#define EXA_DISPATCH_P3(fn, h, a, b)                                                 \
-  switch ((h).cfg.P) {                                                               \
-    case 4: fn<4>(h, a, b); break;                                                   \
-    case 6: fn<6>(h, a, b); break;                                                   \
-    case 8: fn<8>(h, a, b); break;                                                   \
-    case 10: fn<10>(h, a, b); break;                                                 \
-    case 12: fn<12>(h, a, b); break;                                                 \
-    default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");    \
-  }
 
 void run_upward(Handle &h) {
   h.M.resize((size_t)h.ncells * h.nterm);
   h.L.resize((size_t)h.ncells * h.nterm);
   EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream));
   if (h.cfg.basis == 1) return run_upward_cart(h);
-  EXA_DISPATCH_P3(upward_impl, h, 3, h.stream);
+  run_radii(h);
+  run_multipoles(h, h.stream);
 }
 
 // The upward pass split over two streams: radii (needed by the traversal)
@@ -437,7 +477,7 @@ void run_upward_radii(Handle &h) {
   h.M.resize((size_t)h.ncells * h.nterm);
   h.L.resize((size_t)h.ncells * h.nterm);
   EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream));
-  EXA_DISPATCH_P3(upward_impl, h, 2, h.stream);
+  run_radii(h);
   EXA_HIP(hipEventRecord(h.ev[16], h.stream));
 }
 
@@ -449,12 +489,21 @@ void run_upward_mult(Handle &h) {
   run_lattice_tiles(h, h.stream2);
   EXA_HIP(hipEventRecord(h.ev_tiles, h.stream2));
   h.lat_tiles_ready = true;
-  EXA_DISPATCH_P3(upward_impl, h, 1, h.stream3);
+  run_multipoles(h, h.stream3);
   run_lattice_mscale(h, h.stream3);  // the lattice M2L's input
   EXA_HIP(hipEventRecord(h.ev_mult, h.stream3));
 }
 
-void run_multipoles(Handle &h, hipStream_t st) { EXA_DISPATCH_P3(upward_impl, h, 1, st); }
+void run_multipoles(Handle &h, hipStream_t st) {
+  switch (h.cfg.P) {
+    case 4: multipoles_impl<4>(h, st); break;
+    case 6: multipoles_impl<6>(h, st); break;
+    case 8: multipoles_impl<8>(h, st); break;
+    case 10: multipoles_impl<10>(h, st); break;
+    case 12: multipoles_impl<12>(h, st); break;
+    default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");
+  }
+}
 
 void run_downward(Handle &h) {
   if (h.cfg.basis == 1) return run_downward_cart(h);
@@ -466,8 +515,9 @@ void run_downward(Handle &h) {
 // children) of `cells`, and L2L (do_l2l) then L2P at leaves of `cells`.
 template <int P>
 static void upward_cells_impl(Handle &h, const CellSetView &v) {
-  hipLaunchKernelGGL(k_upward<P>, dim3(v.ncell), dim3(64), 0, h.stream, v.cells, v.body, v.cX, v.cRb, v.cChild,
-                     v.cNChild, v.cBody, v.cNBody, v.M, h.cfg.theta, h.cfg.useRmax, 1, 1);
+  hipLaunchKernelGGL(k_p2m<P>, dim3(v.ncell), dim3(64), 0, h.stream, v.cells, v.body, v.cX, v.cNChild, v.cBody,
+                     v.cNBody, v.M);
+  hipLaunchKernelGGL(k_m2m<P>, dim3(v.ncell), dim3(512), 0, h.stream, v.cells, v.cX, v.cChild, v.cNChild, v.M);
 }
 
 template <int P>

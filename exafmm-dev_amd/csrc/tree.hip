@@ -405,6 +405,7 @@ void run_build_uniform(Handle &h) {
   // Level order: the layout is already level-contiguous.
   h.lvl_off.assign(off.begin(), off.begin() + L + 2);
   h.lvl_par = counts;  // (all but the leaves)
+  h.leaf_level = L;
   h.lvl_cells.resize(nc);
   hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
   EXA_HIP(hipGetLastError());
@@ -683,6 +684,8 @@ void run_build_forest(Handle &h) {
   }
   h.lvl_off.assign(loff.begin(), loff.begin() + L + 2);
   h.lvl_par = counts;  // a bound: shallower systems end above
+  h.leaf_level = L;
+  for (const ForestSys &f : fs) h.leaf_level = std::min(h.leaf_level, f.L);
   h.lvl_cells.resize(nc);
   hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
   EXA_HIP(hipGetLastError());

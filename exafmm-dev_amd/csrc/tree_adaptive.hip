@@ -373,6 +373,7 @@ void run_build_adaptive(Handle &h) {
   std::vector<NodeLevel> levels;
   levels.push_back({1, 0});
   h.lvl_par.assign(1, 0);
+  h.leaf_level = 0;
   int total = 1;
   int nact = n > ncrit ? 1 : 0;
   int na = nact ? n : 0;  // bodies of the active nodes
