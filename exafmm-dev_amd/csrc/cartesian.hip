@@ -841,7 +841,8 @@ void run_upward_cart(Handle &h) { EXA_DISPATCH_CART(upward_cart_impl, h); }
 void run_downward_cart(Handle &h) { EXA_DISPATCH_CART(downward_cart_impl, h); }
 void run_m2l_cart(Handle &h) {
   if (h.nm2l_tgt == 0) return;
-  m2l_cart(h, M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p}, h.cX.p, h.M.p, h.ncells,
+  m2l_cart(h, M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p, h.nm2l}, h.cX.p, h.M.p,
+           h.ncells,
            h.L.p);
 }
 void run_periodic_cart(Handle &h) {

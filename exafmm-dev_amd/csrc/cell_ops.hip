@@ -354,7 +354,7 @@ int exafmm_hip_cell_m2l(exafmm_hip_handle *H, const double *Xi, const double *Mi
     h.co_img.resize(2);
     const unsigned char img[2] = {13, 13};  // no image shift
     h2d(h.co_img.p, img, sizeof(img), h);
-    const M2LList lst{v.cells + 5, mutual ? 2 : 1, v.cells, v.cells + 3, h.co_img.p};
+    const M2LList lst{v.cells + 5, mutual ? 2 : 1, v.cells, v.cells + 3, h.co_img.p, mutual ? 2 : 1};
     launch_m2l_arrays(h, lst, h.co_X.p, h.co_M.p, 2, h.co_L.p);
     double *acc = reinterpret_cast<double *>(h.co_L.p + 2 * (size_t)h.nterm);
     h2d(acc, Li, ne * sizeof(double), h);

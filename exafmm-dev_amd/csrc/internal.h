@@ -83,6 +83,7 @@ struct M2LList {
   const int *off;
   const int *src;
   const unsigned char *img;
+  int64_t npairs;
 };
 
 struct Handle {

@@ -125,8 +125,20 @@ static M2LSchedule build_schedule(int P, int ipl, int esz) {
 //   M~_n^m = M_n^m / r^n,  S~_a^b = S_a^b r^(a+1)  (unit-distance harmonics),
 // so L_j^k = r^-(j+1) sum_n sum_m M~ S~, and each finished (j, k, n) partial
 // is multiplied in FP64 by u^(j+1) = r^-(j+1).
-template <int P, typename R>
-__global__ void __launch_bounds__(64)
+//
+// W waves share a target, each with its own tables and slots and a contiguous
+// part of the source list; their slots are added in wave order.  W > 1 where
+// targets are few (the pairs of an adaptive tree that are two or more levels
+// apart: some targets have hundreds, one after another at 5 us each): 15000
+// pairs at P = 12 took 776 us with one wave per target, 300 us with four.
+// With many targets one wave each keeps more targets in flight.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int P, typename R, int W>
+__global__ void __launch_bounds__(64 * W)
     k_m2l(const int *__restrict__ tgt_list, const int *__restrict__ off, const int *__restrict__ src,
           const unsigned char *__restrict__ img, const double4 *__restrict__ cX, const cplx *__restrict__ M,
           cplx *__restrict__ L, const uint32_t *__restrict__ sched, const int *__restrict__ slot0,
@@ -140,12 +152,15 @@ __global__ void __launch_bounds__(64)
   constexpr int NO = (NT + 63) / 64;
   // Single-buffered tables (two barriers per pair) keep the LDS footprint
   // small enough for five or more resident waves per SIMD.
-  __shared__ C sM[NF + 1];
-  __shared__ C sS[NF + 1];
-  __shared__ cplx seg[S::NTRIPLE];
-  __shared__ double sU[P];  // FP32 path: scale * u^(j+1)
+  __shared__ C sMw[W][NF + 1];
+  __shared__ C sSw[W][NF + 1];
+  __shared__ cplx segw[W][S::NTRIPLE];
+  __shared__ double sUw[W][P];  // FP32 path: scale * u^(j+1)
   const int c = tgt_list[blockIdx.x];
-  const int lane = threadIdx.x;
+  const int wave = W > 1 ? (int)threadIdx.x / 64 : 0, lane = W > 1 ? (int)threadIdx.x % 64 : (int)threadIdx.x;
+  C *sM = sMw[wave], *sS = sSw[wave];
+  cplx *seg = segw[wave];
+  double *sU = sUw[wave];
   uint32_t desc[IPL];
 #pragma unroll
   for (int it = 0; it < IPL; it++) desc[it] = sched[it * 64 + lane];
@@ -167,7 +182,8 @@ __global__ void __launch_bounds__(64)
   }
   const double4 Xi = cX[c];
   const double mi0 = mass ? M[(size_t)c * NT].re : 1.0;
-  const int e0 = off[c], e1 = off[c + 1];
+  const int n0 = off[c], np = off[c + 1] - n0;
+  const int e0 = n0 + (int)((int64_t)np * wave / W), e1 = n0 + (int)((int64_t)np * (wave + 1) / W);
   // Prefetch of the first source.
   int s_next = e0 < e1 ? src[e0] : 0;
   int im_next = e0 < e1 ? img[e0] : 13;
@@ -202,7 +218,7 @@ __global__ void __launch_bounds__(64)
     const double us = F32 ? 1.0 : u;  // the FP32 tables use unit distance
     const double ru = us, rsu = st * us, rcp = cp, rsp = sp, cu = ct * us, u2 = us * us;
     const double scale = mass ? mi0 * mj0 : 1.0;
-    __syncthreads();  // the previous pair's items are done with the tables
+    wave_sync();  // the previous pair's items are done with the tables
     if (F32 && lane < P) {
       double f = scale * u;
       for (int i = 0; i < lane; i++) f *= u;
@@ -245,7 +261,7 @@ __global__ void __launch_bounds__(64)
       sM[a * a + a + b] = {sg * (R)mv.re, sg * (R)mv.im};
       if (b > 0) sM[a * a + a - b] = {(R)mv.re, -(R)mv.im};
     }
-    __syncthreads();
+    wave_sync();
     const char *mb = reinterpret_cast<const char *>(sM);
     const char *sb = reinterpret_cast<const char *>(sS);
     R ar = 0, ai = 0;
@@ -271,12 +287,18 @@ __global__ void __launch_bounds__(64)
     }
   }
   __syncthreads();
-  for (int t = lane; t < NT; t += 64) {
+  for (int t = threadIdx.x; t < NT; t += 64 * W) {
     int j = 0;
     while (tri(j + 1) <= t) j++;
     double lr = 0, li = 0;
     for (int n = 0; n < P - j; n++) {
-      const cplx v = seg[outslot[t * P + n]];
+      const int o = outslot[t * P + n];
+      cplx v = segw[0][o];
+#pragma unroll
+      for (int w = 1; w < W; w++) {
+        v.re += segw[w][o].re;
+        v.im += segw[w][o].im;
+      }
       lr += v.re;
       li += v.im;
     }
@@ -287,6 +309,13 @@ __global__ void __launch_bounds__(64)
     L[(size_t)c * NT + t] = o;
   }
 }
+
+// Where several waves share a target: below a few rounds of the resident
+// workgroups (two of 8 waves per CU) the longest list decides the time, and so
+// it does where most lists are short (irregular pairs of an adaptive tree: 3
+// per target on average, over 100 at most).  Long lists on many targets
+// (periodic images: 100 per target) fill the chip by themselves.
+constexpr int kFewTargets = 2048, kShortList = 16;
 
 template <int P>
 static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L, bool f32,
@@ -313,12 +342,16 @@ static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const c
     EXA_HIP(hipEventRecord(h.ev[14], h.stream));
     h.pair_timed = true;
   }
+  auto launch = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(lst.ntgt), dim3(64 * waves), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img, cX, M,
+                       L, desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+  };
+  constexpr int W = P <= 10 ? 8 : 4;  // 55 KB of LDS per workgroup at P = 10, 41 KB at P = 12
+  const bool few = lst.ntgt <= kFewTargets || lst.npairs < (int64_t)kShortList * lst.ntgt;
   if (esz == 8)
-    hipLaunchKernelGGL((k_m2l<P, float>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img,
-                       cX, M, L, desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+    few ? launch(k_m2l<P, float, W>, W) : launch(k_m2l<P, float, 1>, 1);
   else
-    hipLaunchKernelGGL((k_m2l<P, double>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img,
-                       cX, M, L, desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+    few ? launch(k_m2l<P, double, W>, W) : launch(k_m2l<P, double, 1>, 1);
   if (timed) EXA_HIP(hipEventRecord(h.ev[15], h.stream));
   EXA_HIP(hipGetLastError());
 }
@@ -358,7 +391,7 @@ void run_m2l(Handle &h) {
   M2LList lst{};
   if (!run_m2l_lattice(h, lst)) {
     ensure_m2l_grouped(h);
-    lst = M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p};
+    lst = M2LList{h.m2l_tgt.p, h.nm2l_tgt, h.m2l_off.p, h.m2l_src.p, h.m2l_img.p, h.nm2l};
   }
   join_multipoles(h);  // (the lattice path joined them before its contraction)
   h.m2l_last = lst;

@@ -1057,7 +1057,7 @@ static void lattice_run(Handle &h, M2LList &irr) {
                        h.raw_mj.p, h.raw_mimg.p, h.irr_rt.p, h.irr_rs.p, h.irr_ri.p);
     group_pairs(h, nirr, h.irr_rt, h.irr_rs, h.irr_ri, h.irr_off, h.irr_src, h.irr_img, h.irr_tgt, nitl);
   }
-  irr = M2LList{h.irr_tgt.p, nitl, h.irr_off.p, h.irr_src.p, h.irr_img.p};
+  irr = M2LList{h.irr_tgt.p, nitl, h.irr_off.p, h.irr_src.p, h.irr_img.p, nirr};
   h.lat_stats_pairs = np - nirr;
   EXA_HIP(hipGetLastError());
 }
