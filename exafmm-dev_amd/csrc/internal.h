@@ -103,7 +103,7 @@ struct Handle {
   hipEvent_t ev_p2pcnt = nullptr; // P2P target count copied into hpin[9] (stream2)
   hipEvent_t ev_bounds = nullptr; // bounds copied into hpin[kPinBounds..] (main stream)
   int *hpin = nullptr;           // pinned host words for counts read back behind queued work
-  static constexpr int kPinWords = 512;  // hpin: [0..64) counts, [64..322) lattice tile histogram, ...
+  static constexpr int kPinWords = 512;  // hpin: [0..64) counts, [64..80) lattice set-up, [128..) tree build, [400..412) bounds
   static constexpr int kPinBounds = 400;  // hpin: [400, 412) the six bounds (doubles)
 
   // Bodies.
@@ -157,10 +157,14 @@ struct Handle {
   DBuf<int> raw_mi, raw_mj, raw_pi, raw_pj;  // emission-order lists
   DBuf<unsigned char> raw_mimg, raw_pimg;
 
-  // Adaptive-builder scratch (node arrays in creation order).
-  DBuf<double4> at_X, at_aX, at_body2;
-  DBuf<int> at_start, at_count, at_parent, at_leaf, at_level, at_first, at_nchild, at_astart, at_acount, at_agid,
-      at_idx2, at_nnode, at_cellid, at_cursor, at_nl;
+  // Adaptive builder: node arrays in creation order, lists of splitting nodes,
+  // octant boundaries, and the sizes the next build starts from.
+  DBuf<double4> at_X;
+  DBuf<int> at_start, at_count, at_parent, at_level, at_first, at_nchild, at_act0, at_act1, at_lo, at_blk;
+  DBuf<char> at_state;
+  size_t at_cap = 0;
+  int at_depth = 0, at_big = 0;  // levels that split; those from the first with more nodes than one workgroup takes
+  int64_t at_total = 0;          // nodes
 
   // Periodic far field: the lattice sums of the handle's order and basis.
   DBuf<double> per_tab;
@@ -302,6 +306,7 @@ struct CellSetView {
 // Phase implementations (one translation unit each).
 void run_bounds(Handle &h);
 void sync_bounds(Handle &h);
+void upload_bounds(Handle &h);
 void run_build_uniform(Handle &h);
 void run_build_forest(Handle &h);
 void run_build_adaptive(Handle &h);
@@ -395,6 +400,9 @@ void exclusive_scan_int(const int *in, int *out, int n, hipStream_t st, DBuf<uns
 void exclusive_scan_int4(Handle &h, const int4 *in, int4 *out, int n);  // component-wise
 void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bits,
                         bool &result_in_alt);
+// The same over key bits [bit0, bit1), for the tree build (nothing runs beside it).
+void sort_pairs_u64_int_bits(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
+                             int bit1, bool &result_in_alt);
 void sort_pairs_int_int(Handle &h, int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits,
                         bool &result_in_alt);
 void sort_pairs_int_int(int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits, bool &result_in_alt,

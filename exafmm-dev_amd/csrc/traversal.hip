@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "device_util.h"
 #include "internal.h"
 
 namespace exafmm {
@@ -101,46 +102,7 @@ __device__ inline int4 pair_counts(const CellView &cv, int4 f, int a, int mutual
   return pair_counts_n(f, a, mutual, cv.nchild[f.x], cv.nchild[f.y]);
 }
 
-__device__ inline int4 add4(int4 a, int4 b) { return make_int4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-
 constexpr int kTravBlock = 256;
-
-// Exclusive prefix of v over the NT threads of the block (wave scans, then
-// the wave totals); *total receives the block sum.
-template <int NT = kTravBlock>
-__device__ inline int4 block_exscan4(int4 v, int4 *total) {
-  __shared__ int4 wsum[NT / 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int4 inc = v;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int4 t = make_int4(__shfl_up(inc.x, d), __shfl_up(inc.y, d), __shfl_up(inc.z, d), 0);
-    if (lane >= d) inc = add4(inc, t);
-  }
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  int4 base = make_int4(0, 0, 0, 0), tot = make_int4(0, 0, 0, 0);
-  if (NT <= 256) {
-    for (int k = 0; k < NT / 64; k++) {
-      if (k < w) base = add4(base, wsum[k]);
-      tot = add4(tot, wsum[k]);
-    }
-  } else {  // many waves: the first wave scans the wave totals in place
-    if (w == 0) {
-      int4 x = lane < NT / 64 ? wsum[lane] : make_int4(0, 0, 0, 0);
-      for (int d = 1; d < NT / 64; d <<= 1) {
-        const int4 t = make_int4(__shfl_up(x.x, d), __shfl_up(x.y, d), __shfl_up(x.z, d), 0);
-        if (lane >= d) x = add4(x, t);
-      }
-      if (lane < NT / 64) wsum[lane] = x;
-    }
-    __syncthreads();
-    if (w > 0) base = wsum[w - 1];
-    tot = wsum[NT / 64 - 1];
-  }
-  __syncthreads();
-  *total = tot;
-  return make_int4(base.x + inc.x - v.x, base.y + inc.y - v.y, base.z + inc.z - v.z, 0);
-}
 
 // Pass 1 over the frontier: action per pair and the block's output totals.
 __global__ void __launch_bounds__(kTravBlock)
@@ -610,85 +572,18 @@ __global__ void __launch_bounds__(256)
 }
 
 // One wave per target: its indices sorted, then the sources and images in
-// that order.  An entry's place is the number of smaller indices: up to 64
-// entries by lane reads, up to kGroupRank through LDS (quadratic, 1 us at the
-// usual 30 to 100 entries); longer ranges by a stable radix sort, 5 bits at a
-// time, between ord and aux.
-constexpr int kGroupRank = 1024;
+// that order.
 __global__ void __launch_bounds__(64)
     k_group_sort(const int *__restrict__ off, int bits, int *__restrict__ ord, int *__restrict__ aux,
                  const int *__restrict__ src_in, const unsigned char *__restrict__ img_in, int *__restrict__ src_out,
                  unsigned char *__restrict__ img_out) {
-  __shared__ int se[kGroupRank];
-  __shared__ int shist[32];
-  const int lane = threadIdx.x;
+  __shared__ RangeSortLds sh;
   const int o = off[blockIdx.x], n = off[blockIdx.x + 1] - o;
   if (n <= 0) return;
-  if (n <= 64) {
-    const int e = lane < n ? ord[o + lane] : INT_MAX;
-    int rank = 0;
-    for (int k = 0; k < n; k++) rank += __builtin_amdgcn_readlane(e, k) < e;
-    if (lane < n) {
-      src_out[o + rank] = src_in[e];
-      img_out[o + rank] = img_in[e];
-    }
-    return;
-  }
-  if (n <= kGroupRank) {
-    for (int k = lane; k < (n + 3) / 4 * 4; k += 64) se[k] = k < n ? ord[o + k] : INT_MAX;
-    __syncthreads();
-    const int4 *s4 = reinterpret_cast<const int4 *>(se);
-    for (int i = lane; i < n; i += 64) {
-      const int e = se[i];
-      int rank = 0;
-      for (int k = 0; k < (n + 3) / 4; k++) {
-        const int4 v = s4[k];
-        rank += (v.x < e) + (v.y < e) + (v.z < e) + (v.w < e);
-      }
-      src_out[o + rank] = src_in[e];
-      img_out[o + rank] = img_in[e];
-    }
-    return;
-  }
-  int *a = ord + o, *b = aux + o;
-  for (int shift = 0; shift < bits; shift += 5) {
-    if (lane < 32) shist[lane] = 0;
-    __syncthreads();
-    for (int i = lane; i < n; i += 64) atomicAdd(&shist[(a[i] >> shift) & 31], 1);
-    __syncthreads();
-    int h = lane < 32 ? shist[lane] : 0, inc = h;
-    for (int d = 1; d < 32; d <<= 1) {
-      const int t = __shfl_up(inc, d);
-      if (lane >= d) inc += t;
-    }
-    __syncthreads();
-    if (lane < 32) shist[lane] = inc - h;  // where the digit's next entry goes
-    __syncthreads();
-    for (int i0 = 0; i0 < n; i0 += 64) {
-      const int i = i0 + lane;
-      const int e = i < n ? a[i] : 0, d = (e >> shift) & 31;
-      unsigned long long same = __ballot(i < n);
-      for (int k = 0; k < 5; k++) {
-        const unsigned long long m = __ballot((d >> k) & 1);
-        same &= (d >> k) & 1 ? m : ~m;
-      }
-      const int before = (int)__popcll(same & ((1ull << lane) - 1));
-      const int at = i < n ? shist[d] : 0;
-      __syncthreads();
-      if (i < n && before == 0) shist[d] = at + (int)__popcll(same);
-      if (i < n) b[at + before] = e;
-      __syncthreads();
-    }
-    __threadfence_block();
-    __syncthreads();
-    int *t = a;
-    a = b;
-    b = t;
-  }
-  for (int i = lane; i < n; i += 64) {
-    src_out[o + i] = src_in[a[i]];
-    img_out[o + i] = img_in[a[i]];
-  }
+  sort_range(ord + o, aux + o, n, bits, sh, [&](int rank, int e) {
+    src_out[o + rank] = src_in[e];
+    img_out[o + rank] = img_in[e];
+  });
 }
 
 // Grow a buffer, keeping its first `keep` elements.

@@ -105,7 +105,7 @@ void sync_bounds(Handle &h) {
 }
 
 // The device bounds set from the host values (bounds given by the caller).
-static void upload_bounds(Handle &h) {
+void upload_bounds(Handle &h) {
   h.box.reserve(16);
   if (!h.bounds_dev_stale) return;
   const double v[6] = {h.xmin[0], h.xmin[1], h.xmin[2], h.xmax[0], h.xmax[1], h.xmax[2]};

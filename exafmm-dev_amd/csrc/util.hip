@@ -41,10 +41,6 @@ Handle::~Handle() {
   p2p_tgt.release();
   m2l_tgt.release();
   m2l_sched.release();
-  for (auto *b : {&at_X, &at_aX, &at_body2}) b->release();
-  for (auto *b : {&at_start, &at_count, &at_parent, &at_leaf, &at_level, &at_first, &at_nchild, &at_astart,
-                  &at_acount, &at_agid, &at_idx2, &at_nnode, &at_cellid, &at_cursor, &at_nl})
-    b->release();
   raw_mi.release();
   raw_mj.release();
   raw_pi.release();
@@ -142,14 +138,14 @@ constexpr int kOnesweepMin = 1 << 18;
 
 template <typename Config, typename K>
 static void radix_sort_pairs_cfg(K *keys, K *keys_alt, int *vals, int *vals_alt, int n, int bits,
-                                 bool &result_in_alt, hipStream_t st, DBuf<unsigned char> &tmp) {
+                                 bool &result_in_alt, hipStream_t st, DBuf<unsigned char> &tmp, unsigned bit0 = 0) {
   rocprim::double_buffer<K> k(keys, keys_alt);
   rocprim::double_buffer<int> v(vals, vals_alt);
   const unsigned int end_bit = bits > 0 ? bits : 1;
   size_t bytes = 0;
-  EXA_HIP(rocprim::radix_sort_pairs<Config>(nullptr, bytes, k, v, n, 0u, end_bit, st));
+  EXA_HIP(rocprim::radix_sort_pairs<Config>(nullptr, bytes, k, v, n, bit0, end_bit, st));
   tmp.reserve(bytes);
-  EXA_HIP(rocprim::radix_sort_pairs<Config>(tmp.p, bytes, k, v, n, 0u, end_bit, st));
+  EXA_HIP(rocprim::radix_sort_pairs<Config>(tmp.p, bytes, k, v, n, bit0, end_bit, st));
   result_in_alt = k.current() != keys;
 }
 
@@ -165,6 +161,16 @@ static void radix_sort_pairs(K *keys, K *keys_alt, int *vals, int *vals_alt, int
 void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bits,
                         bool &result_in_alt) {
   radix_sort_pairs(keys, keys_alt, vals, vals_alt, n, bits, result_in_alt, h.stream, h.tmp);
+}
+
+void sort_pairs_u64_int_bits(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
+                             int bit1, bool &result_in_alt) {
+  // Alone on the device: onesweep already where its 3 launches per 8 bits are
+  // fewer than those of the merge passes.
+  if (n < (1 << 16))
+    return radix_sort_pairs_cfg<rocprim::default_config>(keys, keys_alt, vals, vals_alt, n, bit1, result_in_alt,
+                                                         h.stream, h.tmp, bit0);
+  radix_sort_pairs_cfg<OnesweepConfig>(keys, keys_alt, vals, vals_alt, n, bit1, result_in_alt, h.stream, h.tmp, bit0);
 }
 
 void sort_pairs_int_int(Handle &h, int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits,
