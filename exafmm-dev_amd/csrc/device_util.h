@@ -7,6 +7,13 @@
 
 namespace exafmm {
 
+// Orders the LDS accesses of one wave (its stores before its later loads by
+// other lanes), where waves of a workgroup use separate parts of LDS.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ inline int4 add4(int4 a, int4 b) { return make_int4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 
 // Exclusive prefix of v over the NT threads of the block (wave scans, then

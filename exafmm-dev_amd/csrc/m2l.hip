@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "device_util.h"
 #include "harmonics.h"
 #include "internal.h"
 
@@ -132,11 +133,6 @@ static M2LSchedule build_schedule(int P, int ipl, int esz) {
 // apart: some targets have hundreds, one after another at 5 us each): 15000
 // pairs at P = 12 took 776 us with one wave per target, 300 us with four.
 // With many targets one wave each keeps more targets in flight.
-__device__ inline void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <int P, typename R, int W>
 __global__ void __launch_bounds__(64 * W)
     k_m2l(const int *__restrict__ tgt_list, const int *__restrict__ off, const int *__restrict__ src,

@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "device_util.h"
 #include "internal.h"
 
 namespace exafmm {
@@ -62,7 +63,8 @@ __device__ inline double rsqrt_pos(double x) {
 // every entry that starts inside the stage marks its first slot, and a
 // running maximum over the slots (four per lane, then across the wave) gives
 // each slot its entry; the body loads of a lane's slots are then issued
-// together.  The workgroup is one wave; every call is uniform across it.
+// together.  Every call is uniform across the wave, whose lanes alone use `sd`
+// and the stage.
 struct SrcWalker {
   int e, sbase, dbase, dcount;
 };
@@ -86,7 +88,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
                                  Put put, int skip = -1) {
   static_assert(STAGE <= kFillMax && STAGE % 64 == 0, "the slot map covers a stage, four slots per lane");
   static_assert((STAGE / 64) % NB == 0, "whole batches of loads");
-  __syncthreads();  // the previous stage (and descriptor batch) are consumed
+  wave_sync();  // the previous stage (and descriptor batch) are consumed
   if (w.e >= w.dbase + w.dcount) {
     w.dbase = w.e;
     w.dcount = min(64, e1 - w.e);
@@ -105,7 +107,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
     }
     sd.pre[lane] = incl - n;
     if (lane == 63) sd.pre[64] = incl;
-    __syncthreads();
+    wave_sync();
   }
   const int first = w.e - w.dbase;
   const int q0 = sd.pre[first] + w.sbase;
@@ -122,7 +124,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
       if (s0 < cnt && sd.pre[e + 1] > sd.pre[e]) sd.map[s0] = e;
     }
   }
-  __syncthreads();
+  wave_sync();
   int4 mv = m4[lane];
   mv.y = max(mv.y, mv.x);
   mv.z = max(mv.z, mv.y);
@@ -139,7 +141,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
   mv.z = max(mv.z, before);
   mv.w = max(mv.w, before);
   m4[lane] = mv;
-  __syncthreads();
+  wave_sync();
   // The lane's slots k = lane + 64 u, NB at a time: their body loads first
   // (slots past the stage's end load a body of the stage and store nothing),
   // then the stores.
@@ -176,7 +178,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
     w.e = w.dbase + lo;
     w.sbase = qn - sd.pre[lo];
   }
-  __syncthreads();  // the stage is filled
+  wave_sync();  // the stage is filled
   return cnt;
 }
 
@@ -187,6 +189,43 @@ __device__ inline int next_leaf(int *next, int lane) {
   if (lane == 0) v = atomicAdd(next, 1);
   return __shfl(v, 0) + (int)gridDim.x;
 }
+
+// Several waves per leaf (k_p2p_f64): wave 0 takes the leaf's own bodies, and
+// each of the W waves a contiguous part of the list through its own stage; the
+// waves' sums of a target are added in wave order.  (Not in the mixed form:
+// the split moves the boundaries of its FP32 runs, so that a system would give
+// other roundings alone than in a batch.)
+template <int W>
+struct Team {
+  double4 part[W > 1 ? W : 1][64];
+  int next;
+
+  __device__ int next_leaf(int *counter, int lane) {
+    if (W == 1) return exafmm::next_leaf(counter, lane);
+    __syncthreads();
+    if (threadIdx.x == 0) next = atomicAdd(counter, 1);
+    __syncthreads();
+    return next + (int)gridDim.x;
+  }
+
+  // Stores the sum of the waves' s (of lanes below n) to trg[lane].
+  __device__ void store(double4 s, int wave, int lane, int n, double4 *trg) {
+    if (W > 1) {
+      __syncthreads();  // the last sums have been read
+      part[wave][lane] = s;
+      __syncthreads();
+      if (wave != 0) return;
+      for (int w = 1; w < W; w++) {
+        const double4 o = part[w][lane];
+        s.x += o.x;
+        s.y += o.y;
+        s.z += o.z;
+        s.w += o.w;
+      }
+    }
+    if (lane < n) trg[lane] = make_double4(s.x, -s.y, -s.z, -s.w);
+  }
+};
 
 __global__ void k_zero_int(int *p) { *p = 0; }
 
@@ -216,35 +255,43 @@ struct TargetPasses {
   }
 };
 
-__global__ void __launch_bounds__(64)
+template <int W>
+__global__ void __launch_bounds__(64 * W)
     k_p2p_f64(const int *__restrict__ tgt_list, int ntl_host, const int *__restrict__ ntl_dev,
               int *__restrict__ next, const int *__restrict__ off, const int *__restrict__ src,
               const unsigned char *__restrict__ img, const int *__restrict__ cBody,
               const int *__restrict__ cNBody, const double4 *__restrict__ body, double4 *__restrict__ trg,
               double cycle) {
-  __shared__ double4 sb[kP2PStage];
+  __shared__ double4 stage[W][kP2PStage];
   // The group partials are combined in the stage buffer (every stage is
   // consumed by then): 8.6 KB of LDS per wave, which leaves more of each CU
   // to the other streams' kernels beside twelve resident waves.
-  double4 *const sacc = sb;
-  __shared__ SrcDesc sd;
-  const int lane = threadIdx.x;
+  __shared__ SrcDesc desc[W];
+  __shared__ Team<W> team;
+  const int lane = W > 1 ? threadIdx.x % 64 : threadIdx.x, wave = W > 1 ? threadIdx.x / 64 : 0;
+  double4 *const sb = stage[wave], *const sacc = sb;
+  SrcDesc &sd = desc[wave];
   // Target leaves: blockIdx.x first, then the next unclaimed one of the
   // work counter (leaves differ in cost; the grid may be smaller than ntl).
   // ntl_dev (if set): the count as the list grouping left it on the device.
   const int ntl = ntl_dev ? *ntl_dev : ntl_host;
-  for (int bi = blockIdx.x; bi < ntl; bi = next_leaf(next, lane)) {
+  for (int bi = blockIdx.x; bi < ntl; bi = team.next_leaf(next, lane)) {
     const int c = tgt_list[bi];
     const int tb0 = cBody[c], tn = cNBody[c];
-    const int e0 = off[c], e1 = off[c + 1];
+    int e0 = off[c], e1 = off[c + 1];
+    if (W > 1) {
+      const int ne = e1 - e0;
+      e1 = e0 + ne * (wave + 1) / W;
+      e0 += ne * wave / W;
+    }
     // Sum the G group partials (lanes gg T + i) of the pass's targets in
     // group order.
     auto combine = [&](const double4 &acc, int T, int G, int n, int tfirst) {
-      __syncthreads();
+      wave_sync();
       sacc[lane] = acc;
-      __syncthreads();
+      wave_sync();
+      double4 s = sacc[lane];
       if (lane < n) {
-        double4 s = sacc[lane];
         for (int gg = 1; gg < G; gg++) {
           const double4 o = sacc[gg * T + lane];
           s.x += o.x;
@@ -252,8 +299,8 @@ __global__ void __launch_bounds__(64)
           s.z += o.z;
           s.w += o.w;
         }
-        trg[tb0 + tfirst + lane] = make_double4(s.x, -s.y, -s.z, -s.w);
       }
+      team.store(s, wave, lane, n, trg + tb0 + tfirst);
     };
     for (int tbase = 0; tbase < tn; tbase += 64) {
       const int nt = min(64, tn - tbase);
@@ -365,7 +412,7 @@ __global__ void __launch_bounds__(64)
         const int g4 = kP2PUnroll * GA;
         const int cntp = (cnt + g4 - 1) / g4 * g4;
         for (int k = cnt + lane; k < cntp; k += 64) sb[k] = make_double4(kFar, kFar, kFar, 0);
-        __syncthreads();
+        wave_sync();
         const int ncp = __builtin_amdgcn_readfirstlane(cntp);
         pass(mask, GA, ncp, xa, ga, acca);
         if (tp.r > 0) pass_b(mask, ncp);
@@ -373,9 +420,9 @@ __global__ void __launch_bounds__(64)
       // The target leaf's own bodies first (masked), then the rest of the
       // list with the own entry left out (the traversal lists every leaf
       // against itself once).
-      for (int s0 = 0; s0 < tn; s0 += kP2PStage) {
+      for (int s0 = 0; wave == 0 && s0 < tn; s0 += kP2PStage) {
         const int cnt = min(kP2PStage, tn - s0);
-        __syncthreads();
+        wave_sync();
         for (int k = lane; k < cnt; k += 64) sb[k] = body[tb0 + s0 + k];
         run(std::true_type{}, cnt);
       }
@@ -1018,19 +1065,39 @@ __global__ void k_count_body_pairs(const int *__restrict__ tgt_list, int ntl, co
   atomicAdd(out, s * (unsigned long long)cNBody[c]);
 }
 
+// Waves per target leaf for a tree of `leaves` of them: the resident grid holds
+// 12 waves per CU, and below a few leaves for each the longest ones and the
+// latency of single waves decide the time.  64 leaves: 19 us with 8 waves each
+// against 85 with one; 994 leaves: 100 against 181; 4744 leaves of 500 000
+// bodies on a sphere: 1870 against 2157.
+static int p2p_team(const Handle &h, int64_t leaves) {
+  const int64_t waves = 12 * (int64_t)h.ncu;
+  if (leaves * 8 <= waves) return 8;
+  return leaves <= 2 * waves ? 4 : 1;
+}
+
 void run_p2p(Handle &h, hipStream_t st) {
   // Every body belongs to a leaf that is in its own list, and every target is
   // written once: the results need no clearing.
   if (h.np2p_tgt == 0) return;
+  // Leaves by the tree alone (with p2p_kmax == 1): the same for every grid.
+  int64_t leaves = h.ncells;
+  for (int l = 0; l + 1 < h.nlevels; l++) leaves -= std::min(h.lvl_par[l], h.lvl_off[l + 1] - h.lvl_off[l]);
+  const int W = h.p2p_kmax == 1 && h.cfg.precision == 0 ? p2p_team(h, std::max<int64_t>(1, leaves)) : 1;
   // A resident grid of p2p_wpc waves per CU that claims target leaves from a
-  // counter (0: one wave per leaf).  A resident grid leaves the rest of each
+  // counter (0: one team per leaf).  A resident grid leaves the rest of each
   // CU to the other stream's kernels (the lattice M2L set-up runs beside P2P
   // instead of queueing behind one wave per leaf); 12 waves (10.6 KB of LDS
   // and at most 128 VGPRs each) leave a third of the LDS and of the VGPRs.
   // The target count is read on the device when the host has not read it
   // back yet and the grid does not depend on it (a resident grid).
   const int *ntl_dev = nullptr;
-  int grid = h.p2p_wpc * h.ncu;
+  int64_t waves = (int64_t)h.p2p_wpc * h.ncu;
+  // Teams take no more of the chip than one wave per leaf would (two waves per
+  // CU at least): the contraction beside them is on the longer path (994
+  // leaves: 840 us per evaluation, 905 with the whole resident grid).
+  if (W > 1) waves = std::min(waves, std::max<int64_t>(leaves, 2 * h.ncu));
+  int grid = std::max(1, (int)(waves / W));
   if (h.np2p_tgt < 0 && h.p2p_wpc > 0) {
     ntl_dev = h.p2p_cnt_dev;
   } else {
@@ -1040,23 +1107,24 @@ void run_p2p(Handle &h, hipStream_t st) {
   }
   h.p2p_next.reserve(1);
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, h.p2p_next.p);
-  if (h.cfg.precision == 1 && h.p2p_kmax == 1)
-    hipLaunchKernelGGL(k_p2p_mixed, dim3(grid), dim3(64), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
+                       h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.body4.p, h.trg4.p, h.cfg.cycle);
+  };
+  auto launch_mixed = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
                        h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.cX.p, h.cRb.p, h.body4.p,
                        h.trg4.p, h.cfg.cycle);
-  else if (h.cfg.precision == 1) {
-    auto *kern = h.p2p_kmax == 3 ? k_p2p_mixed_rb<3> : h.p2p_kmax == 5 ? k_p2p_mixed_rb<5> : k_p2p_mixed_rb<4>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
-                       h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.cX.p, h.cRb.p, h.body4.p,
-                       h.trg4.p, h.cfg.cycle);
-  }
-  else if (h.p2p_kmax == 1)
-    hipLaunchKernelGGL(k_p2p_f64, dim3(grid), dim3(64), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
-                       h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.body4.p, h.trg4.p, h.cfg.cycle);
-  else {
-    auto *kern = h.p2p_kmax == 3 ? k_p2p_f64_rb<3> : h.p2p_kmax == 5 ? k_p2p_f64_rb<5> : k_p2p_f64_rb<4>;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
-                       h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.body4.p, h.trg4.p, h.cfg.cycle);
+  };
+  if (h.cfg.precision == 1) {
+    if (h.p2p_kmax != 1)
+      launch_mixed(h.p2p_kmax == 3 ? k_p2p_mixed_rb<3> : h.p2p_kmax == 5 ? k_p2p_mixed_rb<5> : k_p2p_mixed_rb<4>);
+    else
+      launch_mixed(k_p2p_mixed);
+  } else if (h.p2p_kmax != 1) {
+    launch(h.p2p_kmax == 3 ? k_p2p_f64_rb<3> : h.p2p_kmax == 5 ? k_p2p_f64_rb<5> : k_p2p_f64_rb<4>);
+  } else {
+    launch(W == 8 ? k_p2p_f64<8> : W == 4 ? k_p2p_f64<4> : k_p2p_f64<1>);
   }
   EXA_HIP(hipGetLastError());
 }
