@@ -116,8 +116,13 @@ struct Handle {
   // builder, forests).
   bool key_lvloff = false;
   std::vector<int> sys_off;
-  DBuf<int> sys_offd;
-  DBuf<double> sys_par;  // per-system builder parameters
+  // Uniform builder: per-system parameters and tables (with the host copy of
+  // what the tables were made from), bodies per possible leaf (all zero between
+  // builds if ut_zero) and prefix sums.
+  DBuf<double> ut_sys;
+  DBuf<int> ut_tab, ut_cnt, ut_start, ut_rank, ut_tot;
+  std::vector<int> ut_tab_host;
+  bool ut_zero = false;
   DBuf<double4> in4;     // caller order (x, y, z, q)
   DBuf<double4> body4;   // tree order
   DBuf<int> bidx;        // tree order -> caller index (Body::IBODY)
@@ -398,13 +403,10 @@ void exclusive_scan_int(Handle &h, const int *in, int *out, int n);
 // The same on stream st with temporary storage tmp (concurrent users).
 void exclusive_scan_int(const int *in, int *out, int n, hipStream_t st, DBuf<unsigned char> &tmp);
 void exclusive_scan_int4(Handle &h, const int4 *in, int4 *out, int n);  // component-wise
-void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bits,
-                        bool &result_in_alt);
-// The same over key bits [bit0, bit1), for the tree build (nothing runs beside it).
-void sort_pairs_u64_int_bits(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
-                             int bit1, bool &result_in_alt);
-void sort_pairs_int_int(Handle &h, int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits,
-                        bool &result_in_alt);
+// By key bits [bit0, bit1), for the tree build (nothing runs beside it).
+void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
+                        int bit1, bool &result_in_alt);
+// By the low `bits` of the key, on stream st with temporary storage tmp (concurrent users).
 void sort_pairs_int_int(int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits, bool &result_in_alt,
                         hipStream_t st, DBuf<unsigned char> &tmp);
 

@@ -5,8 +5,11 @@
 // Layout produced (identical to build_tree_omp.h after reverseOrder,
 // :200-211): cells are level-contiguous, root first; inside a level they run
 // in descending Morton order; bodies run in ascending Morton order (stable).
+#include <algorithm>
+#include <climits>
 #include <cmath>
 
+#include "device_util.h"
 #include "internal.h"
 
 namespace exafmm {
@@ -47,7 +50,8 @@ __global__ void __launch_bounds__(256) k_bounds_partial(const double4 *__restric
   if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__ part, int nb, double *__restrict__ out) {
+__global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__ part, int nb, double *__restrict__ out,
+                                                      double *__restrict__ host) {
   __shared__ double s[6][256];
   double r[6];
   for (int d = 0; d < 6; d++) r[d] = part[d];
@@ -68,7 +72,7 @@ __global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__
       }
     __syncthreads();
   }
-  if (threadIdx.x < 6) out[threadIdx.x] = s[threadIdx.x][0];
+  if (threadIdx.x < 6) out[threadIdx.x] = host[threadIdx.x] = s[threadIdx.x][0];
 }
 
 // The bounds stay on the device for the builder; the host copy (xmin,
@@ -86,8 +90,8 @@ void run_bounds(Handle &h) {
   const int nb = std::min(kBoundsBlocks, div_up(h.n, 256));
   h.red.reserve(6 * nb);
   hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(256), 0, h.stream, h.in4.p, h.n, h.red.p);
-  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, h.stream, h.red.p, nb, h.box.p);
-  EXA_HIP(hipMemcpyAsync(h.hpin + Handle::kPinBounds, h.box.p, 6 * sizeof(double), hipMemcpyDeviceToHost, h.stream));
+  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, h.stream, h.red.p, nb, h.box.p,
+                     reinterpret_cast<double *>(h.hpin + Handle::kPinBounds));
   EXA_HIP(hipEventRecord(h.ev_bounds, h.stream));
   h.bounds_pending = true;
   h.have_bounds = true;
@@ -115,316 +119,89 @@ void upload_bounds(Handle &h) {
 }
 
 // ---------------------------------------------------------------------------
-// Uniform builder kernels.
+// Uniform trees: one system, or a forest of independent systems (batched
+// evaluation).  System s owns bodies [begin, end) of the input and gets its own
+// bounds, depth L and Morton keys; level t holds the level-t cells of every
+// system with L >= t, and a system's cells come in the order of its
+// single-system build.
+//
+// A tree of depth L has 8^L possible leaves, at most 8 per ncrit bodies, so
+// leaves are counted and found by index: bodies per leaf (atomic counts), a
+// prefix sum for the leaves' first bodies, bodies scattered into their leaves
+// (in any order) and each leaf's bodies sorted by input index, which is the
+// order a stable sort by key gives.  A cell of any level is a run of leaves, so
+// the same prefix sum says whether it holds bodies, and a second one over the
+// possible cells of all levels numbers those that do.  Bound by launches up to
+// about 100k bodies, then by the counting atomics (50 us at 1M).  A radix sort
+// of the keys with head flags, scans and compactions over all bodies for every
+// level took 24 launches and more; this takes 9 to 12, and whole evaluations of
+// 2000, 100k and 1M bodies and of 32 systems of 1000 to 8000 went from 440 to
+// 380, 875 to 793, 4380 to 4280 and 1720 to 1540 us.
+// A leaf with very many bodies (systems clustered in a corner of their cube) is
+// sorted by one wave, 10 ms at 500k; its P2P takes seconds.
+constexpr int kMaxUniformLevels = 10;  // the reference's int keys hold 3 x 10 bits
 
-// getKey (build_tree_omp.h:36-57): float cell size promoted to double for
-// the division, truncation to int, bit interleave in int.
-// (The key has 3 * level <= 30 bits: it is kept as a 32-bit int for the
-// radix sort; k_widen_keys turns the sorted keys into the 64-bit form.)
-// bounds2box (build_tree_omp.h:21-33) on the device: bb = the bounds
-// (xmin, xmax); box = (x0, y0, z0, d) with d the float leaf cell size of a
-// depth-L grid (:218-220), the same double operations as the reference.
-__global__ void k_box(const double *__restrict__ bb, int L, double *__restrict__ box) {
-  double Xc[3], R0 = 0;
-  for (int d = 0; d < 3; d++) Xc[d] = (bb[3 + d] + bb[d]) / 2;
+struct ForestSys {
+  double x0, y0, z0;  // bounds minimum (the key origin)
+  float d;            // leaf cell size, 2 R0 / 2^L
+  int L;              // depth
+  int begin, end;     // body range
+  int leaf0;          // first of its possible leaves
+};
+
+// Possible cells: level t's are [lev0[t], lev0[t + 1]), system s's part of it
+// from base[t (S + 1) + s] on (8^t of them, none if L < t).
+struct TreeShape {
+  int S, nlev, nleaf, ncell;
+  int lev0[kMaxUniformLevels + 2];
+  const int *base;
+};
+
+// bounds2box (build_tree_omp.h:21-33) and the leaf cell size (:218-220), a
+// float, with the reference's double operations.
+__device__ inline void set_box(const double *mn, const double *mx, ForestSys &f) {
+  double R0 = 0;
   for (int d = 0; d < 3; d++) {  // std::max(a, R0) = a < R0 ? R0 : a
-    const double a = Xc[d] - bb[d], b = bb[3 + d] - Xc[d];
+    const double Xc = (mx[d] + mn[d]) / 2;
+    const double a = Xc - mn[d], b = mx[d] - Xc;
     R0 = a < R0 ? R0 : a;
     R0 = b < R0 ? R0 : b;
   }
   R0 *= 1.00001;
-  const float d = 2 * R0 / (1 << L);
-  box[0] = bb[0];
-  box[1] = bb[1];
-  box[2] = bb[2];
-  box[3] = d;
+  f.x0 = mn[0];
+  f.y0 = mn[1];
+  f.z0 = mn[2];
+  f.d = 2 * R0 / (1 << f.L);
 }
 
-__global__ void k_morton32(const double4 *__restrict__ in, int n, const double *__restrict__ box, int level,
-                           int *__restrict__ key, int *__restrict__ idx) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= n) return;
-  const double4 v = in[b];
-  const double x0 = box[0], y0 = box[1], z0 = box[2];
-  const double dd = (double)(float)box[3];
-  int ix = (int)((v.x - x0) / dd);
-  int iy = (int)((v.y - y0) / dd);
-  int iz = (int)((v.z - z0) / dd);
-  int id = 0;
-  for (int l = 0; l != level; ++l) {
-    id += (ix & 1) << (3 * l);
-    id += (iy & 1) << (3 * l + 1);
-    id += (iz & 1) << (3 * l + 2);
-    ix >>= 1;
-    iy >>= 1;
-    iz >>= 1;
+__global__ void k_box(const double *__restrict__ bb, ForestSys *__restrict__ fs) { set_box(bb, bb + 3, fs[0]); }
+
+// Per-system min/max: chunks (system, first, last body), one workgroup each,
+// then one workgroup per system over its chunks [chunk0[s], chunk0[s + 1]).
+__device__ inline void block_minmax(double *mn, double *mx, double (*s)[256]) {
+  for (int d = 0; d < 3; d++) {
+    s[d][threadIdx.x] = mn[d];
+    s[3 + d][threadIdx.x] = mx[d];
   }
-  key[b] = id;
-  idx[b] = b;
-}
-
-__global__ void k_widen_keys(const int *__restrict__ k32, int n, uint64_t *__restrict__ k64) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) k64[i] = (uint64_t)(int64_t)k32[i];
-}
-
-__global__ void k_gather_bodies(const double4 *__restrict__ in, const int *__restrict__ order, int n,
-                                double4 *__restrict__ out, int *__restrict__ bidx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int s = order[i];
-  out[i] = in[s];
-  bidx[i] = s;
-}
-
-// Head flags of tree level t: body i starts a level-t cell when its key
-// prefix (key >> shift) differs from body i-1's.  flags has n+1 entries; the
-// last is 0 so that the exclusive scan yields the total at index n.
-// out[i] = in[i * stride], i < n (n small).
-constexpr int kMaxUniformLevels = 10;  // the reference's int keys hold 3 x 10 bits
-
-__global__ void k_strided_gather(const int *__restrict__ in, int64_t stride, int n, int *__restrict__ out) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = in[(int64_t)i * stride];
-}
-
-__global__ void k_level_positions(const int *__restrict__ flags, const int *__restrict__ scan, int n,
-                                  int *__restrict__ pos) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (flags[i]) pos[scan[i]] = i;
-}
-
-// All levels at once (level t = blockIdx.y; arrays of stride n + 1 per level).
-__global__ void k_level_heads_all(const uint64_t *__restrict__ key, int n, int L, int64_t stride,
-                                  int *__restrict__ flags) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
-  if (i > n) return;
-  const int shift = 3 * (L - t);
-  int f = 0;
-  if (i < n) f = (i == 0) || ((key[i] >> shift) != (key[i - 1] >> shift));
-  flags[t * stride + i] = f;
-}
-
-// One exclusive scan ran over all levels: subtract each level's start.
-__global__ void k_level_rebase(int *__restrict__ scan, int n, int64_t stride, const int *__restrict__ base) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
-  if (i <= n) scan[t * stride + i] -= base[t];
-}
-
-struct LevelOffsets {
-  int v[kMaxUniformLevels + 1];
-};
-
-__global__ void k_level_positions_all(const int *__restrict__ flags, const int *__restrict__ scan, int n,
-                                      int64_t stride, LevelOffsets posoff, int *__restrict__ pos) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y;
-  if (i >= n) return;
-  if (flags[t * stride + i]) pos[posoff.v[t] + scan[t * stride + i]] = i;
-}
-
-struct LevelArgs {
-  const int *pos;      // heads of this level, ascending
-  const int *scan;     // exclusive scan of this level's flags (n+1)
-  const int *scan_up;  // scan of level t-1 (or nullptr at the root)
-  const int *scan_dn;  // scan of level t+1 (or nullptr at the leaves)
-  int count, count_up, count_dn;
-  int off, off_up, off_dn;
-  int shift;           // 3 * (L - t)
-  int leaf;            // 1 at the finest level
-  int level;
-};
-
-// bodies2leafs / leafs2cells (build_tree_omp.h:130-198) fused with the index
-// arithmetic of reverseOrder: ascending rank r at level t lands at
-// off_t + count_t - 1 - r.
-__device__ inline void level_cell(const LevelArgs &a, const double4 *__restrict__ body,
-                                  const uint64_t *__restrict__ key, int n, int nc, const double *__restrict__ box,
-                                  double4 *__restrict__ cX, double *__restrict__ cRb, int *__restrict__ cParent,
-                                  int *__restrict__ cChild, int *__restrict__ cNChild, int *__restrict__ cBody,
-                                  int *__restrict__ cNBody, uint64_t *__restrict__ cKey, int *__restrict__ cLevel) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= a.count) return;
-  const int start = a.pos[r];
-  const int end = (r + 1 < a.count) ? a.pos[r + 1] : n;
-  const int c = a.off + a.count - 1 - r;
-  const double4 v = body[start];
-  const double x0 = box[0], y0 = box[1], z0 = box[2];
-  float dt = (float)box[3];
-  for (int l = 0; l < a.shift / 3; l++) dt *= 2;  // leafs2cells doubles d per level (:166)
-  const double dd = (double)dt;
-  const int ix = (int)((v.x - x0) / dd);
-  const int iy = (int)((v.y - y0) / dd);
-  const int iz = (int)((v.z - z0) / dd);
-  double4 X;
-  X.x = dd * (ix + .5) + x0;
-  X.y = dd * (iy + .5) + y0;
-  X.z = dd * (iz + .5) + z0;
-  X.w = dd * .5;
-  cX[c] = X;
-  cRb[c] = X.w;
-  cBody[c] = start;
-  cNBody[c] = end - start;
-  cKey[c] = (uint64_t)(int64_t)(int)(key[start] >> a.shift);
-  cLevel[c] = a.level;
-  if (a.leaf) {
-    cNChild[c] = 0;
-    cChild[c] = nc;  // reverseOrder maps ICHILD = 0 of a leaf to numCells
-  } else {
-    const int lo = a.scan_dn[start], hi = a.scan_dn[end];
-    cNChild[c] = hi - lo;
-    cChild[c] = a.off_dn + a.count_dn - hi;
-  }
-  if (a.level == 0) {
-    cParent[c] = nc - 1;  // reverseOrder maps the root's IPARENT = 0 to numCells-1
-  } else {
-    const int rp = a.scan_up[start + 1] - 1;
-    cParent[c] = a.off_up + a.count_up - 1 - rp;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w)
+      for (int d = 0; d < 3; d++) {
+        const double a = s[d][threadIdx.x + w];
+        s[d][threadIdx.x] = a < s[d][threadIdx.x] ? a : s[d][threadIdx.x];
+        const double c = s[3 + d][threadIdx.x + w];
+        s[3 + d][threadIdx.x] = c > s[3 + d][threadIdx.x] ? c : s[3 + d][threadIdx.x];
+      }
+    __syncthreads();
   }
 }
 
-struct LevelArgsAll {
-  LevelArgs a[kMaxUniformLevels + 1];
-};
+constexpr int kBoundsChunk = 4096;
 
-// k_level_cells of every level in one launch (level t = blockIdx.y).
-__global__ void k_level_cells_all(LevelArgsAll all, const double4 *__restrict__ body, const uint64_t *__restrict__ key,
-                                  int n, int nc, const double *__restrict__ box, double4 *__restrict__ cX,
-                                  double *__restrict__ cRb, int *__restrict__ cParent, int *__restrict__ cChild,
-                                  int *__restrict__ cNChild, int *__restrict__ cBody, int *__restrict__ cNBody,
-                                  uint64_t *__restrict__ cKey, int *__restrict__ cLevel) {
-  level_cell(all.a[blockIdx.y], body, key, n, nc, box, cX, cRb, cParent, cChild, cNChild, cBody, cNBody, cKey, cLevel);
-}
-
-__global__ void k_iota(int *__restrict__ a, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = i;
-}
-
-void run_build_uniform(Handle &h) {
-  const int n = h.n;
-  const int ncrit = h.cfg.ncrit;
-  // build_tree_omp.h:218 (integer n / ncrit inside the log).
-  const int L = n >= ncrit ? 1 + int(std::log((double)(n / ncrit)) / M_LN2 / 3) : 0;
-  if (L > 10) throw Error(EXAFMM_HIP_EUNSUP, "uniform tree deeper than 10 levels overflows the reference's int keys");
-  upload_bounds(h);
-  hipLaunchKernelGGL(k_box, dim3(1), dim3(1), 0, h.stream, h.box.p, L, h.box.p + 8);
-
-  h.k64a.reserve(n + 1);
-  h.k64b.reserve(n + 1);
-  h.ia.reserve(n + 1);
-  h.ib.reserve(n + 1);
-  h.body4.resize(n);
-  h.bidx.resize(n);
-  h.trg4.resize(n);
-  const int T = 256;
-  // Keys of 3 L <= 30 bits: sorted as 32-bit ints (a radix sort over 64-bit
-  // keys takes several times as many passes), then widened.  k64b holds the
-  // two 32-bit key buffers.
-  int *k32 = reinterpret_cast<int *>(h.k64b.p), *k32alt = k32 + (n + 1);
-  hipLaunchKernelGGL(k_morton32, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, n, h.box.p + 8, L, k32, h.ia.p);
-  bool alt = false;
-  sort_pairs_int_int(h, k32, k32alt, h.ia.p, h.ib.p, n, 3 * L, alt);
-  hipLaunchKernelGGL(k_widen_keys, dim3(div_up(n, T)), dim3(T), 0, h.stream, alt ? k32alt : k32, n, h.k64a.p);
-  uint64_t *key = h.k64a.p;
-  int *order = alt ? h.ib.p : h.ia.p;
-  hipLaunchKernelGGL(k_gather_bodies, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, order, n, h.body4.p, h.bidx.p);
-
-  // Per-level heads and scans: (L+1) x (n+1) ints each.
-  const size_t stride = (size_t)n + 1;
-  h.ic.reserve(stride * (L + 1));  // flags
-  h.id.reserve(stride * (L + 1));  // scans
-  std::vector<int> counts(L + 1);
-  std::vector<int> tot(L + 1);
-  // Heads of every level, one exclusive scan over all levels, each level's
-  // start subtracted: the per-level exclusive scans.
-  h.cnt.reserve(2 * (L + 1));
-  hipLaunchKernelGGL(k_level_heads_all, dim3(div_up(n + 1, T), L + 1), dim3(T), 0, h.stream, key, n, L,
-                     (int64_t)stride, h.ic.p);
-  exclusive_scan_int(h, h.ic.p, h.id.p, (int)(stride * (L + 1)));
-  hipLaunchKernelGGL(k_strided_gather, dim3(1), dim3(64), 0, h.stream, h.id.p, (int64_t)stride, L + 1,
-                     h.cnt.p + L + 1);
-  hipLaunchKernelGGL(k_level_rebase, dim3(div_up(n + 1, T), L + 1), dim3(T), 0, h.stream, h.id.p, n, (int64_t)stride,
-                     h.cnt.p + L + 1);
-  // Totals: scan[n] of each level, gathered on the device, one read-back.
-  hipLaunchKernelGGL(k_strided_gather, dim3(1), dim3(64), 0, h.stream, h.id.p + n, (int64_t)stride, L + 1, h.cnt.p);
-  EXA_HIP(hipMemcpyAsync(tot.data(), h.cnt.p, (L + 1) * sizeof(int), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipStreamSynchronize(h.stream));
-  sync_bounds(h);  // (arrived before the totals)
-  int nc = 0;
-  std::vector<int> off(L + 2, 0);
-  for (int t = 0; t <= L; t++) {
-    counts[t] = tot[t];
-    off[t] = nc;
-    nc += counts[t];
-  }
-  off[L + 1] = nc;
-  h.ncells = nc;
-  h.nlevels = L + 1;
-  h.ie.reserve(nc + 1);  // positions, level after level
-  LevelOffsets posoff{};
-  {
-    int o = 0;
-    for (int t = 0; t <= L; t++) {
-      posoff.v[t] = o;
-      o += counts[t];
-    }
-  }
-  hipLaunchKernelGGL(k_level_positions_all, dim3(div_up(n, T), L + 1), dim3(T), 0, h.stream, h.ic.p, h.id.p, n,
-                     (int64_t)stride, posoff, h.ie.p);
-  h.cX.resize(nc);
-  h.cRb.resize(nc);
-  h.cParent.resize(nc);
-  h.cChild.resize(nc);
-  h.cNChild.resize(nc);
-  h.cBody.resize(nc);
-  h.cNBody.resize(nc);
-  h.cKey.resize(nc);
-  h.cLevel.resize(nc);
-  LevelArgsAll all{};
-  int maxcount = 0;
-  for (int t = 0; t <= L; t++) {
-    LevelArgs &a = all.a[t];
-    a.pos = h.ie.p + posoff.v[t];
-    a.scan = h.id.p + stride * t;
-    a.scan_up = t > 0 ? h.id.p + stride * (t - 1) : nullptr;
-    a.scan_dn = t < L ? h.id.p + stride * (t + 1) : nullptr;
-    a.count = counts[t];
-    a.count_up = t > 0 ? counts[t - 1] : 0;
-    a.count_dn = t < L ? counts[t + 1] : 0;
-    a.off = off[t];
-    a.off_up = t > 0 ? off[t - 1] : 0;
-    a.off_dn = t < L ? off[t + 1] : 0;
-    a.shift = 3 * (L - t);
-    a.leaf = (t == L);
-    a.level = t;
-    maxcount = std::max(maxcount, counts[t]);
-  }
-  hipLaunchKernelGGL(k_level_cells_all, dim3(div_up(maxcount, T), L + 1), dim3(T), 0, h.stream, all, h.body4.p, key, n,
-                     nc, h.box.p + 8, h.cX.p, h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p,
-                     h.cBody.p, h.cNBody.p, h.cKey.p, h.cLevel.p);
-  // Level order: the layout is already level-contiguous.
-  h.lvl_off.assign(off.begin(), off.begin() + L + 2);
-  h.lvl_par = counts;  // (all but the leaves)
-  h.leaf_level = L;
-  h.lvl_cells.resize(nc);
-  hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
-  EXA_HIP(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Forest of uniform trees (batched evaluation of independent systems).
-// System s owns bodies [off[s], off[s+1]) of the input and gets its own
-// bounds, depth L_s and Morton keys exactly as a single-system build of its
-// bodies would (the same float/int arithmetic); the bodies are sorted by
-// (s, key_s), so systems stay contiguous and in input order.  Level t holds
-// the level-t cells of every system with L_s >= t; a system's cells are the
-// ones its single-system build makes, in the same relative order.
-
-// Per-system min/max, one workgroup per system.
 __global__ void __launch_bounds__(256)
-    k_bounds_seg(const double4 *__restrict__ b, const int *__restrict__ off, double *__restrict__ out) {
+    k_bounds_chunks(const double4 *__restrict__ b, const int2 *__restrict__ chunk, double *__restrict__ out) {
   __shared__ double s[6][256];
-  const int sys = blockIdx.x, i0 = off[sys], i1 = off[sys + 1];
+  const int i0 = chunk[blockIdx.x].x, i1 = chunk[blockIdx.x].y;
   double mn[3] = {b[i0].x, b[i0].y, b[i0].z};
   double mx[3] = {mn[0], mn[1], mn[2]};
   for (int i = i0 + threadIdx.x; i < i1; i += 256) {
@@ -436,52 +213,55 @@ __global__ void __launch_bounds__(256)
     mx[1] = v.y > mx[1] ? v.y : mx[1];
     mx[2] = v.z > mx[2] ? v.z : mx[2];
   }
-  for (int d = 0; d < 3; d++) {
-    s[d][threadIdx.x] = mn[d];
-    s[3 + d][threadIdx.x] = mx[d];
-  }
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-      for (int d = 0; d < 3; d++) {
-        const double a = s[d][threadIdx.x + w], c = s[3 + d][threadIdx.x + w];
-        s[d][threadIdx.x] = a < s[d][threadIdx.x] ? a : s[d][threadIdx.x];
-        s[3 + d][threadIdx.x] = c > s[3 + d][threadIdx.x] ? c : s[3 + d][threadIdx.x];
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) out[6 * sys + threadIdx.x] = s[threadIdx.x][0];
+  block_minmax(mn, mx, s);
+  if (threadIdx.x < 6) out[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
 }
 
-struct ForestSys {
-  double x0, y0, z0;  // bounds minimum (the key origin)
-  float d;            // leaf cell size, 2 R0 / 2^L
-  int L;              // depth
-  int begin, end;     // body range
-};
+__global__ void __launch_bounds__(256)
+    k_bounds_systems(const double *__restrict__ part, const int *__restrict__ chunk0, ForestSys *__restrict__ fs) {
+  __shared__ double s[6][256];
+  const int c0 = chunk0[blockIdx.x], c1 = chunk0[blockIdx.x + 1];
+  double mn[3], mx[3];
+  for (int d = 0; d < 3; d++) {
+    mn[d] = part[6 * c0 + d];
+    mx[d] = part[6 * c0 + 3 + d];
+  }
+  for (int c = c0 + threadIdx.x; c < c1; c += 256)
+    for (int d = 0; d < 3; d++) {
+      const double a = part[6 * c + d], b = part[6 * c + 3 + d];
+      mn[d] = a < mn[d] ? a : mn[d];
+      mx[d] = b > mx[d] ? b : mx[d];
+    }
+  block_minmax(mn, mx, s);
+  if (threadIdx.x == 0) {
+    const double a[3] = {s[0][0], s[1][0], s[2][0]}, b[3] = {s[3][0], s[4][0], s[5][0]};
+    set_box(a, b, fs[blockIdx.x]);
+  }
+}
 
-// System of every body (input order), by binary search over the offsets.
-__global__ void k_sys_of(const int *__restrict__ off, int nsys, int n, int *__restrict__ sys) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int lo = 0, hi = nsys;  // largest s with off[s] <= i
+// Largest s with v[s] <= x, 0 <= s < n (v ascending, v[0] <= x).
+__device__ inline int last_le(const int *__restrict__ v, int n, int x) {
+  int lo = 0, hi = n;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (off[mid] <= i)
+    if (v[mid] <= x)
       lo = mid;
     else
       hi = mid;
   }
-  sys[i] = lo;
+  return lo;
 }
 
-// Sort key (s << 32) | key_s, key_s from getKey at the system's depth.
-__global__ void k_morton_forest(const double4 *__restrict__ in, int n, const int *__restrict__ sys,
-                                const ForestSys *__restrict__ fs, uint64_t *__restrict__ key, int *__restrict__ idx) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// getKey (build_tree_omp.h:36-57): float cell size promoted to double for the
+// division, truncation to int, bit interleave in int.  leaf[b] = the body's
+// leaf among all systems' possible ones, slot[b] = its place there.
+__global__ void __launch_bounds__(256)
+    k_leaf_count(const double4 *__restrict__ in, int n, const ForestSys *__restrict__ fs, int S,
+                 const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ slot,
+                 int *__restrict__ cnt) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
   if (b >= n) return;
-  const int s = sys[b];
-  const ForestSys f = fs[s];
+  const ForestSys f = fs[S > 1 ? last_le(begin, S, b) : 0];
   const double4 v = in[b];
   const double dd = (double)f.d;
   int ix = (int)((v.x - f.x0) / dd);
@@ -496,48 +276,156 @@ __global__ void k_morton_forest(const double4 *__restrict__ in, int n, const int
     iy >>= 1;
     iz >>= 1;
   }
-  key[b] = ((uint64_t)s << 32) | (uint32_t)id;
-  idx[b] = b;
+  leaf[b] = f.leaf0 + id;
+  slot[b] = atomicAdd(&cnt[f.leaf0 + id], 1);
 }
 
-__device__ inline bool forest_prefix(uint64_t k, const ForestSys *__restrict__ fs, int t, int &s, uint32_t &pre) {
-  s = (int)(k >> 32);
-  const int L = fs[s].L;
-  if (t > L) return false;
-  pre = (uint32_t)k >> (3 * (L - t));
-  return true;
+// Level, system and index of possible cell e.
+__device__ inline void cell_of(const TreeShape &sh, int e, int &t, int &s, int &k) {
+  t = 0;
+  while (t + 1 < sh.nlev && e >= sh.lev0[t + 1]) t++;
+  const int *b = sh.base + t * (sh.S + 1);
+  s = sh.S > 1 ? last_le(b, sh.S, e) : 0;
+  k = e - b[s];
 }
 
-__global__ void k_level_heads_forest(const uint64_t *__restrict__ key, int n, int t, const ForestSys *__restrict__ fs,
-                                     int *__restrict__ flags) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > n) return;
-  int f = 0;
-  int s, s2;
-  uint32_t p, p2;
-  if (i < n && forest_prefix(key[i], fs, t, s, p))
-    f = i == 0 || !forest_prefix(key[i - 1], fs, t, s2, p2) || s2 != s || p2 != p;
-  flags[i] = f;
+// First body and end of the run of leaves that cell (t, s, k) covers.
+__device__ inline void cell_bodies(const ForestSys &f, const int *__restrict__ start, int t, int k, int &b0, int &b1) {
+  const int sh = 3 * (f.L - t);
+  b0 = start[f.leaf0 + (k << sh)];
+  b1 = start[f.leaf0 + ((k + 1) << sh)];
 }
 
-// As k_level_cells, with the system's origin and cell size, the cell's body
-// range cut at its system's end, and leaves wherever no child heads follow.
-__global__ void k_level_cells_forest(LevelArgs a, const double4 *__restrict__ body, const uint64_t *__restrict__ key,
-                                     int n, int nc, const ForestSys *__restrict__ fs, double4 *__restrict__ cX,
-                                     double *__restrict__ cRb, int *__restrict__ cParent, int *__restrict__ cChild,
-                                     int *__restrict__ cNChild, int *__restrict__ cBody, int *__restrict__ cNBody,
-                                     uint64_t *__restrict__ cKey, int *__restrict__ cLevel) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= a.count) return;
-  const int start = a.pos[r];
-  const int sys = (int)(key[start] >> 32);
-  const ForestSys f = fs[sys];
-  int end = (r + 1 < a.count) ? a.pos[r + 1] : n;
-  end = end < f.end ? end : f.end;
-  const int c = a.off + a.count - 1 - r;
+__device__ inline int cell_used(const TreeShape &sh, const ForestSys *__restrict__ fs, const int *__restrict__ start,
+                                int e) {
+  if (e >= sh.ncell) return 0;
+  int t, s, k, b0, b1;
+  cell_of(sh, e, t, s, k);
+  cell_bodies(fs[s], start, t, k, b0, b1);
+  return b1 > b0;
+}
+
+// Prefix sums in chunks of kScanChunk: totals per chunk, then each chunk's
+// offsets from the totals before it.  USED: of the cells' flags, else of the
+// counts.
+constexpr int kScanChunk = 4096;
+
+template <bool USED>
+__device__ inline int4 scan_load(const TreeShape &sh, const ForestSys *__restrict__ fs, const int *src, int i, int n) {
+  int v[4];
+  for (int k = 0; k < 4; k++) v[k] = i + k >= n ? 0 : USED ? cell_used(sh, fs, src, i + k) : src[i + k];
+  return make_int4(v[0], v[1], v[2], v[3]);
+}
+
+// The counts, read for the last time, are left at zero for the next build.
+__device__ inline void clear_counts(int *cnt, int i, int n) {
+  for (int k = 0; k < 4; k++)
+    if (i + k < n) cnt[i + k] = 0;
+}
+
+__device__ inline void scan_store(int *__restrict__ out, int i, int n, int at, int4 v) {
+  const int w[4] = {v.x, v.y, v.z, v.w};
+  for (int k = 0; k < 4; k++) {
+    if (i + k <= n) out[i + k] = at;  // out[n]: the total
+    at += w[k];
+  }
+}
+
+template <bool USED>
+__global__ void __launch_bounds__(1024)
+    k_tree_totals(TreeShape sh, const ForestSys *__restrict__ fs, const int *__restrict__ src, int n,
+                  int *__restrict__ tot) {
+  const int4 v = scan_load<USED>(sh, fs, src, blockIdx.x * kScanChunk + 4 * threadIdx.x, n);
+  int4 sum;
+  block_exscan4<1024>(make_int4(v.x + v.y + v.z + v.w, 0, 0, 0), &sum);
+  if (threadIdx.x == 0) tot[blockIdx.x] = sum.x;
+}
+
+template <bool USED>
+__global__ void __launch_bounds__(1024)
+    k_tree_offsets(TreeShape sh, const ForestSys *__restrict__ fs, int *src, int n,
+                   const int *__restrict__ tot, int *__restrict__ out) {
+  int before = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += 1024) before += tot[b];
+  int4 base, sum;
+  block_exscan4<1024>(make_int4(before, 0, 0, 0), &base);
+  const int i = blockIdx.x * kScanChunk + 4 * threadIdx.x;
+  const int4 v = scan_load<USED>(sh, fs, src, i, n);
+  if (!USED) clear_counts(src, i, n);
+  const int4 at = block_exscan4<1024>(make_int4(v.x + v.y + v.z + v.w, 0, 0, 0), &sum);
+  scan_store(out, i, n, base.x + at.x, v);
+}
+
+// Both prefix sums of a small tree in one workgroup.
+constexpr int kScanSmall = 4 * kScanChunk;
+// Cells up to which the cell arrays are sized by what is possible, about 100
+// bytes each, to spare the host a wait for the count.
+constexpr int kCellsUnread = 1 << 21;
+
+__global__ void __launch_bounds__(1024)
+    k_tree_scan_small(TreeShape sh, const ForestSys *__restrict__ fs, int *__restrict__ cnt, int *start,
+                      int *rank) {
+  for (int pass = 0; pass < 2; pass++) {
+    const int n = pass ? sh.ncell : sh.nleaf;
+    int run = 0;
+    for (int c = 0; c <= n; c += kScanChunk) {
+      const int i = c + 4 * threadIdx.x;
+      const int4 v = pass ? scan_load<true>(sh, fs, start, i, n) : scan_load<false>(sh, fs, cnt, i, n);
+      if (!pass) clear_counts(cnt, i, n);
+      int4 sum;
+      const int4 at = block_exscan4<1024>(make_int4(v.x + v.y + v.z + v.w, 0, 0, 0), &sum);
+      scan_store(pass ? rank : start, i, n, run + at.x, v);
+      run += sum.x;
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
+}
+
+// Bodies into their leaves' ranges.
+__global__ void __launch_bounds__(256)
+    k_leaf_scatter(const int *__restrict__ leaf, const int *__restrict__ slot, int n, const int *__restrict__ start,
+                   int *__restrict__ ord) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b < n) ord[start[leaf[b]] + slot[b]] = b;
+}
+
+// Every leaf's bodies in input order.
+__global__ void __launch_bounds__(64)
+    k_leaf_order(const int *__restrict__ start, int bits, int *__restrict__ ord, int *__restrict__ aux,
+                 const double4 *__restrict__ in, double4 *__restrict__ body, int *__restrict__ bidx) {
+  __shared__ RangeSortLds sh;
+  const int b = start[blockIdx.x], n = start[blockIdx.x + 1] - b;
+  if (n <= 0) return;
+  sort_range(ord + b, aux + b, n, bits, sh, [&](int rank, int e) {
+    body[b + rank] = in[e];
+    bidx[b + rank] = e;
+  });
+}
+
+// bodies2leafs / leafs2cells (build_tree_omp.h:130-198) fused with the index
+// arithmetic of reverseOrder: the r-th cell of a level in ascending order
+// lands at the level's offset + count - 1 - r.  rank: prefix sum of the cells'
+// flags, so rank[lev0[t]] is the offset of level t.  Runs before the host
+// knows the number of cells (kCellsUnread).
+__global__ void k_uniform_cells(TreeShape sh, const ForestSys *__restrict__ fs, const int *__restrict__ start,
+                                const int *__restrict__ rank, const double4 *__restrict__ body,
+                                double4 *__restrict__ cX, double *__restrict__ cRb, int *__restrict__ cParent,
+                                int *__restrict__ cChild, int *__restrict__ cNChild, int *__restrict__ cBody,
+                                int *__restrict__ cNBody, uint64_t *__restrict__ cKey, int *__restrict__ cLevel,
+                                int *__restrict__ lvl_cells, int *__restrict__ host_off) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e <= sh.nlev) host_off[e] = rank[sh.lev0[e]];
+  if (e >= sh.ncell || rank[e + 1] == rank[e]) return;
+  int t, s, k, b0, b1;
+  cell_of(sh, e, t, s, k);
+  const ForestSys f = fs[s];
+  cell_bodies(f, start, t, k, b0, b1);
+  const int nc = rank[sh.ncell];
+  const int c = rank[sh.lev0[t]] + rank[sh.lev0[t + 1]] - 1 - rank[e];
+  const double4 v = body[b0];
   float dt = f.d;
-  for (int l = 0; l < f.L - a.level; l++) dt *= 2;  // leafs2cells doubles d per level (:166)
-  const double4 v = body[start];
+  for (int l = 0; l < f.L - t; l++) dt *= 2;  // leafs2cells doubles d per level (:166)
   const double dd = (double)dt;
   const int ix = (int)((v.x - f.x0) / dd);
   const int iy = (int)((v.y - f.y0) / dd);
@@ -549,146 +437,180 @@ __global__ void k_level_cells_forest(LevelArgs a, const double4 *__restrict__ bo
   X.w = dd * .5;
   cX[c] = X;
   cRb[c] = X.w;
-  cBody[c] = start;
-  cNBody[c] = end - start;
-  cKey[c] = (uint64_t)(int64_t)(int)((uint32_t)key[start] >> (3 * (f.L - a.level)));
-  cLevel[c] = a.level;
-  const int nch = a.scan_dn ? a.scan_dn[end] - a.scan_dn[start] : 0;
-  if (nch == 0) {
+  cBody[c] = b0;
+  cNBody[c] = b1 - b0;
+  cKey[c] = (uint64_t)(int64_t)k;
+  cLevel[c] = t;
+  lvl_cells[c] = c;  // level order: the layout is already level-contiguous
+  if (t == f.L) {
     cNChild[c] = 0;
-    cChild[c] = nc;
+    cChild[c] = nc;  // reverseOrder maps ICHILD = 0 of a leaf to numCells
   } else {
-    cNChild[c] = nch;
-    cChild[c] = a.off_dn + a.count_dn - a.scan_dn[end];
+    const int e0 = sh.base[(t + 1) * (sh.S + 1) + s] + 8 * k;
+    const int lo = rank[e0], hi = rank[e0 + 8];
+    cNChild[c] = hi - lo;
+    cChild[c] = rank[sh.lev0[t + 1]] + rank[sh.lev0[t + 2]] - hi;
   }
-  if (a.level == 0) {
-    cParent[c] = nc - 1;
+  if (t == 0) {
+    cParent[c] = nc - 1;  // reverseOrder maps the root's IPARENT = 0 to numCells-1
   } else {
-    const int rp = a.scan_up[start + 1] - 1;
-    cParent[c] = a.off_up + a.count_up - 1 - rp;
+    const int rp = rank[sh.base[(t - 1) * (sh.S + 1) + s] + (k >> 3)];
+    cParent[c] = rank[sh.lev0[t - 1]] + rank[sh.lev0[t]] - 1 - rp;
   }
 }
 
-void run_build_forest(Handle &h) {
-  const int n = h.n, S = h.nsys, ncrit = h.cfg.ncrit;
-  const int T = 256;
-  const std::vector<int> &off = h.sys_off;
-  h.sys_offd.resize(S + 1);
-  EXA_HIP(hipMemcpyAsync(h.sys_offd.p, off.data(), (S + 1) * sizeof(int), hipMemcpyHostToDevice, h.stream));
-  h.red.reserve(6 * (size_t)S);
-  hipLaunchKernelGGL(k_bounds_seg, dim3(S), dim3(256), 0, h.stream, h.in4.p, h.sys_offd.p, h.red.p);
-  std::vector<double> bb(6 * (size_t)S);
-  EXA_HIP(hipMemcpyAsync(bb.data(), h.red.p, bb.size() * sizeof(double), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipStreamSynchronize(h.stream));
-  std::vector<ForestSys> fs(S);
-  int Lmax = 0;
+// Depth of a system of n bodies (build_tree_omp.h:218, integer n / ncrit
+// inside the log).
+static int uniform_depth(int n, int ncrit) {
+  const int L = n >= ncrit ? 1 + int(std::log((double)(n / ncrit)) / M_LN2 / 3) : 0;
+  if (L > kMaxUniformLevels)
+    throw Error(EXAFMM_HIP_EUNSUP, "uniform tree deeper than 10 levels overflows the reference's int keys");
+  return L;
+}
+
+// The trees of the systems [off[s], off[s + 1]): with given bounds (one
+// system), or each with its own.
+static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
+  const int n = h.n, T = 256;
+  // Shape and host tables, uploaded when they change.
+  std::vector<int> L(S);
+  int Lmax = 0, Lmin = kMaxUniformLevels;
   for (int s = 0; s < S; s++) {
-    const int ns = off[s + 1] - off[s];
-    // build_tree_omp.h:218 and bounds2box (:21-33), per system.
-    const int L = ns >= ncrit ? 1 + int(std::log((double)(ns / ncrit)) / M_LN2 / 3) : 0;
-    if (L > 10) throw Error(EXAFMM_HIP_EUNSUP, "uniform tree deeper than 10 levels overflows the reference's int keys");
-    const double *mn = &bb[6 * s], *mx = &bb[6 * s + 3];
-    double Xc[3], R0 = 0;
-    for (int d = 0; d < 3; d++) Xc[d] = (mx[d] + mn[d]) / 2;
-    for (int d = 0; d < 3; d++) {
-      R0 = std::max(Xc[d] - mn[d], R0);
-      R0 = std::max(mx[d] - Xc[d], R0);
-    }
-    R0 *= 1.00001;
-    fs[s] = ForestSys{mn[0], mn[1], mn[2], (float)(2 * R0 / (1 << L)), L, off[s], off[s + 1]};
-    Lmax = std::max(Lmax, L);
+    L[s] = uniform_depth(off[s + 1] - off[s], h.cfg.ncrit);
+    Lmax = std::max(Lmax, L[s]);
+    Lmin = std::min(Lmin, L[s]);
   }
-  h.sys_par.resize(S * sizeof(ForestSys) / sizeof(double) + 1);
-  ForestSys *fsd = reinterpret_cast<ForestSys *>(h.sys_par.p);
-  EXA_HIP(hipMemcpyAsync(fsd, fs.data(), S * sizeof(ForestSys), hipMemcpyHostToDevice, h.stream));
-  h.k64a.reserve(n + 1);
-  h.k64b.reserve(n + 1);
-  h.ia.reserve(n + 1);
-  h.ib.reserve(n + 1);
-  h.ie.reserve(n + 1);
+  TreeShape sh{};
+  sh.S = S;
+  sh.nlev = Lmax + 1;
+  // Words: base [nlev][S + 1], begin [S], chunk0 [S + 1], chunks [][2] at an even word.
+  const size_t begin0 = (size_t)sh.nlev * (S + 1), chunk00 = begin0 + S, chunks0 = (chunk00 + S + 2) / 2 * 2;
+  std::vector<int> tab(chunks0);
+  int64_t e = 0;
+  for (int t = 0; t <= Lmax; t++) {
+    sh.lev0[t] = (int)e;
+    for (int s = 0; s <= S; s++) {
+      tab[(size_t)t * (S + 1) + s] = (int)e;
+      if (s < S && L[s] >= t) e += (int64_t)1 << (3 * t);
+    }
+    if (e > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "build_tree: too many cells");
+  }
+  sh.ncell = (int)e;
+  for (int t = Lmax + 1; t < kMaxUniformLevels + 2; t++) sh.lev0[t] = (int)e;
+  std::vector<ForestSys> fs(S);
+  int64_t leaf0 = 0;
+  for (int s = 0; s < S; s++) {
+    fs[s] = ForestSys{0, 0, 0, 0, L[s], off[s], off[s + 1], (int)leaf0};
+    leaf0 += (int64_t)1 << (3 * L[s]);
+  }
+  if (leaf0 > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "build_tree: too many leaves");
+  sh.nleaf = (int)leaf0;
+  for (int s = 0; s < S; s++) {
+    tab[begin0 + s] = off[s];
+    tab[chunk00 + s] = (int)((tab.size() - chunks0) / 2);
+    for (int b = off[s]; own_bounds && b < off[s + 1]; b += kBoundsChunk) {
+      tab.push_back(b);
+      tab.push_back(std::min(off[s + 1], b + kBoundsChunk));
+    }
+  }
+  const int nchunk = (int)((tab.size() - chunks0) / 2);
+  tab[chunk00 + S] = nchunk;
+  if (tab != h.ut_tab_host) {
+    h.ut_tab_host.clear();
+    h.ut_tab.resize(tab.size() + 1);
+    h.ut_sys.resize(S * sizeof(ForestSys) / sizeof(double));
+    EXA_HIP(hipMemcpyAsync(h.ut_tab.p, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, h.stream));
+    EXA_HIP(hipMemcpyAsync(h.ut_sys.p, fs.data(), S * sizeof(ForestSys), hipMemcpyHostToDevice, h.stream));
+    EXA_HIP(hipStreamSynchronize(h.stream));
+    h.ut_tab_host = std::move(tab);
+  }
+  sh.base = h.ut_tab.p;
+  ForestSys *fsd = reinterpret_cast<ForestSys *>(h.ut_sys.p);
+  if (own_bounds) {
+    h.red.reserve(6 * (size_t)nchunk);
+    const int *chunk = h.ut_tab.p + chunks0;
+    hipLaunchKernelGGL(k_bounds_chunks, dim3(nchunk), dim3(256), 0, h.stream, h.in4.p,
+                       reinterpret_cast<const int2 *>(chunk), h.red.p);
+    hipLaunchKernelGGL(k_bounds_systems, dim3(S), dim3(256), 0, h.stream, h.red.p, h.ut_tab.p + chunk00, fsd);
+  } else {
+    upload_bounds(h);
+    hipLaunchKernelGGL(k_box, dim3(1), dim3(1), 0, h.stream, h.box.p, fsd);
+  }
   h.body4.resize(n);
   h.bidx.resize(n);
   h.trg4.resize(n);
-  hipLaunchKernelGGL(k_sys_of, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.sys_offd.p, S, n, h.ie.p);
-  hipLaunchKernelGGL(k_morton_forest, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, n, h.ie.p, fsd, h.k64a.p,
-                     h.ia.p);
-  int sbits = 1;
-  while ((1 << sbits) < S) sbits++;
-  bool alt = false;
-  sort_pairs_u64_int(h, h.k64a.p, h.k64b.p, h.ia.p, h.ib.p, n, 32 + sbits, alt);
-  uint64_t *key = alt ? h.k64b.p : h.k64a.p;
-  int *order = alt ? h.ib.p : h.ia.p;
-  hipLaunchKernelGGL(k_gather_bodies, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, order, n, h.body4.p, h.bidx.p);
-  const int L = Lmax;
-  const size_t stride = (size_t)n + 1;
-  h.ic.reserve(stride * (L + 1));
-  h.id.reserve(stride * (L + 1));
-  for (int t = 0; t <= L; t++) {
-    int *fl = h.ic.p + stride * t;
-    int *sc = h.id.p + stride * t;
-    hipLaunchKernelGGL(k_level_heads_forest, dim3(div_up(n + 1, T)), dim3(T), 0, h.stream, key, n, t, fsd, fl);
-    exclusive_scan_int(h, fl, sc, n + 1);
+  h.ia.reserve(n + 1);
+  h.ib.reserve(n + 1);
+  h.ic.reserve(n + 1);
+  h.ut_start.resize((size_t)sh.nleaf + 1);
+  h.ut_rank.resize((size_t)sh.ncell + 1);
+  const int nchl = div_up((int64_t)sh.nleaf + 1, kScanChunk), nchc = div_up((int64_t)sh.ncell + 1, kScanChunk);
+  h.ut_tot.reserve(std::max(nchl, nchc));
+  if (!h.ut_zero || (size_t)sh.nleaf >= h.ut_cnt.cap) {
+    h.ut_cnt.reserve((size_t)sh.nleaf + 1);
+    zero_device(h.ut_cnt.p, h.ut_cnt.cap / 2 * 8, h.stream);
   }
-  std::vector<int> counts(L + 1), tot(L + 1);
-  h.cnt.reserve(L + 1);
-  hipLaunchKernelGGL(k_strided_gather, dim3(1), dim3(64), 0, h.stream, h.id.p + n, (int64_t)stride, L + 1, h.cnt.p);
-  EXA_HIP(hipMemcpyAsync(tot.data(), h.cnt.p, (L + 1) * sizeof(int), hipMemcpyDeviceToHost, h.stream));
+  h.ut_zero = false;
+  int *leaf = h.ic.p, *ord = h.ia.p, *aux = h.ib.p, *start = h.ut_start.p, *rank = h.ut_rank.p;
+  hipLaunchKernelGGL(k_leaf_count, dim3(div_up(n, 256)), dim3(256), 0, h.stream, h.in4.p, n, fsd, S,
+                     h.ut_tab.p + begin0, leaf, aux, h.ut_cnt.p);
+  if (sh.ncell <= kScanSmall) {
+    hipLaunchKernelGGL(k_tree_scan_small, dim3(1), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, start, rank);
+  } else {
+    hipLaunchKernelGGL(k_tree_totals<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
+                       h.ut_tot.p);
+    hipLaunchKernelGGL(k_tree_offsets<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
+                       h.ut_tot.p, start);
+    hipLaunchKernelGGL(k_tree_totals<true>, dim3(nchc), dim3(1024), 0, h.stream, sh, fsd, start, sh.ncell,
+                       h.ut_tot.p);
+    hipLaunchKernelGGL(k_tree_offsets<true>, dim3(nchc), dim3(1024), 0, h.stream, sh, fsd, start, sh.ncell,
+                       h.ut_tot.p, rank);
+  }
+  int *host_off = h.hpin + 128;  // (the adaptive builder's words)
+  int ncap = sh.ncell;           // the cell arrays hold every possible cell of trees up to kCellsUnread of them
+  if (ncap > kCellsUnread) {
+    EXA_HIP(hipMemcpyAsync(host_off, rank + ncap, sizeof(int), hipMemcpyDeviceToHost, h.stream));
+    EXA_HIP(hipStreamSynchronize(h.stream));
+    ncap = host_off[0];
+  }
+  for (DBuf<int> *v : {&h.cParent, &h.cChild, &h.cNChild, &h.cBody, &h.cNBody, &h.cLevel, &h.lvl_cells})
+    v->reserve(ncap);
+  h.cX.reserve(ncap);
+  h.cRb.reserve(ncap);
+  h.cKey.reserve(ncap);
+  hipLaunchKernelGGL(k_leaf_scatter, dim3(div_up(n, 256)), dim3(256), 0, h.stream, leaf, aux, n, start, ord);
+  int bits = 1;
+  while (((int64_t)1 << bits) < n) bits++;
+  hipLaunchKernelGGL(k_leaf_order, dim3(sh.nleaf), dim3(64), 0, h.stream, start, bits, ord, aux, h.in4.p, h.body4.p,
+                     h.bidx.p);
+  hipLaunchKernelGGL(k_uniform_cells, dim3(div_up(std::max(sh.ncell, sh.nlev + 1), T)), dim3(T), 0, h.stream, sh, fsd,
+                     start, rank, h.body4.p, h.cX.p, h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p, h.cBody.p,
+                     h.cNBody.p, h.cKey.p, h.cLevel.p, h.lvl_cells.p, host_off);
+  EXA_HIP(hipGetLastError());
+  h.ut_zero = true;
   EXA_HIP(hipStreamSynchronize(h.stream));
-  int nc = 0;
-  std::vector<int> loff(L + 2, 0);
-  for (int t = 0; t <= L; t++) {
-    counts[t] = tot[t];
-    loff[t] = nc;
-    nc += counts[t];
-  }
-  loff[L + 1] = nc;
+  const int nc = host_off[sh.nlev];
   h.ncells = nc;
-  h.nlevels = L + 1;
-  h.ie.reserve(std::max((size_t)nc + 1, (size_t)n + 1));
-  std::vector<int> posoff(L + 1);
-  for (int t = 0, o = 0; t <= L; t++) {
-    posoff[t] = o;
-    o += counts[t];
-  }
-  for (int t = 0; t <= L; t++)
-    hipLaunchKernelGGL(k_level_positions, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.ic.p + stride * t,
-                       h.id.p + stride * t, n, h.ie.p + posoff[t]);
+  h.nlevels = sh.nlev;
+  h.lvl_off.assign(host_off, host_off + sh.nlev + 1);
+  h.lvl_par.assign(sh.nlev, 0);
+  // All cells above the leaves have children; in a forest a bound, as
+  // shallower systems end above.
+  for (int t = 0; t < sh.nlev; t++) h.lvl_par[t] = h.lvl_off[t + 1] - h.lvl_off[t];
+  h.leaf_level = Lmin;
+  for (DBuf<int> *v : {&h.cParent, &h.cChild, &h.cNChild, &h.cBody, &h.cNBody, &h.cLevel, &h.lvl_cells})
+    v->resize(nc);
   h.cX.resize(nc);
   h.cRb.resize(nc);
-  h.cParent.resize(nc);
-  h.cChild.resize(nc);
-  h.cNChild.resize(nc);
-  h.cBody.resize(nc);
-  h.cNBody.resize(nc);
   h.cKey.resize(nc);
-  h.cLevel.resize(nc);
-  for (int t = 0; t <= L; t++) {
-    if (counts[t] == 0) continue;
-    LevelArgs a;
-    a.pos = h.ie.p + posoff[t];
-    a.scan = h.id.p + stride * t;
-    a.scan_up = t > 0 ? h.id.p + stride * (t - 1) : nullptr;
-    a.scan_dn = t < L ? h.id.p + stride * (t + 1) : nullptr;
-    a.count = counts[t];
-    a.count_up = t > 0 ? counts[t - 1] : 0;
-    a.count_dn = t < L ? counts[t + 1] : 0;
-    a.off = loff[t];
-    a.off_up = t > 0 ? loff[t - 1] : 0;
-    a.off_dn = t < L ? loff[t + 1] : 0;
-    a.shift = 0;
-    a.leaf = 0;
-    a.level = t;
-    hipLaunchKernelGGL(k_level_cells_forest, dim3(div_up(counts[t], T)), dim3(T), 0, h.stream, a, h.body4.p, key, n,
-                       nc, fsd, h.cX.p, h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cKey.p,
-                       h.cLevel.p);
-  }
-  h.lvl_off.assign(loff.begin(), loff.begin() + L + 2);
-  h.lvl_par = counts;  // a bound: shallower systems end above
-  h.leaf_level = L;
-  for (const ForestSys &f : fs) h.leaf_level = std::min(h.leaf_level, f.L);
-  h.lvl_cells.resize(nc);
-  hipLaunchKernelGGL(k_iota, dim3(div_up(nc, T)), dim3(T), 0, h.stream, h.lvl_cells.p, nc);
-  EXA_HIP(hipGetLastError());
 }
+
+void run_build_uniform(Handle &h) {
+  const int off[2] = {0, h.n};
+  build_uniform(h, off, 1, false);
+  sync_bounds(h);  // (arrived before the cells)
+}
+
+void run_build_forest(Handle &h) { build_uniform(h, h.sys_off.data(), h.nsys, true); }
 
 }  // namespace exafmm

@@ -477,7 +477,7 @@ void run_build_adaptive(Handle &h) {
     hipLaunchKernelGGL(k_path_keys, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, n, box, levels, h.k64a.p,
                        h.ia.p);
     bool alt = false;
-    sort_pairs_u64_int_bits(h, h.k64a.p, h.k64b.p, h.ia.p, h.ib.p, n, 3 * (kDepth - levels), 3 * kDepth, alt);
+    sort_pairs_u64_int(h, h.k64a.p, h.k64b.p, h.ia.p, h.ib.p, n, 3 * (kDepth - levels), 3 * kDepth, alt);
     key = alt ? h.k64b.p : h.k64a.p;
     idx = alt ? h.ib.p : h.ia.p;
     aux = alt ? h.ia.p : h.ib.p;

@@ -158,24 +158,14 @@ static void radix_sort_pairs(K *keys, K *keys_alt, int *vals, int *vals_alt, int
     radix_sort_pairs_cfg<rocprim::default_config>(keys, keys_alt, vals, vals_alt, n, bits, result_in_alt, st, tmp);
 }
 
-void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bits,
-                        bool &result_in_alt) {
-  radix_sort_pairs(keys, keys_alt, vals, vals_alt, n, bits, result_in_alt, h.stream, h.tmp);
-}
-
-void sort_pairs_u64_int_bits(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
-                             int bit1, bool &result_in_alt) {
+void sort_pairs_u64_int(Handle &h, uint64_t *keys, uint64_t *keys_alt, int *vals, int *vals_alt, int n, int bit0,
+                        int bit1, bool &result_in_alt) {
   // Alone on the device: onesweep already where its 3 launches per 8 bits are
   // fewer than those of the merge passes.
   if (n < (1 << 16))
     return radix_sort_pairs_cfg<rocprim::default_config>(keys, keys_alt, vals, vals_alt, n, bit1, result_in_alt,
                                                          h.stream, h.tmp, bit0);
   radix_sort_pairs_cfg<OnesweepConfig>(keys, keys_alt, vals, vals_alt, n, bit1, result_in_alt, h.stream, h.tmp, bit0);
-}
-
-void sort_pairs_int_int(Handle &h, int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits,
-                        bool &result_in_alt) {
-  radix_sort_pairs(keys, keys_alt, vals, vals_alt, n, bits, result_in_alt, h.stream, h.tmp);
 }
 
 void sort_pairs_int_int(int *keys, int *keys_alt, int *vals, int *vals_alt, int n, int bits, bool &result_in_alt,
