@@ -174,6 +174,8 @@ int exafmm_hip_create(const exafmm_hip_config *cfg, exafmm_hip_handle **out) {
     EXA_HIP(hipEventCreate(&H->h.ev_mult));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_cnt, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_lists, hipEventDisableTiming));
+    EXA_HIP(hipEventCreateWithFlags(&H->h.ev_used, hipEventDisableTiming));
+    EXA_HIP(hipEventCreateWithFlags(&H->h.ev_image, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_tiles, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_p2pcnt, hipEventDisableTiming));
     EXA_HIP(hipEventCreateWithFlags(&H->h.ev_bounds, hipEventDisableTiming));

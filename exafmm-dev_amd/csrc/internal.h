@@ -98,6 +98,8 @@ struct Handle {
   bool mult_pending = false;     // the main stream has not joined ev_mult yet
   bool mult_enqueue = false;     // run_upward_mult not enqueued yet (the traversal does it)
   hipEvent_t ev_cnt = nullptr;   // a device count copied into hpin
+  hipEvent_t ev_used = nullptr;  // image offsets in use flagged (main stream)
+  hipEvent_t ev_image = nullptr; // their matrices done on stream3
   hipEvent_t ev_tiles = nullptr; // lattice tiles done on stream2 (split upward pass)
   hipEvent_t ev_lists = nullptr; // raw lists done (the P2P grouping on stream2 waits for it)
   hipEvent_t ev_p2pcnt = nullptr; // P2P target count copied into hpin[9] (stream2)
@@ -218,6 +220,13 @@ struct Handle {
   DBuf<int> lat_ookey, lat_orow;
   DBuf<unsigned char> lat_hist;
   int lat_noff = 0;
+  // Image offsets (periodic boxes): numbers lat_nreg .. lat_noff, those of the
+  // levels l % 3 = i from lat_img0[i] on; lat_okey: number -> key.  lat_tc_keyn:
+  // keys of the maps above; lat_img_off: too many, left to the per-pair kernel.
+  int lat_nreg = 0, lat_img0[4] = {0, 0, 0, 0}, lat_tc_keyn = 0;
+  DBuf<int> lat_okey;
+  bool lat_img_off = false;
+  std::vector<int> lat_tbase;    // first tile slot of every level
   int lat_tc_rows = 0, lat_tc_P = 0, lat_tc_max = 16384;  // rows; a fuller table starts afresh
   bool lat_tc_f32 = false;
   bool lat_ms_ready = false;     // lat_Ms / lat_Msf already queued for this evaluation

@@ -310,8 +310,11 @@ __global__ void __launch_bounds__(64 * W)
 // workgroups (two of 8 waves per CU) the longest list decides the time, and so
 // it does where most lists are short (irregular pairs of an adaptive tree: 3
 // per target on average, over 100 at most).  Long lists on many targets
-// (periodic images: 100 per target) fill the chip by themselves.
-constexpr int kFewTargets = 2048, kShortList = 16;
+// (periodic images: 100 per target) fill the chip by themselves, from the
+// million pairs on that take it as long (1.8 ns a pair) as a list of 400 takes
+// one wave (5 us a pair): the 237000 images across edges of a box of 64^3
+// bodies took 1930 us with one wave per target, 510 with eight.
+constexpr int kFewTargets = 2048, kShortList = 16, kFewPairs = 1 << 20;
 
 template <int P>
 static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L, bool f32,
@@ -343,7 +346,8 @@ static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const c
                        L, desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
   };
   constexpr int W = P <= 10 ? 8 : 4;  // 55 KB of LDS per workgroup at P = 10, 41 KB at P = 12
-  const bool few = lst.ntgt <= kFewTargets || lst.npairs < (int64_t)kShortList * lst.ntgt;
+  const bool few =
+      lst.ntgt <= kFewTargets || lst.npairs < (int64_t)kShortList * lst.ntgt || lst.npairs < kFewPairs;
   if (esz == 8)
     few ? launch(k_m2l<P, float, W>, W) : launch(k_m2l<P, float, 1>, 1);
   else

@@ -26,9 +26,11 @@
 // T(d) is staged in LDS in MFMA fragment order (only the 16 x 4 blocks that
 // are not identically zero: j + n < P), each lane gathers its column's source
 // multipole scaled by u^-n, and the 4 waves (16 columns each) run
-// v_mfma_f64_16x16x4 (v_mfma_f32_16x16x4 in the mixed form).  Pairs that are
-// not lattice pairs (levels two or more apart, periodic images, MASS mode,
-// offsets beyond kLatD) go to the per-pair kernel.
+// v_mfma_f64_16x16x4 (v_mfma_f32_16x16x4 in the mixed form).  Pairs with a
+// periodic image across one face of the box, on the finest levels, take part
+// with matrices made for their actual offsets in every evaluation.  Pairs that
+// are not lattice pairs (levels two or more apart, other periodic images, MASS
+// mode, offsets beyond kLatD) go to the per-pair kernel.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -46,6 +48,33 @@ constexpr double kLatUnit = 4;                   // u = w / kLatUnit
 constexpr int kLatD = 60;                         // |d_c| <= kLatD (in units of u)
 constexpr int kLatSide = 2 * kLatD + 1;
 constexpr int kLatKeys = kLatSide * kLatSide * kLatSide;
+
+// Image offsets.  The box length is no multiple of a cell width, so a source
+// seen across a face is off the targets' lattice; but all pairs of one level,
+// face and lattice offset have the same actual offset, and with it the same
+// T.  Their keys follow the lattice keys: (level mod 3, face, offset), the
+// offset taken to the nearest lattice image, |d_c| <= kImgD, its components
+// all 0, all 2 or all odd mod 4 (the three level relations).  Unlike the
+// lattice's, their T depends on box and cell sizes and is made anew in every
+// evaluation.
+//
+// Used on the finest kImgLevels levels that are dense, from level 3 on: there
+// a T (61 KB at P = 10, 30 ns to make and to read) serves 100 to 1000 pairs of
+// 1.8 ns each on the per-pair kernel (a lattice of 64^3 bodies, theta = 0.35).
+// Images across an edge of the box share one offset among 40 to 50 pairs, as
+// coarser levels and the few cells of a sparse level do, and gain nothing:
+// they stay with the per-pair kernel, a tenth of the image pairs.
+constexpr int kImgLevels = 3;
+constexpr int kImgD = 44;
+constexpr int kImgN0 = kImgD / 2 + 1, kImgN2 = kImgD / 2, kImgN1 = kImgD;  // values per component
+constexpr int kImgFace = kImgN0 * kImgN0 * kImgN0 + kImgN2 * kImgN2 * kImgN2 + kImgN1 * kImgN1 * kImgN1;
+constexpr int kImgLevelKeys = 6 * kImgFace;
+static_assert(kImgD % 4 == 0, "the offsets of each level relation fill their range");
+
+struct LatImages {
+  int finest = -1;  // finest level of image offsets (-1: none)
+  double cycle = 0;
+};
 
 template <int P>
 struct MfmaShape {
@@ -113,20 +142,65 @@ struct LatState {
   int ntiles;   // tiles with steps
 };
 
-// Key of the lattice offset of target t and source s (image im), or -1.
-__device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ cX, const double *__restrict__ cRb) {
+// Face that image im lies across (-x, +x, -y, ... +z), or -1.
+__device__ inline int image_face(int im) {
+  return im == 4 ? 0 : im == 22 ? 1 : im == 10 ? 2 : im == 16 ? 3 : im == 12 ? 4 : im == 14 ? 5 : -1;
+}
+
+__device__ inline bool image_level(const LatImages &li, int l) { return l >= 3 && l <= li.finest && l > li.finest - kImgLevels; }
+
+// Number of the image offset (x, y, z) among those of one level and face, or
+// -1, and back.
+__device__ inline int image_index(int x, int y, int z) {
+  if (abs(x) > kImgD || abs(y) > kImgD || abs(z) > kImgD) return -1;
+  const int c = (x & 3) == 2 ? 2 : x & 1 ? 1 : 0;
+  if (c == 1 ? !(y & z & 1) : (y & 3) != c || (z & 3) != c) return -1;
+  if (c == 0) return ((x + kImgD) / 4 * kImgN0 + (y + kImgD) / 4) * kImgN0 + (z + kImgD) / 4;
+  constexpr int b2 = kImgN0 * kImgN0 * kImgN0, b1 = b2 + kImgN2 * kImgN2 * kImgN2;
+  if (c == 2) return b2 + ((x + kImgD - 2) / 4 * kImgN2 + (y + kImgD - 2) / 4) * kImgN2 + (z + kImgD - 2) / 4;
+  return b1 + ((x + kImgD - 1) / 2 * kImgN1 + (y + kImgD - 1) / 2) * kImgN1 + (z + kImgD - 1) / 2;
+}
+
+__device__ inline void image_offset(int i, int &x, int &y, int &z) {
+  constexpr int b2 = kImgN0 * kImgN0 * kImgN0, b1 = b2 + kImgN2 * kImgN2 * kImgN2;
+  const int n = i < b2 ? kImgN0 : i < b1 ? kImgN2 : kImgN1, step = i < b1 ? 4 : 2;
+  const int lo = i < b2 ? -kImgD : i < b1 ? 2 - kImgD : 1 - kImgD;
+  i -= i < b2 ? 0 : i < b1 ? b2 : b1;
+  x = lo + step * (i / (n * n));
+  y = lo + step * (i / n % n);
+  z = lo + step * (i % n);
+}
+
+// The lattice's whole number of units nearest to the box length.
+__device__ inline int image_units(double cycle, double rt) { return 4 * (int)rint(cycle / (2 * rt)); }
+static_assert(kLatUnit == 4, "image offsets in units of a quarter cell");
+
+// Key of the offset of target t and source s (image im), or -1.
+__device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ cX, const double *__restrict__ cRb,
+                              const int *__restrict__ cLevel, const LatImages &li) {
   // Same level or one level apart: then the offset's residue mod 4 fixes
   // the level relation (0: same, 2: source one up, odd: source one down).
   const double rt = cRb[t], rs = cRb[s];
-  if (im != 13 || !(rs == rt || rs == 2 * rt || 2 * rs == rt)) return -1;
+  if (!(rs == rt || rs == 2 * rt || 2 * rs == rt)) return -1;
+  int face = -1, l = 0;
+  if (im != 13) {
+    if (li.finest < 0 || (face = image_face(im)) < 0 || !image_level(li, l = cLevel[t])) return -1;
+  }
   // Offsets in units of u = 2 R_t / kLatUnit; the lattice values are whole
   // numbers to far better than the 1e-6 test below.
   const double iu = kLatUnit / (2 * rt);
   const double4 a = cX[t], b = cX[s];
   const double dx = (a.x - b.x) * iu, dy = (a.y - b.y) * iu, dz = (a.z - b.z) * iu;
   const double rx = rint(dx), ry = rint(dy), rz = rint(dz);
-  if (fabs(dx - rx) < 1e-6 && fabs(dy - ry) < 1e-6 && fabs(dz - rz) < 1e-6 && fabs(rx) <= kLatD &&
-      fabs(ry) <= kLatD && fabs(rz) <= kLatD)
+  if (!(fabs(dx - rx) < 1e-6 && fabs(dy - ry) < 1e-6 && fabs(dz - rz) < 1e-6)) return -1;
+  if (im != 13) {
+    if (!(fabs(rx) < 1e6 && fabs(ry) < 1e6 && fabs(rz) < 1e6 && li.cycle < 1e6 * rt)) return -1;
+    const int pc = image_units(li.cycle, rt) * (face & 1 ? 1 : -1);
+    const int i = image_index((int)rx - (face / 2 == 0 ? pc : 0), (int)ry - (face / 2 == 1 ? pc : 0),
+                              (int)rz - (face / 2 == 2 ? pc : 0));
+    return i < 0 ? -1 : kLatKeys + (l % kImgLevels * 6 + face) * kImgFace + i;
+  }
+  if (fabs(rx) <= kLatD && fabs(ry) <= kLatD && fabs(rz) <= kLatD)
     return (((int)rx + kLatD) * kLatSide + ((int)ry + kLatD)) * kLatSide + ((int)rz + kLatD);
   return -1;
 }
@@ -140,7 +214,8 @@ __device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ 
 __global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restrict__ src,
                                const unsigned char *__restrict__ img, int64_t np, const double4 *__restrict__ cX,
                                const double *__restrict__ cRb, const int *__restrict__ o_of_key,
-                               const int *__restrict__ tile_of, int noff, unsigned char *__restrict__ act,
+                               const int *__restrict__ tile_of, const int *__restrict__ cLevel, LatImages li, int nreg,
+                               int noff, unsigned char *__restrict__ act, unsigned char *__restrict__ used,
                                int *__restrict__ pstep, unsigned char *__restrict__ hist, LatState *__restrict__ st) {
   __shared__ int sn;
   if (threadIdx.x == 0) sn = 0;
@@ -148,7 +223,7 @@ __global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restri
   int nirr = 0;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < np; e += (int64_t)gridDim.x * blockDim.x) {
     const int t = ptgt[e];
-    const int key = lat_key(t, src[e], img[e], cX, cRb);
+    const int key = lat_key(t, src[e], img[e], cX, cRb, cLevel, li);
     const int tile = tile_of[t];
     int v = -1;
     if (key >= 0 && tile >= 0) {
@@ -160,6 +235,7 @@ __global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restri
       } else {
         v = tile * noff + o;
         act[v] = 1;
+        if (o >= nreg && !used[o - nreg]) used[o - nreg] = 1;
       }
     }
     pstep[e] = v;
@@ -246,6 +322,97 @@ __global__ void __launch_bounds__(64) k_lat_tmat(const int *__restrict__ okey, R
       T[(size_t)o * TPad<P, R>::TEP + (S::base(rb) + kc) * 64 + lane] = (R)v;
     }
   for (int i = S::NBLK * 64 + lane; i < TPad<P, R>::TEP; i += 64) T[(size_t)o * TPad<P, R>::TEP + i] = 0;
+}
+
+// T of the image offsets in use (numbers nreg + i, used[i]), as k_lat_tmat for
+// the actual offset of their level and face.  A workgroup makes kImgT of them
+// together, so that the entries' index arithmetic is done once for all; bound
+// by the stores: 6800 offsets at P = 10 are 415 MB, 0.32 ms alone with one
+// workgroup per kImgT and 0.45 ms beside P2P and the step lists, which hide it.
+// lvl: for each level mod 3 the first of its cells in lvl_cells.
+constexpr int kImgT = 16, kImgTParts = 4;  // (each in kImgTParts workgroups, for balance)
+struct ImgLevels {
+  int cell[kImgLevels];
+};
+
+template <int P, typename R>
+__global__ void __launch_bounds__(256)
+    k_lat_tmat_image(int nreg, int noff, const int *__restrict__ okey, const int *__restrict__ orow,
+                     const unsigned char *__restrict__ used, ImgLevels lvl, const int *__restrict__ lvl_cells,
+                     const double *__restrict__ cRb, double cycle, R *__restrict__ T, const LatState *__restrict__ st) {
+  using S = MfmaShape<P>;
+  constexpr int NT = S::NT, TEP = TPad<P, R>::TEP;
+  __shared__ double sS[kImgT][2 * P * P];
+  __shared__ int srow[kImgT], sdlev[kImgT];
+  __shared__ Geom sg[kImgT];
+  if (st->unknown) return;
+  const int o0 = nreg + blockIdx.x * kImgT;
+  if (threadIdx.x < kImgT) {
+    const int o = o0 + threadIdx.x;
+    srow[threadIdx.x] = -1;
+    if (o < noff && used[o - nreg]) {
+      const int k = okey[o] - kLatKeys, face = k / kImgFace % 6;
+      int x, y, z;
+      image_offset(k % kImgFace, x, y, z);
+      const double rt = cRb[lvl_cells[lvl.cell[k / kImgLevelKeys]]];
+      // The offset to the nearest lattice image, and what the image is off it.
+      const double p = (face & 1 ? 1 : -1) * (image_units(cycle, rt) - cycle * (kLatUnit / (2 * rt)));
+      sg[threadIdx.x] = make_geom(x + (face / 2 == 0 ? p : 0), y + (face / 2 == 1 ? p : 0), z + (face / 2 == 2 ? p : 0));
+      srow[threadIdx.x] = orow[o];
+      sdlev[threadIdx.x] = (x & 3) == 0 ? 0 : (x & 3) == 2 ? 1 : -1;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kImgT * NT; i += 256) {
+    const int q = i % kImgT, t = i / kImgT;
+    if (srow[q] < 0) continue;
+    int a, b;
+    coef_nm(t, a, b);
+    double re, im;
+    singular_nm(a, b, sg[q], re, im);
+    const double s = (b & 1) ? -1.0 : 1.0;
+    sS[q][2 * (a * a + a + b)] = s * re;
+    sS[q][2 * (a * a + a + b) + 1] = s * im;
+    if (b > 0) {
+      sS[q][2 * (a * a + a - b)] = re;
+      sS[q][2 * (a * a + a - b) + 1] = -im;
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, part = 4 * blockIdx.y + wave;
+  int blk = 0;
+  for (int rb = 0; rb < S::RB; rb++)
+    for (int kc = 0; kc < S::kc_end(rb); kc++, blk++) {
+      if (blk % (4 * kImgTParts) != part) continue;
+      // Entry = c1 S1 + c2 S2, each a component of a harmonic.
+      const int row = rb * 16 + (lane & 15), col = kc * 4 + (lane >> 4);
+      int i1 = 0, i2 = 0, n = 0;
+      double c1 = 0, c2 = 0;
+      if (row < S::NR && col < S::NR) {
+        int j, k, m;
+        coef_nm(row >> 1, j, k);
+        coef_nm(col >> 1, n, m);
+        if (j + n < P) {
+          const int a = j + n, pr = row & 1, pc = col & 1;
+          const double sm = (m & 1) ? -1.0 : 1.0, sj = (j & 1) ? -1.0 : 1.0;
+          i1 = 2 * (a * a + a + m - k) + (pr ^ pc);
+          c1 = sj * (pc & ~pr ? -sm : sm);
+          if (m > 0) {
+            i2 = 2 * (a * a + a - m - k) + (pr ^ pc);
+            c2 = pr & pc ? -sj : sj;
+          }
+        }
+      }
+      const double up = ldexp(1.0, n), down = ldexp(1.0, -n);
+      for (int q = 0; q < kImgT; q++) {
+        const int to = __builtin_amdgcn_readfirstlane(srow[q]), dlev = __builtin_amdgcn_readfirstlane(sdlev[q]);
+        if (to < 0) continue;
+        const double v = c1 * sS[q][i1] + c2 * sS[q][i2];
+        T[(size_t)to * TEP + blk * 64 + lane] = (R)(dlev == 0 ? v : v * (dlev > 0 ? up : down));
+      }
+    }
+  for (int q = part; q < kImgT; q += 4 * kImgTParts)
+    for (int i = S::NBLK * 64 + lane; srow[q] >= 0 && i < TEP; i += 64) T[(size_t)srow[q] * TEP + i] = 0;
 }
 
 // Target tiles: cells grouped by (level, octant), and inside a group ordered
@@ -405,13 +572,32 @@ __global__ void k_tile_assign(int nc, TileLevels tl, const int *__restrict__ ske
   col_of[c] = col;
 }
 
+// The offsets a tile can use: the lattice's, and the image offsets of its level.
+struct LatRanges {
+  int nreg;                           // lattice offsets
+  int nlv;                            // levels with image offsets
+  int tile0[kImgLevels], tile1[kImgLevels];  // tiles of the level
+  int lo[kImgLevels], hi[kImgLevels];        // numbers of its image offsets
+};
+
+__device__ inline void tile_images(const LatRanges &lr, int tile, int &lo, int &hi) {
+  lo = hi = 0;
+  for (int i = 0; i < kImgLevels; i++)
+    if (i < lr.nlv && tile >= lr.tile0[i] && tile < lr.tile1[i]) {
+      lo = lr.lo[i];
+      hi = lr.hi[i];
+    }
+}
+
 // Steps per tile: the flags of its row of act.
 __global__ void __launch_bounds__(256)
-    k_lat_count(const unsigned char *__restrict__ act, int noff, int *__restrict__ cnt) {
+    k_lat_count(const unsigned char *__restrict__ act, int noff, LatRanges lr, int *__restrict__ cnt) {
   __shared__ int sw[4];
   const unsigned char *a = act + (size_t)blockIdx.x * noff;
-  int n = 0;
-  for (int o = threadIdx.x; o < noff; o += 256) n += a[o];
+  int n = 0, lo, hi;
+  tile_images(lr, blockIdx.x, lo, hi);
+  for (int o = threadIdx.x; o < lr.nreg; o += 256) n += a[o];
+  for (int o = lo + threadIdx.x; o < hi; o += 256) n += a[o];
   for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
   if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = n;
   __syncthreads();
@@ -422,7 +608,7 @@ __global__ void __launch_bounds__(256)
 // tiles before it: aidx[tile * noff + o] = step, alist[step] = the offset's T
 // row; their slots are emptied.
 __global__ void __launch_bounds__(256)
-    k_lat_steps(const unsigned char *__restrict__ act, const int *__restrict__ cnt, int noff,
+    k_lat_steps(const unsigned char *__restrict__ act, const int *__restrict__ cnt, int noff, LatRanges lr,
                 const int *__restrict__ orow, int *__restrict__ aidx, int *__restrict__ step0,
                 int *__restrict__ alist, int4 *__restrict__ slot, LatState *__restrict__ st) {
   __shared__ int sw[4], sn[4];
@@ -454,9 +640,12 @@ __global__ void __launch_bounds__(256)
   }
   if (mine == 0) return;
   for (int i = tid; i < mine * 16; i += 256) slot[(size_t)base * 16 + i] = make_int4(-1, -1, -1, -1);
-  for (int b = 0; b < noff; b += 256) {
-    const int o = b + tid;
-    const bool in = o < noff && act[(size_t)tile * noff + o];
+  int lo, hi;
+  tile_images(lr, tile, lo, hi);
+  const int nuse = lr.nreg + hi - lo;
+  for (int b = 0; b < nuse; b += 256) {
+    const int u = b + tid, o = u < lr.nreg ? u : lo + u - lr.nreg;
+    const bool in = u < nuse && act[(size_t)tile * noff + o];
     const unsigned long long m = __ballot(in);
     __syncthreads();
     if (lane == 0) sw[wave] = (int)__popcll(m);
@@ -519,7 +708,7 @@ __global__ void k_lat_flag(const unsigned char *__restrict__ hist, const int *__
 __global__ void k_lat_number(const int *__restrict__ flag, const int *__restrict__ scan,
                              const int *__restrict__ nflag, const int *__restrict__ nscan, int n, int base,
                              int *__restrict__ row_of_key, int *__restrict__ keys, int *__restrict__ o_of_key,
-                             int *__restrict__ orow, unsigned char *__restrict__ hist) {
+                             int *__restrict__ okey, int *__restrict__ orow, unsigned char *__restrict__ hist) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   hist[k] = 0;
@@ -531,7 +720,19 @@ __global__ void k_lat_number(const int *__restrict__ flag, const int *__restrict
     keys[nscan[k]] = k;
   }
   o_of_key[k] = scan[k];
+  okey[scan[k]] = k;
   orow[scan[k]] = row;
+}
+
+// What the host needs of the two scans over n keys: known and new offsets, the
+// new ones of the lattice, and the known ones below each level's image keys.
+__global__ void k_lat_marks(const int *__restrict__ kscan, const int *__restrict__ nscan, int n,
+                            int *__restrict__ host) {
+  const int i = threadIdx.x;
+  if (i == 0) host[0] = kscan[n];
+  if (i == 1) host[1] = nscan[n];
+  if (i == 2) host[2] = nscan[kLatKeys];
+  if (i <= kImgLevels) host[3 + i] = kscan[min(n, kLatKeys + i * kImgLevelKeys)];
 }
 
 // Offsets in use: flags of any tile.
@@ -593,7 +794,7 @@ __global__ void __launch_bounds__(256)
 // and keeps them in its L2.
 constexpr int kLatSeg = 8;
 // Words of Handle::hpin the lattice set-up reads back (LatState; registration counts).
-constexpr int kPinLat = 64, kPinNoff = 64 + 8, kPinNnew = 64 + 9;
+constexpr int kPinLat = 64, kPinMarks = 64 + 4;
 
 typedef __attribute__((address_space(3))) void lds_void;
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt left alone.
@@ -784,16 +985,31 @@ static void mscale_impl(Handle &h, hipStream_t st) {
 // Largest slot array sized by the all-steps-active bound (512 MB of int).
 constexpr int64_t kSlotBound = (int64_t)1 << 27;
 
+// Levels of the current tree whose image pairs take part.
+static LatImages lat_images(const Handle &h) {
+  LatImages li;
+  if (h.cfg.images == 0 || h.lat_img_off) return li;
+  for (int l = 3; l < std::min(h.nlevels, kTileLevels - 1) && l <= 20; l++)
+    if (2 * (int64_t)(h.lvl_off[l + 1] - h.lvl_off[l]) >= (int64_t)1 << (3 * l)) li.finest = l;
+  li.cycle = h.cfg.cycle;
+  return li;
+}
+
+// Offset keys: the lattice's, and the image offsets' in a periodic box.
+static int lat_keys(const Handle &h) { return kLatKeys + (h.cfg.images > 0 ? kImgLevels * kImgLevelKeys : 0); }
+
 // An empty T table for expansion order P in FP32 or FP64, no offset known.
 static void tc_reset(Handle &h, int P, bool f32) {
-  h.lat_tc_map.resize(kLatKeys + 1);
-  h.lat_ookey.resize(kLatKeys + 1);
-  h.lat_hist.resize(kLatKeys + 8);
+  const int nk = lat_keys(h);
+  h.lat_tc_map.resize(nk + 1);
+  h.lat_ookey.resize(nk + 1);
+  h.lat_hist.resize(nk + 8);
   for (int *p : {h.lat_tc_map.p, h.lat_ookey.p})
-    hipLaunchKernelGGL(k_fill_int, dim3(div_up(kLatKeys + 1, 256)), dim3(256), 0, h.stream, p, (int64_t)kLatKeys + 1,
-                       -1);
-  zero_device(h.lat_hist.p, kLatKeys + 7, h.stream);
-  h.lat_tc_rows = h.lat_noff = 0;
+    hipLaunchKernelGGL(k_fill_int, dim3(div_up(nk + 1, 256)), dim3(256), 0, h.stream, p, (int64_t)nk + 1, -1);
+  zero_device(h.lat_hist.p, nk + 7, h.stream);
+  h.lat_tc_rows = h.lat_noff = h.lat_nreg = 0;
+  for (int &i : h.lat_img0) i = 0;
+  h.lat_tc_keyn = nk;
   h.lat_tc_P = P;
   h.lat_tc_f32 = f32;
 }
@@ -855,6 +1071,7 @@ void run_lattice_tiles(Handle &h, hipStream_t st) {
     base += 8 * div_up(group, 64);
   }
   h.lat_ntiles = base;
+  h.lat_tbase.assign(tl.base, tl.base + kTileLevels + 1);
   h.lat_tile_of.resize(nc);
   h.lat_col_of.resize(nc);
   h.lat_tile_tgt.resize((size_t)std::max(1, base) * 64);
@@ -881,30 +1098,63 @@ void run_lattice_tiles(Handle &h, hipStream_t st) {
   EXA_HIP(hipGetLastError());
 }
 
-// Steps and slots of the current M2L list with the offsets known so far.
-// Nothing waits for the device; whether every offset was known, and how many
-// pairs are irregular, is read back behind it (ev_cnt).
+// Steps and slots of the current M2L list with the offsets known so far, and
+// the matrices of its image offsets.  Nothing waits for the device; whether
+// every offset was known, and how many pairs are irregular, is read back
+// behind it (ev_cnt).
+template <int P>
 static void lattice_steps(Handle &h) {
   const int64_t np = h.nm2l, nall = (int64_t)h.lat_ntiles * h.lat_noff;
   const int TPB = 256, gp = div_up(np, TPB);
   const int *ptgt = h.raw_mi.p, *psrc = h.raw_mj.p;
   if (nall > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
-  h.lat_act.resize(sizeof(LatState) + nall + 8);
+  const LatImages li = lat_images(h);
+  const int nimg = h.lat_noff - h.lat_nreg;
+  LatRanges lr{};
+  ImgLevels lvl{};
+  lr.nreg = h.lat_nreg;
+  int64_t nbound = (int64_t)h.lat_ntiles * h.lat_nreg;  // most steps
+  for (int l = std::max(3, li.finest - kImgLevels + 1); l <= li.finest; l++) {
+    const int i = lr.nlv++, slot = l % kImgLevels;
+    lvl.cell[slot] = h.lvl_off[l];
+    lr.tile0[i] = h.lat_tbase[l];
+    lr.tile1[i] = h.lat_tbase[l + 1];
+    lr.lo[i] = h.lat_img0[slot];
+    lr.hi[i] = h.lat_img0[slot + 1];
+    nbound += (int64_t)(lr.tile1[i] - lr.tile0[i]) * (lr.hi[i] - lr.lo[i]);
+  }
+  h.lat_act.resize(sizeof(LatState) + nall + nimg + 8);
   h.lat_aidx.resize(nall + 1);
   h.lat_pslot.resize(np);
   h.lat_tcnt.resize(h.lat_ntiles + 1);
   h.lat_step0.resize(h.lat_ntiles + 1);
-  unsigned char *act = h.lat_act.p + sizeof(LatState);
-  zero_device(h.lat_act.p, sizeof(LatState) + (nall + 7) / 8 * 8, h.stream);
+  unsigned char *act = h.lat_act.p + sizeof(LatState), *used = act + nall;
+  zero_device(h.lat_act.p, sizeof(LatState) + (nall + nimg + 7) / 8 * 8, h.stream);
   hipLaunchKernelGGL(k_lat_classify, dim3(std::min(gp, 4096)), dim3(TPB), 0, h.stream, ptgt, psrc, h.raw_mimg.p, np,
-                     h.cX.p, h.cRb.p, h.lat_ookey.p, h.lat_tile_of.p, h.lat_noff, act, h.lat_pslot.p, h.lat_hist.p,
-                     lat_state(h));
+                     h.cX.p, h.cRb.p, h.lat_ookey.p, h.lat_tile_of.p, h.cLevel.p, li, h.lat_nreg, h.lat_noff, act,
+                     used, h.lat_pslot.p, h.lat_hist.p, lat_state(h));
+  // The image offsets' matrices beside the step lists (third stream).
+  const bool image = nimg > 0 && li.finest >= 0;
+  if (image) {
+    const dim3 grid(div_up(nimg, kImgT), kImgTParts);
+    EXA_HIP(hipEventRecord(h.ev_used, h.stream));
+    EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev_used, 0));
+    if (h.lat_tc_f32)
+      hipLaunchKernelGGL((k_lat_tmat_image<P, float>), grid, dim3(256), 0, h.stream3, h.lat_nreg, h.lat_noff,
+                         h.lat_okey.p, h.lat_orow.p, used, lvl, h.lvl_cells.p, h.cRb.p, li.cycle, h.lat_Tf.p,
+                         lat_state(h));
+    else
+      hipLaunchKernelGGL((k_lat_tmat_image<P, double>), grid, dim3(256), 0, h.stream3, h.lat_nreg, h.lat_noff,
+                         h.lat_okey.p, h.lat_orow.p, used, lvl, h.lvl_cells.p, h.cRb.p, li.cycle, h.lat_T.p,
+                         lat_state(h));
+    EXA_HIP(hipEventRecord(h.ev_image, h.stream3));
+  }
   if (nall > 0) {
-    hipLaunchKernelGGL(k_lat_count, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_noff, h.lat_tcnt.p);
+    hipLaunchKernelGGL(k_lat_count, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_noff, lr, h.lat_tcnt.p);
     // Step lists sized for every (tile, offset) being in use, so that the
     // host need not wait for the count, unless that bound is large.
-    int64_t nact = nall;
-    if (nall * 64 > kSlotBound) {
+    int64_t nact = nbound;
+    if (nbound * 64 > kSlotBound) {
       std::vector<int> cnt(h.lat_ntiles);
       EXA_HIP(hipMemcpyAsync(cnt.data(), h.lat_tcnt.p, h.lat_ntiles * sizeof(int), hipMemcpyDeviceToHost, h.stream));
       EXA_HIP(hipStreamSynchronize(h.stream));
@@ -914,7 +1164,7 @@ static void lattice_steps(Handle &h) {
     if (nact * 64 > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
     h.lat_alist.resize(nact > 0 ? nact : 1);
     h.lat_slot.resize(nact > 0 ? nact * 64 : 4);
-    hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff,
+    hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff, lr,
                        h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
                        reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h));
     hipLaunchKernelGGL(h.bounds_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
@@ -922,6 +1172,7 @@ static void lattice_steps(Handle &h) {
   }
   EXA_HIP(hipMemcpyAsync(h.hpin + kPinLat, lat_state(h), sizeof(LatState), hipMemcpyDeviceToHost, h.stream));
   EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
+  if (image) EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_image, 0));
   EXA_HIP(hipGetLastError());
 }
 
@@ -930,43 +1181,51 @@ static void lattice_steps(Handle &h) {
 // come in the same order whatever the table held before) and rows of T(d).
 template <int P>
 static void lattice_register(Handle &h) {
-  const int TPB = 256, gk = div_up(kLatKeys + 1, TPB);
+  const int TPB = 256, nk = h.lat_tc_keyn, gk = div_up(nk + 1, TPB);
   const bool f32 = h.lat_tc_f32;
-  h.lat_flag.resize(kLatKeys + 1);
-  h.lat_kscan.resize(kLatKeys + 1);
-  h.lat_tc_flag.resize(kLatKeys + 1);
-  h.lat_tc_scan.resize(kLatKeys + 1);
+  const int *marks = h.hpin + kPinMarks;
+  h.lat_flag.resize(nk + 1);
+  h.lat_kscan.resize(nk + 1);
+  h.lat_tc_flag.resize(nk + 1);
+  h.lat_tc_scan.resize(nk + 1);
   for (int again = 0;; again++) {
-    hipLaunchKernelGGL(k_lat_flag, dim3(gk), dim3(TPB), 0, h.stream, h.lat_hist.p, h.lat_ookey.p, h.lat_tc_map.p,
-                       kLatKeys, h.lat_flag.p, h.lat_tc_flag.p);
-    exclusive_scan_int(h, h.lat_flag.p, h.lat_kscan.p, kLatKeys + 1);
-    exclusive_scan_int(h, h.lat_tc_flag.p, h.lat_tc_scan.p, kLatKeys + 1);
-    EXA_HIP(hipMemcpyAsync(h.hpin + kPinNoff, h.lat_kscan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost, h.stream));
-    EXA_HIP(hipMemcpyAsync(h.hpin + kPinNnew, h.lat_tc_scan.p + kLatKeys, sizeof(int), hipMemcpyDeviceToHost,
-                           h.stream));
+    hipLaunchKernelGGL(k_lat_flag, dim3(gk), dim3(TPB), 0, h.stream, h.lat_hist.p, h.lat_ookey.p, h.lat_tc_map.p, nk,
+                       h.lat_flag.p, h.lat_tc_flag.p);
+    exclusive_scan_int(h, h.lat_flag.p, h.lat_kscan.p, nk + 1);
+    exclusive_scan_int(h, h.lat_tc_flag.p, h.lat_tc_scan.p, nk + 1);
+    hipLaunchKernelGGL(k_lat_marks, dim3(1), dim3(64), 0, h.stream, h.lat_kscan.p, h.lat_tc_scan.p, nk,
+                       h.hpin + kPinMarks);
     EXA_HIP(hipStreamSynchronize(h.stream));
-    if (again || h.lat_tc_rows == 0 || h.lat_tc_rows + h.hpin[kPinNnew] <= h.lat_tc_max) break;
+    // Image offsets that would make too many steps: none from here on.
+    const bool drop = (int64_t)h.lat_ntiles * marks[0] > INT_MAX && marks[0] > marks[3] && !h.lat_img_off;
+    if (drop) h.lat_img_off = true;
+    if (!drop && (again || h.lat_tc_rows == 0 || h.lat_tc_rows + marks[1] <= h.lat_tc_max)) break;
     tc_reset(h, P, f32);  // start the table afresh with this list's offsets alone
-    lattice_steps(h);
+    lattice_steps<P>(h);
   }
-  const int noff = h.hpin[kPinNoff], nnew = h.hpin[kPinNnew];
+  const int noff = marks[0], nnew = marks[1], nlat = marks[2];
+  for (int i = 0; i <= kImgLevels; i++) h.lat_img0[i] = marks[3 + i];
+  h.lat_nreg = marks[3];
+  h.lat_okey.resize(std::max(1, noff));
   h.lat_tc_keys.resize(std::max(1, nnew));
   h.lat_orow.resize(std::max(1, noff));
   hipLaunchKernelGGL(k_lat_number, dim3(gk), dim3(TPB), 0, h.stream, h.lat_flag.p, h.lat_kscan.p, h.lat_tc_flag.p,
-                     h.lat_tc_scan.p, kLatKeys, h.lat_tc_rows, h.lat_tc_map.p, h.lat_tc_keys.p, h.lat_ookey.p,
+                     h.lat_tc_scan.p, nk, h.lat_tc_rows, h.lat_tc_map.p, h.lat_tc_keys.p, h.lat_ookey.p, h.lat_okey.p,
                      h.lat_orow.p, h.lat_hist.p);
   h.lat_noff = noff;
   if (nnew > 0) {
     if (f32) {
       constexpr size_t TEP = TPad<P, float>::TEP;
       grow_keep_rows(h, h.lat_Tf, (size_t)(h.lat_tc_rows + nnew) * TEP, (size_t)h.lat_tc_rows * TEP);
-      hipLaunchKernelGGL((k_lat_tmat<P, float>), dim3(nnew), dim3(64), 0, h.stream, h.lat_tc_keys.p,
-                         h.lat_Tf.p + (size_t)h.lat_tc_rows * TEP);
+      if (nlat > 0)
+        hipLaunchKernelGGL((k_lat_tmat<P, float>), dim3(nlat), dim3(64), 0, h.stream, h.lat_tc_keys.p,
+                           h.lat_Tf.p + (size_t)h.lat_tc_rows * TEP);
     } else {
       constexpr size_t TEP = TPad<P, double>::TEP;
       grow_keep_rows(h, h.lat_T, (size_t)(h.lat_tc_rows + nnew) * TEP, (size_t)h.lat_tc_rows * TEP);
-      hipLaunchKernelGGL((k_lat_tmat<P, double>), dim3(nnew), dim3(64), 0, h.stream, h.lat_tc_keys.p,
-                         h.lat_T.p + (size_t)h.lat_tc_rows * TEP);
+      if (nlat > 0)
+        hipLaunchKernelGGL((k_lat_tmat<P, double>), dim3(nlat), dim3(64), 0, h.stream, h.lat_tc_keys.p,
+                           h.lat_T.p + (size_t)h.lat_tc_rows * TEP);
     }
     h.lat_tc_rows += nnew;
   }
@@ -987,13 +1246,15 @@ static void lattice_begin(Handle &h) {
   else
     run_lattice_tiles(h, h.stream);
   h.lat_tiles_ready = false;
-  if (h.lat_tc_P != P || h.lat_tc_f32 != f32 || (int64_t)h.lat_ntiles * h.lat_noff > INT_MAX) tc_reset(h, P, f32);
-  lattice_steps(h);
+  if (h.lat_tc_P != P || h.lat_tc_f32 != f32 || h.lat_tc_keyn != lat_keys(h) ||
+      (int64_t)h.lat_ntiles * h.lat_noff > INT_MAX)
+    tc_reset(h, P, f32);
+  lattice_steps<P>(h);
   if (h.lat_noff == 0) {  // no offset known yet: register them before P2P fills the GPU
     EXA_HIP(hipEventSynchronize(h.ev_cnt));
     if (reinterpret_cast<const LatState *>(h.hpin + kPinLat)->unknown) {
       lattice_register<P>(h);
-      lattice_steps(h);
+      lattice_steps<P>(h);
     }
   }
   h.lat_begun = true;
@@ -1036,7 +1297,7 @@ static void lattice_run(Handle &h, M2LList &irr) {
     if (!ls->unknown) break;
     if (again) throw Error(EXAFMM_HIP_EDEVICE, "lattice M2L: offsets unknown after their registration");
     lattice_register<P>(h);
-    lattice_steps(h);
+    lattice_steps<P>(h);
   }
   const int nirr = ls->nirr;
   h.lat_stats_steps = h.lat_run_ntiles ? ls->nsteps : 0;

@@ -66,6 +66,8 @@ Handle::~Handle() {
   if (ev_mult) (void)hipEventDestroy(ev_mult);
   if (ev_cnt) (void)hipEventDestroy(ev_cnt);
   if (ev_lists) (void)hipEventDestroy(ev_lists);
+  if (ev_used) (void)hipEventDestroy(ev_used);
+  if (ev_image) (void)hipEventDestroy(ev_image);
   if (ev_tiles) (void)hipEventDestroy(ev_tiles);
   if (ev_p2pcnt) (void)hipEventDestroy(ev_p2pcnt);
   if (ev_bounds) (void)hipEventDestroy(ev_bounds);
