@@ -206,11 +206,8 @@ struct Handle {
   DBuf<int> lat_tkey, lat_tval, lat_aidx, lat_alist, lat_step0, lat_tcnt;
   DBuf<unsigned char> lat_act;  // state of the set-up (LatState), then flags of the (tile, offset) steps in use
   DBuf<double> lat_part;
-  DBuf<int> lat_flag, lat_kscan, lat_tile_tgt, lat_tile_of, lat_col_of, lat_slot, lat_irr, lat_scan, irr_off, irr_src,
-      irr_tgt;
+  DBuf<int> lat_flag, lat_kscan, lat_tile_tgt, lat_tile_of, lat_col_of, lat_slot, irr_off, irr_src, irr_tgt;
   DBuf<unsigned char> irr_img;
-  DBuf<int> irr_rt, irr_rs;     // irregular pairs in emission order (target, source)
-  DBuf<unsigned char> irr_ri;   // ... and image
   DBuf<int> lat_pslot;          // per-pair step (-1: irregular)
   // T(d) table kept across evaluations: offset key -> row of lat_T / lat_Tf
   // (-1: not computed yet), for expansion order lat_tc_P and FP32 or FP64.
@@ -230,6 +227,7 @@ struct Handle {
   int lat_tc_rows = 0, lat_tc_P = 0, lat_tc_max = 16384;  // rows; a fuller table starts afresh
   bool lat_tc_f32 = false;
   bool lat_ms_ready = false;     // lat_Ms / lat_Msf already queued for this evaluation
+  bool lat_reduce_pending = false;  // contraction queued, its reduction left to lattice_finish
   bool lat_begun = false;        // lattice set-up's first part queued (m2l_begin)
   bool lat_tiles_ready = false;  // tiles of this tree queued on the second stream (ev_tiles)
   int lat_ntiles = 0;            // tile slots of the tree
@@ -353,10 +351,9 @@ inline void resolve_p2p_count(Handle &h) {
 }
 // The M2L list grouped by target (run_lists leaves it raw for the lattice M2L).
 void ensure_m2l_grouped(Handle &h);
-// Pairs (tgt, src, img) grouped by target into CSR (off, src_out, img_out)
-// and the targets with pairs (tlist, ntl); waits for the device.
-void group_pairs(Handle &h, int64_t np, DBuf<int> &tgt, DBuf<int> &src, DBuf<unsigned char> &img, DBuf<int> &off,
-                 DBuf<int> &src_out, DBuf<unsigned char> &img_out, DBuf<int> &tlist, int &ntl);
+// The nirr irregular pairs of the M2L list grouped by target (irr_off, irr_src,
+// irr_img, the ntl targets irr_tgt) on stream st; waits for it.
+void group_irregular(Handle &h, hipStream_t st, int64_t nirr, int &ntl);
 void run_p2p(Handle &h, hipStream_t st);
 void run_m2l(Handle &h);
 // The lattice contraction and reduction / the whole M2L of the last
@@ -373,6 +370,7 @@ void run_direct_arrays(Handle &h, int nt, const double *t_xyzq, int ns, const do
 void run_mass_normalise(Handle &h);
 void run_ropt(Handle &h);
 bool run_m2l_lattice(Handle &h, M2LList &irr);
+void lattice_finish(Handle &h);
 void run_lattice_mscale(Handle &h, hipStream_t st);
 // Target tiles of the lattice contraction for the current tree.
 void run_lattice_tiles(Handle &h, hipStream_t st);

@@ -317,8 +317,8 @@ __global__ void __launch_bounds__(64 * W)
 constexpr int kFewTargets = 2048, kShortList = 16, kFewPairs = 1 << 20;
 
 template <int P>
-static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L, bool f32,
-                       bool timed) {
+static void m2l_launch(Handle &h, hipStream_t st, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L,
+                       bool f32, bool timed) {
   using S = M2LShape<P>;
   const int esz = f32 ? 8 : 16;  // bytes of one table entry
   const int key = P * 100 + esz;
@@ -328,9 +328,8 @@ static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const c
     for (int v : sc.slot0) blob.push_back((uint32_t)v);
     for (int v : sc.outslot) blob.push_back((uint32_t)v);
     h.m2l_sched.resize(blob.size());
-    EXA_HIP(hipMemcpyAsync(h.m2l_sched.p, blob.data(), blob.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
-                           h.stream));
-    EXA_HIP(hipStreamSynchronize(h.stream));
+    EXA_HIP(hipMemcpyAsync(h.m2l_sched.p, blob.data(), blob.size() * sizeof(uint32_t), hipMemcpyHostToDevice, st));
+    EXA_HIP(hipStreamSynchronize(st));
     h.m2l_sched_P = key;
   }
   const uint32_t *desc = h.m2l_sched.p;
@@ -338,12 +337,12 @@ static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const c
   const int *outslot = slot0 + 64;
   if (lst.ntgt == 0) return;
   if (timed) {
-    EXA_HIP(hipEventRecord(h.ev[14], h.stream));
+    EXA_HIP(hipEventRecord(h.ev[14], st));
     h.pair_timed = true;
   }
   auto launch = [&](auto kernel, int waves) {
-    hipLaunchKernelGGL(kernel, dim3(lst.ntgt), dim3(64 * waves), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img, cX, M,
-                       L, desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+    hipLaunchKernelGGL(kernel, dim3(lst.ntgt), dim3(64 * waves), 0, st, lst.tgt, lst.off, lst.src, lst.img, cX, M, L,
+                       desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
   };
   constexpr int W = P <= 10 ? 8 : 4;  // 55 KB of LDS per workgroup at P = 10, 41 KB at P = 12
   const bool few =
@@ -352,23 +351,23 @@ static void m2l_launch(Handle &h, const M2LList &lst, const double4 *cX, const c
     few ? launch(k_m2l<P, float, W>, W) : launch(k_m2l<P, float, 1>, 1);
   else
     few ? launch(k_m2l<P, double, W>, W) : launch(k_m2l<P, double, 1>, 1);
-  if (timed) EXA_HIP(hipEventRecord(h.ev[15], h.stream));
+  if (timed) EXA_HIP(hipEventRecord(h.ev[15], st));
   EXA_HIP(hipGetLastError());
 }
 
 template <int P>
-static void m2l_impl(Handle &h, const M2LList &lst) {
-  m2l_launch<P>(h, lst, h.cX.p, h.M.p, h.L.p, h.cfg.precision == 1, true);
+static void m2l_impl(Handle &h, hipStream_t st, const M2LList &lst) {
+  m2l_launch<P>(h, st, lst, h.cX.p, h.M.p, h.L.p, h.cfg.precision == 1, true);
 }
 
 void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L) {
   if (h.cfg.basis == 1) return launch_m2l_cart_arrays(h, lst, cX, M, nc, L);
   switch (h.cfg.P) {
-    case 4: m2l_launch<4>(h, lst, cX, M, L, false, false); break;
-    case 6: m2l_launch<6>(h, lst, cX, M, L, false, false); break;
-    case 8: m2l_launch<8>(h, lst, cX, M, L, false, false); break;
-    case 10: m2l_launch<10>(h, lst, cX, M, L, false, false); break;
-    case 12: m2l_launch<12>(h, lst, cX, M, L, false, false); break;
+    case 4: m2l_launch<4>(h, h.stream, lst, cX, M, L, false, false); break;
+    case 6: m2l_launch<6>(h, h.stream, lst, cX, M, L, false, false); break;
+    case 8: m2l_launch<8>(h, h.stream, lst, cX, M, L, false, false); break;
+    case 10: m2l_launch<10>(h, h.stream, lst, cX, M, L, false, false); break;
+    case 12: m2l_launch<12>(h, h.stream, lst, cX, M, L, false, false); break;
     default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");
   }
 }
@@ -395,14 +394,16 @@ void run_m2l(Handle &h) {
   }
   join_multipoles(h);  // (the lattice path joined them before its contraction)
   h.m2l_last = lst;
+  const hipStream_t st = h.lat_reduce_pending ? h.stream3 : h.stream;
   switch (h.cfg.P) {
-    case 4: m2l_impl<4>(h, lst); break;
-    case 6: m2l_impl<6>(h, lst); break;
-    case 8: m2l_impl<8>(h, lst); break;
-    case 10: m2l_impl<10>(h, lst); break;
-    case 12: m2l_impl<12>(h, lst); break;
+    case 4: m2l_impl<4>(h, st, lst); break;
+    case 6: m2l_impl<6>(h, st, lst); break;
+    case 8: m2l_impl<8>(h, st, lst); break;
+    case 10: m2l_impl<10>(h, st, lst); break;
+    case 12: m2l_impl<12>(h, st, lst); break;
     default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");
   }
+  lattice_finish(h);
 }
 
 // The M2L of the last run_m2l again on the current multipoles: the lattice
@@ -413,11 +414,11 @@ void run_m2l_replay(Handle &h) {
   lattice_replay(h);
   const bool f32 = h.cfg.precision == 1;
   switch (h.cfg.P) {
-    case 4: m2l_launch<4>(h, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
-    case 6: m2l_launch<6>(h, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
-    case 8: m2l_launch<8>(h, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
-    case 10: m2l_launch<10>(h, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
-    case 12: m2l_launch<12>(h, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
+    case 4: m2l_launch<4>(h, h.stream, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
+    case 6: m2l_launch<6>(h, h.stream, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
+    case 8: m2l_launch<8>(h, h.stream, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
+    case 10: m2l_launch<10>(h, h.stream, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
+    case 12: m2l_launch<12>(h, h.stream, h.m2l_last, h.cX.p, h.M.p, h.L.p, f32, false); break;
     default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");
   }
 }

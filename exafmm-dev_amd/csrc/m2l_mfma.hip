@@ -59,7 +59,7 @@ constexpr int kLatKeys = kLatSide * kLatSide * kLatSide;
 // evaluation.
 //
 // Used on the finest kImgLevels levels that are dense, from level 3 on: there
-// a T (61 KB at P = 10, 30 ns to make and to read) serves 100 to 1000 pairs of
+// a T (31 KB at P = 10, 30 ns to make and to read) serves 100 to 1000 pairs of
 // 1.8 ns each on the per-pair kernel (a lattice of 64^3 bodies, theta = 0.35).
 // Images across an edge of the box share one offset among 40 to 50 pairs, as
 // coarser levels and the few cells of a sparse level do, and gain nothing:
@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(64) k_lat_tmat(const int *__restrict__ okey, R
 // T of the image offsets in use (numbers nreg + i, used[i]), as k_lat_tmat for
 // the actual offset of their level and face.  A workgroup makes kImgT of them
 // together, so that the entries' index arithmetic is done once for all; bound
-// by the stores: 6800 offsets at P = 10 are 415 MB, 0.32 ms alone with one
+// by the stores: 6800 offsets at P = 10 are 212 MB, 0.32 ms alone with one
 // workgroup per kImgT and 0.45 ms beside P2P and the step lists, which hide it.
 // lvl: for each level mod 3 the first of its cells in lvl_cells.
 constexpr int kImgT = 16, kImgTParts = 4;  // (each in kImgTParts workgroups, for balance)
@@ -686,11 +686,6 @@ __global__ void k_lat_slots(const int *__restrict__ ptgt, const int *__restrict_
   }
 }
 
-__global__ void k_irr_flag(const int *__restrict__ pstep, int64_t np, int *__restrict__ irr) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e <= np) irr[e] = e < np && pstep[e] < 0 ? 1 : 0;
-}
-
 // Offsets known after this set-up (the known ones and those hist flags, to
 // be numbered in key order), and those of them with no row in the T table.
 __global__ void k_lat_flag(const unsigned char *__restrict__ hist, const int *__restrict__ o_of_key,
@@ -747,18 +742,6 @@ __global__ void k_lat_used(const unsigned char *__restrict__ act, int ntiles, in
 __global__ void k_fill_int(int *__restrict__ p, int64_t n, int v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
-}
-
-// The irregular pairs (irr[e] = 1) in emission order.
-__global__ void k_irr_compact(const int *__restrict__ irr, const int *__restrict__ scan, int64_t np,
-                              const int *__restrict__ tgt, const int *__restrict__ src,
-                              const unsigned char *__restrict__ img, int *__restrict__ tgt_irr,
-                              int *__restrict__ src_irr, unsigned char *__restrict__ img_irr) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= np || !irr[e]) return;
-  tgt_irr[scan[e]] = tgt[e];
-  src_irr[scan[e]] = src[e];
-  img_irr[scan[e]] = img[e];
 }
 
 // ---------------------------------------------------------------------------
@@ -960,7 +943,13 @@ __global__ void __launch_bounds__(256)
     const double iw = 1.0 / (2 * cRb[tgt] / kLatUnit);
     double f = iw;
     for (int q = 0; q < deg.n[(r0 + row) >> 1]; q++) f *= iw;
-    Lr[(size_t)tgt * NR + r0 + row] += sv[row][c] * f;
+    // Rounded before it is added: the sum with the per-pair kernel's part is
+    // then the same whichever of the two comes first.
+    {
+#pragma clang fp contract(off)
+      const double v = sv[row][c] * f;
+      Lr[(size_t)tgt * NR + r0 + row] += v;
+    }
   }
 }
 
@@ -1272,6 +1261,12 @@ static void lattice_run(Handle &h, M2LList &irr) {
   const int ntiles = h.lat_ntiles;
   h.lat_stats_tiles = 0;
   join_multipoles(h);  // the set-up above did not need them
+  // Irregular pairs are expected: they are grouped and translated on the third
+  // stream beside the contraction, and the reduction adds to their result
+  // (lattice_finish).  Behind the reduction on the main stream instead, a box
+  // of 64^3 bodies (237000 of 11.5 M pairs irregular) took 5.09 ms, not 4.81,
+  // and 4.2 M clustered bodies 22.7 ms, not 22.2.
+  const bool irregular = (h.cfg.images > 0 || h.cfg.builder == 1) && !h.serial_heavy;
   // The contraction (timed by ev[12..13]) and the reduction: queued on the
   // set-up as it is; both do nothing if it met an unknown offset, and are
   // queued again after that offset has its row.
@@ -1291,7 +1286,7 @@ static void lattice_run(Handle &h, M2LList &irr) {
       h.lat_timed = true;
       lattice_contract<P>(h);
       EXA_HIP(hipEventRecord(h.ev[13], h.stream));
-      lattice_reduce<P>(h);
+      if (!irregular) lattice_reduce<P>(h);
     }
     EXA_HIP(hipEventSynchronize(h.ev_cnt));
     if (!ls->unknown) break;
@@ -1302,25 +1297,31 @@ static void lattice_run(Handle &h, M2LList &irr) {
   const int nirr = ls->nirr;
   h.lat_stats_steps = h.lat_run_ntiles ? ls->nsteps : 0;
   h.lat_stats_tiles = h.lat_run_ntiles ? ls->ntiles : 0;
-  // The irregular pairs (none for a uniform free-space tree), in emission
-  // order, grouped by target (a stable sort: within a target the order of the
-  // full list grouped by target), queued behind the contraction.
+  h.lat_reduce_pending = irregular && h.lat_run_ntiles > 0;
   int nitl = 0;
   if (nirr) {
-    h.lat_irr.resize(np + 1);
-    h.lat_scan.resize(np + 1);
-    hipLaunchKernelGGL(k_irr_flag, dim3(div_up(np + 1, TPB)), dim3(TPB), 0, h.stream, h.lat_pslot.p, np, h.lat_irr.p);
-    exclusive_scan_int(h, h.lat_irr.p, h.lat_scan.p, (int)(np + 1));
-    h.irr_rt.resize(nirr);
-    h.irr_rs.resize(nirr);
-    h.irr_ri.resize(nirr);
-    hipLaunchKernelGGL(k_irr_compact, dim3(gp), dim3(TPB), 0, h.stream, h.lat_irr.p, h.lat_scan.p, np, h.raw_mi.p,
-                       h.raw_mj.p, h.raw_mimg.p, h.irr_rt.p, h.irr_rs.p, h.irr_ri.p);
-    group_pairs(h, nirr, h.irr_rt, h.irr_rs, h.irr_ri, h.irr_off, h.irr_src, h.irr_img, h.irr_tgt, nitl);
+    if (h.lat_reduce_pending) EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev_cnt, 0));
+    group_irregular(h, h.lat_reduce_pending ? h.stream3 : h.stream, nirr, nitl);
   }
   irr = M2LList{h.irr_tgt.p, nitl, h.irr_off.p, h.irr_src.p, h.irr_img.p, nirr};
   h.lat_stats_pairs = np - nirr;
   EXA_HIP(hipGetLastError());
+}
+
+// The reduction left by run_m2l_lattice, behind the per-pair kernel on the
+// third stream.
+void lattice_finish(Handle &h) {
+  if (!h.lat_reduce_pending) return;
+  h.lat_reduce_pending = false;
+  EXA_HIP(hipEventRecord(h.ev_image, h.stream3));
+  EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_image, 0));
+  switch (h.cfg.P) {
+    case 4: lattice_reduce<4>(h); break;
+    case 6: lattice_reduce<6>(h); break;
+    case 8: lattice_reduce<8>(h); break;
+    case 10: lattice_reduce<10>(h); break;
+    case 12: lattice_reduce<12>(h); break;
+  }
 }
 
 // Distinct offsets of the last contraction (a reduction over its step flags).
@@ -1386,7 +1387,7 @@ void lattice_replay(Handle &h) {
 }
 
 bool run_m2l_lattice(Handle &h, M2LList &irr) {
-  h.lat_timed = false;
+  h.lat_timed = h.lat_reduce_pending = false;
   h.lat_run_ntiles = 0;
   h.lat_stats_pairs = 0;
   h.lat_stats_tiles = 0;

@@ -493,10 +493,17 @@ __device__ inline bool wave_run(int t, int lane, int &first, int &len) {
   return t >= 0;
 }
 
-__global__ void __launch_bounds__(256) k_group_count(const int *__restrict__ tgt, int64_t n, int *__restrict__ cnt) {
+// An entry's target; -1 for none and for the entries that skip marks (>= 0) as
+// somebody else's.
+__device__ inline int group_target(const int *__restrict__ tgt, const int *__restrict__ skip, int64_t e, int64_t n) {
+  return e < n && !(skip && skip[e] >= 0) ? tgt[e] : -1;
+}
+
+__global__ void __launch_bounds__(256) k_group_count(const int *__restrict__ tgt, const int *__restrict__ skip,
+                                                     int64_t n, int *__restrict__ cnt) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
-  const int t = e < n ? tgt[e] : -1;
+  const int t = group_target(tgt, skip, e, n);
   int first, len;
   if (wave_run(t, lane, first, len) && lane == first) atomicAdd(&cnt[t], len);
 }
@@ -559,11 +566,11 @@ __global__ void __launch_bounds__(1024)
 
 // ord: the entries' indices, grouped; the counts run back to zero.
 __global__ void __launch_bounds__(256)
-    k_group_scatter(const int *__restrict__ tgt, int64_t n, const int *__restrict__ off, int *__restrict__ cnt,
-                    int *__restrict__ ord) {
+    k_group_scatter(const int *__restrict__ tgt, const int *__restrict__ skip, int64_t n, const int *__restrict__ off,
+                    int *__restrict__ cnt, int *__restrict__ ord) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
-  const int t = e < n ? tgt[e] : -1;
+  const int t = group_target(tgt, skip, e, n);
   int first, len, at = 0;
   const bool in = wave_run(t, lane, first, len);
   if (in && lane == first) at = off[t] + atomicSub(&cnt[t], len) - len;
@@ -606,19 +613,22 @@ static void grow_keep(Handle &h, DBuf<T> &b, size_t want, size_t keep) {
 // w.r.t. emission order), and the compact list of targets with at least one
 // entry, whose count is written to *ntl_host (pinned; valid after st is
 // synchronised) and left on the device at *ntl_dev (if given; valid until the
-// next grouping with g).  Nothing waits for the device.
+// next grouping with g).  With skip, only the nout entries k with skip[k] < 0.
+// Nothing waits for the device.
 static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t np, DBuf<int> &tgt, DBuf<int> &src,
                             DBuf<unsigned char> &img, DBuf<int> &off, DBuf<int> &src_out, DBuf<unsigned char> &img_out,
-                            DBuf<int> &tlist, int *ntl_host, const int **ntl_dev = nullptr) {
+                            DBuf<int> &tlist, int *ntl_host, const int **ntl_dev = nullptr,
+                            const int *skip = nullptr, int64_t nout = -1) {
   const int nc = h.ncells;
   if (np > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "list grouping: more than 2^31 - 1 entries");
   const int chunks = div_up(nc, kGroupChunk);
   off.resize(nc + 1);
-  src_out.resize(np);
-  img_out.resize(np);
+  if (!skip) nout = np;
+  src_out.resize(nout);
+  img_out.resize(nout);
   tlist.resize(nc);
-  g.ord.reserve(np + 1);
-  g.aux.reserve(np + 1);
+  g.ord.reserve(nout + 1);
+  g.aux.reserve(nout + 1);
   g.tot.reserve(2 * (size_t)chunks + 2);
   int2 *tot = reinterpret_cast<int2 *>(g.tot.p);
   int *ntl = g.tot.p + 2 * (size_t)chunks;
@@ -628,13 +638,14 @@ static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t 
   }
   g.zero = false;
   if (np > 0)
-    hipLaunchKernelGGL(k_group_count, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, np, g.cnt.p);
+    hipLaunchKernelGGL(k_group_count, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, skip, np, g.cnt.p);
   if (chunks > 1) hipLaunchKernelGGL(k_group_totals, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot);
   hipLaunchKernelGGL(k_group_offsets, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot, off.p, tlist.p, ntl, ntl_host);
   if (np > 0) {
     int bits = 1;
     while (((int64_t)1 << bits) < np) bits++;
-    hipLaunchKernelGGL(k_group_scatter, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, np, off.p, g.cnt.p, g.ord.p);
+    hipLaunchKernelGGL(k_group_scatter, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, skip, np, off.p, g.cnt.p,
+                       g.ord.p);
     hipLaunchKernelGGL(k_group_sort, dim3(nc), dim3(64), 0, st, off.p, bits, g.ord.p, g.aux.p, src.p, img.p, src_out.p,
                        img_out.p);
   }
@@ -801,11 +812,10 @@ void ensure_m2l_grouped(Handle &h) {
   h.m2l_grouped = true;
 }
 
-void group_pairs(Handle &h, int64_t np, DBuf<int> &tgt, DBuf<int> &src, DBuf<unsigned char> &img, DBuf<int> &off,
-                 DBuf<int> &src_out, DBuf<unsigned char> &img_out, DBuf<int> &tlist, int &ntl) {
-  group_by_target(h, h.grp1, h.stream, np, tgt, src, img, off, src_out, img_out,
-                  tlist, h.hpin + 10);
-  EXA_HIP(hipStreamSynchronize(h.stream));
+void group_irregular(Handle &h, hipStream_t st, int64_t nirr, int &ntl) {
+  group_by_target(h, h.grp1, st, h.nm2l, h.raw_mi, h.raw_mj, h.raw_mimg, h.irr_off, h.irr_src, h.irr_img, h.irr_tgt,
+                  h.hpin + 10, nullptr, h.lat_pslot.p, nirr);
+  EXA_HIP(hipStreamSynchronize(st));
   ntl = h.hpin[10];
 }
 
