@@ -796,8 +796,15 @@ typedef __attribute__((address_space(1))) void glb_void;
 // and the step loop is unrolled by two, so every access names its buffer
 // statically (no register copy between steps).  The segment's partial
 // expansions (unscaled) go to part[] for k_lat_reduce.
+//
+// A wave without a pair in its 16 columns sits the step out: in adaptive trees
+// half the columns of a step and more are empty (250k clustered bodies, P = 12,
+// FP32: 1.66 ms, 1.55 without them).  Up to P = 8 in FP64 and P = 10 in FP32 the
+// registers allow three or four workgroups per CU: 4.2 M clustered bodies, P =
+// 8, took 8.5 ms with two and 7.5 with three; 1 M bodies, P = 10, FP32, 0.69
+// and 0.64.
 template <int P, typename R>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 10 ? 2 : 1, 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 10 ? 2 : 1, 4)))
     k_m2l_mfma(int nc, int nitems, const int *__restrict__ step0, const int *__restrict__ alist,
                const int *__restrict__ slot, const R *__restrict__ T, const R *__restrict__ Ms,
                double *__restrict__ part, const LatState *__restrict__ st) {
@@ -851,34 +858,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 1
     };
     // Step i from buffers CUR = (i - i0) & 1 while step i + 1 is fetched
     // into the other ones.
+    bool busy = false;
     auto step = [&](auto curc, int i) {
       constexpr int CUR = decltype(curc)::value;
       const R *sTc = CUR ? sT1 : sT0;
       R *sTn = CUR ? sT0 : sT1;
       const R *b = CUR ? b1 : b0;
       R *bn = CUR ? b0 : b1;
-      const bool more = i + 1 < i1;
+      const bool more = i + 1 < i1, busy_next = more && __any(sn <= -2);
       int snn = -1;
       if (more) {
-        load_col(bn, sn);
+        if (busy_next) load_col(bn, sn);
         fetch_T(sTn, i + 1);
         if (i + 2 < i1) snn = slot[(size_t)(i + 2) * 64 + col];
       }
+      if (busy) {
 #pragma unroll
-      for (int rb = 0; rb < RB; rb++) {
+        for (int rb = 0; rb < RB; rb++) {
 #pragma unroll
-        for (int kc = 0; kc < S::kc_end(rb); kc++)
-          acc[rb] = A::mac(sTc[(S::base(rb) + kc) * 64 + lane], b[kc], acc[rb]);
-      }
-      if (F32) {
+          for (int kc = 0; kc < S::kc_end(rb); kc++)
+            acc[rb] = A::mac(sTc[(S::base(rb) + kc) * 64 + lane], b[kc], acc[rb]);
+        }
+        if (F32) {
 #pragma unroll
-        for (int rb = 0; rb < (F32 ? RB : 1); rb++)
-          for (int r = 0; r < 4; r++) {
-            acc64[rb][r] += (double)acc[rb][r];
-            acc[rb][r] = 0;
-          }
+          for (int rb = 0; rb < (F32 ? RB : 1); rb++)
+            for (int r = 0; r < 4; r++) {
+              acc64[rb][r] += (double)acc[rb][r];
+              acc[rb][r] = 0;
+            }
+        }
       }
       if (more) sn = snn;
+      busy = busy_next;
       __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this wave's DMA and loads have landed
       __syncthreads();
     };
@@ -886,6 +897,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 1
     if (i0 < i1) {
       fetch_T(sT0, i0);
       sn = slot[(size_t)i0 * 64 + col];
+      busy = __any(sn <= -2);
       load_col(b0, sn);
       sn = i0 + 1 < i1 ? slot[(size_t)(i0 + 1) * 64 + col] : -1;
     }
