@@ -159,6 +159,7 @@ struct Handle {
   DBuf<unsigned char> p2p_img, m2l_img;
   DBuf<int> p2p_tgt, m2l_tgt;      // compact target lists
   DBuf<int> p2p_next;              // P2P work counter (next target leaf)
+  bool p2p_next_clear = false;     // cleared by the list grouping, for one run_p2p
   int np2p_tgt = 0, nm2l_tgt = 0;  // np2p_tgt < 0: on the device only (p2p_cnt_dev)
   const int *p2p_cnt_dev = nullptr;
   DBuf<int> raw_mi, raw_mj, raw_pi, raw_pj;  // emission-order lists

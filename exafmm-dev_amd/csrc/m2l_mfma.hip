@@ -610,7 +610,8 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(256)
     k_lat_steps(const unsigned char *__restrict__ act, const int *__restrict__ cnt, int noff, LatRanges lr,
                 const int *__restrict__ orow, int *__restrict__ aidx, int *__restrict__ step0,
-                int *__restrict__ alist, int4 *__restrict__ slot, LatState *__restrict__ st) {
+                int *__restrict__ alist, int4 *__restrict__ slot, LatState *__restrict__ st,
+                LatState *__restrict__ host) {
   __shared__ int sw[4], sn[4];
   const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int base = 0, full = 0;
@@ -636,6 +637,7 @@ __global__ void __launch_bounds__(256)
       step0[tile + 1] = base + mine;
       st->nsteps = base + mine;
       st->ntiles = sn[0] + sn[1] + sn[2] + sn[3] + (mine > 0);
+      *host = *st;  // (pinned)
     }
   }
   if (mine == 0) return;
@@ -1108,6 +1110,7 @@ static void lattice_steps(Handle &h) {
   const int64_t np = h.nm2l, nall = (int64_t)h.lat_ntiles * h.lat_noff;
   const int TPB = 256, gp = div_up(np, TPB);
   const int *ptgt = h.raw_mi.p, *psrc = h.raw_mj.p;
+  LatState *const host = reinterpret_cast<LatState *>(h.hpin + kPinLat);
   if (nall > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "lattice M2L: too many (tile, offset) steps");
   const LatImages li = lat_images(h);
   const int nimg = h.lat_noff - h.lat_nreg;
@@ -1167,12 +1170,15 @@ static void lattice_steps(Handle &h) {
     h.lat_slot.resize(nact > 0 ? nact * 64 : 4);
     hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff, lr,
                        h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
-                       reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h));
+                       reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h), host);
+    if (!h.bounds_given) EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
     hipLaunchKernelGGL(h.bounds_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
                        psrc, np, h.lat_col_of.p, h.lat_aidx.p, h.lat_pslot.p, h.lat_slot.p, lat_state(h));
   }
-  EXA_HIP(hipMemcpyAsync(h.hpin + kPinLat, lat_state(h), sizeof(LatState), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
+  if (nall == 0 || h.bounds_given) {  // (k_lat_slots may add irregular pairs)
+    EXA_HIP(hipMemcpyAsync(host, lat_state(h), sizeof(LatState), hipMemcpyDeviceToHost, h.stream));
+    EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
+  }
   if (image) EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_image, 0));
   EXA_HIP(hipGetLastError());
 }

@@ -1105,8 +1105,8 @@ void run_p2p(Handle &h, hipStream_t st) {
     if (h.np2p_tgt == 0) return;
     grid = h.p2p_wpc > 0 ? std::min(h.np2p_tgt, grid) : h.np2p_tgt;
   }
-  h.p2p_next.reserve(1);
-  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, h.p2p_next.p);
+  if (!h.p2p_next_clear) hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, h.p2p_next.p);
+  h.p2p_next_clear = false;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, st, h.p2p_tgt.p, h.np2p_tgt, ntl_dev, h.p2p_next.p,
                        h.p2p_off.p, h.p2p_src.p, h.p2p_img.p, h.cBody.p, h.cNBody.p, h.body4.p, h.trg4.p, h.cfg.cycle);

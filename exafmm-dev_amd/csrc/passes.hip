@@ -476,7 +476,6 @@ void run_upward(Handle &h) {
 void run_upward_radii(Handle &h) {
   h.M.resize((size_t)h.ncells * h.nterm);
   h.L.resize((size_t)h.ncells * h.nterm);
-  EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream));
   run_radii(h);
   EXA_HIP(hipEventRecord(h.ev[16], h.stream));
 }
@@ -484,6 +483,7 @@ void run_upward_radii(Handle &h) {
 void run_upward_mult(Handle &h) {
   EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev[16], 0));
   EXA_HIP(hipEventRecord(h.ev[17], h.stream3));
+  EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream3));  // (read with the multipoles)
   // The tiles on the second stream, idle until the lists are there.
   EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev[16], 0));
   run_lattice_tiles(h, h.stream2);

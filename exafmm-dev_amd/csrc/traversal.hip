@@ -224,6 +224,9 @@ struct TravState {
   int done_blocks;               // k_emit_dev blocks finished (the last one advances the level)
 };
 
+constexpr int kPinTrav = 16;  // words of Handle::hpin that receive the state
+static_assert(kPinTrav * sizeof(int) % 8 == 0 && sizeof(TravState) <= 48 * sizeof(int), "pinned words");
+
 constexpr int kSmallFrontier = 512;  // levels up to this size run in one workgroup
 constexpr int kSmallBlock = 1024;
 
@@ -245,35 +248,34 @@ __device__ inline void chunk_of(int nf, int &i0, int &i1) {
   i1 = min(nf, i0 + c);
 }
 
-__global__ void k_trav_init(TravState *st, int nf) {
-  st->nm = st->np = 0;
-  st->nf = nf;
-  st->fsel = 0;
-  st->overflow = 0;
-  st->levels = 0;
-  st->levels_small = 0;
-  st->done_blocks = 0;
+// The first frontier: the root against itself for every image, or (a forest)
+// every root against itself, no images: the traversal never pairs cells of two
+// systems.
+__device__ inline int2 first_pair(const int *__restrict__ roots, int images, int i) {
+  return roots ? pack_pair(roots[i], roots[i], 13) : pack_pair(0, 0, images == 0 ? 13 : i);
 }
 
 // The first levels, while 0 < nf <= kSmallFrontier, in one workgroup: both
 // passes of a level back to back (the frontier in 1024-pair chunks, in
-// order), no launch per level.
+// order), no launch per level.  Makes the first frontier of nf0 pairs itself;
+// the state goes to the host (pinned) with every kernel that changes it.
 __global__ void __launch_bounds__(kSmallBlock)
-    k_trav_small(CellView cv, int2 *__restrict__ fa, int2 *__restrict__ fb, TravState *st, double cycle,
-                 int nspawn, int mutual, unsigned char *__restrict__ act, int *__restrict__ m2l_i,
+    k_trav_small(CellView cv, const int *__restrict__ roots, int images, int nf0, int2 *fa, int2 *fb, TravState *st,
+                 TravState *__restrict__ host, double cycle, int nspawn, int mutual, unsigned char *__restrict__ act, int *__restrict__ m2l_i,
                  int *__restrict__ m2l_j, unsigned char *__restrict__ m2l_img, int *__restrict__ p2p_i,
                  int *__restrict__ p2p_j, unsigned char *__restrict__ p2p_img, long long cap_m2l, long long cap_p2p,
                  int cap_f) {
   __shared__ int s_nf, s_fsel;
   __shared__ long long s_nm, s_np;
+  for (int i = threadIdx.x; i < nf0; i += kSmallBlock) fa[i] = first_pair(roots, images, i);
   if (threadIdx.x == 0) {
-    s_nf = st->nf;
-    s_fsel = st->fsel;
-    s_nm = st->nm;
-    s_np = st->np;
+    s_nf = nf0;
+    s_fsel = 0;
+    s_nm = s_np = 0;
   }
   __syncthreads();
   int levels = 0;
+  bool overflow = false;  // (the same for all threads)
   while (true) {
     const int nf = s_nf;
     if (nf == 0 || nf > kSmallFrontier) break;
@@ -295,7 +297,7 @@ __global__ void __launch_bounds__(kSmallBlock)
       acc = add4(acc, tot);
     }
     if (!(nm + acc.x <= cap_m2l && np + acc.y <= cap_p2p && acc.z <= cap_f)) {
-      if (threadIdx.x == 0) st->overflow = 1;
+      overflow = true;
       break;
     }
     int4 run = make_int4(0, 0, 0, 0);
@@ -323,18 +325,8 @@ __global__ void __launch_bounds__(kSmallBlock)
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    if (st->overflow) {
-      st->nf = 0;
-    } else {
-      st->nf = s_nf;
-      st->fsel = s_fsel;
-      st->nm = s_nm;
-      st->np = s_np;
-      st->levels += levels;
-      st->levels_small = levels;
-    }
-  }
+  if (threadIdx.x == 0)
+    *host = *st = TravState{s_nm, s_np, overflow ? 0 : s_nf, s_fsel, overflow ? 1 : 0, levels, levels, 0};
 }
 
 template <int NT, int K>
@@ -375,7 +367,8 @@ __global__ void __launch_bounds__(NT, NT / 128)  // two blocks per CU
 // last block to finish moves the state to the next level.
 template <int NT, int K>
 __global__ void __launch_bounds__(NT, NT / 128)  // two blocks per CU
-    k_emit_dev(CellView cv, int2 *__restrict__ fa, int2 *__restrict__ fb, TravState *st, int mutual,
+    k_emit_dev(CellView cv, int2 *__restrict__ fa, int2 *__restrict__ fb, TravState *st,
+               TravState *__restrict__ host, int mutual,
                const unsigned char *__restrict__ act, const int4 *__restrict__ blk, long long cap_m2l,
                long long cap_p2p, int cap_f, int *__restrict__ m2l_i, int *__restrict__ m2l_j,
                unsigned char *__restrict__ m2l_img, int *__restrict__ p2p_i, int *__restrict__ p2p_j,
@@ -455,23 +448,13 @@ __global__ void __launch_bounds__(NT, NT / 128)  // two blocks per CU
       st->fsel = fsel ^ 1;
       st->levels++;
     }
+    *host = *st;
   }
 }
 
-__global__ void k_init_frontier(int2 *__restrict__ fr, int images) {
-  const int i = threadIdx.x;
-  if (images == 0) {
-    if (i == 0) fr[0] = pack_pair(0, 0, 13);
-  } else if (i < 27) {
-    fr[i] = pack_pair(0, 0, i);
-  }
-}
-
-// A forest (batched systems): every root against itself, no images; the
-// traversal never pairs cells of two systems.
-__global__ void k_init_frontier_roots(int2 *__restrict__ fr, const int *__restrict__ roots, int nroots) {
+__global__ void k_init_frontier(int2 *__restrict__ fr, const int *__restrict__ roots, int images, int nf) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nroots) fr[i] = pack_pair(roots[i], roots[i], 13);
+  if (i < nf) fr[i] = first_pair(roots, images, i);
 }
 
 // Grouping a list by target: entries counted per target, offsets by a scan,
@@ -526,10 +509,12 @@ __global__ void __launch_bounds__(1024)
 }
 
 // off[c] = entries of the targets before c, tlist = the non-empty targets;
-// the number of those to *ntl and *ntl_host (pinned).
+// the number of those to *ntl and *ntl_host (pinned); *next (if given) is
+// cleared, the work counter of what reads the list.
 __global__ void __launch_bounds__(1024)
     k_group_offsets(const int *__restrict__ cnt, int nc, const int2 *__restrict__ tot, int *__restrict__ off,
-                    int *__restrict__ tlist, int *__restrict__ ntl, int *__restrict__ ntl_host) {
+                    int *__restrict__ tlist, int *__restrict__ ntl, int *__restrict__ ntl_host,
+                    int *__restrict__ next) {
   __shared__ int sbase[2];
   int4 v = make_int4(0, 0, 0, 0), sum;
   for (int b = threadIdx.x; b < (int)blockIdx.x; b += 1024) {
@@ -561,6 +546,7 @@ __global__ void __launch_bounds__(1024)
     off[nc] = sbase[0] + sum.x;
     *ntl = sbase[1] + sum.y;
     *ntl_host = sbase[1] + sum.y;
+    if (next) *next = 0;
   }
 }
 
@@ -613,12 +599,12 @@ static void grow_keep(Handle &h, DBuf<T> &b, size_t want, size_t keep) {
 // w.r.t. emission order), and the compact list of targets with at least one
 // entry, whose count is written to *ntl_host (pinned; valid after st is
 // synchronised) and left on the device at *ntl_dev (if given; valid until the
-// next grouping with g).  With skip, only the nout entries k with skip[k] < 0.
+// next grouping with g); *next is cleared.  With skip, only the nout entries k with skip[k] < 0.
 // Nothing waits for the device.
 static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t np, DBuf<int> &tgt, DBuf<int> &src,
                             DBuf<unsigned char> &img, DBuf<int> &off, DBuf<int> &src_out, DBuf<unsigned char> &img_out,
                             DBuf<int> &tlist, int *ntl_host, const int **ntl_dev = nullptr,
-                            const int *skip = nullptr, int64_t nout = -1) {
+                            const int *skip = nullptr, int64_t nout = -1, int *next = nullptr) {
   const int nc = h.ncells;
   if (np > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "list grouping: more than 2^31 - 1 entries");
   const int chunks = div_up(nc, kGroupChunk);
@@ -640,7 +626,8 @@ static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t 
   if (np > 0)
     hipLaunchKernelGGL(k_group_count, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, skip, np, g.cnt.p);
   if (chunks > 1) hipLaunchKernelGGL(k_group_totals, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot);
-  hipLaunchKernelGGL(k_group_offsets, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot, off.p, tlist.p, ntl, ntl_host);
+  hipLaunchKernelGGL(k_group_offsets, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot, off.p, tlist.p, ntl, ntl_host,
+                     next);
   if (np > 0) {
     int bits = 1;
     while (((int64_t)1 << bits) < np) bits++;
@@ -656,10 +643,11 @@ static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t 
 
 // Levels of device-driven passes, enqueued without waiting; returns false
 // (nothing usable emitted) when an output did not fit its buffer or the
-// traversal did not end within kMaxLevels levels.  The frontier starts in fa.
-static bool traverse_on_device(Handle &h, const CellView &cv, int nf0, int mutual, int64_t &nm, int64_t &np) {
+// traversal did not end within kMaxLevels levels.
+static bool traverse_on_device(Handle &h, const CellView &cv, const int *roots, int nf0, int mutual, int64_t &nm,
+                               int64_t &np) {
   constexpr int kMaxLevels = 256;
-  // (fa and fb were sized by the caller before the frontier was written.)
+  // (fa and fb were sized by the caller.)
   h.ia.reserve(std::max(h.trav_fcap, nf0) + 1);
   h.ib.reserve(4 * (size_t)kTravGrid);
   h.trav_state.reserve(sizeof(TravState));
@@ -669,26 +657,26 @@ static bool traverse_on_device(Handle &h, const CellView &cv, int nf0, int mutua
   const int cap_fr = (int)std::min(std::min(h.fa.cap, h.fb.cap), h.ia.cap) - 1;  // frontier and action slots
   int4 *blk = reinterpret_cast<int4 *>(h.ib.p);
   unsigned char *act = reinterpret_cast<unsigned char *>(h.ia.p);
-  hipLaunchKernelGGL(k_trav_init, dim3(1), dim3(1), 0, h.stream, st, nf0);
-  hipLaunchKernelGGL(k_trav_small, dim3(1), dim3(kSmallBlock), 0, h.stream, cv, h.fa.p, h.fb.p, st, h.cfg.cycle,
-                     h.cfg.nspawn, mutual, act, h.raw_mi.p, h.raw_mj.p, h.raw_mimg.p, h.raw_pi.p, h.raw_pj.p,
+  TravState *const host = reinterpret_cast<TravState *>(h.hpin + kPinTrav);
+  hipLaunchKernelGGL(k_trav_small, dim3(1), dim3(kSmallBlock), 0, h.stream, cv, roots, h.cfg.images, nf0, h.fa.p,
+                     h.fb.p, st, host, h.cfg.cycle, h.cfg.nspawn, mutual, act, h.raw_mi.p, h.raw_mj.p, h.raw_mimg.p, h.raw_pi.p, h.raw_pj.p,
                      h.raw_pimg.p, cap_m, cap_p, cap_fr);
-  TravState hs{};
+  const volatile TravState &hs = *host;
   int enq = 0;
   // The levels after the small ones: as many as the last traversal had (its
   // last level leaves an empty frontier), then more in batches if needed.
-  int batch = h.trav_levels > 0 ? h.trav_levels : 8;
+  int batch = h.trav_levels;
   while (true) {
     for (int l = 0; l < batch; l++) {
       hipLaunchKernelGGL((k_classify_dev<kClassifyBlock, 1>), dim3(kTravGrid), dim3(kClassifyBlock), 0, h.stream, cv,
                          h.fa.p, h.fb.p, st, h.cfg.cycle, h.cfg.nspawn, mutual, act, blk);
       hipLaunchKernelGGL((k_emit_dev<kEmitBlock, kEmitItems>), dim3(kTravGrid), dim3(kEmitBlock), 0, h.stream, cv,
-                         h.fa.p, h.fb.p, st, mutual, act, blk, cap_m, cap_p, cap_fr, h.raw_mi.p, h.raw_mj.p,
+                         h.fa.p, h.fb.p, st, host, mutual, act, blk, cap_m, cap_p, cap_fr, h.raw_mi.p, h.raw_mj.p,
                          h.raw_mimg.p, h.raw_pi.p, h.raw_pj.p, h.raw_pimg.p);
     }
     enq += batch;
     enqueue_multipoles(h);  // the second stream's work, while these levels run
-    EXA_HIP(hipMemcpyAsync(&hs, st, sizeof(TravState), hipMemcpyDeviceToHost, h.stream));
+    EXA_HIP(hipGetLastError());
     EXA_HIP(hipStreamSynchronize(h.stream));
     if (hs.overflow) return false;
     if (hs.nf == 0) break;
@@ -714,18 +702,11 @@ void run_lists(Handle &h) {
   // Periodic images are traversed non-mutually (traversal.h:250-259).
   const int mutual = (h.cfg.mutual && h.cfg.images == 0) ? 1 : 0;
   if (h.nsys > 1) nf = h.lvl_off[1] - h.lvl_off[0];  // the roots: level 0 of the forest
+  const int *roots = h.nsys > 1 ? h.lvl_cells.p + h.lvl_off[0] : nullptr;
   // Frontier buffers sized before the first frontier is written (a reserve
   // that grows a buffer drops its contents).
   h.fa.reserve(std::max(nf + 64, h.trav_fcap));
   if (h.trav_fcap > 0) h.fb.reserve(std::max(nf + 64, h.trav_fcap));
-  auto init_frontier = [&]() {
-    if (h.nsys > 1)
-      hipLaunchKernelGGL(k_init_frontier_roots, dim3(div_up(nf, 256)), dim3(256), 0, h.stream, h.fa.p,
-                         h.lvl_cells.p + h.lvl_off[0], nf);
-    else
-      hipLaunchKernelGGL(k_init_frontier, dim3(1), dim3(64), 0, h.stream, h.fa.p, h.cfg.images);
-  };
-  init_frontier();
   // Start the raw lists at a capacity that covers uniform trees without
   // regrowth (about 180 M2L and 65 P2P sources per cell at theta = 0.4).
   grow_keep(h, mi, (size_t)h.ncells * 128 + 1024, 0);
@@ -737,12 +718,13 @@ void run_lists(Handle &h) {
   h.cnt.reserve(4);
   const int nf0 = nf;
   bool done = false;
-  if (h.trav_fcap > 0) {
-    done = traverse_on_device(h, cv, nf0, mutual, nm, np);
-    if (!done) init_frontier();  // the per-level passes start over
+  if (h.trav_fcap > 0) done = traverse_on_device(h, cv, roots, nf0, mutual, nm, np);
+  if (!done) {  // the per-level passes
+    hipLaunchKernelGGL(k_init_frontier, dim3(div_up(nf, 256)), dim3(256), 0, h.stream, h.fa.p, roots, h.cfg.images,
+                       nf);
+    h.trav_levels = 0;
+    enqueue_multipoles(h);
   }
-  if (!done) h.trav_levels = 0;
-  if (!done) enqueue_multipoles(h);
   int max_nf = nf0;
   while (!done && nf > 0) {
     const int nb = div_up(nf, kTravBlock);
@@ -791,8 +773,10 @@ void run_lists(Handle &h) {
   if (h.m2l_grouped)
     group_by_target(h, h.grp1, h.stream, nm, mi, mj, mimg, h.m2l_off,
                     h.m2l_src, h.m2l_img, h.m2l_tgt, h.hpin + 8);
+  h.p2p_next.reserve(1);
   group_by_target(h, h.grp2, h.stream2, np, pi, pj, pimg, h.p2p_off,
-                  h.p2p_src, h.p2p_img, h.p2p_tgt, h.hpin + 9, &h.p2p_cnt_dev);
+                  h.p2p_src, h.p2p_img, h.p2p_tgt, h.hpin + 9, &h.p2p_cnt_dev, nullptr, -1, h.p2p_next.p);
+  h.p2p_next_clear = true;
   EXA_HIP(hipEventRecord(h.ev_p2pcnt, h.stream2));
   h.np2p_tgt = -1;
   h.nm2l_tgt = 0;

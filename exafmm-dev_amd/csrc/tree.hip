@@ -17,8 +17,11 @@ namespace exafmm {
 // ---------------------------------------------------------------------------
 // Bounds: grid-stride min/max, one partial per block, then one block.
 constexpr int kBoundsBlocks = 512;
+constexpr int kBoundsOne = 4096;  // bodies up to which one block is no slower than a second launch
 
-__global__ void __launch_bounds__(256) k_bounds_partial(const double4 *__restrict__ b, int n, double *__restrict__ part) {
+// (host: with one block, the pinned copy of the result.)
+__global__ void __launch_bounds__(256) k_bounds_partial(const double4 *__restrict__ b, int n, double *__restrict__ part,
+                                                        double *__restrict__ host) {
   __shared__ double s[6][256];
   double mn[3] = {b[0].x, b[0].y, b[0].z};
   double mx[3] = {mn[0], mn[1], mn[2]};
@@ -48,6 +51,7 @@ __global__ void __launch_bounds__(256) k_bounds_partial(const double4 *__restric
     __syncthreads();
   }
   if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
+  if (host && threadIdx.x < 6) host[threadIdx.x] = s[threadIdx.x][0];
 }
 
 __global__ void __launch_bounds__(256) k_bounds_final(const double *__restrict__ part, int nb, double *__restrict__ out,
@@ -87,11 +91,15 @@ void run_bounds(Handle &h) {
     h.have_bounds = true;
     return;
   }
-  const int nb = std::min(kBoundsBlocks, div_up(h.n, 256));
-  h.red.reserve(6 * nb);
-  hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(256), 0, h.stream, h.in4.p, h.n, h.red.p);
-  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, h.stream, h.red.p, nb, h.box.p,
-                     reinterpret_cast<double *>(h.hpin + Handle::kPinBounds));
+  double *host = reinterpret_cast<double *>(h.hpin + Handle::kPinBounds);
+  if (h.n <= kBoundsOne) {
+    hipLaunchKernelGGL(k_bounds_partial, dim3(1), dim3(256), 0, h.stream, h.in4.p, h.n, h.box.p, host);
+  } else {
+    const int nb = std::min(kBoundsBlocks, div_up(h.n, 256));
+    h.red.reserve(6 * nb);
+    hipLaunchKernelGGL(k_bounds_partial, dim3(nb), dim3(256), 0, h.stream, h.in4.p, h.n, h.red.p, nullptr);
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(256), 0, h.stream, h.red.p, nb, h.box.p, host);
+  }
   EXA_HIP(hipEventRecord(h.ev_bounds, h.stream));
   h.bounds_pending = true;
   h.have_bounds = true;
@@ -174,8 +182,6 @@ __device__ inline void set_box(const double *mn, const double *mx, ForestSys &f)
   f.d = 2 * R0 / (1 << f.L);
 }
 
-__global__ void k_box(const double *__restrict__ bb, ForestSys *__restrict__ fs) { set_box(bb, bb + 3, fs[0]); }
-
 // Per-system min/max: chunks (system, first, last body), one workgroup each,
 // then one workgroup per system over its chunks [chunk0[s], chunk0[s + 1]).
 __device__ inline void block_minmax(double *mn, double *mx, double (*s)[256]) {
@@ -256,12 +262,21 @@ __device__ inline int last_le(const int *__restrict__ v, int n, int x) {
 // division, truncation to int, bit interleave in int.  leaf[b] = the body's
 // leaf among all systems' possible ones, slot[b] = its place there.
 __global__ void __launch_bounds__(256)
-    k_leaf_count(const double4 *__restrict__ in, int n, const ForestSys *__restrict__ fs, int S,
-                 const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ slot,
+    k_leaf_count(const double4 *__restrict__ in, int n, const double *__restrict__ box, ForestSys *__restrict__ fs,
+                 int S, const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ slot,
                  int *__restrict__ cnt) {
   const int b = blockIdx.x * 256 + threadIdx.x;
   if (b >= n) return;
-  const ForestSys f = fs[S > 1 ? last_le(begin, S, b) : 0];
+  ForestSys f = fs[S > 1 ? last_le(begin, S, b) : 0];
+  if (box) {  // one system: its box, for the kernels behind this one too
+    set_box(box, box + 3, f);
+    if (b == 0) {
+      fs->x0 = f.x0;
+      fs->y0 = f.y0;
+      fs->z0 = f.z0;
+      fs->d = f.d;
+    }
+  }
   const double4 v = in[b];
   const double dd = (double)f.d;
   int ix = (int)((v.x - f.x0) / dd);
@@ -534,7 +549,6 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
     hipLaunchKernelGGL(k_bounds_systems, dim3(S), dim3(256), 0, h.stream, h.red.p, h.ut_tab.p + chunk00, fsd);
   } else {
     upload_bounds(h);
-    hipLaunchKernelGGL(k_box, dim3(1), dim3(1), 0, h.stream, h.box.p, fsd);
   }
   h.body4.resize(n);
   h.bidx.resize(n);
@@ -552,8 +566,8 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
   }
   h.ut_zero = false;
   int *leaf = h.ic.p, *ord = h.ia.p, *aux = h.ib.p, *start = h.ut_start.p, *rank = h.ut_rank.p;
-  hipLaunchKernelGGL(k_leaf_count, dim3(div_up(n, 256)), dim3(256), 0, h.stream, h.in4.p, n, fsd, S,
-                     h.ut_tab.p + begin0, leaf, aux, h.ut_cnt.p);
+  hipLaunchKernelGGL(k_leaf_count, dim3(div_up(n, 256)), dim3(256), 0, h.stream, h.in4.p, n,
+                     own_bounds ? nullptr : h.box.p, fsd, S, h.ut_tab.p + begin0, leaf, aux, h.ut_cnt.p);
   if (sh.ncell <= kScanSmall) {
     hipLaunchKernelGGL(k_tree_scan_small, dim3(1), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, start, rank);
   } else {
