@@ -80,12 +80,13 @@ struct SrcDesc {
 
 // skip: a cell whose unshifted entry (image 13) is left out (-1: none).
 // put(k, v, im) stores body v (x, y, z, q) with image im into slot k; NB
-// body loads are in flight at a time (registers against latency).
+// body loads are in flight at a time (registers against latency).  At most
+// `most` bodies are taken.
 template <int STAGE, int NB = 4, typename Put>
 __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__restrict__ src,
                                  const unsigned char *__restrict__ img, const int *__restrict__ cBody,
                                  const int *__restrict__ cNBody, const double4 *__restrict__ body, SrcDesc &sd,
-                                 Put put, int skip = -1) {
+                                 Put put, int skip = -1, int most = STAGE) {
   static_assert(STAGE <= kFillMax && STAGE % 64 == 0, "the slot map covers a stage, four slots per lane");
   static_assert((STAGE / 64) % NB == 0, "whole batches of loads");
   wave_sync();  // the previous stage (and descriptor batch) are consumed
@@ -112,7 +113,7 @@ __device__ inline int fill_stage(SrcWalker &w, int e1, int lane, const int *__re
   const int first = w.e - w.dbase;
   const int q0 = sd.pre[first] + w.sbase;
   const int qend = sd.pre[64];
-  const int cnt = min(STAGE, qend - q0);
+  const int cnt = min(most < STAGE ? most : STAGE, qend - q0);
   // Slot map: entry `first` from slot 0, each later entry with bodies from
   // its first slot in the stage; a running maximum fills the rest.
   int4 *m4 = reinterpret_cast<int4 *>(sd.map);
@@ -191,14 +192,52 @@ __device__ inline int next_leaf(int *next, int lane) {
 }
 
 // Several waves per leaf (k_p2p_f64): wave 0 takes the leaf's own bodies, and
-// each of the W waves a contiguous part of the list through its own stage; the
-// waves' sums of a target are added in wave order.  (Not in the mixed form:
+// each of the W waves a contiguous part of the list's bodies through its own
+// stage, so that all have the same number; the waves' sums of a target are added
+// in wave order.  (Equal numbers of list entries instead: 1960 us for a new charge
+// vector on 500 000 bodies on a sphere, of which P2P is all but 250; now 1800.)  (Not in the mixed form:
 // the split moves the boundaries of its FP32 runs, so that a system would give
 // other roundings alone than in a batch.)
 template <int W>
 struct Team {
   double4 part[W > 1 ? W : 1][64];
   int next;
+
+  // This wave's part of the list [e0, e1) of leaf c (n bodies, wave 0's beside
+  // its part): where it starts, and how many bodies it has.
+  __device__ int share(int e0, int e1, int c, int n, int wave, int lane, const int *__restrict__ src,
+                       const unsigned char *__restrict__ img, const int *__restrict__ cNBody, SrcWalker &w) const {
+    auto bodies = [&](int e) {
+      if (e >= e1) return 0;
+      const int s = src[e];
+      return s == c && img[e] == 13 ? 0 : cNBody[s];
+    };
+    int total = 0;
+    for (int b = e0; b < e1; b += 64) total += bodies(b + lane);
+    for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor(total, d);
+    // Wave w ends where (w + 1) / W of all bodies are done, the own ones first.
+    auto end = [&](int k) { return max(0, (int)((int64_t)(total + n) * k / W) - n); };
+    const int q0 = wave == 0 ? 0 : end(wave), q1 = end(wave + 1);
+    w = SrcWalker{e0, 0, e0, 0};
+    int before = 0;  // bodies of the entries before b
+    for (int b = e0; b < e1 && q0 > 0; b += 64) {
+      const int m = bodies(b + lane);
+      int incl = m;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int t = __shfl_up(incl, d);
+        if (lane >= d) incl += t;
+      }
+      const unsigned long long past = __ballot(before + incl > q0);  // the first of these holds body q0
+      if (past) {
+        const int k = __ffsll(past) - 1;
+        w.e = w.dbase = b + k;
+        w.sbase = q0 - before - (__shfl(incl, k) - __shfl(m, k));
+        break;
+      }
+      before += __shfl(incl, 63);
+    }
+    return q1 - q0;
+  }
 
   __device__ int next_leaf(int *counter, int lane) {
     if (W == 1) return exafmm::next_leaf(counter, lane);
@@ -278,12 +317,9 @@ __global__ void __launch_bounds__(64 * W)
   for (int bi = blockIdx.x; bi < ntl; bi = team.next_leaf(next, lane)) {
     const int c = tgt_list[bi];
     const int tb0 = cBody[c], tn = cNBody[c];
-    int e0 = off[c], e1 = off[c + 1];
-    if (W > 1) {
-      const int ne = e1 - e0;
-      e1 = e0 + ne * (wave + 1) / W;
-      e0 += ne * wave / W;
-    }
+    const int e0 = off[c], e1 = off[c + 1];
+    SrcWalker first{e0, 0, e0, 0};
+    const int share = W > 1 ? team.share(e0, e1, c, tn, wave, lane, src, img, cNBody, first) : 0;
     // Sum the G group partials (lanes gg T + i) of the pass's targets in
     // group order.
     auto combine = [&](const double4 &acc, int T, int G, int n, int tfirst) {
@@ -426,8 +462,9 @@ __global__ void __launch_bounds__(64 * W)
         for (int k = lane; k < cnt; k += 64) sb[k] = body[tb0 + s0 + k];
         run(std::true_type{}, cnt);
       }
-      SrcWalker w{e0, 0, e0, 0};
-      while (w.e < e1) {
+      SrcWalker w = first;
+      int left = share;  // (W > 1)
+      while (w.e < e1 && (W == 1 || left > 0)) {
         // Fill: consecutive source leaves (or parts of one) up to kP2PStage
         // bodies, each shifted by its periodic image.
         bool imaged = false;
@@ -445,7 +482,8 @@ __global__ void __launch_bounds__(64 * W)
               }
               sb[k] = v;
             },
-            c);
+            c, W > 1 ? left : kP2PStage);
+        left -= cnt;
         if (cnt == 0) continue;
         if (__any(imaged))
           run(std::true_type{}, cnt);
@@ -1069,7 +1107,7 @@ __global__ void k_count_body_pairs(const int *__restrict__ tgt_list, int ntl, co
 // 12 waves per CU, and below a few leaves for each the longest ones and the
 // latency of single waves decide the time.  64 leaves: 19 us with 8 waves each
 // against 85 with one; 994 leaves: 100 against 181; 4744 leaves of 500 000
-// bodies on a sphere: 1870 against 2157.
+// bodies on a sphere, a new charge vector: 1800 with 4, 2110 with 8, 2290 with one.
 static int p2p_team(const Handle &h, int64_t leaves) {
   const int64_t waves = 12 * (int64_t)h.ncu;
   if (leaves * 8 <= waves) return 8;
