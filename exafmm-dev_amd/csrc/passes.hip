@@ -376,16 +376,25 @@ __global__ void __launch_bounds__(64)
 static int first_leaf(const Handle &h) { return h.lvl_off[std::min(h.leaf_level, h.nlevels - 1)]; }
 
 template <int P>
-static void multipoles_impl(Handle &h, hipStream_t st) {
+static void p2m_impl(Handle &h, hipStream_t st) {
+  const int l0 = first_leaf(h), n = h.ncells - l0;
+  hipLaunchKernelGGL(k_p2m<P>, dim3(n), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p, h.cNChild.p,
+                     h.cBody.p, h.cNBody.p, h.M.p);
+}
+
+// Parents up to which a level runs per cell: the product on the matrix cores
+// reads all eight octants' operators whatever their number (P = 10, 1 to 64
+// parents: 21 us, 11 to 14 per cell; 512 parents: 25 against 29).
+constexpr int kM2MFew = 64;
+
+template <int P>
+static void m2m_impl(Handle &h, hipStream_t st) {
   const bool mf = updown_mfma_enabled(h);
-  const int l0 = first_leaf(h);
-  hipLaunchKernelGGL(k_p2m<P>, dim3(h.ncells - l0), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
-                     h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p);
   for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;
     const int *cells = h.lvl_cells.p + h.lvl_off[t];
-    if (mf)
+    if (mf && cnt > kM2MFew)
       run_m2m_level_mfma(h, cells, cnt, st);
     else
       hipLaunchKernelGGL(k_m2m<P>, dim3(cnt), dim3(512), 0, st, cells, h.cX.p, h.cChild.p, h.cNChild.p, h.M.p);
@@ -467,42 +476,48 @@ void run_upward(Handle &h) {
   run_multipoles(h, h.stream);
 }
 
+#define EXA_DISPATCH_ST(fn, h, st)                                                   \
+  switch ((h).cfg.P) {                                                               \
+    case 4: fn<4>(h, st); break;                                                     \
+    case 6: fn<6>(h, st); break;                                                     \
+    case 8: fn<8>(h, st); break;                                                     \
+    case 10: fn<10>(h, st); break;                                                   \
+    case 12: fn<12>(h, st); break;                                                   \
+    default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");    \
+  }
+
 // The upward pass split over two streams: radii (needed by the traversal)
 // on the main stream, multipoles (needed only by M2L) on the third stream
-// after the radii, joined by the main stream through h.ev_mult before M is
-// read (join_multipoles).  run_upward_mult is enqueued by the traversal once its
-// own first kernels are queued (its launches would otherwise hold the host
-// while the main stream idles).
+// behind the tree (ev[2]), joined by the main stream through h.ev_mult before M
+// is read (join_multipoles).  P2M is queued with the radii and runs beside
+// them; run_upward_mult queues the rest, called by the traversal once its own
+// first kernels are queued (its launches would otherwise hold the host while
+// the main stream idles).
 void run_upward_radii(Handle &h) {
   h.M.resize((size_t)h.ncells * h.nterm);
   h.L.resize((size_t)h.ncells * h.nterm);
   run_radii(h);
   EXA_HIP(hipEventRecord(h.ev[16], h.stream));
+  EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev[2], 0));
+  EXA_HIP(hipEventRecord(h.ev[17], h.stream3));
+  EXA_DISPATCH_ST(p2m_impl, h, h.stream3);
 }
 
 void run_upward_mult(Handle &h) {
-  EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev[16], 0));
-  EXA_HIP(hipEventRecord(h.ev[17], h.stream3));
-  EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream3));  // (read with the multipoles)
   // The tiles on the second stream, idle until the lists are there.
   EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev[16], 0));
   run_lattice_tiles(h, h.stream2);
   EXA_HIP(hipEventRecord(h.ev_tiles, h.stream2));
   h.lat_tiles_ready = true;
-  run_multipoles(h, h.stream3);
+  EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream3));  // (read with the multipoles)
+  EXA_DISPATCH_ST(m2m_impl, h, h.stream3);
   run_lattice_mscale(h, h.stream3);  // the lattice M2L's input
   EXA_HIP(hipEventRecord(h.ev_mult, h.stream3));
 }
 
 void run_multipoles(Handle &h, hipStream_t st) {
-  switch (h.cfg.P) {
-    case 4: multipoles_impl<4>(h, st); break;
-    case 6: multipoles_impl<6>(h, st); break;
-    case 8: multipoles_impl<8>(h, st); break;
-    case 10: multipoles_impl<10>(h, st); break;
-    case 12: multipoles_impl<12>(h, st); break;
-    default: throw Error(EXAFMM_HIP_EUNSUP, "P must be one of 4, 6, 8, 10, 12");
-  }
+  EXA_DISPATCH_ST(p2m_impl, h, st);
+  EXA_DISPATCH_ST(m2m_impl, h, st);
 }
 
 void run_downward(Handle &h) {
