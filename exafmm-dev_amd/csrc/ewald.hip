@@ -293,11 +293,13 @@ constexpr int kEwStage = 128;
 // power of two targets, replicated over 64 / T lane groups that split the
 // staged bodies; a leaf whose size leaves more than a quarter of T idle takes
 // a second, smaller pass.  Lanes select the source leaves of a chunk; their
-// bodies fill the stage in parallel through a slot map.  A pair is about 65
+// bodies within the cut-off of the targets' box fill the stage in parallel
+// through a slot map (without that test 23% of the pairs evaluated were out of
+// range, with it 15%; 2.31 ms and 2.28).  A pair is about 65
 // FP64 operations (erfc and exp as polynomials with one reciprocal square
 // root and one reciprocal, instead of the library's erfc, exp, sqrt and
 // divide), which bounds the kernel: about 90 issued with the tests and LDS
-// reads.  32768 bodies, cut-off half the box: 2.3 ms (3.0 ms with the
+// reads.  32768 bodies, cut-off half the box: 2.28 ms (3.0 ms with the
 // coefficients in VGPRs), 8.47 ms with the library functions, at least 16
 // lanes per leaf and leaves staged one after another.
 __global__ void __launch_bounds__(64)
@@ -327,6 +329,18 @@ __global__ void __launch_bounds__(64)
     const bool active = ti < rem;
     const double4 xi = active ? body[tb0 + tbase + ti] : make_double4(0, 0, 0, 0);
     double pot = 0, gx = 0, gy = 0, gz = 0;
+    // The targets' box.
+    double lo[3], hi[3];
+    for (int d = 0; d < 3; d++) {
+      const double x = d == 0 ? xi.x : d == 1 ? xi.y : xi.z;
+      lo[d] = active ? x : 1e300;
+      hi[d] = active ? x : -1e300;
+    }
+    for (int w = 32; w >= 1; w >>= 1)
+      for (int d = 0; d < 3; d++) {
+        lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
+        hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
+      }
     for (int base = 64 * blockIdx.y; base < ncells; base += 64 * gridDim.y) {
       // Lanes select the source leaves of this chunk and their images.
       const int cj = base + lane;
@@ -372,17 +386,25 @@ __global__ void __launch_bounds__(64)
         __syncthreads();
         for (int k = max(first, w0); k < min(end, w0 + kEwStage); k++) smap[k - w0] = (unsigned char)lane;
         __syncthreads();
-        for (int k = lane; k < cnt; k += 64) {
-          const int l = smap[k];
-          double4 v = body[sfrom[l] + w0 + k];
+        int nst = 0;  // staged bodies: those within the cut-off of the targets' box
+        for (int k0 = 0; k0 < cnt; k0 += 64) {
+          const int k = k0 + lane;
+          bool in = k < cnt;
+          const int l = smap[in ? k : 0];
+          double4 v = body[sfrom[l] + w0 + (in ? k : 0)];
           const double4 p = sshift[l];
           v.x += p.x;
           v.y += p.y;
           v.z += p.z;
-          sb[k] = v;
+          const double dx = fmax(fmax(lo[0] - v.x, v.x - hi[0]), 0.0), dy = fmax(fmax(lo[1] - v.y, v.y - hi[1]), 0.0),
+                       dz = fmax(fmax(lo[2] - v.z, v.z - hi[2]), 0.0);
+          in = in && dx * dx + dy * dy + dz * dz < cut2 * (1 + 1e-9);
+          const unsigned long long m = __ballot(in);
+          if (in) sb[nst + (int)__popcll(m & ((1ull << lane) - 1))] = v;
+          nst += (int)__popcll(m);
         }
         __syncthreads();
-        for (int k = g; k < cnt; k += G) {
+        for (int k = g; k < nst; k += G) {
           const double4 xj = sb[k];
           const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
           const double R2 = dx * dx + dy * dy + dz * dz;
