@@ -53,13 +53,23 @@ static void enqueue_numeric(Handle &h) {
   EXA_HIP(hipGetLastError());
   zero_device(h.L.p, (size_t)h.ncells * h.nterm * sizeof(cplx), h.stream);
   EXA_HIP(hipEventRecord(h.ev_fork, h.stream));
+  auto p2p = [&] {
+    EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev_fork, 0));
+    run_p2p(h, h.stream2);
+    EXA_HIP(hipEventRecord(h.ev_gp2p, h.stream2));
+  };
+  // The order of launches: P2P first, beside the multipoles, where its resident
+  // grid of single waves leaves them room (20 000 bodies, mixed, 289 us and 324;
+  // 500 000 on a sphere, mixed, 1560 and 1600; 1 M bodies the same); behind them
+  // where teams of waves take the LDS of every CU (200 000 bodies, P = 8, 825 us
+  // first and 750 behind).
+  const bool first = p2p_waves_per_leaf(h) == 1;
+  if (first) p2p();
   EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev_fork, 0));
   run_multipoles(h, h.stream3);
   run_lattice_mscale(h, h.stream3);
   EXA_HIP(hipEventRecord(h.ev_gmult, h.stream3));
-  EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev_fork, 0));
-  run_p2p(h, h.stream2);
-  EXA_HIP(hipEventRecord(h.ev_gp2p, h.stream2));
+  if (!first) p2p();
   EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_gmult, 0));
   run_m2l_replay(h);
   if (h.cfg.images > 0) run_periodic(h);

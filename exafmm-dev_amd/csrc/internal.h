@@ -356,6 +356,7 @@ void ensure_m2l_grouped(Handle &h);
 // irr_img, the ntl targets irr_tgt) on stream st; waits for it.
 void group_irregular(Handle &h, hipStream_t st, int64_t nirr, int &ntl);
 void run_p2p(Handle &h, hipStream_t st);
+int p2p_waves_per_leaf(const Handle &h);
 void run_m2l(Handle &h);
 // The lattice contraction and reduction / the whole M2L of the last
 // run_m2l again, on the current multipoles (its set-up reused).

@@ -1114,14 +1114,23 @@ static int p2p_team(const Handle &h, int64_t leaves) {
   return leaves <= 2 * waves ? 4 : 1;
 }
 
+// Leaves by the tree alone (with p2p_kmax == 1): the same for every grid.
+static int64_t tree_leaves(const Handle &h) {
+  int64_t leaves = h.ncells;
+  for (int l = 0; l + 1 < h.nlevels; l++) leaves -= std::min(h.lvl_par[l], h.lvl_off[l + 1] - h.lvl_off[l]);
+  return std::max<int64_t>(1, leaves);
+}
+
+int p2p_waves_per_leaf(const Handle &h) {
+  return h.p2p_kmax == 1 && h.cfg.precision == 0 ? p2p_team(h, tree_leaves(h)) : 1;
+}
+
 void run_p2p(Handle &h, hipStream_t st) {
   // Every body belongs to a leaf that is in its own list, and every target is
   // written once: the results need no clearing.
   if (h.np2p_tgt == 0) return;
-  // Leaves by the tree alone (with p2p_kmax == 1): the same for every grid.
-  int64_t leaves = h.ncells;
-  for (int l = 0; l + 1 < h.nlevels; l++) leaves -= std::min(h.lvl_par[l], h.lvl_off[l + 1] - h.lvl_off[l]);
-  const int W = h.p2p_kmax == 1 && h.cfg.precision == 0 ? p2p_team(h, std::max<int64_t>(1, leaves)) : 1;
+  const int64_t leaves = tree_leaves(h);
+  const int W = p2p_waves_per_leaf(h);
   // A resident grid of p2p_wpc waves per CU that claims target leaves from a
   // counter (0: one team per leaf).  A resident grid leaves the rest of each
   // CU to the other stream's kernels (the lattice M2L set-up runs beside P2P
