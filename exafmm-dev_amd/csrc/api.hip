@@ -314,9 +314,9 @@ static void evaluate_all(Handle &h) {
       do_build(h);
     }
     EXA_HIP(hipEventRecord(h.ev[2], h.stream));
-    // Inside one evaluation the multipoles (P2M, M2M) run on the second
+    // Inside one evaluation the multipoles (P2M, M2M) run on the third
     // stream while the main stream computes radii and builds the lists.
-    const bool split = h.cfg.basis == 0 && !h.cfg.useRopt;
+    const bool split = !h.cfg.useRopt;
     if (split) {
       ensure(h.have_tree, "upward_pass: tree not built");
       run_upward_radii(h);

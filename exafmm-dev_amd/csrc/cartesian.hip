@@ -136,7 +136,8 @@ struct CartTab {
 
 // ---------------------------------------------------------------------------
 // Upward pass: P2M (:590-598) at leaves, M2M (:600-612) at parents, then
-// setRmax and R /= theta as in the spherical pass.
+// setRmax and R /= theta as in the spherical pass (radii = 0: left out, where
+// the radii are made beside the multipoles).
 
 __device__ inline void cart_radius(double4 *cX, int c, double rb, double rmax, double theta, int useRmax) {
   double R = rb;
@@ -162,7 +163,7 @@ template <int P>
 __global__ void __launch_bounds__(64)
     k_p2m_cart(const int *__restrict__ cells, const double4 *__restrict__ body, double4 *__restrict__ cX,
                const double *__restrict__ cRb, const int *__restrict__ cNChild, const int *__restrict__ cBody,
-               const int *__restrict__ cNBody, cplx *__restrict__ M, double theta, int useRmax) {
+               const int *__restrict__ cNBody, cplx *__restrict__ M, double theta, int useRmax, int radii) {
 #pragma clang fp contract(off)
   constexpr int NT = Cart<P>::NT;
   constexpr int NO = (NT + 63) / 64;
@@ -208,7 +209,7 @@ __global__ void __launch_bounds__(64)
   for (int o = 0; o < NO; o++)
     if (lane + 64 * o < NT) M[(size_t)c * NT + lane + 64 * o] = {acc[o], 0.0};
   rmax = wave_max(rmax);
-  if (lane == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
+  if (radii && lane == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
 }
 
 // The parents among `cells` (one level), one wave per child; the children's
@@ -219,7 +220,7 @@ template <int P>
 __global__ void __launch_bounds__(512)
     k_m2m_cart(const int *__restrict__ cells, double4 *__restrict__ cX, const double *__restrict__ cRb,
                const int *__restrict__ cChild, const int *__restrict__ cNChild, cplx *__restrict__ M, double theta,
-               int useRmax) {
+               int useRmax, int radii) {
 #pragma clang fp contract(off)
   constexpr int NT = Cart<P>::NT;
   __shared__ double sC[8][NT], sM[8][NT], s0[8][NT], s1[8][NT];
@@ -270,7 +271,7 @@ __global__ void __launch_bounds__(512)
       }
   }
   if ((int)threadIdx.x < NT) M[(size_t)c * NT + threadIdx.x] = {acc, 0.0};
-  if (threadIdx.x == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
+  if (radii && threadIdx.x == 0) cart_radius(cX, c, cRb[c], rmax, theta, useRmax);
 }
 
 // ---------------------------------------------------------------------------
@@ -804,15 +805,19 @@ static void periodic_cart_impl(Handle &h) {
 // ---------------------------------------------------------------------------
 // All leaves first (they need nothing), then the parents level by level.
 template <int P>
-static void upward_cart_impl(Handle &h) {
+static void p2m_cart_impl(Handle &h, hipStream_t st, int radii) {
   const int l0 = h.lvl_off[std::min(h.leaf_level, h.nlevels - 1)];  // the cells that can be leaves
-  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells - l0), dim3(64), 0, h.stream, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
-                     h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
+  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells - l0), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
+                     h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
+}
+
+template <int P>
+static void m2m_cart_impl(Handle &h, hipStream_t st, int radii) {
   for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;
-    hipLaunchKernelGGL(k_m2m_cart<P>, dim3(cnt), dim3(512), 0, h.stream, h.lvl_cells.p + h.lvl_off[t], h.cX.p,
-                       h.cRb.p, h.cChild.p, h.cNChild.p, h.M.p, h.cfg.theta, h.cfg.useRmax);
+    hipLaunchKernelGGL(k_m2m_cart<P>, dim3(cnt), dim3(512), 0, st, h.lvl_cells.p + h.lvl_off[t], h.cX.p, h.cRb.p,
+                       h.cChild.p, h.cNChild.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
   }
   EXA_HIP(hipGetLastError());
 }
@@ -837,7 +842,20 @@ static void downward_cart_impl(Handle &h) {
     default: throw Error(EXAFMM_HIP_EUNSUP, "Cartesian P must be one of 4, 6, 8"); \
   }
 
-void run_upward_cart(Handle &h) { EXA_DISPATCH_CART(upward_cart_impl, h); }
+#define EXA_DISPATCH_CART_UP(fn, h, st, radii)                                    \
+  switch ((h).cfg.P) {                                                            \
+    case 4: fn<4>(h, st, radii); break;                                           \
+    case 6: fn<6>(h, st, radii); break;                                           \
+    case 8: fn<8>(h, st, radii); break;                                           \
+    default: throw Error(EXAFMM_HIP_EUNSUP, "Cartesian P must be one of 4, 6, 8"); \
+  }
+
+void run_upward_cart(Handle &h) {
+  EXA_DISPATCH_CART_UP(p2m_cart_impl, h, h.stream, 1);
+  EXA_DISPATCH_CART_UP(m2m_cart_impl, h, h.stream, 1);
+}
+void run_p2m_cart(Handle &h, hipStream_t st) { EXA_DISPATCH_CART_UP(p2m_cart_impl, h, st, 0); }
+void run_m2m_cart(Handle &h, hipStream_t st) { EXA_DISPATCH_CART_UP(m2m_cart_impl, h, st, 0); }
 void run_downward_cart(Handle &h) { EXA_DISPATCH_CART(downward_cart_impl, h); }
 void run_m2l_cart(Handle &h) {
   if (h.nm2l_tgt == 0) return;
@@ -854,9 +872,9 @@ void run_periodic_cart(Handle &h) {
 template <int P>
 static void upward_cart_cells_impl(Handle &h, const CellSetView &v) {
   hipLaunchKernelGGL(k_p2m_cart<P>, dim3(v.ncell), dim3(64), 0, h.stream, v.cells, v.body, v.cX, v.cRb, v.cNChild,
-                     v.cBody, v.cNBody, v.M, h.cfg.theta, h.cfg.useRmax);
+                     v.cBody, v.cNBody, v.M, h.cfg.theta, h.cfg.useRmax, 1);
   hipLaunchKernelGGL(k_m2m_cart<P>, dim3(v.ncell), dim3(512), 0, h.stream, v.cells, v.cX, v.cRb, v.cChild, v.cNChild,
-                     v.M, h.cfg.theta, h.cfg.useRmax);
+                     v.M, h.cfg.theta, h.cfg.useRmax, 1);
 }
 
 template <int P>

@@ -382,6 +382,9 @@ bool lattice_applies(const Handle &h);
 void run_m2m_level_mfma(Handle &h, const int *cells, int cnt, hipStream_t st);
 void run_l2l_level_mfma(Handle &h, const int *cells, int cnt);
 void run_upward_cart(Handle &h);
+// Its multipoles alone (the split upward pass), on stream st.
+void run_p2m_cart(Handle &h, hipStream_t st);
+void run_m2m_cart(Handle &h, hipStream_t st);
 void run_downward_cart(Handle &h);
 void run_m2l_cart(Handle &h);
 void run_periodic_cart(Handle &h);

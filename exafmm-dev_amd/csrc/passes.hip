@@ -492,7 +492,10 @@ void run_upward(Handle &h) {
 // is read (join_multipoles).  P2M is queued with the radii and runs beside
 // them; run_upward_mult queues the rest, called by the traversal once its own
 // first kernels are queued (its launches would otherwise hold the host while
-// the main stream idles).
+// the main stream idles).  In the Cartesian basis the multipole kernels make
+// the radii as well when the pass runs alone; here they leave them out: 48^3
+// periodic P = 6 1000 -> 930 us, 50k Plummer 925 -> 803 us, 5k P = 4 361 ->
+// 340 us.
 void run_upward_radii(Handle &h) {
   h.M.resize((size_t)h.ncells * h.nterm);
   h.L.resize((size_t)h.ncells * h.nterm);
@@ -500,6 +503,7 @@ void run_upward_radii(Handle &h) {
   EXA_HIP(hipEventRecord(h.ev[16], h.stream));
   EXA_HIP(hipStreamWaitEvent(h.stream3, h.ev[2], 0));
   EXA_HIP(hipEventRecord(h.ev[17], h.stream3));
+  if (h.cfg.basis == 1) return run_p2m_cart(h, h.stream3);
   EXA_DISPATCH_ST(p2m_impl, h, h.stream3);
 }
 
@@ -510,7 +514,11 @@ void run_upward_mult(Handle &h) {
   EXA_HIP(hipEventRecord(h.ev_tiles, h.stream2));
   h.lat_tiles_ready = true;
   EXA_HIP(hipMemsetAsync(h.L.p, 0, h.L.bytes(), h.stream3));  // (read with the multipoles)
-  EXA_DISPATCH_ST(m2m_impl, h, h.stream3);
+  if (h.cfg.basis == 1) {
+    run_m2m_cart(h, h.stream3);
+  } else {
+    EXA_DISPATCH_ST(m2m_impl, h, h.stream3);
+  }
   run_lattice_mscale(h, h.stream3);  // the lattice M2L's input
   EXA_HIP(hipEventRecord(h.ev_mult, h.stream3));
 }
