@@ -16,12 +16,9 @@
 //
 // The upward pass follows the reference's operation order without FMA
 // contraction (multipoles bit-identical to the reference).  M2L takes one
-// wave per target cell and, at P = 4 and 6, one lane per pair with everything
-// in registers; at P = 8 each lane builds one pair's derivative tensor in LDS
-// and the lanes run a host-built, load-balanced schedule of (a, b) terms over
-// the whole batch.
+// wave per target cell and one lane per pair with everything in registers.
 #include <algorithm>
-#include <vector>
+#include <utility>
 
 #include "harmonics.h"
 #include "internal.h"
@@ -360,177 +357,20 @@ __global__ void __launch_bounds__(64)
 }
 
 // ---------------------------------------------------------------------------
-// M2L over the CSR interaction list, one 64-lane workgroup per target cell.
-// Schedule (host): the terms (a, b) of every output a, b in index order, cut
-// into chunks of at most kCartChunk terms and packed onto the 64 lanes by
-// longest-first.  Descriptor: bits [0,10) b, [10,20) index of a+b, bit 20
-// end of chunk.  Padding items use b = NT (a zero column) and a+b = 0.
-constexpr int kCartChunk = 8;
-
-struct CartSchedule {
-  std::vector<uint32_t> desc;  // ipl x 64, item-major
-  std::vector<int> slot0;      // 64
-  std::vector<int> outslot;    // NT x maxc (-1 padded)
-  int ipl = 0, maxc = 0, nslots = 0;
-};
-
-static CartSchedule build_cart_schedule(int P) {
-  const int NT = P * (P + 1) * (P + 2) / 6;
-  struct Chunk {
-    int a;
-    std::vector<uint32_t> items;
-  };
-  std::vector<Chunk> chunks;
-  std::vector<int> nchunk(NT, 0);
-  for (int a = 0; a < NT; a++) {
-    int xa, ya, za;
-    cmi(a, xa, ya, za);
-    const int da = xa + ya + za;
-    Chunk cur{a, {}};
-    for (int b = 0; b < NT; b++) {
-      int xb, yb, zb;
-      cmi(b, xb, yb, zb);
-      if (!m2l_term(P, da, xb + yb + zb)) continue;
-      cur.items.push_back((uint32_t)b | ((uint32_t)cidx(xa + xb, ya + yb, za + zb) << 10));
-      if ((int)cur.items.size() == kCartChunk) {
-        chunks.push_back(cur);
-        nchunk[a]++;
-        cur.items.clear();
-      }
-    }
-    if (!cur.items.empty()) {
-      chunks.push_back(cur);
-      nchunk[a]++;
-    }
-  }
-  std::vector<int> order(chunks.size());
-  for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int x, int y) { return chunks[x].items.size() > chunks[y].items.size(); });
-  std::vector<std::vector<int>> lanes(64);
-  std::vector<int> load(64, 0);
-  for (int ch : order) {
-    int best = 0;
-    for (int l = 1; l < 64; l++)
-      if (load[l] < load[best]) best = l;
-    lanes[best].push_back(ch);
-    load[best] += (int)chunks[ch].items.size();
-  }
-  CartSchedule s;
-  s.ipl = *std::max_element(load.begin(), load.end());
-  s.maxc = *std::max_element(nchunk.begin(), nchunk.end());
-  s.desc.assign((size_t)s.ipl * 64, (uint32_t)NT);
-  s.slot0.assign(64, 0);
-  s.outslot.assign((size_t)NT * s.maxc, -1);
-  std::vector<int> fill(NT, 0);
-  // Slots are numbered lane-major; outslot lists each output's chunks in
-  // term order (chunk creation order).
-  std::vector<int> chunk_slot(chunks.size());
-  int slot = 0;
-  for (int l = 0; l < 64; l++) {
-    s.slot0[l] = slot;
-    int it = 0;
-    for (int ch : lanes[l]) {
-      const auto &items = chunks[ch].items;
-      for (size_t i = 0; i < items.size(); i++) {
-        uint32_t d = items[i];
-        if (i + 1 == items.size()) d |= 1u << 20;
-        s.desc[(size_t)it * 64 + l] = d;
-        it++;
-      }
-      chunk_slot[ch] = slot++;
-    }
-  }
-  s.nslots = slot;
-  for (size_t ch = 0; ch < chunks.size(); ch++) {
-    const int a = chunks[ch].a;
-    s.outslot[(size_t)a * s.maxc + fill[a]++] = chunk_slot[ch];
-  }
-  return s;
-}
-
-template <int P>
-struct CartM2LShape {
-  static constexpr int NT = Cart<P>::NT;
-  static constexpr int RS = NT + 1;               // LDS row stride (zero column at NT)
-  static constexpr int B = NT <= 64 ? 64 : 32;     // pairs per batch
-  static constexpr int NCHUNK = 3 * NT + 256;      // slot capacity (checked on the host)
-};
-
-template <int P, int IPL>
-__global__ void __launch_bounds__(64)
-    k_m2l_cart(const int *__restrict__ tgt_list, const int *__restrict__ off, const int *__restrict__ src,
-               const unsigned char *__restrict__ img, const double4 *__restrict__ cX, const cplx *__restrict__ M,
-               cplx *__restrict__ L, const uint32_t *__restrict__ sched, const int *__restrict__ slot0,
-               const int *__restrict__ outslot, int maxc, double cycle, int mass) {
-  using S = CartM2LShape<P>;
-  constexpr int NT = S::NT, RS = S::RS, B = S::B;
-  __shared__ double sC[B * RS];
-  __shared__ double sM[B * RS];
-  __shared__ double slots[S::NCHUNK];
-  __shared__ int ssrc[B];
-  const int c = tgt_list[blockIdx.x];
-  const int lane = threadIdx.x;
-  uint32_t desc[IPL];
-#pragma unroll
-  for (int it = 0; it < IPL; it++) desc[it] = sched[it * 64 + lane];
-  const int myslot0 = slot0[lane];
-  for (int t = lane; t < S::NCHUNK; t += 64) slots[t] = 0;
-  const double4 Xi = cX[c];
-  const double mi0 = M[(size_t)c * NT].re;
-  const int e0 = off[c], e1 = off[c + 1];
-  for (int base = e0; base < e1; base += B) {
-    const int cnt = min(B, e1 - base);
-    __syncthreads();  // the previous batch is done with the tables
-    if (lane < cnt) {
-      const int s = src[base + lane];
-      const int im = img[base + lane];
-      ssrc[lane] = s;
-      const double4 Xj = cX[s];
-      const double px = (im / 9 - 1) * cycle, py = ((im / 3) % 3 - 1) * cycle, pz = (im % 3 - 1) * cycle;
-      const double dx = Xi.x - Xj.x - px, dy = Xi.y - Xj.y - py, dz = Xi.z - Xj.z - pz;
-      double r2 = 0;
-      r2 += dx * dx;
-      r2 += dy * dy;
-      r2 += dz * dz;
-      const double invR2 = 1 / r2;
-      const double invR = mass ? mi0 * M[(size_t)s * NT].re * sqrt(invR2) : sqrt(invR2);
-      cart_coef<P>(sC + lane * RS, dx, dy, dz, invR2, invR);
-      sC[lane * RS + NT] = 0;
-    }
-    __syncthreads();
-    for (int p = 0; p < cnt; p++) {
-      const int s = ssrc[p];
-      for (int t = lane; t < NT; t += 64) sM[p * RS + t] = (t == 0 && mass) ? 1.0 : M[(size_t)s * NT + t].re;
-      if (lane == 0) sM[p * RS + NT] = 0;
-    }
-    __syncthreads();
-    double acc = 0;
-    int slot = myslot0;
-#pragma unroll
-    for (int it = 0; it < IPL; it++) {
-      const uint32_t d = desc[it];
-      const int b = d & 0x3FF, ab = (d >> 10) & 0x3FF;
-      for (int p = 0; p < cnt; p++) acc += sM[p * RS + b] * sC[p * RS + ab];
-      if (d & (1u << 20)) {
-        slots[slot] += acc;
-        slot++;
-        acc = 0;
-      }
-    }
-  }
-  __syncthreads();
-  for (int a = lane; a < NT; a += 64) {
-    double sum = 0;
-    for (int k = 0; k < maxc; k++) {
-      const int sl = outslot[a * maxc + k];
-      if (sl >= 0) sum += slots[sl];
-    }
-    cplx o = L[(size_t)c * NT + a];
-    o.re += sum;
-    L[(size_t)c * NT + a] = o;
-  }
-}
+// M2L over the CSR interaction list: one wave per target cell and one lane per
+// pair, the pair's derivative tensor and the target's sums in registers, every
+// index fixed at compile time; the lanes' sums are added in lane order through
+// LDS at the end.  FP64 issue bounds it: at P = 6 a pair is 462 multiply-adds
+// and about 400 operations of the recurrence, and 448 bytes of its source's
+// multipole; 2 x 56 doubles leave two waves per SIMD.  1.41 M pairs over 4680
+// targets at P = 6: 315 us; 2180 us with a batch of tensors in LDS and a term
+// list per lane (62 KB for one wave left two waves per CU).
+// At P = 8 the 2 x 120 doubles do not fit 512 registers, so two kernels each
+// make the tensor and sum a part of the outputs, those up to degree 4 (35
+// outputs, 1358 of the 1716 terms) and the others: a cube of 100k bodies
+// evaluates in 1045 us (1170 us with all outputs in one kernel, 163 registers
+// spilled; 1080 and 1058 us cut after degree 3 and 5; 5150 us with tensors in
+// LDS), 5k bodies in 468 us (478, 462, 471; 990).
 
 // Real parts of the multipoles, packed (what k_m2l_cart_reg reads).
 __global__ void k_cart_pack(const cplx *__restrict__ M, int64_t n, double *__restrict__ Mp) {
@@ -538,16 +378,59 @@ __global__ void k_cart_pack(const cplx *__restrict__ M, int64_t n, double *__res
   if (i < n) Mp[i] = M[i].re;
 }
 
-// P = 4 and 6: one wave per target cell and one lane per pair, the pair's
-// derivative tensor and the target's sums in registers (2 x 56 doubles at P =
-// 6, two waves per SIMD), every index fixed at compile time; the lanes' sums
-// are added in lane order through LDS at the end.  A pair is 462 multiply-adds
-// and about 400 operations of the recurrence at P = 6, and 448 bytes of its
-// source's multipole.  1.41 M pairs over 4680 targets: 315 us; 2180 us with a
-// batch of tensors in LDS and a term list per lane (62 KB for one wave left
-// two waves per CU), which stays for P = 8, whose 2 x 120 doubles do not fit.
-template <int P>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+// One Taylor coefficient (Kernels::derivative, :187-191) from the lower ones.
+template <int P, int T>
+__device__ __forceinline__ void cart_taylor(double (&C)[Cart<P>::NT], const double (&d)[3], double invR2) {
+  constexpr CartTab<P> tab{};
+  constexpr int x = tab.x[T], y = tab.y[T], z = tab.z[T], n = x + y + z;
+  double s1 = 0, s2 = 0;
+  if constexpr (x >= 1) s1 += d[0] * C[CartTab<P>::idx(x - 1, y, z)];
+  if constexpr (x >= 2) s2 += C[CartTab<P>::idx(x - 2, y, z)];
+  if constexpr (y >= 1) s1 += d[1] * C[CartTab<P>::idx(x, y - 1, z)];
+  if constexpr (y >= 2) s2 += C[CartTab<P>::idx(x, y - 2, z)];
+  if constexpr (z >= 1) s1 += d[2] * C[CartTab<P>::idx(x, y, z - 1)];
+  if constexpr (z >= 2) s2 += C[CartTab<P>::idx(x, y, z - 2)];
+  C[T] = ((1.0 - 2 * n) / n * s1 + (1.0 - n) / n * s2) * invR2;
+}
+
+
+// C[1..] from C[0], times k!.
+template <int P, int... T>
+__device__ __forceinline__ void cart_tensor(double (&C)[Cart<P>::NT], const double (&d)[3], double invR2,
+                                            std::integer_sequence<int, T...>) {
+  constexpr CartTab<P> tab{};
+  (cart_taylor<P, T + 1>(C, d, invR2), ...);
+  ((C[T + 1] *= (int)factorial(tab.x[T + 1]) * (int)factorial(tab.y[T + 1]) * (int)factorial(tab.z[T + 1])), ...);
+}
+
+// The terms of the multipole's coefficient B on the outputs [A0, A1).
+template <int P, int A0, int A1, int B>
+__device__ __forceinline__ void cart_terms(double (&l)[A1 - A0], const double (&C)[Cart<P>::NT], double m) {
+  constexpr CartTab<P> tab{};
+  constexpr int db = tab.x[B] + tab.y[B] + tab.z[B], da = P - db;  // outputs of a lower degree than da
+  constexpr int n = da * (da + 1) * (da + 2) / 6, end = n < A1 ? n : A1;
+#pragma unroll
+  for (int a = A0; a < end; a++)
+    if (m2l_term(P, tab.x[a] + tab.y[a] + tab.z[a], db))
+      l[a - A0] += m * C[CartTab<P>::idx(tab.x[a] + tab.x[B], tab.y[a] + tab.y[B], tab.z[a] + tab.z[B])];
+}
+
+template <int P, int A0, int A1, int... B2>
+__device__ __forceinline__ void cart_contract(double (&l)[A1 - A0], const double (&C)[Cart<P>::NT],
+                                              const double2 *__restrict__ mp, int mass,
+                                              std::integer_sequence<int, B2...>) {
+  (
+      [&] {
+        const double2 m2 = mp[B2];
+        cart_terms<P, A0, A1, 2 * B2>(l, C, mass && B2 == 0 ? 1.0 : m2.x);
+        cart_terms<P, A0, A1, 2 * B2 + 1>(l, C, m2.y);
+      }(),
+      ...);
+}
+
+// Outputs [A0, A1).
+template <int P, int A0, int A1>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P <= 6 ? 2 : 1)))
     k_m2l_cart_reg(const int *__restrict__ tgt_list, const int *__restrict__ off, const int *__restrict__ src,
                    const unsigned char *__restrict__ img, const double4 *__restrict__ cX,
                    const double *__restrict__ Mp, cplx *__restrict__ L, double cycle, int mass) {
@@ -558,9 +441,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
   const int c = tgt_list[blockIdx.x], lane = threadIdx.x;
   const double4 Xi = cX[c];
   const double mi0 = mass ? Mp[(size_t)c * NT] : 1.0;
-  double l[NT];
+  constexpr int NA = A1 - A0;
+  double l[NA];
 #pragma unroll
-  for (int a = 0; a < NT; a++) l[a] = 0;
+  for (int a = 0; a < NA; a++) l[a] = 0;
   const int e0 = off[c], e1 = off[c + 1];
   for (int e = e0 + lane; e < e1; e += 64) {
     const int s = src[e], im = img[e];
@@ -572,55 +456,25 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
     // Taylor coefficients (Kernels::derivative, :187-191), then times k!.
     double C[NT];
     C[0] = (mass ? mi0 * Mp[(size_t)s * NT] : 1.0) * sqrt(invR2);
-#pragma unroll
-    for (int t = 1; t < NT; t++) {
-      const int k[3] = {tab.x[t], tab.y[t], tab.z[t]}, n = k[0] + k[1] + k[2];
-      double s1 = 0, s2 = 0;
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        const int ux = q == 0, uy = q == 1, uz = q == 2;
-        if (k[q] >= 1) s1 += d[q] * C[CartTab<P>::idx(k[0] - ux, k[1] - uy, k[2] - uz)];
-        if (k[q] >= 2) s2 += C[CartTab<P>::idx(k[0] - 2 * ux, k[1] - 2 * uy, k[2] - 2 * uz)];
-      }
-      C[t] = ((1.0 - 2 * n) / n * s1 + (1.0 - n) / n * s2) * invR2;
-    }
-#pragma unroll
-    for (int t = 1; t < NT; t++) {
-      int f = 1;
-#pragma unroll
-      for (int q = 2; q < P; q++) f *= (tab.x[t] >= q ? q : 1) * (tab.y[t] >= q ? q : 1) * (tab.z[t] >= q ? q : 1);
-      C[t] *= f;
-    }
-#pragma unroll
-    for (int b2 = 0; b2 < NT / 2; b2++) {
-      const double2 m2 = mp[b2];
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const int b = 2 * b2 + u;
-        const double m = u == 0 ? (mass && b == 0 ? 1.0 : m2.x) : m2.y;
-#pragma unroll
-        for (int a = 0; a < NT; a++)
-          if (m2l_term(P, tab.x[a] + tab.y[a] + tab.z[a], tab.x[b] + tab.y[b] + tab.z[b]))
-            l[a] += m * C[CartTab<P>::idx(tab.x[a] + tab.x[b], tab.y[a] + tab.y[b], tab.z[a] + tab.z[b])];
-      }
-    }
+    cart_tensor<P>(C, d, invR2, std::make_integer_sequence<int, NT - 1>{});
+    cart_contract<P, A0, A1>(l, C, mp, mass, std::make_integer_sequence<int, NT / 2>{});
   }
 #pragma unroll
-  for (int a0 = 0; a0 < NT; a0 += kRow) {
+  for (int a0 = 0; a0 < NA; a0 += kRow) {
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kRow; r++)
-      if (a0 + r < NT) sh[r][lane] = l[a0 + r];
+      if (a0 + r < NA) sh[r][lane] = l[a0 + r];
     __syncthreads();
     const int r = lane >> 1, half = 32 * (lane & 1);  // two lanes per output
     double v = 0;
     if (r < kRow)
       for (int i = 0; i < 32; i++) v += sh[r][half + i];
     v += __shfl_xor(v, 1);
-    if (r < kRow && a0 + r < NT && half == 0) {
-      cplx o = L[(size_t)c * NT + a0 + r];
+    if (r < kRow && a0 + r < NA && half == 0) {
+      cplx o = L[(size_t)c * NT + A0 + a0 + r];
       o.re += v;
-      L[(size_t)c * NT + a0 + r] = o;
+      L[(size_t)c * NT + A0 + a0 + r] = o;
     }
   }
 }
@@ -631,38 +485,12 @@ static void m2l_cart_reg(Handle &h, const M2LList &lst, const double4 *cX, const
   if (lst.ntgt == 0) return;
   h.cart_M.resize(nc * NT);
   hipLaunchKernelGGL(k_cart_pack, dim3(div_up(nc * NT, 256)), dim3(256), 0, h.stream, M, nc * NT, h.cart_M.p);
-  hipLaunchKernelGGL(k_m2l_cart_reg<P>, dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src, lst.img, cX,
-                     h.cart_M.p, L, h.cfg.cycle, h.cfg.mass);
-  EXA_HIP(hipGetLastError());
-}
-
-// Items per lane at P = 8, rounded up to the compiled register budget.
-constexpr int kCartIPL8 = 40;
-
-static void m2l_cart_sched8(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, cplx *L) {
-  using S = CartM2LShape<8>;
-  const int key = 1008;
-  if (h.m2l_sched_P != key) {
-    const CartSchedule sc = build_cart_schedule(8);
-    if (sc.ipl > kCartIPL8 || sc.nslots > S::NCHUNK)
-      throw Error(EXAFMM_HIP_EUNSUP, "Cartesian M2L schedule exceeds its compiled budget");
-    std::vector<uint32_t> blob(sc.desc);
-    blob.resize((size_t)kCartIPL8 * 64, (uint32_t)S::NT);  // pad to the compiled item count
-    for (int v : sc.slot0) blob.push_back((uint32_t)v);
-    for (int v : sc.outslot) blob.push_back((uint32_t)v);
-    h.m2l_sched.resize(blob.size());
-    EXA_HIP(hipMemcpyAsync(h.m2l_sched.p, blob.data(), blob.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
-                           h.stream));
-    EXA_HIP(hipStreamSynchronize(h.stream));
-    h.m2l_sched_P = key;
-    h.cart_maxc = sc.maxc;
-  }
-  const uint32_t *desc = h.m2l_sched.p;
-  const int *slot0 = reinterpret_cast<const int *>(desc + 64 * kCartIPL8);
-  const int *outslot = slot0 + 64;
-  if (lst.ntgt > 0)
-    hipLaunchKernelGGL((k_m2l_cart<8, kCartIPL8>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src,
-                       lst.img, cX, M, L, desc, slot0, outslot, h.cart_maxc, h.cfg.cycle, h.cfg.mass);
+  constexpr int A1 = P <= 6 ? NT : 35;
+  hipLaunchKernelGGL((k_m2l_cart_reg<P, 0, A1>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src,
+                     lst.img, cX, h.cart_M.p, L, h.cfg.cycle, h.cfg.mass);
+  if constexpr (A1 < NT)
+    hipLaunchKernelGGL((k_m2l_cart_reg<P, A1, NT>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src,
+                       lst.img, cX, h.cart_M.p, L, h.cfg.cycle, h.cfg.mass);
   EXA_HIP(hipGetLastError());
 }
 
@@ -671,7 +499,7 @@ static void m2l_cart(Handle &h, const M2LList &lst, const double4 *cX, const cpl
   switch (h.cfg.P) {
     case 4: m2l_cart_reg<4>(h, lst, cX, M, nc, L); break;
     case 6: m2l_cart_reg<6>(h, lst, cX, M, nc, L); break;
-    case 8: m2l_cart_sched8(h, lst, cX, M, L); break;
+    case 8: m2l_cart_reg<8>(h, lst, cX, M, nc, L); break;
     default: throw Error(EXAFMM_HIP_EUNSUP, "Cartesian P must be one of 4, 6, 8");
   }
 }

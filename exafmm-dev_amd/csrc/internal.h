@@ -241,11 +241,10 @@ struct Handle {
   int64_t lat_stats_steps = 0;
   bool lat_timed = false, pair_timed = false;  // ev[12..13]: MFMA kernel, ev[14..15]: per-pair kernel
 
-  // M2L lane schedule (a pure function of P, the basis and the table type).
+  // M2L lane schedule (a pure function of P and the table type).
   DBuf<uint32_t> m2l_sched;
   int m2l_sched_P = -1;
   DBuf<double> cart_M;  // real parts of the multipoles, packed (Cartesian M2L)
-  int cart_maxc = 0;  // Cartesian schedule: chunks per output (outslot row length)
 
   // Scratch.
   DBuf<unsigned char> tmp;         // hipCUB temporary storage
