@@ -107,7 +107,7 @@ static void do_traverse(Handle &h) {
   m2l_begin(h);
   if (h.mult_pending) EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev_mult, 0));
   EXA_HIP(hipEventRecord(h.ev[9], h.stream2));
-  run_p2p(h, h.stream2);
+  run_p2p(h, h.stream2, true);
   EXA_HIP(hipEventRecord(h.ev[10], h.stream2));
   run_m2l(h);
   join_multipoles(h);  // if no M2L path did

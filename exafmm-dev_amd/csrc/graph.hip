@@ -55,7 +55,7 @@ static void enqueue_numeric(Handle &h) {
   EXA_HIP(hipEventRecord(h.ev_fork, h.stream));
   auto p2p = [&] {
     EXA_HIP(hipStreamWaitEvent(h.stream2, h.ev_fork, 0));
-    run_p2p(h, h.stream2);
+    run_p2p(h, h.stream2, false);
     EXA_HIP(hipEventRecord(h.ev_gp2p, h.stream2));
   };
   // The order of launches: P2P first, beside the multipoles, where its resident

@@ -354,7 +354,8 @@ void ensure_m2l_grouped(Handle &h);
 // The nirr irregular pairs of the M2L list grouped by target (irr_off, irr_src,
 // irr_img, the ntl targets irr_tgt) on stream st; waits for it.
 void group_irregular(Handle &h, hipStream_t st, int64_t nirr, int &ntl);
-void run_p2p(Handle &h, hipStream_t st);
+// setup: the M2L set-up runs beside it.
+void run_p2p(Handle &h, hipStream_t st, bool setup);
 int p2p_waves_per_leaf(const Handle &h);
 void run_m2l(Handle &h);
 // The lattice contraction and reduction / the whole M2L of the last

@@ -1125,7 +1125,24 @@ int p2p_waves_per_leaf(const Handle &h) {
   return h.p2p_kmax == 1 && h.cfg.precision == 0 ? p2p_team(h, tree_leaves(h)) : 1;
 }
 
-void run_p2p(Handle &h, hipStream_t st) {
+// Where the resident grid of single waves takes between one and two rounds and
+// the M2L beside it, with its set-up, is the longer path, half as many waves as
+// leaves: two full rounds instead of one and a nearly empty one, and room for
+// the M2L's kernels on every CU meanwhile.  (For new charges, without the set-up,
+// the full grid is as good or better: 100 000 bodies 520 us and 540.)  By flops (20 per body pair, the pairs
+// estimated from the mean leaf): 4096 leaves, mixed, P2P 0.1 to 0.9 of the M2L:
+// 35 000 bodies at P = 10 676 -> 609 us, 100 000 735 -> 650 and at P = 12 827 ->
+// 777, 130 000 787 -> 766, 100 000 on a sphere 1057 -> 949; but 1.3 of it (160 000
+// in a cube) 878 -> 862, 2.1 (200 000) 1015 -> 1090 and 3.2 (100 000 at P = 6)
+// 585 -> 610.
+static bool p2p_two_rounds(const Handle &h, int64_t leaves, int64_t waves) {
+  if (h.cfg.basis != 0 || h.p2p_kmax != 1 || leaves <= waves || leaves > 2 * waves) return false;
+  const double P = h.cfg.P, per = (double)h.n / leaves;
+  const double m2l = (double)h.nm2l * 8 * P * (P + 1) * (P + 1) * (P + 2) / 12;
+  return 20.0 * h.np2p * per * per < 1.25 * m2l;
+}
+
+void run_p2p(Handle &h, hipStream_t st, bool setup) {
   // Every body belongs to a leaf that is in its own list, and every target is
   // written once: the results need no clearing.
   if (h.np2p_tgt == 0) return;
@@ -1144,6 +1161,8 @@ void run_p2p(Handle &h, hipStream_t st) {
   // CU at least): the contraction beside them is on the longer path (994
   // leaves: 840 us per evaluation, 905 with the whole resident grid).
   if (W > 1) waves = std::min(waves, std::max<int64_t>(leaves, 2 * h.ncu));
+  else if (setup && p2p_two_rounds(h, leaves, waves))
+    waves = (leaves + 1) / 2;
   int grid = std::max(1, (int)(waves / W));
   if (h.np2p_tgt < 0 && h.p2p_wpc > 0) {
     ntl_dev = h.p2p_cnt_dev;
