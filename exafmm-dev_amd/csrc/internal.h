@@ -125,6 +125,7 @@ struct Handle {
   DBuf<int> ut_tab, ut_cnt, ut_start, ut_rank, ut_tot;
   std::vector<int> ut_tab_host;
   bool ut_zero = false;
+  bool ut_sort = false;  // the last tree had a leaf that calls for a sort of the bodies
   DBuf<double4> in4;     // caller order (x, y, z, q)
   DBuf<double4> body4;   // tree order
   DBuf<int> bidx;        // tree order -> caller index (Body::IBODY)

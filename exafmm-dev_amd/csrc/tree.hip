@@ -133,20 +133,23 @@ void upload_bounds(Handle &h) {
 // system with L >= t, and a system's cells come in the order of its
 // single-system build.
 //
-// A tree of depth L has 8^L possible leaves, at most 8 per ncrit bodies, so
-// leaves are counted and found by index: bodies per leaf (atomic counts), a
-// prefix sum for the leaves' first bodies, bodies scattered into their leaves
-// (in any order) and each leaf's bodies sorted by input index, which is the
-// order a stable sort by key gives.  A cell of any level is a run of leaves, so
-// the same prefix sum says whether it holds bodies, and a second one over the
-// possible cells of all levels numbers those that do.  Bound by launches up to
-// about 100k bodies, then by the counting atomics (50 us at 1M).  A radix sort
-// of the keys with head flags, scans and compactions over all bodies for every
-// level took 24 launches and more; this takes 9 to 12, and whole evaluations of
-// 2000, 100k and 1M bodies and of 32 systems of 1000 to 8000 went from 440 to
-// 380, 875 to 793, 4380 to 4280 and 1720 to 1540 us.
-// A leaf with very many bodies (systems clustered in a corner of their cube) is
-// sorted by one wave, 10 ms at 500k; its P2P takes seconds.
+// A tree of depth L has 8^L possible leaves, at most 8 per ncrit bodies, so a
+// cell of any level is a run of leaves: where the leaves' first bodies are known,
+// they say whether a cell holds bodies, and a prefix sum over the possible cells
+// of all levels numbers those that do (no key sort, scan and compaction over the
+// bodies for every level, which took 24 launches and more).
+// The bodies come into leaf order, those of a leaf in input order, as a stable
+// sort by key gives, in one of two ways:
+//   up to kCountMost bodies by counting, in 9 to 12 launches: bodies per leaf
+//   (atomic counts), a prefix sum for the leaves' first bodies, bodies scattered
+//   into their leaves in any order, and each body's rank among its leaf's.
+//   2000 bodies 30 us (75 by sorts per level), 100k 47 (118), 262144 68 (147).
+//   With a leaf beyond kLeafRank bodies the sort follows, and it comes at once in
+//   the handle's next build.
+//   beyond, by a stable sort of (leaf, body), the starts found by bisection:
+//   1 M bodies 147 us, 4 M 330, however clustered (by counting 156 and 468, and
+//   4 M clustered bodies 900 us and more: the atomic counts of few leaves follow
+//   each other).
 constexpr int kMaxUniformLevels = 10;  // the reference's int keys hold 3 x 10 bits
 
 struct ForestSys {
@@ -259,14 +262,10 @@ __device__ inline int last_le(const int *__restrict__ v, int n, int x) {
 }
 
 // getKey (build_tree_omp.h:36-57): float cell size promoted to double for the
-// division, truncation to int, bit interleave in int.  leaf[b] = the body's
-// leaf among all systems' possible ones, slot[b] = its place there.
-__global__ void __launch_bounds__(256)
-    k_leaf_count(const double4 *__restrict__ in, int n, const double *__restrict__ box, ForestSys *__restrict__ fs,
-                 int S, const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ slot,
-                 int *__restrict__ cnt) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= n) return;
+// division, truncation to int, bit interleave in int.  The body's leaf among
+// all systems' possible ones.
+__device__ inline int body_leaf(const double4 *__restrict__ in, int b, const double *__restrict__ box,
+                                ForestSys *__restrict__ fs, int S, const int *__restrict__ begin) {
   ForestSys f = fs[S > 1 ? last_le(begin, S, b) : 0];
   if (box) {  // one system: its box, for the kernels behind this one too
     set_box(box, box + 3, f);
@@ -291,14 +290,90 @@ __global__ void __launch_bounds__(256)
     iy >>= 1;
     iz >>= 1;
   }
-  leaf[b] = f.leaf0 + id;
-  slot[b] = atomicAdd(&cnt[f.leaf0 + id], 1);
+  return f.leaf0 + id;
+}
+
+// leaf[b] and slot[b], the body's place in it.  A workgroup counts its bodies
+// per leaf in an LDS table first (open addressing, half full at most) and adds
+// one count per leaf: additions to one line of counters follow each other, and
+// 65536 bodies in one leaf took 745 us with an addition each, 10 with one per
+// workgroup.
+constexpr int kCountTable = 512;
+
+__global__ void __launch_bounds__(256)
+    k_leaf_count(const double4 *__restrict__ in, int n, const double *__restrict__ box, ForestSys *__restrict__ fs,
+                 int S, const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ slot,
+                 int *__restrict__ cnt) {
+  __shared__ int key[kCountTable], num[kCountTable];
+  const int tid = threadIdx.x, b = blockIdx.x * 256 + tid;
+  for (int i = tid; i < kCountTable; i += 256) {
+    key[i] = -1;
+    num[i] = 0;
+  }
+  __syncthreads();
+  int at = 0, before = 0;
+  if (b < n) {
+    const int id = body_leaf(in, b, box, fs, S, begin);
+    leaf[b] = id;
+    at = (int)(((unsigned)id * 2654435761u >> 16) % kCountTable);
+    while (true) {
+      const int k = atomicCAS(&key[at], -1, id);
+      if (k == -1 || k == id) break;
+      at = (at + 1) % kCountTable;
+    }
+    before = atomicAdd(&num[at], 1);
+  }
+  __syncthreads();
+  for (int i = tid; i < kCountTable; i += 256)
+    if (num[i] > 0) num[i] = atomicAdd(&cnt[key[i]], num[i]);
+  __syncthreads();
+  if (b < n) slot[b] = num[at] + before;
+}
+
+// leaf[b] and the bodies' indices, for the sort by leaf.
+__global__ void __launch_bounds__(256)
+    k_leaf_keys(const double4 *__restrict__ in, int n, const double *__restrict__ box, ForestSys *__restrict__ fs,
+                int S, const int *__restrict__ begin, int *__restrict__ leaf, int *__restrict__ ord) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= n) return;
+  leaf[b] = body_leaf(in, b, box, fs, S, begin);
+  ord[b] = b;
+}
+
+// First of the n sorted keys that is not below v, in [lo, hi].
+__device__ inline int first_not_below(const int *__restrict__ key, int lo, int hi, int v) {
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (key[mid] < v)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+// start[l] = first body of leaf l (l = nleaf: n) among the sorted keys, PER leaves
+// a thread; the two ends of a workgroup's leaves bound the others' search.
+template <int PER>
+__global__ void __launch_bounds__(256)
+    k_leaf_starts(const int *__restrict__ key, int n, int nleaf, int *__restrict__ start) {
+  __shared__ int ends[2];
+  const int64_t l0 = (int64_t)blockIdx.x * 256 * PER;
+  if (threadIdx.x < 2)
+    ends[threadIdx.x] = first_not_below(key, 0, n, (int)min<int64_t>(nleaf, l0 + 256 * PER * threadIdx.x));
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const int64_t l = l0 + 256 * j + threadIdx.x;
+    if (l <= nleaf) start[l] = first_not_below(key, ends[0], ends[1], (int)l);
+  }
 }
 
 // Level, system and index of possible cell e.
 __device__ inline void cell_of(const TreeShape &sh, int e, int &t, int &s, int &k) {
   t = 0;
-  while (t + 1 < sh.nlev && e >= sh.lev0[t + 1]) t++;
+#pragma unroll
+  for (int l = 1; l <= kMaxUniformLevels; l++) t += e >= sh.lev0[l];  // (ncell from lev0[nlev] on)
   const int *b = sh.base + t * (sh.S + 1);
   s = sh.S > 1 ? last_le(b, sh.S, e) : 0;
   k = e - b[s];
@@ -311,15 +386,6 @@ __device__ inline void cell_bodies(const ForestSys &f, const int *__restrict__ s
   b1 = start[f.leaf0 + ((k + 1) << sh)];
 }
 
-__device__ inline int cell_used(const TreeShape &sh, const ForestSys *__restrict__ fs, const int *__restrict__ start,
-                                int e) {
-  if (e >= sh.ncell) return 0;
-  int t, s, k, b0, b1;
-  cell_of(sh, e, t, s, k);
-  cell_bodies(fs[s], start, t, k, b0, b1);
-  return b1 > b0;
-}
-
 // Prefix sums in chunks of kScanChunk: totals per chunk, then each chunk's
 // offsets from the totals before it.  USED: of the cells' flags, else of the
 // counts.
@@ -327,8 +393,24 @@ constexpr int kScanChunk = 4096;
 
 template <bool USED>
 __device__ inline int4 scan_load(const TreeShape &sh, const ForestSys *__restrict__ fs, const int *src, int i, int n) {
-  int v[4];
-  for (int k = 0; k < 4; k++) v[k] = i + k >= n ? 0 : USED ? cell_used(sh, fs, src, i + k) : src[i + k];
+  int v[4] = {0, 0, 0, 0};
+  if (USED) {  // a cell's end is the next one's first body, within its level and system
+    int t, s, k, end = 0, step = 0, at = 0, b = 0;
+    for (int j = 0; j < 4 && i + j < n; j++, at += step) {
+      if (i + j >= end) {
+        cell_of(sh, i + j, t, s, k);
+        end = sh.base[t * (sh.S + 1) + s + 1];
+        step = 1 << 3 * (fs[s].L - t);
+        at = fs[s].leaf0 + k * step;
+        b = src[at];
+      }
+      const int e = src[at + step];
+      v[j] = e > b;
+      b = e;
+    }
+  } else {
+    for (int k = 0; k < 4; k++) v[k] = i + k >= n ? 0 : src[i + k];
+  }
   return make_int4(v[0], v[1], v[2], v[3]);
 }
 
@@ -405,30 +487,67 @@ __global__ void __launch_bounds__(256)
   if (b < n) ord[start[leaf[b]] + slot[b]] = b;
 }
 
-// Every leaf's bodies in input order.
-__global__ void __launch_bounds__(64)
-    k_leaf_order(const int *__restrict__ start, int bits, int *__restrict__ ord, int *__restrict__ aux,
+// Every leaf's bodies in input order, a thread per place: its body's rank in the
+// leaf is the number of the leaf's bodies with a smaller index.  Work follows
+// the bodies, whatever the number of possible leaves (with a workgroup for each,
+// 262144 bodies at ncrit = 1, 2.1 M possible leaves, took 565 us a build, now
+// 121; 2^26 and more were not launched at all).  Leaves beyond kLeafRank bodies,
+// where the quadratic count costs more than a sort of all bodies, are left to it.
+constexpr int kLeafRank = 1024, kLeafFew = 8;
+
+__global__ void __launch_bounds__(256)
+    k_leaf_order(const int *__restrict__ leaf, const int *__restrict__ start, int n, const int *__restrict__ ord,
                  const double4 *__restrict__ in, double4 *__restrict__ body, int *__restrict__ bidx) {
-  __shared__ RangeSortLds sh;
-  const int b = start[blockIdx.x], n = start[blockIdx.x + 1] - b;
-  if (n <= 0) return;
-  sort_range(ord + b, aux + b, n, bits, sh, [&](int rank, int e) {
-    body[b + rank] = in[e];
-    bidx[b + rank] = e;
-  });
+  const int p = min(blockIdx.x * 256 + (int)threadIdx.x, n - 1);  // (the last place may be done more than once)
+  const int e = ord[p], l = leaf[e], s = start[l], t = start[l + 1];
+  bool todo = t - s <= kLeafRank;
+  int rank = 0;
+  if (todo && t - s <= kLeafFew) {  // by lane
+    for (int k = s; k < t; k++) rank += ord[k] < e;
+    todo = false;
+  }
+  // The wave's larger leaves one by one, their indices by scalar loads.
+  while (__any(todo)) {
+    const int who = __ffsll(__ballot(todo)) - 1;
+    const int s0 = __builtin_amdgcn_readlane(s, who), t0 = __builtin_amdgcn_readlane(t, who);
+    int r = 0, k = s0;
+    for (; k + 16 <= t0; k += 16)
+#pragma unroll
+      for (int u = 0; u < 16; u++) r += ord[k + u] < e;
+    for (; k < t0; k++) r += ord[k] < e;
+    if (todo && s == s0) {
+      rank = r;
+      todo = false;
+    }
+  }
+  if (t - s > kLeafRank) return;
+  body[s + rank] = in[e];
+  bidx[s + rank] = e;
+}
+
+// The bodies in the order ord (a stable sort by leaf).
+__global__ void __launch_bounds__(256)
+    k_body_gather(const int *__restrict__ ord, int n, const double4 *__restrict__ in, double4 *__restrict__ body,
+                  int *__restrict__ bidx) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= n) return;
+  const int e = ord[p];
+  body[p] = in[e];
+  bidx[p] = e;
 }
 
 // bodies2leafs / leafs2cells (build_tree_omp.h:130-198) fused with the index
 // arithmetic of reverseOrder: the r-th cell of a level in ascending order
 // lands at the level's offset + count - 1 - r.  rank: prefix sum of the cells'
 // flags, so rank[lev0[t]] is the offset of level t.  Runs before the host
-// knows the number of cells (kCellsUnread).
+// knows the number of cells (kCellsUnread).  *host_big: a leaf has more than
+// kLeafRank bodies.
 __global__ void k_uniform_cells(TreeShape sh, const ForestSys *__restrict__ fs, const int *__restrict__ start,
                                 const int *__restrict__ rank, const double4 *__restrict__ body,
                                 double4 *__restrict__ cX, double *__restrict__ cRb, int *__restrict__ cParent,
                                 int *__restrict__ cChild, int *__restrict__ cNChild, int *__restrict__ cBody,
                                 int *__restrict__ cNBody, uint64_t *__restrict__ cKey, int *__restrict__ cLevel,
-                                int *__restrict__ lvl_cells, int *__restrict__ host_off) {
+                                int *__restrict__ lvl_cells, int *__restrict__ host_off, int *__restrict__ host_big) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e <= sh.nlev) host_off[e] = rank[sh.lev0[e]];
   if (e >= sh.ncell || rank[e + 1] == rank[e]) return;
@@ -458,6 +577,7 @@ __global__ void k_uniform_cells(TreeShape sh, const ForestSys *__restrict__ fs, 
   cLevel[c] = t;
   lvl_cells[c] = c;  // level order: the layout is already level-contiguous
   if (t == f.L) {
+    if (b1 - b0 > kLeafRank) *host_big = 1;
     cNChild[c] = 0;
     cChild[c] = nc;  // reverseOrder maps ICHILD = 0 of a leaf to numCells
   } else {
@@ -482,6 +602,10 @@ static int uniform_depth(int n, int ncrit) {
     throw Error(EXAFMM_HIP_EUNSUP, "uniform tree deeper than 10 levels overflows the reference's int keys");
   return L;
 }
+
+// Bodies up to which the leaves are counted (see above); leaves from which a
+// thread finds the starts of several.
+constexpr int kCountMost = 1 << 18, kStartsMany = 1 << 21;
 
 // The trees of the systems [off[s], off[s + 1]): with given bounds (one
 // system), or each with its own.
@@ -560,25 +684,58 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
   h.ut_rank.resize((size_t)sh.ncell + 1);
   const int nchl = div_up((int64_t)sh.nleaf + 1, kScanChunk), nchc = div_up((int64_t)sh.ncell + 1, kScanChunk);
   h.ut_tot.reserve(std::max(nchl, nchc));
-  if (!h.ut_zero || (size_t)sh.nleaf >= h.ut_cnt.cap) {
-    h.ut_cnt.reserve((size_t)sh.nleaf + 1);
-    zero_device(h.ut_cnt.p, h.ut_cnt.cap / 2 * 8, h.stream);
-  }
-  h.ut_zero = false;
   int *leaf = h.ic.p, *ord = h.ia.p, *aux = h.ib.p, *start = h.ut_start.p, *rank = h.ut_rank.p;
-  hipLaunchKernelGGL(k_leaf_count, dim3(div_up(n, 256)), dim3(256), 0, h.stream, h.in4.p, n,
-                     own_bounds ? nullptr : h.box.p, fsd, S, h.ut_tab.p + begin0, leaf, aux, h.ut_cnt.p);
-  if (sh.ncell <= kScanSmall) {
+  const double *box = own_bounds ? nullptr : h.box.p;
+  const int *begin = h.ut_tab.p + begin0;
+  const int nb = div_up(n, 256);
+  // Bodies by a stable sort, and the leaves' starts from the sorted keys.
+  auto sort_bodies = [&] {
+    int bits = 1;
+    while (((int64_t)1 << bits) < sh.nleaf) bits++;
+    h.id.reserve(n + 1);
+    hipLaunchKernelGGL(k_leaf_keys, dim3(nb), dim3(256), 0, h.stream, h.in4.p, n, box, fsd, S, begin, leaf, ord);
+    bool alt = false;
+    sort_pairs_int_int(leaf, h.id.p, ord, aux, n, bits, alt, h.stream, h.tmp);
+    auto starts = [&](auto kernel, int per) {
+      hipLaunchKernelGGL(kernel, dim3(div_up((int64_t)sh.nleaf + 1, 256 * per)), dim3(256), 0, h.stream,
+                         alt ? h.id.p : leaf, n, sh.nleaf, start);
+    };
+    // (16.7 M leaves: 250 us with one leaf a thread, 132 with four; 262144: 13 and 25.)
+    sh.nleaf >= kStartsMany ? starts(k_leaf_starts<4>, 4) : starts(k_leaf_starts<1>, 1);
+    hipLaunchKernelGGL(k_body_gather, dim3(nb), dim3(256), 0, h.stream, alt ? aux : ord, n, h.in4.p, h.body4.p,
+                       h.bidx.p);
+  };
+  const bool sort = n > kCountMost || h.ut_sort;
+  if (sort) {
+    sort_bodies();
+  } else {
+    if (!h.ut_zero || (size_t)sh.nleaf >= h.ut_cnt.cap) {
+      h.ut_cnt.reserve((size_t)sh.nleaf + 1);
+      zero_device(h.ut_cnt.p, h.ut_cnt.cap / 2 * 8, h.stream);
+    }
+    h.ut_zero = false;
+    hipLaunchKernelGGL(k_leaf_count, dim3(nb), dim3(256), 0, h.stream, h.in4.p, n, box, fsd, S, begin, leaf, aux,
+                       h.ut_cnt.p);
+  }
+  if (!sort && sh.ncell <= kScanSmall) {
     hipLaunchKernelGGL(k_tree_scan_small, dim3(1), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, start, rank);
   } else {
-    hipLaunchKernelGGL(k_tree_totals<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
-                       h.ut_tot.p);
-    hipLaunchKernelGGL(k_tree_offsets<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
-                       h.ut_tot.p, start);
+    if (!sort) {
+      hipLaunchKernelGGL(k_tree_totals<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
+                         h.ut_tot.p);
+      hipLaunchKernelGGL(k_tree_offsets<false>, dim3(nchl), dim3(1024), 0, h.stream, sh, fsd, h.ut_cnt.p, sh.nleaf,
+                         h.ut_tot.p, start);
+    }
     hipLaunchKernelGGL(k_tree_totals<true>, dim3(nchc), dim3(1024), 0, h.stream, sh, fsd, start, sh.ncell,
                        h.ut_tot.p);
     hipLaunchKernelGGL(k_tree_offsets<true>, dim3(nchc), dim3(1024), 0, h.stream, sh, fsd, start, sh.ncell,
                        h.ut_tot.p, rank);
+  }
+  if (!sort) {
+    hipLaunchKernelGGL(k_leaf_scatter, dim3(nb), dim3(256), 0, h.stream, leaf, aux, n, start, ord);
+    hipLaunchKernelGGL(k_leaf_order, dim3(nb), dim3(256), 0, h.stream, leaf, start, n, ord, h.in4.p, h.body4.p,
+                       h.bidx.p);
+    h.ut_zero = true;
   }
   int *host_off = h.hpin + 128;  // (the adaptive builder's words)
   int ncap = sh.ncell;           // the cell arrays hold every possible cell of trees up to kCellsUnread of them
@@ -592,17 +749,21 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
   h.cX.reserve(ncap);
   h.cRb.reserve(ncap);
   h.cKey.reserve(ncap);
-  hipLaunchKernelGGL(k_leaf_scatter, dim3(div_up(n, 256)), dim3(256), 0, h.stream, leaf, aux, n, start, ord);
-  int bits = 1;
-  while (((int64_t)1 << bits) < n) bits++;
-  hipLaunchKernelGGL(k_leaf_order, dim3(sh.nleaf), dim3(64), 0, h.stream, start, bits, ord, aux, h.in4.p, h.body4.p,
-                     h.bidx.p);
-  hipLaunchKernelGGL(k_uniform_cells, dim3(div_up(std::max(sh.ncell, sh.nlev + 1), T)), dim3(T), 0, h.stream, sh, fsd,
-                     start, rank, h.body4.p, h.cX.p, h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p, h.cBody.p,
-                     h.cNBody.p, h.cKey.p, h.cLevel.p, h.lvl_cells.p, host_off);
-  EXA_HIP(hipGetLastError());
-  h.ut_zero = true;
-  EXA_HIP(hipStreamSynchronize(h.stream));
+  volatile int *host_big = host_off + sh.nlev + 1;
+  auto cells = [&] {
+    *host_big = 0;
+    hipLaunchKernelGGL(k_uniform_cells, dim3(div_up(std::max(sh.ncell, sh.nlev + 1), T)), dim3(T), 0, h.stream, sh,
+                       fsd, start, rank, h.body4.p, h.cX.p, h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p, h.cBody.p,
+                       h.cNBody.p, h.cKey.p, h.cLevel.p, h.lvl_cells.p, host_off, const_cast<int *>(host_big));
+    EXA_HIP(hipGetLastError());
+    EXA_HIP(hipStreamSynchronize(h.stream));
+  };
+  cells();
+  h.ut_sort = *host_big != 0;
+  if (h.ut_sort && !sort) {  // the large leaves' bodies, and the cells again (a cell's centre comes from its first)
+    sort_bodies();
+    cells();
+  }
   const int nc = host_off[sh.nlev];
   h.ncells = nc;
   h.nlevels = sh.nlev;
