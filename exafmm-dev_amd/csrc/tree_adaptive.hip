@@ -388,19 +388,49 @@ __global__ void k_validate(TreeState *__restrict__ st, int room, int n, const in
   if (!ok) atomicAdd(&st->bad, 1);
 }
 
-// Each leaf's bodies in the order of their indices.
+// Each leaf's bodies in the order of their indices, one wave a leaf, where no
+// leaf is larger than that takes well (kRangeRank).
 __global__ void __launch_bounds__(64)
-    k_leaf_bodies(Nodes nd, const TreeState *__restrict__ st, int room, int bits, int *__restrict__ idx,
+    k_leaf_bodies(int g0, Nodes nd, const TreeState *__restrict__ st, int room, int bits, int *__restrict__ idx,
                   int *__restrict__ aux, const double4 *__restrict__ in, double4 *__restrict__ body,
                   int *__restrict__ bidx) {
   __shared__ RangeSortLds sh;
-  const int g = blockIdx.x;
+  const int g = g0 + blockIdx.x;
   if (g >= node_count(st, room) || nd.nchild[g] != 0) return;
   const int b = nd.start[g];
   sort_range(idx + b, aux + b, nd.count[g], bits, sh, [&](int rank, int e) {
     body[b + rank] = in[e];
     bidx[b + rank] = e;
   });
+}
+
+// Larger leaves: key[e] = the first body of body e's leaf, for a stable sort of
+// (key, e) in input order.  (100000 bodies, a leaf for all or ncrit = 20000: 3650
+// and 570 us a build by one wave a leaf, 71 and 170 so.)
+__global__ void __launch_bounds__(256)
+    k_leaf_keys(Nodes nd, const TreeState *__restrict__ st, int room, const int *__restrict__ idx,
+                int *__restrict__ key, int *__restrict__ val) {
+  const int total = node_count(st, room);
+  for (int g = blockIdx.x; g < total; g += gridDim.x) {
+    if (nd.nchild[g] != 0) continue;
+    const int b = nd.start[g], n = nd.count[g];
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const int e = idx[b + i];
+      key[e] = b;
+      val[e] = e;
+    }
+  }
+}
+
+// The bodies in the order ord (only written for a finished build).
+__global__ void __launch_bounds__(256)
+    k_body_gather(const TreeState *__restrict__ st, int room, const int *__restrict__ ord, int n,
+                  const double4 *__restrict__ in, double4 *__restrict__ body, int *__restrict__ bidx) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= n || node_count(st, room) == 0) return;
+  const int e = ord[p];
+  body[p] = in[e];
+  bidx[p] = e;
 }
 
 }  // namespace
@@ -430,7 +460,9 @@ void run_build_adaptive(Handle &h) {
   int bits = 1;
   while (((int64_t)1 << bits) < n) bits++;
   const uint64_t *key = nullptr;
+  uint64_t *spare = nullptr;  // the keys' other buffer
   int *idx = nullptr, *aux = nullptr;
+  const bool one = n <= ncrit;  // the root is a leaf: its bodies stay in input order
   // The cells of up to `room` nodes, the bodies in tree order and the check.
   auto emit = [&](int room) {
     h.cX.reserve(room);
@@ -445,11 +477,28 @@ void run_build_adaptive(Handle &h) {
     h.lvl_cells.reserve(room);
     h.ic.reserve((size_t)n + 2);
     h.id.reserve((size_t)n + 2);
-    hipLaunchKernelGGL(k_leaf_bodies, dim3(room), dim3(64), 0, h.stream, nd, st, room, bits, idx, aux, h.in4.p,
-                       h.body4.p, h.bidx.p);
-    zero_device(h.ic.p, ((size_t)n + 1) / 2 * 8, h.stream);
-    hipLaunchKernelGGL(k_block_sizes, dim3(div_up(room, T)), dim3(T), 0, h.stream, nd, st, room, h.ic.p);
-    exclusive_scan_int(h, h.ic.p, h.id.p, n);
+    const int *ord = idx;
+    if (!one && ncrit <= kRangeRank) {
+      for (int g = 0; g < room; g += std::min(room - g, kWaveGrid))
+        hipLaunchKernelGGL(k_leaf_bodies, dim3(std::min(room - g, kWaveGrid)), dim3(64), 0, h.stream, g, nd, st, room,
+                           bits, idx, aux, h.in4.p, h.body4.p, h.bidx.p);
+      ord = nullptr;
+    } else if (!one) {
+      int *k = reinterpret_cast<int *>(spare);
+      h.ie.reserve(n + 1);
+      hipLaunchKernelGGL(k_leaf_keys, dim3(std::min(room, 1 << 20)), dim3(T), 0, h.stream, nd, st, room, idx, k, aux);
+      bool alt = false;
+      sort_pairs_int_int(k, k + n + 1, aux, h.ie.p, n, bits, alt, h.stream, h.tmp);
+      ord = alt ? h.ie.p : aux;
+    }
+    if (ord)
+      hipLaunchKernelGGL(k_body_gather, dim3(div_up(n, T)), dim3(T), 0, h.stream, st, room, ord, n, h.in4.p, h.body4.p,
+                         h.bidx.p);
+    if (!one) {
+      zero_device(h.ic.p, ((size_t)n + 1) / 2 * 8, h.stream);
+      hipLaunchKernelGGL(k_block_sizes, dim3(div_up(room, T)), dim3(T), 0, h.stream, nd, st, room, h.ic.p);
+      exclusive_scan_int(h, h.ic.p, h.id.p, n);
+    }
     EXA_HIP(hipMemsetAsync(h.cNChild.p, 0xff, room * sizeof(int), h.stream));  // -1: not written
     hipLaunchKernelGGL(k_emit_cells, dim3(div_up(room, T)), dim3(T), 0, h.stream, nd, st, room, h.id.p, box, h.cX.p,
                        h.cRb.p, h.cParent.p, h.cChild.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cKey.p, h.cLevel.p,
@@ -477,8 +526,9 @@ void run_build_adaptive(Handle &h) {
     hipLaunchKernelGGL(k_path_keys, dim3(div_up(n, T)), dim3(T), 0, h.stream, h.in4.p, n, box, levels, h.k64a.p,
                        h.ia.p);
     bool alt = false;
-    sort_pairs_u64_int(h, h.k64a.p, h.k64b.p, h.ia.p, h.ib.p, n, 3 * (kDepth - levels), 3 * kDepth, alt);
+    if (!one) sort_pairs_u64_int(h, h.k64a.p, h.k64b.p, h.ia.p, h.ib.p, n, 3 * (kDepth - levels), 3 * kDepth, alt);
     key = alt ? h.k64b.p : h.k64a.p;
+    spare = alt ? h.k64a.p : h.k64b.p;
     idx = alt ? h.ib.p : h.ia.p;
     aux = alt ? h.ia.p : h.ib.p;
     hipLaunchKernelGGL(k_tree_small, dim3(1), dim3(8 * kTreeSmall), 0, h.stream, nd, key, ncrit, levels, st);
