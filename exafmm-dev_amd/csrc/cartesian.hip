@@ -373,9 +373,10 @@ __global__ void __launch_bounds__(64)
 // LDS), 5k bodies in 468 us (478, 462, 471; 990).
 
 // Real parts of the multipoles, packed (what k_m2l_cart_reg reads).
+constexpr int kPackGrid = 1 << 20;  // workgroups at most
 __global__ void k_cart_pack(const cplx *__restrict__ M, int64_t n, double *__restrict__ Mp) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) Mp[i] = M[i].re;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    Mp[i] = M[i].re;
 }
 
 // One Taylor coefficient (Kernels::derivative, :187-191) from the lower ones.
@@ -484,7 +485,7 @@ static void m2l_cart_reg(Handle &h, const M2LList &lst, const double4 *cX, const
   constexpr int NT = Cart<P>::NT;
   if (lst.ntgt == 0) return;
   h.cart_M.resize(nc * NT);
-  hipLaunchKernelGGL(k_cart_pack, dim3(div_up(nc * NT, 256)), dim3(256), 0, h.stream, M, nc * NT, h.cart_M.p);
+  hipLaunchKernelGGL(k_cart_pack, dim3(std::min(div_up(nc * NT, 256), kPackGrid)), dim3(256), 0, h.stream, M, nc * NT, h.cart_M.p);
   constexpr int A1 = P <= 6 ? NT : 35;
   hipLaunchKernelGGL((k_m2l_cart_reg<P, 0, A1>), dim3(lst.ntgt), dim3(64), 0, h.stream, lst.tgt, lst.off, lst.src,
                      lst.img, cX, h.cart_M.p, L, h.cfg.cycle, h.cfg.mass);
@@ -635,8 +636,10 @@ static void periodic_cart_impl(Handle &h) {
 template <int P>
 static void p2m_cart_impl(Handle &h, hipStream_t st, int radii) {
   const int l0 = h.lvl_off[std::min(h.leaf_level, h.nlevels - 1)];  // the cells that can be leaves
-  hipLaunchKernelGGL(k_p2m_cart<P>, dim3(h.ncells - l0), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p,
-                     h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
+  launch_ranges(h.ncells - l0, 64, [&](int c, int cnt) {
+    hipLaunchKernelGGL(k_p2m_cart<P>, dim3(cnt), dim3(64), 0, st, h.lvl_cells.p + l0 + c, h.body4.p, h.cX.p, h.cRb.p,
+                       h.cNChild.p, h.cBody.p, h.cNBody.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
+  });
 }
 
 template <int P>
@@ -644,8 +647,10 @@ static void m2m_cart_impl(Handle &h, hipStream_t st, int radii) {
   for (int t = h.nlevels - 2; t >= 0; t--) {
     const int cnt = h.lvl_off[t + 1] - h.lvl_off[t];
     if (cnt == 0) continue;
-    hipLaunchKernelGGL(k_m2m_cart<P>, dim3(cnt), dim3(512), 0, st, h.lvl_cells.p + h.lvl_off[t], h.cX.p, h.cRb.p,
-                       h.cChild.p, h.cNChild.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
+    launch_ranges(cnt, 512, [&](int c, int n) {
+      hipLaunchKernelGGL(k_m2m_cart<P>, dim3(n), dim3(512), 0, st, h.lvl_cells.p + h.lvl_off[t] + c, h.cX.p, h.cRb.p,
+                         h.cChild.p, h.cNChild.p, h.M.p, h.cfg.theta, h.cfg.useRmax, radii);
+    });
   }
   EXA_HIP(hipGetLastError());
 }

@@ -7,10 +7,6 @@
 
 namespace exafmm {
 
-// Workgroups of 64 in one launch, which takes fewer than 2^32 threads: longer
-// ranges go in several.
-constexpr int kWaveGrid = 1 << 25;
-
 // Orders the LDS accesses of one wave (its stores before its later loads by
 // other lanes), where waves of a workgroup use separate parts of LDS.
 __device__ inline void wave_sync() {

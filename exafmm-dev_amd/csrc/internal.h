@@ -76,6 +76,17 @@ struct GroupScratch {
   bool zero = false;
 };
 
+// n workgroups of `threads` threads in as many launches as it takes (one takes
+// fewer than 2^32 threads): launch(first, count).
+template <typename F>
+inline void launch_ranges(int n, int threads, F launch) {
+  const int most = (int)(((int64_t)1 << 31) / threads);
+  for (int i = 0, c; i < n; i += c) {
+    c = n - i < most ? n - i : most;
+    launch(i, c);
+  }
+}
+
 // A CSR interaction list by target cell (targets with work listed in tgt).
 struct M2LList {
   const int *tgt;

@@ -341,8 +341,10 @@ static void m2l_launch(Handle &h, hipStream_t st, const M2LList &lst, const doub
     h.pair_timed = true;
   }
   auto launch = [&](auto kernel, int waves) {
-    hipLaunchKernelGGL(kernel, dim3(lst.ntgt), dim3(64 * waves), 0, st, lst.tgt, lst.off, lst.src, lst.img, cX, M, L,
-                       desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+    launch_ranges(lst.ntgt, 64 * waves, [&](int t, int cnt) {
+      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(64 * waves), 0, st, lst.tgt + t, lst.off, lst.src, lst.img, cX, M, L,
+                         desc, slot0, outslot, h.cfg.cycle, h.cfg.mass);
+    });
   };
   constexpr int W = P <= 10 ? 8 : 4;  // 55 KB of LDS per workgroup at P = 10, 41 KB at P = 12
   const bool few =

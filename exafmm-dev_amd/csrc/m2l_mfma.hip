@@ -752,12 +752,12 @@ __global__ void k_fill_int(int *__restrict__ p, int64_t n, int v) {
 // all zero and stands for an empty column.
 template <int P, typename R>
 __global__ void __launch_bounds__(256)
-    k_lat_mscale(int nc, const double *__restrict__ cRb, const cplx *__restrict__ M, R *__restrict__ Ms) {
+    k_lat_mscale(int b0, int nc, const double *__restrict__ cRb, const cplx *__restrict__ M, R *__restrict__ Ms) {
   using S = MfmaShape<P>;
   using MR = MsRow<P, R>;
   constexpr int NR = S::NR, NKP = MR::NKP, VL = MR::VL;
   constexpr DegreeTable<P> deg{};
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = (int64_t)(b0 + blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= (int64_t)(nc + 1) * NKP) return;
   const int c = (int)(i / NKP), p = (int)(i % NKP);
   const int r = p % (4 * VL), kq = r / VL, kc = (p / (4 * VL)) * VL + r % VL;
@@ -976,12 +976,14 @@ static void mscale_impl(Handle &h, hipStream_t st) {
   const int64_t nmd = (int64_t)(nc + 1) * MsRow<P, double>::NKP;
   if (h.cfg.precision == 1) {
     h.lat_Msf.resize(nms);
-    hipLaunchKernelGGL((k_lat_mscale<P, float>), dim3(div_up(nms, 256)), dim3(256), 0, st, nc, h.cRb.p, h.M.p,
-                       h.lat_Msf.p);
+    launch_ranges(div_up(nms, 256), 256, [&](int b0, int nb) {
+      hipLaunchKernelGGL((k_lat_mscale<P, float>), dim3(nb), dim3(256), 0, st, b0, nc, h.cRb.p, h.M.p, h.lat_Msf.p);
+    });
   } else {
     h.lat_Ms.resize(nmd);
-    hipLaunchKernelGGL((k_lat_mscale<P, double>), dim3(div_up(nmd, 256)), dim3(256), 0, st, nc, h.cRb.p, h.M.p,
-                       h.lat_Ms.p);
+    launch_ranges(div_up(nmd, 256), 256, [&](int b0, int nb) {
+      hipLaunchKernelGGL((k_lat_mscale<P, double>), dim3(nb), dim3(256), 0, st, b0, nc, h.cRb.p, h.M.p, h.lat_Ms.p);
+    });
   }
 }
 

@@ -378,8 +378,10 @@ static int first_leaf(const Handle &h) { return h.lvl_off[std::min(h.leaf_level,
 template <int P>
 static void p2m_impl(Handle &h, hipStream_t st) {
   const int l0 = first_leaf(h), n = h.ncells - l0;
-  hipLaunchKernelGGL(k_p2m<P>, dim3(n), dim3(64), 0, st, h.lvl_cells.p + l0, h.body4.p, h.cX.p, h.cNChild.p,
-                     h.cBody.p, h.cNBody.p, h.M.p);
+  launch_ranges(n, 64, [&](int c, int cnt) {
+    hipLaunchKernelGGL(k_p2m<P>, dim3(cnt), dim3(64), 0, st, h.lvl_cells.p + l0 + c, h.body4.p, h.cX.p, h.cNChild.p,
+                       h.cBody.p, h.cNBody.p, h.M.p);
+  });
 }
 
 // Parents up to which a level runs per cell: the product on the matrix cores
@@ -397,7 +399,9 @@ static void m2m_impl(Handle &h, hipStream_t st) {
     if (mf && cnt > kM2MFew)
       run_m2m_level_mfma(h, cells, cnt, st);
     else
-      hipLaunchKernelGGL(k_m2m<P>, dim3(cnt), dim3(512), 0, st, cells, h.cX.p, h.cChild.p, h.cNChild.p, h.M.p);
+      launch_ranges(cnt, 512, [&](int c, int n) {
+        hipLaunchKernelGGL(k_m2m<P>, dim3(n), dim3(512), 0, st, cells + c, h.cX.p, h.cChild.p, h.cNChild.p, h.M.p);
+      });
   }
   EXA_HIP(hipGetLastError());
 }
@@ -405,8 +409,10 @@ static void m2m_impl(Handle &h, hipStream_t st) {
 // Leaves of every level first, then the parents from the bottom up.
 static void run_radii(Handle &h) {
   const int l0 = first_leaf(h), nleaf = h.ncells - l0;
-  hipLaunchKernelGGL(k_radii_leaves, dim3(div_up(nleaf, 4)), dim3(256), 0, h.stream, h.lvl_cells.p + l0, nleaf,
-                     h.body4.p, h.cX.p, h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cfg.theta, h.cfg.useRmax);
+  launch_ranges(nleaf, 64, [&](int c, int cnt) {
+    hipLaunchKernelGGL(k_radii_leaves, dim3(div_up(cnt, 4)), dim3(256), 0, h.stream, h.lvl_cells.p + l0 + c, cnt,
+                       h.body4.p, h.cX.p, h.cRb.p, h.cNChild.p, h.cBody.p, h.cNBody.p, h.cfg.theta, h.cfg.useRmax);
+  });
   TopLevels tl{};
   const int np = h.nlevels - 1;  // levels that can hold parents
   while (tl.n < np && tl.n < 32 && h.lvl_off[tl.n + 1] - h.lvl_off[tl.n] <= kRadiiTop) tl.n++;

@@ -567,11 +567,11 @@ __global__ void __launch_bounds__(256)
 // One wave per target: its indices sorted, then the sources and images in
 // that order.
 __global__ void __launch_bounds__(64)
-    k_group_sort(const int *__restrict__ off, int bits, int *__restrict__ ord, int *__restrict__ aux,
+    k_group_sort(int c0, const int *__restrict__ off, int bits, int *__restrict__ ord, int *__restrict__ aux,
                  const int *__restrict__ src_in, const unsigned char *__restrict__ img_in, int *__restrict__ src_out,
                  unsigned char *__restrict__ img_out) {
   __shared__ RangeSortLds sh;
-  const int o = off[blockIdx.x], n = off[blockIdx.x + 1] - o;
+  const int c = c0 + blockIdx.x, o = off[c], n = off[c + 1] - o;
   if (n <= 0) return;
   sort_range(ord + o, aux + o, n, bits, sh, [&](int rank, int e) {
     src_out[o + rank] = src_in[e];
@@ -633,8 +633,10 @@ static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t 
     while (((int64_t)1 << bits) < np) bits++;
     hipLaunchKernelGGL(k_group_scatter, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, skip, np, off.p, g.cnt.p,
                        g.ord.p);
-    hipLaunchKernelGGL(k_group_sort, dim3(nc), dim3(64), 0, st, off.p, bits, g.ord.p, g.aux.p, src.p, img.p, src_out.p,
-                       img_out.p);
+    launch_ranges(nc, 64, [&](int c, int cnt) {
+      hipLaunchKernelGGL(k_group_sort, dim3(cnt), dim3(64), 0, st, c, off.p, bits, g.ord.p, g.aux.p, src.p, img.p,
+                         src_out.p, img_out.p);
+    });
   }
   EXA_HIP(hipGetLastError());
   g.zero = true;

@@ -479,9 +479,10 @@ void run_build_adaptive(Handle &h) {
     h.id.reserve((size_t)n + 2);
     const int *ord = idx;
     if (!one && ncrit <= kRangeRank) {
-      for (int g = 0; g < room; g += std::min(room - g, kWaveGrid))
-        hipLaunchKernelGGL(k_leaf_bodies, dim3(std::min(room - g, kWaveGrid)), dim3(64), 0, h.stream, g, nd, st, room,
-                           bits, idx, aux, h.in4.p, h.body4.p, h.bidx.p);
+      launch_ranges(room, 64, [&](int g, int cnt) {
+        hipLaunchKernelGGL(k_leaf_bodies, dim3(cnt), dim3(64), 0, h.stream, g, nd, st, room, bits, idx, aux, h.in4.p,
+                           h.body4.p, h.bidx.p);
+      });
       ord = nullptr;
     } else if (!one) {
       int *k = reinterpret_cast<int *>(spare);
