@@ -654,6 +654,7 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
   }
   const int nchunk = (int)((tab.size() - chunks0) / 2);
   tab[chunk00 + S] = nchunk;
+  h.drop_tree();
   if (tab != h.ut_tab_host) {
     h.ut_tab_host.clear();
     h.ut_tab.resize(tab.size() + 1);

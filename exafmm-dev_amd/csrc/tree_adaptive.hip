@@ -433,11 +433,19 @@ __global__ void __launch_bounds__(256)
   bidx[p] = e;
 }
 
+constexpr const char *kDegenerate = "build_tree: degenerate bounds (box radius 0)";
+
 }  // namespace
 
 void run_build_adaptive(Handle &h) {
   const int n = h.n, ncrit = h.cfg.ncrit;
   const int T = 256;
+  if (!h.bounds_pending) {  // (otherwise the device's radius is read back)
+    bool extent = false;
+    for (int d = 0; d < 3; d++) extent = extent || h.xmax[d] > h.xmin[d];
+    if (!extent) throw Error(EXAFMM_HIP_EINVAL, kDegenerate);
+  }
+  h.drop_tree();
   upload_bounds(h);
   h.body4.resize(n);
   h.bidx.resize(n);
@@ -550,7 +558,7 @@ void run_build_adaptive(Handle &h) {
       if (hs.overflow || hs.nact == 0 || hs.lev >= levels) break;
       batch = 4;
     }
-    if (!(hs.R0 > 0)) throw Error(EXAFMM_HIP_EINVAL, "build_tree: degenerate bounds (box radius 0)");
+    if (!(hs.R0 > 0)) throw Error(EXAFMM_HIP_EINVAL, kDegenerate);
     if (hs.overflow) {
       cap *= 2;
       continue;
