@@ -64,7 +64,13 @@ static void ensure(bool cond, const char *msg) {
   if (!cond) throw Error(EXAFMM_HIP_EINVAL, msg);
 }
 
+// Before another tree or upward pass: an evaluation that failed in its traversal
+// has left multipoles that the next traversal would queue or wait for, and they
+// are not those of what comes now.
+static void drop_multipoles(Handle &h) { h.mult_enqueue = h.mult_pending = false; }
+
 static void do_build(Handle &h) {
+  drop_multipoles(h);
   ensure(h.have_bounds, "build_tree: bounds not computed");
   ensure(h.n > 0, "build_tree: no bodies");
   if (h.nsys > 1)
@@ -81,6 +87,7 @@ static void do_build(Handle &h) {
 
 static void do_upward(Handle &h) {
   ensure(h.have_tree, "upward_pass: tree not built");
+  drop_multipoles(h);
   h.lat_ms_ready = h.lat_tiles_ready = false;  // the lattice M2L rescales these multipoles itself
   run_upward(h);
   run_ropt(h);
@@ -160,6 +167,8 @@ int exafmm_hip_create(const exafmm_hip_config *cfg, exafmm_hip_handle **out) {
   }
   if (const char *m = std::getenv("EXAFMM_HIP_LAT_WG")) H->h.lat_wg_cu = std::atoi(m);
   if (const char *m = std::getenv("EXAFMM_HIP_SERIAL")) H->h.serial_heavy = std::atoi(m) != 0;
+  // Fewer cells than a traversal could take (tests of what follows a refusal).
+  if (const char *m = std::getenv("EXAFMM_HIP_MAX_CELLS")) H->h.max_cells = std::min(H->h.max_cells, std::atoi(m));
   // Rows of the lattice T(d) table kept across evaluations (16384 rows are
   // 0.5 GB in FP64 at P = 10).
   if (const char *m = std::getenv("EXAFMM_HIP_TCACHE_ROWS")) H->h.lat_tc_max = std::max(1, std::atoi(m));
@@ -305,6 +314,7 @@ static void evaluate_all(Handle &h) {
     if (h.nsys > 1) {  // a forest: per-system bounds inside the builder
       h.have_bounds = true;
       EXA_HIP(hipEventRecord(h.ev[1], h.stream));
+      drop_multipoles(h);
       run_build_forest(h);
       h.have_tree = true;
       h.have_up = h.have_trav = false;

@@ -108,6 +108,7 @@ struct Handle {
   hipEvent_t ev_mult = nullptr;  // multipoles done on stream3 (split upward pass)
   bool mult_pending = false;     // the main stream has not joined ev_mult yet
   bool mult_enqueue = false;     // run_upward_mult not enqueued yet (the traversal does it)
+  int max_cells = 1 << 27;       // a traversal takes fewer cells than this (its pairs hold 27-bit indices)
   hipEvent_t ev_cnt = nullptr;   // a device count copied into hpin
   hipEvent_t ev_used = nullptr;  // image offsets in use flagged (main stream)
   hipEvent_t ev_image = nullptr; // their matrices done on stream3
@@ -352,6 +353,10 @@ inline void join_multipoles(Handle &h) {
   EXA_HIP(hipStreamWaitEvent(h.stream, h.ev_mult, 0));
   h.mult_pending = false;
 }
+// What a failed call has queued runs out before the next one changes its arrays.
+inline void settle(Handle &h) {
+  for (hipStream_t st : {h.stream, h.stream2, h.stream3}) (void)hipStreamSynchronize(st);
+}
 void run_lists(Handle &h);
 // The first part of the lattice M2L set-up (nothing waits for the device),
 // queued on the main stream before P2P; run_m2l does the rest.
@@ -456,9 +461,11 @@ static int guarded(exafmm_hip_handle *H, F &&f) {
     H->h.err.clear();
     return EXAFMM_HIP_OK;
   } catch (const exafmm::Error &e) {
+    exafmm::settle(H->h);
     H->h.err = e.what();
     return e.code;
   } catch (const std::exception &e) {
+    exafmm::settle(H->h);
     H->h.err = e.what();
     return EXAFMM_HIP_EDEVICE;
   }

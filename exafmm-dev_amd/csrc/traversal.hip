@@ -693,7 +693,8 @@ static bool traverse_on_device(Handle &h, const CellView &cv, const int *roots, 
 
 void run_lists(Handle &h) {
   const int T = 256;
-  if (h.ncells >= (1 << kImgShift))
+  static_assert(kImgShift == 27, "Handle::max_cells");
+  if (h.ncells >= h.max_cells)
     throw Error(EXAFMM_HIP_EUNSUP, "traversal: more than 2^27 cells (frontier pairs hold 27-bit cell indices)");
   CellView cv{h.cX.p, h.cChild.p, h.cNChild.p, h.cNBody.p};
   // Raw (emission-order) lists, kept on the handle across evaluations.

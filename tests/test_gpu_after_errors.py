@@ -48,3 +48,34 @@ def test_refused_tree():
     f.build_tree(f.get_bounds())
     assert np.array_equal(passes(f), want)
     f.close()
+
+
+@pytest.mark.parametrize("kw", [dict(P=8, ncrit=64), dict(P=6, ncrit=64, builder="adaptive", precision="mixed"),
+                                dict(P=4, ncrit=64, basis="cartesian")])
+@pytest.mark.parametrize("then", ["passes", "evaluate", "passes of the same tree"])
+def test_refused_evaluation(kw, then, monkeypatch):
+    x, big = unit_cube(20000, 2), unit_cube(60000, 3)
+    f = X.FMM(**kw)
+    f.set_bodies(x)
+    limit = f.build_tree(f.get_bounds()) + 1
+    f.close()
+    want = fresh(x, **kw)
+    monkeypatch.setenv("EXAFMM_HIP_MAX_CELLS", str(limit))
+    f = X.FMM(**kw)
+    f.set_bodies(big)
+    print(f"[gpu] evaluation of more than {limit} cells refused, then {then}", flush=True)
+    with pytest.raises(X.ExafmmError, match="cells"):
+        f.evaluate()
+    if then == "passes of the same tree":
+        f.upward_pass()
+        with pytest.raises(X.ExafmmError, match="cells"):
+            f.traverse()
+    f.set_bodies(x)
+    if then == "evaluate":
+        f.evaluate()
+        got = f.results()
+    else:
+        f.build_tree(f.get_bounds())
+        got = passes(f)
+    assert np.array_equal(got, want)
+    f.close()
