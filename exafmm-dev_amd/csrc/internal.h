@@ -391,6 +391,7 @@ void run_direct_arrays(Handle &h, int nt, const double *t_xyzq, int ns, const do
 void run_mass_normalise(Handle &h);
 void run_ropt(Handle &h);
 bool run_m2l_lattice(Handle &h, M2LList &irr);
+void lattice_reset(Handle &h);  // no contraction run, no pairs counted
 void lattice_finish(Handle &h);
 void run_lattice_mscale(Handle &h, hipStream_t st);
 // Target tiles of the lattice contraction for the current tree.

@@ -375,6 +375,8 @@ void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const c
 }
 
 void run_m2l(Handle &h) {
+  h.pair_timed = false;
+  lattice_reset(h);  // (nothing of the last run is this one's)
   if (h.nm2l == 0) {
     // No pair reads the scaled multipoles the split upward pass may have
     // queued: a later traversal must rebuild them for its own tree.
@@ -388,7 +390,6 @@ void run_m2l(Handle &h) {
   }
   // Lattice pairs on the matrix cores first (from the raw list; lst becomes
   // the irregular pairs grouped by target); otherwise every pair per pair.
-  h.pair_timed = false;
   M2LList lst{};
   if (!run_m2l_lattice(h, lst)) {
     ensure_m2l_grouped(h);

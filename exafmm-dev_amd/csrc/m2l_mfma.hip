@@ -1406,12 +1406,15 @@ void lattice_replay(Handle &h) {
   }
 }
 
-bool run_m2l_lattice(Handle &h, M2LList &irr) {
+void lattice_reset(Handle &h) {
   h.lat_timed = h.lat_reduce_pending = false;
   h.lat_run_ntiles = 0;
   h.lat_stats_pairs = 0;
   h.lat_stats_tiles = 0;
   h.lat_stats_steps = 0;
+}
+
+bool run_m2l_lattice(Handle &h, M2LList &irr) {
   if (!lattice_applies(h) || h.nm2l == 0) {
     h.lat_ms_ready = h.lat_tiles_ready = false;
     return false;
