@@ -634,7 +634,7 @@ int exafmm_hip_get_stats(exafmm_hip_handle *H, exafmm_hip_stats *s) {
     h.stats.num_cells = h.ncells;
     h.stats.num_levels = h.nlevels;
     h.stats.num_m2l_lattice = h.lat_stats_pairs;
-    h.stats.num_m2l_offsets = h.have_trav ? lattice_offsets_used(h) : 0;
+    h.stats.num_m2l_offsets = h.lat_stats_noff;
     h.stats.num_m2l_tiles = h.lat_stats_tiles;
     h.stats.num_m2l_steps = h.lat_stats_steps;
     *s = h.stats;

@@ -252,7 +252,7 @@ struct Handle {
   int lat_run_ntiles = 0, lat_run_ngrid = 0;  // the last contraction's tiles and grid (0 tiles: none ran)
   M2LList m2l_last{};                          // the pairs the last run_m2l gave the per-pair kernel
   int64_t lat_stats_pairs = 0;
-  int lat_stats_tiles = 0;
+  int lat_stats_tiles = 0, lat_stats_noff = 0;
   int64_t lat_stats_steps = 0;
   bool lat_timed = false, pair_timed = false;  // ev[12..13]: MFMA kernel, ev[14..15]: per-pair kernel
 
@@ -396,7 +396,6 @@ void lattice_finish(Handle &h);
 void run_lattice_mscale(Handle &h, hipStream_t st);
 // Target tiles of the lattice contraction for the current tree.
 void run_lattice_tiles(Handle &h, hipStream_t st);
-int lattice_offsets_used(Handle &h);
 bool updown_mfma_enabled(const Handle &h);
 bool lattice_applies(const Handle &h);
 void run_m2m_level_mfma(Handle &h, const int *cells, int cnt, hipStream_t st);

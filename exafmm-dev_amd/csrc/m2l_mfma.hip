@@ -140,7 +140,10 @@ struct LatState {
   int nirr;     // irregular pairs
   int nsteps;   // (tile, offset) steps
   int ntiles;   // tiles with steps
+  int noffs;    // offsets with steps
+  int pad;
 };
+static_assert(sizeof(LatState) % 8 == 0, "cleared by whole words");
 
 // Face that image im lies across (-x, +x, -y, ... +z), or -1.
 __device__ inline int image_face(int im) {
@@ -207,7 +210,8 @@ __device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ 
 
 // Every M2L pair's step, tile * noff + o (o: number of its offset among the
 // noff known ones), into pstep, -1 for a pair that is not on the lattice (or
-// whose target is in no tile); act flags the steps in use.  A pair with an
+// whose target is in no tile); act flags the steps in use, used the image
+// offsets (the others by k_lat_count).  A pair with an
 // unknown offset flags it in hist and makes the set-up unusable.  (A fixed grid
 // and one atomic per workgroup for the irregular count: one per wave took 500 us
 // in a periodic list of 11 M pairs, a fifth of them irregular.)
@@ -235,7 +239,7 @@ __global__ void k_lat_classify(const int *__restrict__ ptgt, const int *__restri
       } else {
         v = tile * noff + o;
         act[v] = 1;
-        if (o >= nreg && !used[o - nreg]) used[o - nreg] = 1;
+        if (o >= nreg && !used[o]) used[o] = 1;
       }
     }
     pstep[e] = v;
@@ -324,7 +328,7 @@ __global__ void __launch_bounds__(64) k_lat_tmat(const int *__restrict__ okey, R
   for (int i = S::NBLK * 64 + lane; i < TPad<P, R>::TEP; i += 64) T[(size_t)o * TPad<P, R>::TEP + i] = 0;
 }
 
-// T of the image offsets in use (numbers nreg + i, used[i]), as k_lat_tmat for
+// T of the image offsets in use (numbers from nreg on), as k_lat_tmat for
 // the actual offset of their level and face.  A workgroup makes kImgT of them
 // together, so that the entries' index arithmetic is done once for all; bound
 // by the stores: 6800 offsets at P = 10 are 212 MB, 0.32 ms alone with one
@@ -350,7 +354,7 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x < kImgT) {
     const int o = o0 + threadIdx.x;
     srow[threadIdx.x] = -1;
-    if (o < noff && used[o - nreg]) {
+    if (o < noff && used[o]) {
       const int k = okey[o] - kLatKeys, face = k / kImgFace % 6;
       int x, y, z;
       image_offset(k % kImgFace, x, y, z);
@@ -589,14 +593,19 @@ __device__ inline void tile_images(const LatRanges &lr, int tile, int &lo, int &
     }
 }
 
-// Steps per tile: the flags of its row of act.
+// Steps per tile: the flags of its row of act.  Flags the lattice offsets in use.
 __global__ void __launch_bounds__(256)
-    k_lat_count(const unsigned char *__restrict__ act, int noff, LatRanges lr, int *__restrict__ cnt) {
+    k_lat_count(const unsigned char *__restrict__ act, int noff, LatRanges lr, int *__restrict__ cnt,
+                unsigned char *__restrict__ used) {
   __shared__ int sw[4];
   const unsigned char *a = act + (size_t)blockIdx.x * noff;
   int n = 0, lo, hi;
   tile_images(lr, blockIdx.x, lo, hi);
-  for (int o = threadIdx.x; o < lr.nreg; o += 256) n += a[o];
+  for (int o = threadIdx.x; o < lr.nreg; o += 256)
+    if (a[o]) {
+      n++;
+      if (!used[o]) used[o] = 1;
+    }
   for (int o = lo + threadIdx.x; o < hi; o += 256) n += a[o];
   for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
   if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = n;
@@ -609,10 +618,10 @@ __global__ void __launch_bounds__(256)
 // row; their slots are emptied.
 __global__ void __launch_bounds__(256)
     k_lat_steps(const unsigned char *__restrict__ act, const int *__restrict__ cnt, int noff, LatRanges lr,
-                const int *__restrict__ orow, int *__restrict__ aidx, int *__restrict__ step0,
+                const unsigned char *__restrict__ used, const int *__restrict__ orow, int *__restrict__ aidx, int *__restrict__ step0,
                 int *__restrict__ alist, int4 *__restrict__ slot, LatState *__restrict__ st,
                 LatState *__restrict__ host) {
-  __shared__ int sw[4], sn[4];
+  __shared__ int sw[4], sn[4], su[4];
   const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int base = 0, full = 0;
   for (int t = tid; t < tile; t += 256) {
@@ -620,13 +629,17 @@ __global__ void __launch_bounds__(256)
     base += c;
     full += c > 0;
   }
+  int offs = 0;
+  for (int o = tid; tile == (int)gridDim.x - 1 && o < noff; o += 256) offs += used[o];
   for (int d = 32; d >= 1; d >>= 1) {
     base += __shfl_xor(base, d);
     full += __shfl_xor(full, d);
+    offs += __shfl_xor(offs, d);
   }
   if (lane == 0) {
     sw[wave] = base;
     sn[wave] = full;
+    su[wave] = offs;
   }
   __syncthreads();
   base = sw[0] + sw[1] + sw[2] + sw[3];
@@ -637,6 +650,7 @@ __global__ void __launch_bounds__(256)
       step0[tile + 1] = base + mine;
       st->nsteps = base + mine;
       st->ntiles = sn[0] + sn[1] + sn[2] + sn[3] + (mine > 0);
+      st->noffs = su[0] + su[1] + su[2] + su[3];
       *host = *st;  // (pinned)
     }
   }
@@ -732,15 +746,6 @@ __global__ void k_lat_marks(const int *__restrict__ kscan, const int *__restrict
   if (i <= kImgLevels) host[3 + i] = kscan[min(n, kLatKeys + i * kImgLevelKeys)];
 }
 
-// Offsets in use: flags of any tile.
-__global__ void k_lat_used(const unsigned char *__restrict__ act, int ntiles, int noff, int *__restrict__ count) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  bool u = false;
-  for (int t = 0; o < noff && t < ntiles && !u; t++) u = act[(size_t)t * noff + o];
-  const unsigned long long m = __ballot(u);
-  if (m && (threadIdx.x & 63) == 0) atomicAdd(count, (int)__popcll(m));
-}
-
 __global__ void k_fill_int(int *__restrict__ p, int64_t n, int v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -779,7 +784,8 @@ __global__ void __launch_bounds__(256)
 // and keeps them in its L2.
 constexpr int kLatSeg = 8;
 // Words of Handle::hpin the lattice set-up reads back (LatState; registration counts).
-constexpr int kPinLat = 64, kPinMarks = 64 + 4;
+constexpr int kPinLat = 64, kPinMarks = kPinLat + 8;
+static_assert(sizeof(LatState) <= 8 * sizeof(int), "pinned words");
 
 typedef __attribute__((address_space(3))) void lds_void;
 // s_waitcnt immediate for vmcnt(0) with expcnt and lgkmcnt left alone.
@@ -1129,13 +1135,13 @@ static void lattice_steps(Handle &h) {
     lr.hi[i] = h.lat_img0[slot + 1];
     nbound += (int64_t)(lr.tile1[i] - lr.tile0[i]) * (lr.hi[i] - lr.lo[i]);
   }
-  h.lat_act.resize(sizeof(LatState) + nall + nimg + 8);
+  h.lat_act.resize(sizeof(LatState) + nall + h.lat_noff + 8);
   h.lat_aidx.resize(nall + 1);
   h.lat_pslot.resize(np);
   h.lat_tcnt.resize(h.lat_ntiles + 1);
   h.lat_step0.resize(h.lat_ntiles + 1);
   unsigned char *act = h.lat_act.p + sizeof(LatState), *used = act + nall;
-  zero_device(h.lat_act.p, sizeof(LatState) + (nall + nimg + 7) / 8 * 8, h.stream);
+  zero_device(h.lat_act.p, sizeof(LatState) + (nall + h.lat_noff + 7) / 8 * 8, h.stream);
   hipLaunchKernelGGL(k_lat_classify, dim3(std::min(gp, 4096)), dim3(TPB), 0, h.stream, ptgt, psrc, h.raw_mimg.p, np,
                      h.cX.p, h.cRb.p, h.lat_ookey.p, h.lat_tile_of.p, h.cLevel.p, li, h.lat_nreg, h.lat_noff, act,
                      used, h.lat_pslot.p, h.lat_hist.p, lat_state(h));
@@ -1156,7 +1162,8 @@ static void lattice_steps(Handle &h) {
     EXA_HIP(hipEventRecord(h.ev_image, h.stream3));
   }
   if (nall > 0) {
-    hipLaunchKernelGGL(k_lat_count, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_noff, lr, h.lat_tcnt.p);
+    hipLaunchKernelGGL(k_lat_count, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_noff, lr, h.lat_tcnt.p,
+                       used);
     // Step lists sized for every (tile, offset) being in use, so that the
     // host need not wait for the count, unless that bound is large.
     int64_t nact = nbound;
@@ -1171,7 +1178,7 @@ static void lattice_steps(Handle &h) {
     h.lat_alist.resize(nact > 0 ? nact : 1);
     h.lat_slot.resize(nact > 0 ? nact * 64 : 4);
     hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff, lr,
-                       h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
+                       used, h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
                        reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h), host);
     if (!h.bounds_given) EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
     hipLaunchKernelGGL(h.bounds_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
@@ -1317,6 +1324,7 @@ static void lattice_run(Handle &h, M2LList &irr) {
   const int nirr = ls->nirr;
   h.lat_stats_steps = h.lat_run_ntiles ? ls->nsteps : 0;
   h.lat_stats_tiles = h.lat_run_ntiles ? ls->ntiles : 0;
+  h.lat_stats_noff = h.lat_run_ntiles ? ls->noffs : 0;
   h.lat_reduce_pending = irregular && h.lat_run_ntiles > 0;
   int nitl = 0;
   if (nirr) {
@@ -1342,20 +1350,6 @@ void lattice_finish(Handle &h) {
     case 10: lattice_reduce<10>(h); break;
     case 12: lattice_reduce<12>(h); break;
   }
-}
-
-// Distinct offsets of the last contraction (a reduction over its step flags).
-int lattice_offsets_used(Handle &h) {
-  if (h.lat_run_ntiles == 0) return 0;
-  h.cnt.reserve(4);
-  int n = 0;
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, h.stream, h.cnt.p, (int64_t)1, 0);
-  hipLaunchKernelGGL(k_lat_used, dim3(div_up(h.lat_noff, 256)), dim3(256), 0, h.stream, h.lat_act.p + sizeof(LatState),
-                     h.lat_run_ntiles, h.lat_noff, h.cnt.p);
-  EXA_HIP(hipGetLastError());
-  EXA_HIP(hipMemcpyAsync(&n, h.cnt.p, sizeof(int), hipMemcpyDeviceToHost, h.stream));
-  EXA_HIP(hipStreamSynchronize(h.stream));
-  return n;
 }
 
 bool lattice_applies(const Handle &h) {
@@ -1410,7 +1404,7 @@ void lattice_reset(Handle &h) {
   h.lat_timed = h.lat_reduce_pending = false;
   h.lat_run_ntiles = 0;
   h.lat_stats_pairs = 0;
-  h.lat_stats_tiles = 0;
+  h.lat_stats_tiles = h.lat_stats_noff = 0;
   h.lat_stats_steps = 0;
 }
 

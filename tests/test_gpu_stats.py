@@ -1,4 +1,6 @@
-"""What get_stats says of the M2L: nothing of an earlier system."""
+"""What get_stats says of the M2L: nothing of an earlier system, and as many
+offsets as the list has."""
+import numpy as np
 import pytest
 
 import exafmm_hip as X
@@ -21,4 +23,21 @@ def test_no_pairs_after_a_larger_system(precision):
     s = f.stats()
     assert s["num_m2l_pairs"] == 0
     assert {k: s[k] for k in names + ("t_m2l_pairs",)} == dict.fromkeys(names + ("t_m2l_pairs",), 0)
+    f.close()
+
+
+def test_offsets_of_the_list():
+    f = X.FMM(P=4, ncrit=32)
+    for n in (20000, 1500, 9000):  # one handle: it knows the offsets of the larger trees
+        f.set_bodies(unit_cube(n, n))
+        f.evaluate()
+        c, l, s = f.cells(), f.lists(), f.stats()
+        print(f"[gpu] {n} bodies, {s['num_m2l_offsets']} offsets", flush=True)
+        assert s["num_m2l_lattice"] == s["num_m2l_pairs"] == len(l["m2l_i"])
+        # In quarters of the target's width, which is twice its distance to the parent's centre in any
+        # coordinate (the residues modulo 4 tell the source's level).
+        up = np.abs(c["X"] - c["X"][c["iparent"]]).max(1)
+        i, j = l["m2l_i"], l["m2l_j"]
+        d = np.rint((c["X"][i] - c["X"][j]) / (0.5 * up[i])[:, None]).astype(int)
+        assert s["num_m2l_offsets"] == len(np.unique(d, axis=0))
     f.close()
