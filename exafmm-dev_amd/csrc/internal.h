@@ -118,6 +118,7 @@ struct Handle {
   hipEvent_t ev_bounds = nullptr; // bounds copied into hpin[kPinBounds..] (main stream)
   int *hpin = nullptr;           // pinned host words for counts read back behind queued work
   static constexpr int kPinWords = 512;  // hpin: [0..64) counts, [64..80) lattice set-up, [128..) tree build, [400..412) bounds
+  static constexpr int kPinBare = 11;     // set by the P2P grouping: some leaf is no P2P target
   static constexpr int kPinBounds = 400;  // hpin: [400, 412) the six bounds (doubles)
 
   // Bodies.

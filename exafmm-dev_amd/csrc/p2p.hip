@@ -1143,8 +1143,10 @@ static bool p2p_two_rounds(const Handle &h, int64_t leaves, int64_t waves) {
 }
 
 void run_p2p(Handle &h, hipStream_t st, bool setup) {
-  // Every body belongs to a leaf that is in its own list, and every target is
-  // written once: the results need no clearing.
+  // Every target's results are written once, and those of leaves that are no
+  // target were cleared with the list grouping: they are cleared here only for a
+  // run from kept lists.
+  if (h.np2p_tgt >= 0 && h.hpin[Handle::kPinBare]) zero_device(h.trg4.p, (size_t)h.n * sizeof(double4), st);
   if (h.np2p_tgt == 0) return;
   const int64_t leaves = tree_leaves(h);
   const int W = p2p_waves_per_leaf(h);

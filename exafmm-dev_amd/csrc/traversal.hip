@@ -510,11 +510,21 @@ __global__ void __launch_bounds__(1024)
 
 // off[c] = entries of the targets before c, tlist = the non-empty targets;
 // the number of those to *ntl and *ntl_host (pinned); *next (if given) is
-// cleared, the work counter of what reads the list.
+// cleared, the work counter of what reads the list.  bare.trg (if given): the
+// results of leaves that are no target, which nothing else writes, are cleared
+// and *bare.any set.  (A leaf is in its own list unless its centre lies off its
+// parent's by more than the parent's radius: rounded centres, or bounds from the
+// caller that do not enclose the bodies.)
+struct BareLeaves {
+  const int *nchild, *body, *nbody;
+  double4 *trg;
+  int *any;
+};
+
 __global__ void __launch_bounds__(1024)
     k_group_offsets(const int *__restrict__ cnt, int nc, const int2 *__restrict__ tot, int *__restrict__ off,
                     int *__restrict__ tlist, int *__restrict__ ntl, int *__restrict__ ntl_host,
-                    int *__restrict__ next) {
+                    int *__restrict__ next, BareLeaves bare) {
   __shared__ int sbase[2];
   int4 v = make_int4(0, 0, 0, 0), sum;
   for (int b = threadIdx.x; b < (int)blockIdx.x; b += 1024) {
@@ -540,6 +550,11 @@ __global__ void __launch_bounds__(1024)
   for (int k = 0; k < 4; k++) {
     if (c0 + k < nc) off[c0 + k] = o;
     if (n[k] > 0) tlist[t++] = c0 + k;
+    if (bare.trg && n[k] == 0 && c0 + k < nc && bare.nchild[c0 + k] == 0) {
+      const int b = bare.body[c0 + k], nb = bare.nbody[c0 + k];
+      for (int i = 0; i < nb; i++) bare.trg[b + i] = make_double4(0, 0, 0, 0);
+      if (nb > 0) *bare.any = 1;
+    }
     o += n[k];
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
@@ -604,7 +619,8 @@ static void grow_keep(Handle &h, DBuf<T> &b, size_t want, size_t keep) {
 static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t np, DBuf<int> &tgt, DBuf<int> &src,
                             DBuf<unsigned char> &img, DBuf<int> &off, DBuf<int> &src_out, DBuf<unsigned char> &img_out,
                             DBuf<int> &tlist, int *ntl_host, const int **ntl_dev = nullptr,
-                            const int *skip = nullptr, int64_t nout = -1, int *next = nullptr) {
+                            const int *skip = nullptr, int64_t nout = -1, int *next = nullptr,
+                            const BareLeaves &bare = {}) {
   const int nc = h.ncells;
   if (np > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "list grouping: more than 2^31 - 1 entries");
   const int chunks = div_up(nc, kGroupChunk);
@@ -627,7 +643,7 @@ static void group_by_target(Handle &h, GroupScratch &g, hipStream_t st, int64_t 
     hipLaunchKernelGGL(k_group_count, dim3(div_up(np, 256)), dim3(256), 0, st, tgt.p, skip, np, g.cnt.p);
   if (chunks > 1) hipLaunchKernelGGL(k_group_totals, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot);
   hipLaunchKernelGGL(k_group_offsets, dim3(chunks), dim3(1024), 0, st, g.cnt.p, nc, tot, off.p, tlist.p, ntl, ntl_host,
-                     next);
+                     next, bare);
   if (np > 0) {
     int bits = 1;
     while (((int64_t)1 << bits) < np) bits++;
@@ -777,8 +793,10 @@ void run_lists(Handle &h) {
     group_by_target(h, h.grp1, h.stream, nm, mi, mj, mimg, h.m2l_off,
                     h.m2l_src, h.m2l_img, h.m2l_tgt, h.hpin + 8);
   h.p2p_next.reserve(1);
+  h.hpin[Handle::kPinBare] = 0;
   group_by_target(h, h.grp2, h.stream2, np, pi, pj, pimg, h.p2p_off,
-                  h.p2p_src, h.p2p_img, h.p2p_tgt, h.hpin + 9, &h.p2p_cnt_dev, nullptr, -1, h.p2p_next.p);
+                  h.p2p_src, h.p2p_img, h.p2p_tgt, h.hpin + 9, &h.p2p_cnt_dev, nullptr, -1, h.p2p_next.p,
+                  BareLeaves{h.cNChild.p, h.cBody.p, h.cNBody.p, h.trg4.p, h.hpin + Handle::kPinBare});
   h.p2p_next_clear = true;
   EXA_HIP(hipEventRecord(h.ev_p2pcnt, h.stream2));
   h.np2p_tgt = -1;
