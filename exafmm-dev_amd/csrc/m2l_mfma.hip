@@ -46,6 +46,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr double kLatUnit = 4;                   // u = w / kLatUnit
 constexpr int kLatD = 60;                         // |d_c| <= kLatD (in units of u)
+constexpr double kLatFar = (double)((int64_t)1 << 40);  // |centre| (in units of u), 2^12 below what FP64 resolves
 constexpr int kLatSide = 2 * kLatD + 1;
 constexpr int kLatKeys = kLatSide * kLatSide * kLatSide;
 
@@ -193,6 +194,9 @@ __device__ inline int lat_key(int t, int s, int im, const double4 *__restrict__ 
   // numbers to far better than the 1e-6 test below.
   const double iu = kLatUnit / (2 * rt);
   const double4 a = cX[t], b = cX[s];
+  // Centres far from the origin are rounded; where that is not far below a unit,
+  // cells of one level may have one centre and would share a slot.
+  if (!(fmax(fmax(fabs(a.x), fabs(a.y)), fabs(a.z)) * iu < kLatFar)) return -1;
   const double dx = (a.x - b.x) * iu, dy = (a.y - b.y) * iu, dz = (a.z - b.z) * iu;
   const double rx = rint(dx), ry = rint(dy), rz = rint(dz);
   if (!(fabs(dx - rx) < 1e-6 && fabs(dy - ry) < 1e-6 && fabs(dz - rz) < 1e-6)) return -1;
@@ -571,6 +575,10 @@ __global__ void k_tile_assign(int nc, TileLevels tl, const int *__restrict__ ske
       hi = mid;
   }
   const int r = p - lo, t = tl.base[g >> 3] + (r / 64) * 8 + (g & 7), col = r % 64;
+  if (r >= tl.cap[g >> 3]) {  // beyond the group's slots, as in k_tiles
+    tile_of[c] = -1;
+    return;
+  }
   tile_tgt[t * 64 + col] = c;
   tile_of[c] = t;
   col_of[c] = col;
