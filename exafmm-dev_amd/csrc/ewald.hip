@@ -518,8 +518,12 @@ static void wave_part(Handle &h, int K, double alpha, double sigma, double cycle
   const int4 *srows = reinterpret_cast<const int4 *>(h.ew_rows.p);
   const int2 *rows = reinterpret_cast<const int2 *>(srows + nsrows), *idx = rows + nrows;
   const int ny = div_up(nrows, 64), nz = div_up(K + 1, kNT), nrp = 64 * ny;
-  // About 1024 workgroups at most, so that the partials stay small.
-  const int per = kDftBodies * div_up(n, (int64_t)kDftBodies * std::max(1, 1024 / (ny * nz)));
+  // About 1024 workgroups at most, so that the partials stay small; few bodies
+  // and waves take one round of the stage per workgroup, to fill more CUs (wave
+  // part of 1728 bodies, ksize 2, 86 -> 69 us; from 64 workgroups on the partials
+  // cost what it gains).
+  const int least = (int64_t)ny * nz * div_up(n, kDftBodies) < 64 ? kDftBodies / 4 : kDftBodies;
+  const int per = least * div_up(n, (int64_t)least * std::max(1, 1024 / (ny * nz)));
   const int groups = div_up(n, per);
   const size_t npart = (size_t)groups * nz * 8 * kNT * nrp;
   h.ew_waves.resize(npart + (size_t)nsrows * (K + 1) * 4);
@@ -559,7 +563,10 @@ void run_ewald(Handle &h, int ksize, double alpha, double sigma, double cutoff, 
   // Slots: the row splits of the back transform (enough workgroups to fill
   // the chip), then the source splits of the real part.
   int nwave = 0, nreal = 0;
-  if ((parts & 1) && ksize > 0) nwave = std::min(16, std::max(1, div_up((int64_t)4096 * 64, n)));
+  if ((parts & 1) && ksize > 0) {
+    nwave = std::min(16, std::max(1, div_up((int64_t)4096 * 64, n)));
+    if (ksize < 4) nwave = std::min(nwave, ksize == 1 ? 3 : ksize == 2 ? 7 : 15);  // no more than rows
+  }
   if (parts & 2) {
     const int chunks = div_up(h.ncells, 64);
     nreal = std::max(1, std::min(chunks, std::min(64, 8192 / h.ncells)));
