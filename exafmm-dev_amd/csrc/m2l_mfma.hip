@@ -457,6 +457,12 @@ __device__ inline int face_class(uint64_t kk, int l) {
 // builders leave their number), and level l gets 8 ceil(parents / 64) slots
 // from base[l] on, chunk q of octant o at base[l] + 8 q + o (consecutive
 // tiles cover one region of space).  Slots without cells are skipped later.
+// Each costs its partial results (0.13 MB at P = 4, 0.46 at P = 10) and its row
+// of step flags all the same, and parents have half as many children on surfaces
+// as they could, a third with a body to a leaf: from kTilesUnread slots on the
+// host waits for the octants' counts (3.1 M bodies, ncrit = 1, P = 4: 63.4 ms and
+// 67 GB with the bound, 52.9 ms and 39 GB with the counts; 1 M: 15.0 and 14.5 ms).
+constexpr int kTilesUnread = 1 << 14;
 constexpr int kTileLevels = 32;  // deeper cells are in no tile (their pairs go per pair)
 struct TileLevels {
   int nlevels;
@@ -468,6 +474,22 @@ struct TileLevels {
 // What cKey adds to the Morton index of a level's cells.
 __device__ inline uint64_t level_offset(int l, bool key_lvloff) {
   return key_lvloff ? ((1ull << (3 * l)) - 1) / 7 : 0;
+}
+
+// Cells of each (level, octant), 8 l + o.
+__global__ void __launch_bounds__(256)
+    k_tile_octants(int nc, const int *__restrict__ lvl, const uint64_t *__restrict__ ckey, bool key_lvloff,
+                   int *__restrict__ cnt) {
+  __shared__ int s[8 * kTileLevels];
+  static_assert(8 * kTileLevels == 256, "one count a thread");
+  s[threadIdx.x] = 0;
+  __syncthreads();
+  for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256) {
+    const int l = lvl[c];
+    if (l < kTileLevels) atomicAdd(&s[8 * l + (int)((ckey[c] - level_offset(l, key_lvloff)) & 7)], 1);
+  }
+  __syncthreads();
+  if (s[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], s[threadIdx.x]);
 }
 
 // One workgroup per (octant, level): its cells in cell order, sorted by class
@@ -1080,14 +1102,30 @@ void run_lattice_tiles(Handle &h, hipStream_t st) {
   TileLevels tl{};
   int base = 0, most = 0;
   tl.nlevels = std::min(h.nlevels, kTileLevels - 1);
-  for (int l = 0; l <= kTileLevels; l++) {
-    tl.off[l] = h.lvl_off[std::min(l, h.nlevels)];
-    tl.base[l] = base;
-    if (l == 0 || l >= tl.nlevels) continue;
-    const int group = std::min(h.lvl_par[l - 1], h.lvl_off[l + 1] - h.lvl_off[l]);
-    tl.cap[l] = group;
-    most = std::max(most, group);
-    base += 8 * div_up(group, 64);
+  auto layout = [&](const int *octants) {
+    base = most = 0;
+    for (int l = 0; l <= kTileLevels; l++) {
+      tl.off[l] = h.lvl_off[std::min(l, h.nlevels)];
+      tl.base[l] = base;
+      if (l == 0 || l >= tl.nlevels) continue;
+      int group = std::min(h.lvl_par[l - 1], h.lvl_off[l + 1] - h.lvl_off[l]);
+      if (octants) group = std::min(group, *std::max_element(octants + 8 * l, octants + 8 * l + 8));
+      tl.cap[l] = group;
+      most = std::max(most, group);
+      base += 8 * div_up(group, 64);
+    }
+  };
+  layout(nullptr);
+  if (base > kTilesUnread) {
+    int octants[8 * kTileLevels];
+    h.lat_tcnt.resize(8 * kTileLevels);
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, st, h.lat_tcnt.p, (int64_t)(8 * kTileLevels), 0);
+    hipLaunchKernelGGL(k_tile_octants, dim3(std::min(1024, div_up(nc, 256))), dim3(256), 0, st, nc, h.cLevel.p,
+                       h.cKey.p, h.key_lvloff, h.lat_tcnt.p);
+    EXA_HIP(hipGetLastError());
+    EXA_HIP(hipMemcpyAsync(octants, h.lat_tcnt.p, sizeof(octants), hipMemcpyDeviceToHost, st));
+    EXA_HIP(hipStreamSynchronize(st));
+    layout(octants);
   }
   h.lat_ntiles = base;
   h.lat_tbase.assign(tl.base, tl.base + kTileLevels + 1);
