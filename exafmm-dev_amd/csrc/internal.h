@@ -143,10 +143,9 @@ struct Handle {
   DBuf<double4> body4;   // tree order
   DBuf<int> bidx;        // tree order -> caller index (Body::IBODY)
   DBuf<double4> trg4;    // tree order results (pot, gx, gy, gz)
-  DBuf<float4> trgf;     // scratch of the mixed-precision P2P
   double xmin[3] = {0, 0, 0}, xmax[3] = {0, 0, 0};
-  // Device copy: [0, 6) the bounds (xmin, xmax), [8, 12) the uniform box
-  // (x0, y0, z0, leaf cell size).  bounds_pending: xmin/xmax still wait for
+  // Device copy: [0, 6) the bounds (xmin, xmax), [8, 12) the adaptive tree's box
+  // (centre, R0).  bounds_pending: xmin/xmax still wait for
   // the copy behind ev_bounds (sync_bounds); bounds_dev_stale: the host
   // values were set by the caller and the device copy is out of date.
   DBuf<double> box;
@@ -170,7 +169,7 @@ struct Handle {
   DBuf<int> lvl_cells;             // cells sorted by level (stable)
 
   // Interaction lists (CSR by target cell).
-  int64_t np2p = 0, nm2l = 0, np2p_bodies = 0;
+  int64_t np2p = 0, nm2l = 0;
   DBuf<int> p2p_off, p2p_src, m2l_off, m2l_src;
   DBuf<unsigned char> p2p_img, m2l_img;
   DBuf<int> p2p_tgt, m2l_tgt;      // compact target lists
@@ -269,7 +268,7 @@ struct Handle {
   GroupScratch grp1, grp2;
   DBuf<unsigned char> tmp3;        // ... and of sorts on stream2
   DBuf<uint64_t> k64a, k64b;
-  DBuf<int> ia, ib, ic, id, ie, ifl;
+  DBuf<int> ia, ib, ic, id, ie;
   DBuf<int2> fa, fb;               // traversal frontiers (ci, cj | img << 27)
   // Device-driven traversal: its state, the frontier capacity and the level
   // count of the last traversal (0: run the per-level passes).
@@ -425,10 +424,9 @@ void launch_downward_cart_cells(Handle &h, const CellSetView &v);
 void launch_m2l_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L);
 void launch_m2l_cart_arrays(Handle &h, const M2LList &lst, const double4 *cX, const cplx *M, int nc, cplx *L);
 
-// Zero / copy device memory with a kernel (bytes a multiple of 8), so the
-// work can be recorded in a HIP graph (no memset or copy nodes).
+// Zero device memory with a kernel (bytes a multiple of 8), so the work can be
+// recorded in a HIP graph (no memset nodes).
 void zero_device(void *p, size_t bytes, hipStream_t st);
-void copy_device(void *d, const void *s, size_t bytes, hipStream_t st);
 
 // Scan / sort helpers (hipCUB) in util.hip.
 void exclusive_scan_int(Handle &h, const int *in, int *out, int n);

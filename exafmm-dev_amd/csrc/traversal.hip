@@ -693,7 +693,7 @@ static bool traverse_on_device(Handle &h, const CellView &cv, const int *roots, 
                          h.raw_mimg.p, h.raw_pi.p, h.raw_pj.p, h.raw_pimg.p);
     }
     enq += batch;
-    enqueue_multipoles(h);  // the second stream's work, while these levels run
+    enqueue_multipoles(h);  // the third stream's work, while these levels run
     EXA_HIP(hipGetLastError());
     EXA_HIP(hipStreamSynchronize(h.stream));
     if (hs.overflow) return false;

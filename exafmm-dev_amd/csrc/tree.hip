@@ -156,7 +156,6 @@ struct ForestSys {
   double x0, y0, z0;  // bounds minimum (the key origin)
   float d;            // leaf cell size, 2 R0 / 2^L
   int L;              // depth
-  int begin, end;     // body range
   int leaf0;          // first of its possible leaves
 };
 
@@ -639,7 +638,7 @@ static void build_uniform(Handle &h, const int *off, int S, bool own_bounds) {
   std::vector<ForestSys> fs(S);
   int64_t leaf0 = 0;
   for (int s = 0; s < S; s++) {
-    fs[s] = ForestSys{0, 0, 0, 0, L[s], off[s], off[s + 1], (int)leaf0};
+    fs[s] = ForestSys{0, 0, 0, 0, L[s], (int)leaf0};
     leaf0 += (int64_t)1 << (3 * L[s]);
   }
   if (leaf0 > INT_MAX) throw Error(EXAFMM_HIP_EUNSUP, "build_tree: too many leaves");

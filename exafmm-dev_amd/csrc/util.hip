@@ -19,7 +19,6 @@ Handle::~Handle() {
   body4.release();
   bidx.release();
   trg4.release();
-  trgf.release();
   cX.release();
   cRb.release();
   cParent.release();
@@ -55,7 +54,6 @@ Handle::~Handle() {
   ic.release();
   id.release();
   ie.release();
-  ifl.release();
   fa.release();
   fb.release();
   cnt.release();
@@ -77,15 +75,10 @@ Handle::~Handle() {
   if (stream3) (void)hipStreamDestroy(stream3);
 }
 
-// Zero / copy device memory by kernel (graph-capturable; bytes a multiple of 8).
+// Zero device memory by kernel (graph-capturable; bytes a multiple of 8).
 __global__ void k_zero_u64(unsigned long long *__restrict__ p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = 0;
-}
-
-__global__ void k_copy_u64(unsigned long long *__restrict__ d, const unsigned long long *__restrict__ s, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    d[i] = s[i];
 }
 
 void zero_device(void *p, size_t bytes, hipStream_t st) {
@@ -93,14 +86,6 @@ void zero_device(void *p, size_t bytes, hipStream_t st) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_zero_u64, dim3((int)std::min<int64_t>(div_up(n, 256), 8192)), dim3(256), 0, st,
                      (unsigned long long *)p, n);
-  EXA_HIP(hipGetLastError());
-}
-
-void copy_device(void *d, const void *s, size_t bytes, hipStream_t st) {
-  const int64_t n = (int64_t)(bytes / 8);
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_copy_u64, dim3((int)std::min<int64_t>(div_up(n, 256), 8192)), dim3(256), 0, st,
-                     (unsigned long long *)d, (const unsigned long long *)s, n);
   EXA_HIP(hipGetLastError());
 }
 
