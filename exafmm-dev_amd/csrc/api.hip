@@ -80,6 +80,7 @@ static void do_build(Handle &h) {
   else
     run_build_adaptive(h);
   h.key_lvloff = h.nsys == 1 && h.cfg.builder == 1;
+  h.tree_given = h.bounds_given && h.nsys == 1;
   h.have_tree = true;
   h.have_up = h.have_trav = false;
   h.lat_ms_ready = h.lat_tiles_ready = false;  // of an older tree
@@ -316,6 +317,7 @@ static void evaluate_all(Handle &h) {
       EXA_HIP(hipEventRecord(h.ev[1], h.stream));
       drop_multipoles(h);
       run_build_forest(h);
+      h.tree_given = false;
       h.have_tree = true;
       h.have_up = h.have_trav = false;
     } else {

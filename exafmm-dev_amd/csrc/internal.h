@@ -151,6 +151,7 @@ struct Handle {
   DBuf<double> box;
   bool bounds_pending = false, bounds_dev_stale = false;
   bool bounds_given = false;  // by the caller: they may not enclose every body
+  bool tree_given = false;    // the tree was built from such bounds
   bool have_bounds = false, have_tree = false, have_up = false, have_trav = false;
   // Before a build writes to the tree: one that fails from there on leaves none.
   void drop_tree() { have_tree = have_up = have_trav = false; }

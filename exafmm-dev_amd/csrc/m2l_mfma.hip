@@ -1226,11 +1226,11 @@ static void lattice_steps(Handle &h) {
     hipLaunchKernelGGL(k_lat_steps, dim3(h.lat_ntiles), dim3(256), 0, h.stream, act, h.lat_tcnt.p, h.lat_noff, lr,
                        used, h.lat_orow.p, h.lat_aidx.p, h.lat_step0.p, h.lat_alist.p,
                        reinterpret_cast<int4 *>(h.lat_slot.p), lat_state(h), host);
-    if (!h.bounds_given) EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
-    hipLaunchKernelGGL(h.bounds_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
+    if (!h.tree_given) EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
+    hipLaunchKernelGGL(h.tree_given ? k_lat_slots<true> : k_lat_slots<false>, dim3(gp), dim3(TPB), 0, h.stream, ptgt,
                        psrc, np, h.lat_col_of.p, h.lat_aidx.p, h.lat_pslot.p, h.lat_slot.p, lat_state(h));
   }
-  if (nall == 0 || h.bounds_given) {  // (k_lat_slots may add irregular pairs)
+  if (nall == 0 || h.tree_given) {  // (k_lat_slots may add irregular pairs)
     EXA_HIP(hipMemcpyAsync(host, lat_state(h), sizeof(LatState), hipMemcpyDeviceToHost, h.stream));
     EXA_HIP(hipEventRecord(h.ev_cnt, h.stream));
   }

@@ -33,3 +33,23 @@ def test_rounded_centres(edge, builder, far, monkeypatch):
         res.append(f.results())
         f.close()
     assert rel_l2(res[0], res[1]) < 1e-12
+
+
+@pytest.mark.parametrize("lo,hi", [(-0.2, 0.3), (-1.5, 1.2)])
+def test_bounds_asked_for_after_the_build(lo, hi):
+    """The tree keeps the bounds it was built from, whatever get_bounds computes before its lists are made."""
+    x = np.random.default_rng(5).uniform(-1, 1, (3000, 4))
+    res = []
+    for ask in (False, True):
+        f = X.FMM(P=6, ncrit=16)
+        f.set_bodies(x)
+        f.build_tree((np.full(3, lo), np.full(3, hi)))
+        f.upward_pass()
+        print(f"[gpu] bounds {lo} to {hi} from the caller, asked for again: {ask}", flush=True)
+        if ask:
+            f.get_bounds()
+        f.traverse()
+        f.downward_pass()
+        res.append(f.results())
+        f.close()
+    assert rel_l2(res[1], res[0]) < 1e-12
