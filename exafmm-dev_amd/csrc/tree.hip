@@ -143,13 +143,13 @@ void upload_bounds(Handle &h) {
 //   up to kCountMost bodies by counting, in 9 to 12 launches: bodies per leaf
 //   (atomic counts), a prefix sum for the leaves' first bodies, bodies scattered
 //   into their leaves in any order, and each body's rank among its leaf's.
-//   2000 bodies 30 us (75 by sorts per level), 100k 47 (118), 262144 68 (147).
+//   2000 bodies 30 us (75 by sorts per level), 100k 46 (124), 400k 81 (165).
 //   With a leaf beyond kLeafRank bodies the sort follows, and it comes at once in
 //   the handle's next build.
-//   beyond, by a stable sort of (leaf, body), the starts found by bisection:
-//   1 M bodies 147 us, 4 M 330, however clustered (by counting 156 and 468, and
-//   4 M clustered bodies 900 us and more: the atomic counts of few leaves follow
-//   each other).
+//   beyond, by a stable sort of (leaf, body), the starts found by bisection: 400k
+//   bodies 130 us, 1 M 150, 4 M 330, however clustered (1 M and 4 M by counting 147
+//   and 468, and 4 M clustered bodies 900 us and more: the atomic counts of few
+//   leaves follow each other).
 constexpr int kMaxUniformLevels = 10;  // the reference's int keys hold 3 x 10 bits
 
 struct ForestSys {
@@ -604,7 +604,7 @@ static int uniform_depth(int n, int ncrit) {
 
 // Bodies up to which the leaves are counted (see above); leaves from which a
 // thread finds the starts of several.
-constexpr int kCountMost = 1 << 18, kStartsMany = 1 << 21;
+constexpr int kCountMost = 1 << 20, kStartsMany = 1 << 21;
 
 // The trees of the systems [off[s], off[s + 1]): with given bounds (one
 // system), or each with its own.

@@ -1,7 +1,7 @@
 """The uniform tree where its build is sized by what is possible: trees of more
 than 2^26 possible leaves (depth 9, a workgroup for each would be more than a
 launch takes) and of more than 2^21 possible cells, and leaves of more than 1024
-bodies or trees of more than 2^18, whose order comes from a sort.  Against the same tree made here from the
+bodies or trees of more than 2^20, whose order comes from a sort.  Against the same tree made here from the
 bodies' Morton keys: body order, cells per level, their keys and body ranges,
 all to the bit."""
 import ctypes
@@ -93,7 +93,7 @@ def test_large_leaves():
         print(f"[gpu] uniform build, {m} of {n} in one leaf", flush=True)
         check_tree(f, corner(n, m, n + m), 64)
     f.close()
-    for n in (1024, 1025, 1 << 18, (1 << 18) + 1):
+    for n in (1024, 1025, 1 << 20, (1 << 20) + 1):
         f = X.FMM(P=4, ncrit=1200)
         check_tree(f, unit_cube(n, n), 1200)
         check_tree(f, unit_cube(n, n + 1), 1200)
