@@ -28,14 +28,22 @@ __global__ void k_mass_normalise(cplx *__restrict__ M, int ncells, int nt) {
   }
 }
 
+__global__ void k_monopoles(const cplx *__restrict__ M, int ncells, int nt, double *__restrict__ m0) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < ncells) m0[c] = M[(size_t)c * nt].re;
+}
+
 void run_ropt(Handle &h) {
   if (!h.cfg.useRopt) return;
   const int nc = h.ncells, nt = h.nterm, P = h.cfg.P;
   const double theta = h.cfg.theta;
   std::vector<double> m0(nc);
   std::vector<double4> X(nc);
-  EXA_HIP(hipMemcpy2DAsync(m0.data(), sizeof(double), h.M.p, nt * sizeof(cplx), sizeof(double), nc,
-                           hipMemcpyDeviceToHost, h.stream));
+  // (Gathered first: a strided copy to the host goes row by row, 35 ms for 4681
+  // cells.)
+  h.red.reserve(nc);
+  hipLaunchKernelGGL(k_monopoles, dim3(div_up(nc, 256)), dim3(256), 0, h.stream, h.M.p, nc, nt, h.red.p);
+  EXA_HIP(hipMemcpyAsync(m0.data(), h.red.p, nc * sizeof(double), hipMemcpyDeviceToHost, h.stream));
   EXA_HIP(hipMemcpyAsync(X.data(), h.cX.p, nc * sizeof(double4), hipMemcpyDeviceToHost, h.stream));
   EXA_HIP(hipStreamSynchronize(h.stream));
   const double c0 = (1 - theta) * (1 - theta) / std::pow(theta, P + 2) / powf((float)std::fabs(m0[0]), (float)(1.0 / 3));
