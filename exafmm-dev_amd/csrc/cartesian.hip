@@ -16,7 +16,7 @@
 //
 // The upward pass follows the reference's operation order without FMA
 // contraction (multipoles bit-identical to the reference).  M2L takes one
-// wave per target cell and one lane per pair with everything in registers.
+// wave per target cell and one lane per pair, in registers.
 #include <algorithm>
 #include <utility>
 
@@ -360,11 +360,13 @@ __global__ void __launch_bounds__(64)
 // M2L over the CSR interaction list: one wave per target cell and one lane per
 // pair, the pair's derivative tensor and the target's sums in registers, every
 // index fixed at compile time; the lanes' sums are added in lane order through
-// LDS at the end.  FP64 issue bounds it: at P = 6 a pair is 462 multiply-adds
-// and about 400 operations of the recurrence, and 448 bytes of its source's
-// multipole; 2 x 56 doubles leave two waves per SIMD.  1.41 M pairs over 4680
-// targets at P = 6: 315 us; 2180 us with a batch of tensors in LDS and a term
-// list per lane (62 KB for one wave left two waves per CU).
+// LDS at the end.  At P = 6 a pair is 462 multiply-adds and about 400 operations
+// of the recurrence, and 448 bytes of its source's multipole; 2 x 56 doubles
+// leave two waves per SIMD, with 26 registers spilled, so latency bounds it: the
+// VALU issues 36% of the time, loads hit the L2 to 98%.  1.41 M pairs over 4680
+// targets at P = 6: 105 us alone and 302 beside P2P, which takes 283 alone; 2180
+// us beside P2P with a batch of tensors in LDS and a term list per lane (62 KB for
+// one wave left two waves per CU).
 // At P = 8 the 2 x 120 doubles do not fit 512 registers, so two kernels each
 // make the tensor and sum a part of the outputs, those up to degree 4 (35
 // outputs, 1358 of the 1716 terms) and the others: a cube of 100k bodies
